@@ -333,6 +333,58 @@ def test_prefill_rows_of_any_length_and_alignment(L, offset):
     assert bool(torch.isnan(guard).all()), "elements outside the output tensor were written"
 
 
+TILES = [  # D, L, block_len, dtype, a_dtype, log_a, offset: edges of the 16-row x 64-step tiles, their granules and halos
+    (16, 64, 16, torch.float32, None, False, 0),           # one whole tile, 16-byte granules
+    (16, 260, 16, torch.float32, None, False, 0),          # 17 blocks: workgroup edge, partial last block
+    (16, 1000, 16, torch.float32, None, True, 0),          # several workgroups per row
+    (16, 77, 16, torch.float32, None, False, 1),           # rows off the 16-byte grid
+    (48, 200, 32, torch.bfloat16, None, False, 0),
+    (16, 203, 32, torch.float16, None, False, 0),          # 16-bit rows start on either half of a word
+    (16, 203, 33, torch.bfloat16, None, False, 1),         # 16-bit rows on 2-byte boundaries
+    (5, 97, 5, torch.bfloat16, torch.float32, False, 0),   # several blocks per lane, channel rows of two gate rows per tile
+    (1, 65, 1, torch.float32, None, False, 0),
+    (24, 131, 24, torch.float32, None, False, 2),
+    (16, 129, 65, torch.bfloat16, None, False, 0),         # blocks longer than a tile of 64 steps
+    (16, 600, 256, torch.float32, None, False, 0),         # the longest block of a tile
+    (16, 600, 257, torch.float32, None, False, 0),         # and the first that is not
+]
+
+
+@pytest.mark.parametrize("D,L,bl,dtype,a_dtype,log_a,offset", TILES)
+def test_prefill_tiles_of_any_type_block_length_and_head_size(D, L, bl, dtype, a_dtype, log_a, offset):
+    """Output, state and sequential form with a carry against the oracle; the elements around the output stay untouched."""
+    from spear_amd import _btp
+
+    B, H = 2, 3
+    A, X, C, V = make(B, H, D, L, seed=L + bl, dtype=dtype, a_dtype=a_dtype, log_a=log_a)
+    carry = torch.randn(B, H, D, generator=torch.Generator().manual_seed(bl))
+
+    def shifted(t):
+        buf = torch.full((t.numel() + 16,), float("nan"), dtype=t.dtype, device=DEV)
+        view = buf[offset:offset + t.numel()].view(t.shape)
+        view.copy_(t)
+        return buf, view
+
+    (_, a), (_, x), (_, c), (_, v) = (shifted(t) for t in (A, X, C, V))
+    ybuf, y = shifted(torch.full(X.shape, float("nan"), dtype=X.dtype))
+    h, cp = (torch.full((B, H, D), float("nan"), device=DEV) for _ in range(2))
+    r = torch.full((B, H), float("nan"), device=DEV)
+    print(f"tiles D={D} L={L} bl={bl} {dtype} offset={offset}", flush=True)
+    _btp.jagged_prefill(a, x, c, v, None, y, h, r, cp, bl, log_a)
+    torch.cuda.synchronize()
+    rY, rst = jag.prefill(f64(A), f64(X), f64(C), f64(V), block_len=bl, use_log_a=log_a)
+    assert_close(f64(y), rY, *tol(dtype), "Y")
+    for name, got, want in (("h", h, rst.h_loc), ("c_prev", cp, rst.c_prev_loc), ("r", r, rst.r_pref)):
+        assert_close(f64(got), want, F32_ATOL, F32_RTOL, name)
+    guard = torch.cat([ybuf[:offset], ybuf[offset + X.numel():]])
+    assert bool(torch.isnan(guard).all()), "elements outside the output tensor were written"
+
+    _btp.jagged_prefill(a, x, None, None, carry.to(DEV), y, None, None, None, bl, log_a)
+    torch.cuda.synchronize()
+    want = jag.sequential(f64(X), f64(A), bl, use_log_a=log_a, carry_init=f64(carry))
+    assert_close(f64(y), want, *tol(dtype), "sequential form")
+
+
 @pytest.mark.parametrize("case", ["full", "ragged", "short", "one_block", "bl4"])
 def test_kernels_match_the_reference_vectors(case):
     """The HIP prefill and decode kernels against vectors computed by the reference's own
