@@ -23,7 +23,7 @@
  *     y           [B, H, 16, L]      out_dtype  (in_dtype or fp32)
  *     dy          [B, H, 16, L]      dy_dtype   (in_dtype or fp32)
  *     checkpoint  [B, H, L/16, 16]   fp32       slot i-1 = local terminal state of block i-1
- *     dA          [B, H, L]          fp32       every element is written (no accumulation)
+ *     dA          [B, H, L]          fp32       every element is written (no accumulation); in_dtype with SPEAR_BTP_DA_16
  *
  * Requirements: L is a positive multiple of 16; every pointer is 16-byte aligned; k is 1 or 2.
  * Calls are asynchronous on `stream` (a hipStream_t passed as void*, NULL = default stream),
@@ -57,6 +57,9 @@ extern "C" {
 
 #define SPEAR_BTP_DX_F32 0x10u          /* backward: check mode, `dx` is fp32 [B, H, 16, L] and receives the    */
                                         /* kernel's fp32 values instead of their rounding to in_dtype           */
+#define SPEAR_BTP_DA_16 0x20u           /* backward: `dA` is in in_dtype, the fp32 values rounded to nearest even by   */
+                                        /* the kernel (what autograd does to the gradient of a 16-bit coefficient, with   */
+                                        /* one launch and 6 bytes per step less). Not with SPEAR_BTP_PATH_MFMA            */
 
 /* error codes */
 #define SPEAR_BTP_EINVAL (-1)  /* bad shape, dtype, k, flag or alignment                       */
@@ -75,7 +78,7 @@ int spear_btp_forward(const void* coeff, const void* x, void* y, float* checkpoi
  * (_bindings.cu:52-54), which stays the default; SPEAR_BTP_DX_F32 is the fp32 check mode (arithmetic is fp32
  * either way, the flag only drops the final rounding so that dx can be compared at fp32 tolerances). */
 int spear_btp_backward(const void* coeff, const void* x, const void* dy, const float* checkpoint,
-                       void* dx, float* dA, int B, int H, int L, int k, int in_dtype, int dy_dtype,
+                       void* dx, void* dA, int B, int H, int L, int k, int in_dtype, int dy_dtype,
                        unsigned flags, void* stream);
 
 /* Log-space gate variants. They have no counterpart function in the reference, whose op takes

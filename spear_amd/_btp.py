@@ -20,7 +20,7 @@ import threading
 
 import torch
 
-__all__ = ["forward", "backward", "forward_log", "backward_log", "mix_forward", "mix_backward", "jagged_prefill", "jagged_step", "library_path", "load_library", "load_extension", "FLAG_WRITE_CHECKPOINT", "FLAG_PATH_MFMA", "FLAG_JAGGED_LOG_A", "FLAG_JAGGED_LOG_R", "FLAG_MIX_QKV_GATE", "FLAG_MIX_F32_RESULTS", "FLAG_DX_F32", "mix_backward_sum_rows", "mix_backward_bias", "mix_step"]
+__all__ = ["forward", "backward", "forward_log", "backward_log", "mix_forward", "mix_backward", "jagged_prefill", "jagged_step", "library_path", "load_library", "load_extension", "FLAG_WRITE_CHECKPOINT", "FLAG_PATH_MFMA", "FLAG_JAGGED_LOG_A", "FLAG_JAGGED_LOG_R", "FLAG_MIX_QKV_GATE", "FLAG_MIX_F32_RESULTS", "FLAG_DX_F32", "FLAG_DA_16", "mix_backward_sum_rows", "mix_backward_bias", "mix_step"]
 
 _BF16, _F16, _F32 = 0, 1, 2
 FLAG_WRITE_CHECKPOINT = 0x1
@@ -30,6 +30,7 @@ FLAG_JAGGED_LOG_R = 0x8
 FLAG_MIX_QKV_GATE = 0x1
 FLAG_MIX_F32_RESULTS = 0x2
 FLAG_DX_F32 = 0x10
+FLAG_DA_16 = 0x20
 _ABI_VERSION = 18
 _SUPPORTED_WPB = (4, 8, 16, 32)
 
@@ -243,7 +244,8 @@ def backward(
 
     Every element of ``dA`` is written, so it need not arrive zero-filled. ``checkpoint`` is
     accepted for signature compatibility and not read. ``flags`` is an extension: with ``FLAG_DX_F32``
-    ``dx`` is a float32 tensor and receives the kernel's fp32 values unrounded (fp32 check mode).
+    ``dx`` is a float32 tensor and receives the kernel's fp32 values unrounded (fp32 check mode), with
+    ``FLAG_DA_16`` ``dA`` is a tensor of ``coeff``'s dtype and receives the rounded values.
     """
     _check(
         coeff.is_cuda and x.is_cuda and dy.is_cuda and checkpoint.is_cuda,
@@ -255,7 +257,10 @@ def backward(
         _check(dx.dtype == torch.float32, "dx must be float32 in the fp32 check mode.")
     else:
         _check(dx.dtype == x.dtype, "dx dtype must match x.")
-    _check(dA.dtype == torch.float32, "dA must be float32.")
+    if flags & FLAG_DA_16:
+        _check(dA.dtype == coeff.dtype, "dA must match coeff dtype.")
+    else:
+        _check(dA.dtype == torch.float32, "dA must be float32.")
     _check(dy.dtype == torch.float32 or dy.dtype == x.dtype, "dy must be float32 or match x dtype.")
     B, H, _, L = x.shape
     _check(L % 16 == 0, "Length L must be multiple of 16")

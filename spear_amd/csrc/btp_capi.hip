@@ -90,12 +90,12 @@ int spear_btp_forward(const void* coeff, const void* x, void* y, float* checkpoi
   return 0;
 }
 
-int spear_btp_backward(const void* coeff, const void* x, const void* dy, const float* checkpoint, void* dx, float* dA,
+int spear_btp_backward(const void* coeff, const void* x, const void* dy, const float* checkpoint, void* dx, void* dA,
                        int B, int H, int L, int k, int in_dtype, int dy_dtype, unsigned flags, void* stream) {
   (void)checkpoint;  // carries are recomputed from coeff and x
   g_error[0] = '\0';
   if (int rc = check_common("spear_btp_backward", B, H, L, k, in_dtype, dy_dtype, "dy", flags,
-                            SPEAR_BTP_PATH_MFMA | SPEAR_BTP_DX_F32))
+                            SPEAR_BTP_PATH_MFMA | SPEAR_BTP_DX_F32 | SPEAR_BTP_DA_16))
     return rc;
   if ((long long)B * H == 0 || L == 0) return 0;
   if (!coeff || !x || !dy || !dx || !dA) return fail(SPEAR_BTP_ENULL, "spear_btp_backward: NULL tensor pointer");
@@ -104,13 +104,16 @@ int spear_btp_backward(const void* coeff, const void* x, const void* dy, const f
   const bool mfma = (flags & SPEAR_BTP_PATH_MFMA) != 0;
   if (mfma && (flags & SPEAR_BTP_DX_F32))
     return fail(SPEAR_BTP_EINVAL, "spear_btp_backward: the MFMA path has no fp32 dx (SPEAR_BTP_DX_F32)");
+  if (mfma && (flags & SPEAR_BTP_DA_16))
+    return fail(SPEAR_BTP_EINVAL, "spear_btp_backward: the MFMA path stores dA as fp32 only (SPEAR_BTP_DA_16)");
   if (mfma && dy_dtype == SPEAR_BTP_F32)
     return fail(SPEAR_BTP_EINVAL,
                 "spear_btp_backward: the MFMA path takes dy in the inputs' 16-bit type (the matrix instruction's operand "
                 "width) and does not round a float32 dy silently; use the default path, or give the forward an output "
                 "in the inputs' dtype so that dy arrives in it");
 
-  spear_btp::BwdArgs a{coeff, x, dy, dx, dA, B, H, L, k, in_dtype, dy_dtype, false, (flags & SPEAR_BTP_DX_F32) != 0};
+  spear_btp::BwdArgs a{coeff, x, dy, dx, dA, B, H, L, k, in_dtype, dy_dtype, false, (flags & SPEAR_BTP_DX_F32) != 0,
+                       (flags & SPEAR_BTP_DA_16) != 0};
   const hipStream_t hs = static_cast<hipStream_t>(stream);
   const hipError_t err = mfma ? spear_btp::mfma_backward(a, hs) : spear_btp::scan_backward(a, hs);
   if (err != hipSuccess) return fail(SPEAR_BTP_ELAUNCH, "spear_btp_backward: launch failed: %s", hipGetErrorString(err));

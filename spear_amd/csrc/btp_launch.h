@@ -25,11 +25,12 @@ struct BwdArgs {
   const void* x;
   const void* dy;
   void* dx;
-  float* dA;  // d/d coeff, or d/d gate when log_gate is set
+  void* dA;  // d/d coeff, or d/d gate when log_gate is set: fp32, or in_dtype with da_16
   int B, H, L, k;
   int in_dtype, dy_dtype;
   bool log_gate = false;
   bool dx_f32 = false;  // check mode: dx is fp32 [B, H, 16, L] (the kernel's fp32 values, not rounded to in_dtype)
+  bool da_16 = false;   // dA is stored in in_dtype (linear-space coefficients only)
 };
 
 // Exact-fp32 recurrence kernels (btp_scan.hip).

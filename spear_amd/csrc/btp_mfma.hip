@@ -492,7 +492,7 @@ hipError_t mfma_backward(const BwdArgs& p, hipStream_t s) {
     const auto* x = static_cast<const uint16_t*>(p.x);
     auto* dx = static_cast<uint16_t*>(p.dx);
     hipLaunchKernelGGL((btp_bwd_mfma_kernel<E, kIn>), dim3(g.blocks), dim3(64 * kWaves), 0, s, c, x,
-                       static_cast<const uint16_t*>(p.dy), dx, p.dA, p.L, g.spans_per_row, g.total_spans, p.k);
+                       static_cast<const uint16_t*>(p.dy), dx, static_cast<float*>(p.dA), p.L, g.spans_per_row, g.total_spans, p.k);
   };
   const bool st = stream_inputs(g);
   if (p.in_dtype == kBf16) {

@@ -287,8 +287,8 @@ template <class E, class C, class GradT, class DxT, bool kStreamIn, int kW, bool
 __device__ __forceinline__ void btp_bwd_scan_body(
     unsigned char (*lds)[4096 + (std::is_same<GradT, float>::value ? 8192 : 4096) + kCoeffLdsBytes],
     const typename C::elem* __restrict__ coeff, const uint16_t* __restrict__ x, const GradT* __restrict__ dy,
-    DxT* __restrict__ dx, float* __restrict__ dA, int L, int spans_per_row, long total_spans,
-    int k) {
+    DxT* __restrict__ dx, void* __restrict__ dA, int L, int spans_per_row, long total_spans,
+    int k, int da16) {
   constexpr bool kGradF32 = std::is_same<GradT, float>::value;
   constexpr bool kDxF32 = std::is_same<DxT, float>::value;  // check mode: dx leaves unrounded
   constexpr int kGradBytes = kGradF32 ? 8192 : 4096;
@@ -530,9 +530,19 @@ __device__ __forceinline__ void btp_bwd_scan_body(
     dA_B *= a_lds[coeff_slot(32 * j) + 16 + d];
   }
   SPEAR_BTP_PRIO(3);
-  float* dArow = dA + sc.row * (long)L + sc.s0 + 32 * j + d;
-  if (32 * j < sc.nvalid) __builtin_nontemporal_store(dA_A, dArow);
-  if (32 * j + 16 < sc.nvalid) __builtin_nontemporal_store(dA_B, dArow + 16);
+  const long dA_at = sc.row * (long)L + sc.s0 + 32 * j + d;
+  if (da16) {
+    // rounded to the coefficients' type here rather than by whoever consumes the gradient: even lanes store their
+    // step and the next one as a word
+    const uint32_t wA = E::pack2(dA_A, row_xor<1>(dA_A)), wB = E::pack2(dA_B, row_xor<1>(dA_B));
+    uint32_t* words = reinterpret_cast<uint32_t*>(static_cast<uint16_t*>(dA) + dA_at);
+    if (32 * j < sc.nvalid && !(d & 1)) __builtin_nontemporal_store(wA, words);
+    if (32 * j + 16 < sc.nvalid && !(d & 1)) __builtin_nontemporal_store(wB, words + 8);
+  } else {
+    float* dArow = static_cast<float*>(dA) + dA_at;
+    if (32 * j < sc.nvalid) __builtin_nontemporal_store(dA_A, dArow);
+    if (32 * j + 16 < sc.nvalid) __builtin_nontemporal_store(dA_B, dArow + 16);
+  }
 
   if constexpr (kDxF32) {
     // fp32 dx: an 8 KiB image (512 B per channel row) laid over the x and dy images, both dead by now
@@ -568,10 +578,10 @@ __device__ __forceinline__ void btp_bwd_scan_body(
 template <class E, class C, bool kStreamIn, int kW = bwd_waves<true, kStreamIn>(), bool kLines = false, bool kFlat = false>
 __global__ __launch_bounds__((64 * kW)) SPEAR_BTP_BWD_OCC void btp_bwd_scan_kernel(
     const typename C::elem* __restrict__ coeff, const uint16_t* __restrict__ x, const uint16_t* __restrict__ dy,
-    uint16_t* __restrict__ dx, float* __restrict__ dA, int L, int spans_per_row, long total_spans, int k) {
+    uint16_t* __restrict__ dx, void* __restrict__ dA, int L, int spans_per_row, long total_spans, int k, int da16) {
   __shared__ __align__(16) unsigned char lds[kW][4096 + 4096 + kCoeffLdsBytes];
   btp_bwd_scan_body<E, C, uint16_t, uint16_t, kStreamIn, kW, kLines, kFlat>(lds, coeff, x, dy, dx, dA, L, spans_per_row,
-                                                                        total_spans, k);
+                                                                        total_spans, k, da16);
 }
 
 // fp32 dy (twice the staging registers and LDS), log-space gates (an exponential per coefficient)
@@ -579,12 +589,12 @@ __global__ __launch_bounds__((64 * kW)) SPEAR_BTP_BWD_OCC void btp_bwd_scan_kern
 template <class E, class C, class GradT, class DxT, bool kStreamIn, bool kLines = false, bool kFlat = false>
 __global__ __launch_bounds__((64 * bwd_waves<false, kStreamIn>())) void btp_bwd_scan_kernel_relaxed(
     const typename C::elem* __restrict__ coeff, const uint16_t* __restrict__ x, const GradT* __restrict__ dy,
-    DxT* __restrict__ dx, float* __restrict__ dA, int L, int spans_per_row, long total_spans, int k) {
+    DxT* __restrict__ dx, void* __restrict__ dA, int L, int spans_per_row, long total_spans, int k, int da16) {
   constexpr int kGradBytes = std::is_same<GradT, float>::value ? 8192 : 4096;
   constexpr int kW = bwd_waves<false, kStreamIn>();
   __shared__ __align__(16) unsigned char lds[kW][4096 + kGradBytes + kCoeffLdsBytes];
   btp_bwd_scan_body<E, C, GradT, DxT, kStreamIn, kW, kLines, kFlat>(lds, coeff, x, dy, dx, dA, L, spans_per_row,
-                                                                    total_spans, k);
+                                                                    total_spans, k, da16);
 }
 
 template <class E, class C, class OutT, bool kCheckpoint, bool kStreamIn, bool kLines = false, bool kFlat = false>
@@ -632,7 +642,7 @@ void launch_bwd_as(const BwdArgs& p, const Grid& g, hipStream_t s) {
   const auto* dy = static_cast<const GradT*>(p.dy);
   auto go = [&](auto kernel, auto* dx) {
     hipLaunchKernelGGL(kernel, dim3(g.blocks), dim3(64 * g.waves), 0, s, c, x, dy, dx, p.dA, p.L, g.spans_per_row,
-                       g.total_spans, p.k);
+                       g.total_spans, p.k, p.da_16 ? 1 : 0);
   };
   auto* dx16 = static_cast<uint16_t*>(p.dx);
   if (p.dx_f32) {  // fp32 check mode

@@ -98,7 +98,11 @@ void backward(const at::Tensor& coeff, const at::Tensor& x, const at::Tensor& dy
   } else {
     TORCH_CHECK(dx.scalar_type() == x.scalar_type(), "dx dtype must match x.");
   }
-  TORCH_CHECK(dA.scalar_type() == at::kFloat, "dA must be float32.");
+  if (flags & SPEAR_BTP_DA_16) {
+    TORCH_CHECK(dA.scalar_type() == coeff.scalar_type(), "dA must match coeff dtype.");
+  } else {
+    TORCH_CHECK(dA.scalar_type() == at::kFloat, "dA must be float32.");
+  }
   TORCH_CHECK(dy.scalar_type() == at::kFloat || dy.scalar_type() == x.scalar_type(), "dy must be float32 or match x dtype.");
   const int64_t B = x.size(0), H = x.size(1), L = x.size(3);
   TORCH_CHECK(L % 16 == 0, "Length L must be multiple of 16");
@@ -111,7 +115,7 @@ void backward(const at::Tensor& coeff, const at::Tensor& x, const at::Tensor& dy
   const c10::DeviceGuard guard(x.device());
   const int rc = spear_btp_backward(coeff.data_ptr(), x.data_ptr(), dy.data_ptr(),
                                     checkpoint.numel() ? static_cast<const float*>(checkpoint.data_ptr()) : nullptr,
-                                    dx.data_ptr(), static_cast<float*>(dA.data_ptr()), (int)B, (int)H, (int)L, (int)k,
+                                    dx.data_ptr(), dA.data_ptr(), (int)B, (int)H, (int)L, (int)k,
                                     tag_of(x.scalar_type()), tag_of(dy.scalar_type()), (unsigned)flags, stream_of(x));
   if (rc != 0) raise_native(rc);
 }
@@ -194,9 +198,12 @@ struct BtpNode : public torch::autograd::Function<BtpNode> {
     const at::Tensor &coeff = saved[0], &x = saved[1], &checkpoint = saved[2];
     const at::Tensor dy = grad_outputs[0].contiguous();
     at::Tensor dx = at::empty(x.sizes(), x.options());
-    at::Tensor dA = at::empty(coeff.sizes(), coeff.options().dtype(at::kFloat));
-    ::backward(coeff, x, dy, checkpoint, dx, dA, ctx->saved_data["k"].toInt(), ctx->saved_data["wpb"].toInt(),
-               ctx->saved_data["flags"].toInt());
+    // The engine hands the gradient on in coeff's dtype; the kernel can round it there itself (the matrix-core path
+    // stores fp32 and leaves the rounding to the engine).
+    int64_t flags = ctx->saved_data["flags"].toInt();
+    if (!(flags & SPEAR_BTP_PATH_MFMA)) flags |= SPEAR_BTP_DA_16;
+    at::Tensor dA = at::empty(coeff.sizes(), (flags & SPEAR_BTP_DA_16) ? coeff.options() : coeff.options().dtype(at::kFloat));
+    ::backward(coeff, x, dy, checkpoint, dx, dA, ctx->saved_data["k"].toInt(), ctx->saved_data["wpb"].toInt(), flags);
     return {dA, dx, at::Tensor(), at::Tensor(), at::Tensor(), at::Tensor(), at::Tensor()};
   }
 };

@@ -624,3 +624,27 @@ def test_concurrent_callers_on_their_own_streams():
     assert not errors, errors
     for (y, dx, dA), (y0, (dx0, dA0)) in zip(results, alone):
         assert torch.equal(y, y0) and torch.equal(dx, dx0) and torch.equal(dA, dA0)
+
+
+@pytest.mark.parametrize("dy_f32", [False, True], ids=["dy16", "dy32"])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "f16"])
+@pytest.mark.parametrize("L", [16, 48, 112, 128, 144, 192, 272, 1168])
+def test_backward_stores_the_coefficient_gradient_rounded(L, dtype, dy_f32):
+    """FLAG_DA_16: every instance's dA in the coefficients' type is the rounding of its fp32 dA, dx is the same, and
+    nothing beside the tensor is written."""
+    from spear_amd import _btp
+
+    B, H = 2, 3
+    coeff, x, dy = (t.to(dtype).to(DEV) for t in make_inputs(B, H, L, seed=4100 + L))
+    dy = dy.float() if dy_f32 else dy
+    ck = torch.empty(0, device=DEV)
+    dx32, dx16 = torch.empty_like(x), torch.empty_like(x)
+    dA32 = torch.empty(B, H, L, device=DEV)
+    buf = torch.full((B * H * L + 32,), float("nan"), device=DEV, dtype=dtype)
+    dA16 = buf[16:16 + B * H * L].view(B, H, L)
+    print(f"dA in 16 bits L={L} {dtype} dy_f32={dy_f32}", flush=True)
+    _btp.backward(coeff, x, dy, ck, dx32, dA32, 2, 32)
+    _btp.backward(coeff, x, dy, ck, dx16, dA16, 2, 32, flags=_btp.FLAG_DA_16)
+    torch.cuda.synchronize()
+    assert torch.equal(dA16, dA32.to(dtype)) and torch.equal(dx16, dx32)
+    assert bool(torch.isnan(buf[:16]).all()) and bool(torch.isnan(buf[-16:]).all())
