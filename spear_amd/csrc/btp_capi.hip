@@ -9,6 +9,7 @@
 #include <stdlib.h>
 
 #include "../../include/spear_btp.h"
+#include "../../include/spear_layer.h"
 #include "btp_launch.h"
 
 namespace {
@@ -63,7 +64,7 @@ int check_common(const char* who, int B, int H, int L, int k, int in_dtype, int 
 
 extern "C" {
 
-int spear_btp_abi_version(void) { return 18; }
+int spear_btp_abi_version(void) { return 19; }
 
 const char* spear_btp_last_error(void) { return g_error; }
 
@@ -161,34 +162,58 @@ int spear_phalanx_mix_forward(const void* a_logit, const void* b_logit, const vo
   return spear_phalanx_mix_prefill(a_logit, b_logit, c, v, out, nullptr, B, L, H, kv_heads, dtype, flags, stream);
 }
 
+// Checks shared by the fused forward entry points; 1 = nothing to do (empty tensors), 0 = go on.
+static int check_mix_forward(const char* who, const void* const (&ptrs)[5], int B, int L, int H, int kv_heads, int dtype, bool f32) {
+  if (B < 0 || L < 0 || H < 0) return fail(SPEAR_BTP_EINVAL, "%s: negative dimension (B=%d L=%d H=%d)", who, B, L, H);
+  if (kv_heads <= 0 || H % kv_heads != 0)
+    return fail(SPEAR_BTP_EINVAL, "%s: heads (%d) must be divisible by kv_heads (%d)", who, H, kv_heads);
+  if (dtype != SPEAR_BTP_BF16 && dtype != SPEAR_BTP_F16)
+    return fail(SPEAR_BTP_EINVAL, "%s: tensors must be float16 or bfloat16.", who);
+  if ((long long)B * L * H * 16ll >= (1ll << 40)) return fail(SPEAR_BTP_EINVAL, "%s: tensor too large", who);
+  if ((long long)L * H * (f32 ? 64ll : 32ll) >= (1ll << 31))  // a batch row is addressed through one 32-bit buffer resource
+    return fail(SPEAR_BTP_EINVAL, "%s: one batch row (L * H * 16 elements) must stay below 2 GiB", who);
+  if ((long long)B * H == 0 || L == 0) return 1;
+  if (spear_btp::fused_mix_workgroups(B, H, H / kv_heads, L, false) >= (1ll << 31))
+    return fail(SPEAR_BTP_EINVAL, "%s: too many tiles for one launch (B * L / 64 * H / 8 must stay below 2^31)", who);
+  for (const void* q : ptrs) {
+    if (!q) return fail(SPEAR_BTP_ENULL, "%s: NULL tensor pointer", who);
+    if (!aligned16(q)) return fail(SPEAR_BTP_EINVAL, "%s: tensor pointers must be 16-byte aligned", who);
+  }
+  return 0;
+}
+
 int spear_phalanx_mix_prefill(const void* a_logit, const void* b_logit, const void* c, const void* v, void* out,
                               float* c_prev_tail, int B, int L, int H, int kv_heads, int dtype, unsigned flags,
                               void* stream) {
   g_error[0] = '\0';
   const char* who = c_prev_tail ? "spear_phalanx_mix_prefill" : "spear_phalanx_mix_forward";
-  if (B < 0 || L < 0 || H < 0) return fail(SPEAR_BTP_EINVAL, "%s: negative dimension (B=%d L=%d H=%d)", who, B, L, H);
   if (L % 16 != 0) return fail(SPEAR_BTP_EINVAL, "%s: Length L must be multiple of 16 (got %d)", who, L);
-  if (kv_heads <= 0 || H % kv_heads != 0)
-    return fail(SPEAR_BTP_EINVAL, "%s: heads (%d) must be divisible by kv_heads (%d)", who, H, kv_heads);
-  if (dtype != SPEAR_BTP_BF16 && dtype != SPEAR_BTP_F16)
-    return fail(SPEAR_BTP_EINVAL, "%s: tensors must be float16 or bfloat16.", who);
   const unsigned known = SPEAR_MIX_QKV_GATE | SPEAR_MIX_F32_RESULTS;
   if (flags & ~known) return fail(SPEAR_BTP_EINVAL, "%s: unknown flag bits 0x%x", who, flags & ~known);
   const bool f32 = (flags & SPEAR_MIX_F32_RESULTS) != 0;
-  if ((long long)B * L * H * 16ll >= (1ll << 40)) return fail(SPEAR_BTP_EINVAL, "%s: tensor too large", who);
-  if ((long long)L * H * (f32 ? 64ll : 32ll) >= (1ll << 31))  // a batch row is addressed through one 32-bit buffer resource
-    return fail(SPEAR_BTP_EINVAL, "%s: one batch row (L * H * 16 elements) must stay below 2 GiB", who);
-  if ((long long)B * H == 0 || L == 0) return 0;
-  if (spear_btp::fused_mix_workgroups(B, H, H / kv_heads, L, false) >= (1ll << 31))
-    return fail(SPEAR_BTP_EINVAL, "%s: too many tiles for one launch (B * L / 64 * H / 8 must stay below 2^31)", who);
-  if (!a_logit || !b_logit || !c || !v || !out) return fail(SPEAR_BTP_ENULL, "%s: NULL tensor pointer", who);
-  if (!aligned16(a_logit) || !aligned16(b_logit) || !aligned16(c) || !aligned16(v) || !aligned16(out))
-    return fail(SPEAR_BTP_EINVAL, "%s: tensor pointers must be 16-byte aligned", who);
+  const void* const ptrs[5] = {a_logit, b_logit, c, v, out};
+  if (int rc = check_mix_forward(who, ptrs, B, L, H, kv_heads, dtype, f32)) return rc < 0 ? rc : 0;
   if (c_prev_tail && !aligned16(c_prev_tail)) return fail(SPEAR_BTP_EINVAL, "%s: tensor pointers must be 16-byte aligned", who);
   if (c_prev_tail && (flags & SPEAR_MIX_QKV_GATE))
     return fail(SPEAR_BTP_EINVAL, "%s: the hand-over state belongs to the layer form, not SPEAR_MIX_QKV_GATE", who);
   spear_btp::MixArgs a{a_logit, b_logit, c, v, out, B, L, H, H / kv_heads, dtype, (flags & SPEAR_MIX_QKV_GATE) != 0, f32,
                        c_prev_tail};
+  const hipError_t err = spear_btp::fused_mix_forward(a, static_cast<hipStream_t>(stream));
+  if (err != hipSuccess) return fail(SPEAR_BTP_ELAUNCH, "%s: launch failed: %s", who, hipGetErrorString(err));
+  return 0;
+}
+
+int spear_layer_prefill(const void* a_logit, const void* b_logit, const void* c, const void* v, void* out, float* h, float* r,
+                        float* c_prev, int* pos, int B, int L, int H, int kv_heads, int dtype, void* stream) {
+  g_error[0] = '\0';
+  const char* who = "spear_layer_prefill";
+  const void* const ptrs[5] = {a_logit, b_logit, c, v, out};
+  if (int rc = check_mix_forward(who, ptrs, B, L, H, kv_heads, dtype, false)) return rc < 0 ? rc : 0;
+  if (!h || !r || !c_prev || !pos) return fail(SPEAR_BTP_ENULL, "%s: NULL tensor pointer", who);
+  if (!aligned16(h) || !aligned16(c_prev)) return fail(SPEAR_BTP_EINVAL, "%s: tensor pointers must be 16-byte aligned", who);
+  if ((reinterpret_cast<uintptr_t>(r) & 3u) || (reinterpret_cast<uintptr_t>(pos) & 3u))
+    return fail(SPEAR_BTP_EINVAL, "%s: r and pos must be 4-byte aligned", who);
+  spear_btp::MixArgs a{a_logit, b_logit, c, v, out, B, L, H, H / kv_heads, dtype, false, false, c_prev, h, r, pos};
   const hipError_t err = spear_btp::fused_mix_forward(a, static_cast<hipStream_t>(stream));
   if (err != hipSuccess) return fail(SPEAR_BTP_ELAUNCH, "%s: launch failed: %s", who, hipGetErrorString(err));
   return 0;

@@ -105,9 +105,9 @@ struct GatePlace {
 };
 
 template <bool kQkv>
-__device__ __forceinline__ GatePlace gate_place(int first, int H, int lane) {
+__device__ __forceinline__ GatePlace gate_place(int first, int H, int lane, int last_step = kTile - 1) {
   constexpr int kGateBytes = kQkv ? 4 : 2;
-  const int gt = lane & 15, h0 = first + 2 * (lane >> 4);
+  const int gt = min(lane & 15, last_step), h0 = first + 2 * (lane >> 4);
   GatePlace g;
   g.split = !kQkv && (((H | first) & 1) != 0);
   if (kQkv || g.split) {
@@ -736,18 +736,23 @@ void phalanx_mix_bwd_tile_kernel(
 // and runs that recurrence itself. A kv head shared by several heads is resolved by indexing (head h reads b, c of
 // kv head h / group), for any group size. The wavefront of a row's last block also stores the streaming state for
 // decoding after this prompt, when asked.
+// kRagged: rows whose last block is not whole (prompts of any length). That block's steps past the end read the row's last step
+// and are not stored, and its state is the one after the row's last step: one launch for the whole prompt where the steps of
+// the last block used to go through the decode kernel one launch each, between transposes and a concatenation of the two parts
+// (B=64 L=1003 dim=512: 45 us for the whole prompt; the 11 steps and the copies around them took 350 us more).
 // kW wavefronts per workgroup, one head slot x kW consecutive blocks (2 head slots x kW / 2 blocks measured
 // slower at every shape): 4 or 8. Microseconds for 4 / 8, B L H:
 //   1024 128 32: 87.3 / 91.5    256 512 32: 89.8 / 86.0    16 8192 32: 89.4 / 87.1
 //   512 128 64: 91.6 / 90.2     16 8192 64: 167.5 / 170.6  64 2048 128: 336.1 / 338.3
 //   256 128 128: 87.7 / 90.1    4096 128 8: 92.9 / 88.1    1024 128 48: 132.9 / 125.3
 // ==========================================================================================
-template <class E, int kW, bool kQkv, bool kF32>
+template <class E, int kW, bool kQkv, bool kF32, bool kRagged>
 __global__ __launch_bounds__(64 * kW) __attribute__((amdgpu_waves_per_eu(SPEAR_FUSED_TILE_WAVES_PER_EU)))
 void phalanx_mix_fwd_tile_kernel(const uint16_t* __restrict__ a_logit, const uint16_t* __restrict__ b_logit,
                                  const uint16_t* __restrict__ c_in, const uint16_t* __restrict__ v_in,
-                                 uint16_t* __restrict__ out, float* __restrict__ c_prev_tail, int L, int H,
-                                 int kv_groups, int tiles) {
+                                 uint16_t* __restrict__ out, float* __restrict__ c_prev_tail, float* __restrict__ h_tail,
+                                 float* __restrict__ r_tail, int* __restrict__ pos_tail, int L, int H, int kv_groups,
+                                 int tiles) {
   __shared__ __align__(16) float gate_tiles[kW][2][kHeadsPerWave * kGateRow];  // own block, block before the edge
   __shared__ float2 carry_out[kW][64];  // terminal local state of the wavefront's block, per lane
 
@@ -786,6 +791,8 @@ void phalanx_mix_fwd_tile_kernel(const uint16_t* __restrict__ a_logit, const uin
   const int gt = lane & 15;
   const GatePlace gp = gate_place<kQkv>(ho, H, lane);
   constexpr int kNt = 2;
+  const int steps = kRagged ? min(kTile, L - t0) : kTile;  // of this wavefront's block
+  auto at_step = [&](int r) { return kRagged ? t0 + min(r, steps - 1) : t0 + r; };  // loads stay inside the row
 
   const bool halo = valid && bl == 0 && t0 > 0;  // needs the terminal local state of block t0 - 16
   const int th = t0 - kTile;
@@ -794,7 +801,7 @@ void phalanx_mix_fwd_tile_kernel(const uint16_t* __restrict__ a_logit, const uin
   uint32_t b[16], c[16], v[16], hb[16], hv[16];
   GateWords araw = {0u, 0u}, haraw = {0u, 0u};
   if (valid) {
-    araw = load_gate_words<kQkv>(ra, gp, t0, H);
+    araw = load_gate_words<kQkv>(ra, kRagged ? gate_place<kQkv>(ho, H, lane, steps - 1) : gp, t0, H);
     if (halo) {
       haraw = load_gate_words<kQkv>(ra, gp, th, H);
 #pragma unroll
@@ -805,11 +812,11 @@ void phalanx_mix_fwd_tile_kernel(const uint16_t* __restrict__ a_logit, const uin
     }
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
-      b[r] = __builtin_amdgcn_raw_buffer_load_b32(rb, kv_lane, (t0 + r) * kv_stride, kNt);
-      v[r] = __builtin_amdgcn_raw_buffer_load_b32(rv, f_lane, (t0 + r) * stride, kNt);
+      b[r] = __builtin_amdgcn_raw_buffer_load_b32(rb, kv_lane, at_step(r) * kv_stride, kNt);
+      v[r] = __builtin_amdgcn_raw_buffer_load_b32(rv, f_lane, at_step(r) * stride, kNt);
     }
 #pragma unroll
-    for (int r = 0; r < 16; ++r) c[r] = __builtin_amdgcn_raw_buffer_load_b32(rc, kv_lane, (t0 + r) * kv_stride, kNt);
+    for (int r = 0; r < 16; ++r) c[r] = __builtin_amdgcn_raw_buffer_load_b32(rc, kv_lane, at_step(r) * kv_stride, kNt);
   }
   __builtin_amdgcn_sched_barrier(0);
 
@@ -854,14 +861,12 @@ void phalanx_mix_fwd_tile_kernel(const uint16_t* __restrict__ a_logit, const uin
     for (int r = 0; r < 16; ++r) {
       x0[r] = input_gate<kQkv>(E::lo(b[r])) * E::lo(v[r]);
       x1[r] = input_gate<kQkv>(E::hi(b[r])) * E::hi(v[r]);
-      l0 = fmaf(a[r], l0, x0[r]);
-      l1 = fmaf(a[r], l1, x1[r]);
+      if (!kRagged || r < steps) {  // wave-uniform: a block that ends early keeps the state after its last step
+        l0 = fmaf(a[r], l0, x0[r]);
+        l1 = fmaf(a[r], l1, x1[r]);
+      }
     }
     carry_out[wave][lane] = make_float2(l0, l1);
-    // Hand-over for token-by-token decoding after this prompt: the terminal local state of the row's last block is
-    // what the next block's steps need as c_prev (the block-local state restarts at 0 and the gate product at 1).
-    if (c_prev_tail != nullptr && t0 + kTile == L && real)
-      *reinterpret_cast<float2*>(c_prev_tail + (brow * H + head) * kChan + d0) = make_float2(l0, l1);
   }
   __syncthreads();  // the kernel's only workgroup barrier; wavefronts without a block arrive here directly
   if (!valid) return;
@@ -871,6 +876,29 @@ void phalanx_mix_fwd_tile_kernel(const uint16_t* __restrict__ a_logit, const uin
     cin0 = q.x;
     cin1 = q.y;
   }
+  // Hand-over for token-by-token decoding after this prompt, by the wavefront of the row's last block. After a whole block
+  // the next steps need its terminal local state as c_prev and start at h = 0, r = 1; inside a block they go on from the
+  // block-local state and gate product with the carry this block was given.
+  if (c_prev_tail != nullptr && t0 + kTile >= L) {
+    const bool full = !kRagged || steps == kTile;
+    const float2 own = carry_out[wave][lane];
+    const long o = (brow * H + head) * kChan + d0;
+    if (real) {
+      *reinterpret_cast<float2*>(c_prev_tail + o) = full ? own : make_float2(cin0, cin1);
+      if (h_tail != nullptr) {
+        *reinterpret_cast<float2*>(h_tail + o) = full ? make_float2(0.0f, 0.0f) : own;
+        if (d0 == 0) {
+          float p = 1.0f;
+          if (!full) {
+#pragma unroll
+            for (int r = 0; r < 16; ++r) p *= r < steps ? a[r] : 1.0f;
+          }
+          r_tail[brow * H + head] = p;
+        }
+      }
+    }
+    if (pos_tail != nullptr && at.slot == 0 && lane == 0) pos_tail[brow] = full ? 0 : steps;
+  }
   // the carry-started recurrence and the output mix
   float y0 = cin0, y1 = cin1;
 #pragma unroll
@@ -878,11 +906,12 @@ void phalanx_mix_fwd_tile_kernel(const uint16_t* __restrict__ a_logit, const uin
     y0 = fmaf(a[r], y0, x0[r]);
     y1 = fmaf(a[r], y1, x1[r]);
     const float o0 = fmaf(y0, E::lo(c[r]), E::lo(v[r])), o1 = fmaf(y1, E::hi(c[r]), E::hi(v[r]));
+    const int off = !kRagged || r < steps ? o_lane : kNowhere;
     if constexpr (kF32) {
       const u32x2_t ow = {__float_as_uint(o0), __float_as_uint(o1)};
-      __builtin_amdgcn_raw_buffer_store_b64(ow, ro, o_lane, (t0 + r) * stride * 2, kNt);
+      __builtin_amdgcn_raw_buffer_store_b64(ow, ro, off, at_step(r) * stride * 2, kNt);
     } else {
-      __builtin_amdgcn_raw_buffer_store_b32(E::pack2(o0, o1), ro, o_lane, (t0 + r) * stride, kNt);
+      __builtin_amdgcn_raw_buffer_store_b32(E::pack2(o0, o1), ro, off, at_step(r) * stride, kNt);
     }
   }
 }
@@ -965,7 +994,7 @@ struct TileGrid {
   long wgs;
 };
 TileGrid tile_grid(long B, int slots, int L, int waves) {
-  const int nb = L / kTile;
+  const int nb = (L + kTile - 1) / kTile;
   TileGrid g;
   g.tiles = (nb + waves - 1) / waves;
   const int tg = g.tiles < SPEAR_FUSED_TILE_TIME_GROUP ? g.tiles : SPEAR_FUSED_TILE_TIME_GROUP;  // tile_place()
@@ -977,13 +1006,13 @@ TileGrid tile_grid(long B, int slots, int L, int waves) {
 // (table at the forward kernel).
 bool forward_takes_eight_waves(int H, int L) { return H < 16 || (L >= 512 && H <= 32); }
 
-template <class E, int kW, bool kQkv, bool kF32 = false>
+template <class E, int kW, bool kQkv, bool kF32 = false, bool kRagged = false>
 void launch_mix_fwd_tile(const MixArgs& p, hipStream_t s) {
   const TileGrid g = tile_grid(p.B, (p.H + kHeadsPerWave - 1) / kHeadsPerWave, p.L, kW);
-  hipLaunchKernelGGL((phalanx_mix_fwd_tile_kernel<E, kW, kQkv, kF32>), dim3((unsigned)g.wgs), dim3(64 * kW), 0, s,
+  hipLaunchKernelGGL((phalanx_mix_fwd_tile_kernel<E, kW, kQkv, kF32, kRagged>), dim3((unsigned)g.wgs), dim3(64 * kW), 0, s,
                      static_cast<const uint16_t*>(p.a_logit), static_cast<const uint16_t*>(p.b_logit),
                      static_cast<const uint16_t*>(p.c), static_cast<const uint16_t*>(p.v), static_cast<uint16_t*>(p.out),
-                     p.c_prev_tail, p.L, p.H, p.kv_groups, g.tiles);
+                     p.c_prev_tail, p.h_tail, p.r_tail, p.pos_tail, p.L, p.H, p.kv_groups, g.tiles);
 }
 
 // Groups of 1, 2, 4, 8 heads per kv head are summed inside a wavefront's 8 heads; the others take slots cut at
@@ -1024,6 +1053,13 @@ hipError_t fused_mix_forward(const MixArgs& p, hipStream_t s) {
   const bool eight = forward_takes_eight_waves(p.H, p.L);
   auto by_form = [&](auto e, auto q) {
     using E = decltype(e);
+    if constexpr (!decltype(q)::value) {
+      if (p.L % kTile != 0) {  // prompts, layer form with 16-bit results only (the caller has checked)
+        if (eight) launch_mix_fwd_tile<E, 8, false, false, true>(p, s);
+        else launch_mix_fwd_tile<E, 4, false, false, true>(p, s);
+        return;
+      }
+    }
     if (p.f32_out) launch_mix_fwd_tile<E, 4, decltype(q)::value, true>(p, s);  // check mode: one instance per form
     else if (eight) launch_mix_fwd_tile<E, 8, decltype(q)::value>(p, s);
     else launch_mix_fwd_tile<E, 4, decltype(q)::value>(p, s);

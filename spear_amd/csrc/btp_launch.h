@@ -57,6 +57,10 @@ struct MixArgs {
   // null, or fp32 [B, H, 16]: receives the terminal local state of every row's last block (the c_prev of the
   // streaming state after this prompt)
   float* c_prev_tail = nullptr;
+  // with c_prev_tail, all three or none: the rest of the streaming state after any number of steps, fp32 [B, H, 16] block-local
+  // state, fp32 [B, H] gate product, int32 [B] position inside the block. L % 16 != 0 is for these calls.
+  float *h_tail = nullptr, *r_tail = nullptr;
+  int* pos_tail = nullptr;
 };
 hipError_t fused_mix_forward(const MixArgs& p, hipStream_t s);
 // Workgroups the forward / backward kernel launches for a shape (must fit a 31-bit grid).

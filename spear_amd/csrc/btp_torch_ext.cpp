@@ -17,6 +17,7 @@
 #include <vector>
 
 #include "../../include/spear_btp.h"
+#include "../../include/spear_layer.h"
 
 namespace {
 
@@ -217,7 +218,7 @@ struct MixShape {
   int64_t B, L, F, Fkv;
 };
 
-MixShape check_mix_inputs(const at::Tensor& a_logit, const at::Tensor& b_logit, const at::Tensor& c, const at::Tensor& v,
+MixShape check_mix_shapes(const at::Tensor& a_logit, const at::Tensor& b_logit, const at::Tensor& c, const at::Tensor& v,
                           int64_t heads, int64_t kv_heads, bool qkv_gate) {
   TORCH_CHECK(a_logit.is_cuda() && b_logit.is_cuda() && c.is_cuda() && v.is_cuda(), "All tensors must be CUDA.");
   TORCH_CHECK(v.dim() == 3 && v.size(2) == heads * 16, "v must be [B, L, heads * 16].");
@@ -230,11 +231,17 @@ MixShape check_mix_inputs(const at::Tensor& a_logit, const at::Tensor& b_logit, 
     TORCH_CHECK(a_logit.scalar_type() == v.scalar_type(), "all tensors must share one dtype.");
   }
   const MixShape s{v.size(0), v.size(1), v.size(2), kv_heads * 16};
-  TORCH_CHECK(s.L % 16 == 0, "Length L must be multiple of 16");
   check_layout("a_logit", a_logit, {s.B, s.L, heads});
   check_layout("b_logit", b_logit, {s.B, s.L, s.Fkv});
   check_layout("c", c, {s.B, s.L, s.Fkv});
   check_layout("v", v, {s.B, s.L, s.F});
+  return s;
+}
+
+MixShape check_mix_inputs(const at::Tensor& a_logit, const at::Tensor& b_logit, const at::Tensor& c, const at::Tensor& v,
+                          int64_t heads, int64_t kv_heads, bool qkv_gate) {
+  const MixShape s = check_mix_shapes(a_logit, b_logit, c, v, heads, kv_heads, qkv_gate);
+  TORCH_CHECK(s.L % 16 == 0, "Length L must be multiple of 16");
   return s;
 }
 
@@ -373,6 +380,22 @@ at::Tensor mix_autograd(const at::Tensor& a_logit, const at::Tensor& b_logit, co
   return MixNode::apply(a_logit, b_logit, c, v, heads, kv_heads, qkv_gate);
 }
 
+// A prompt through the mixing stage: out and the streaming state after it (h, r, c_prev, pos), all allocated here. Any L >= 1.
+std::vector<at::Tensor> mix_prefill(const at::Tensor& a_logit, const at::Tensor& b_logit, const at::Tensor& c, const at::Tensor& v,
+                                    int64_t heads, int64_t kv_heads) {
+  const MixShape s = check_mix_shapes(a_logit, b_logit, c, v, heads, kv_heads, false);
+  check_same_device({&a_logit, &b_logit, &c, &v});
+  const auto f32 = v.options().dtype(at::kFloat);
+  at::Tensor out = at::empty_like(v), h = at::empty({s.B, heads, 16}, f32), r = at::empty({s.B, heads}, f32),
+             c_prev = at::empty({s.B, heads, 16}, f32), pos = at::empty({s.B}, v.options().dtype(at::kInt));
+  const c10::DeviceGuard guard(v.device());
+  const int rc = spear_layer_prefill(a_logit.data_ptr(), b_logit.data_ptr(), c.data_ptr(), v.data_ptr(), out.data_ptr(),
+                                     h.data_ptr<float>(), r.data_ptr<float>(), c_prev.data_ptr<float>(), pos.data_ptr<int>(),
+                                     (int)s.B, (int)s.L, (int)heads, (int)kv_heads, tag_of(v.scalar_type()), stream_of(v));
+  if (rc != 0) raise_native(rc);
+  return {out, h, r, c_prev, pos};
+}
+
 }  // namespace
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
@@ -397,6 +420,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("mix_autograd", &mix_autograd, py::arg("a_logit"), py::arg("b_logit"), py::arg("c"), py::arg("v"), py::arg("heads"),
         py::arg("kv_heads"), py::arg("qkv_gate") = false,
         "out = phalanx_mix(...) (or the q/k/v/gate form) with its autograd node (contiguous plain tensors)");
+  m.def("mix_prefill", &mix_prefill, py::arg("a_logit"), py::arg("b_logit"), py::arg("c"), py::arg("v"), py::arg("heads"),
+        py::arg("kv_heads"), "[out, h, r, c_prev, pos]: a prompt of any length through the mixing stage, with the state after it");
   m.def("abi_version", []() { return spear_btp_abi_version(); });
   m.def("mix_backward_sum_rows", [](int64_t B, int64_t L, int64_t heads) {
     return (int64_t)spear_phalanx_mix_backward_sum_rows((int)B, (int)L, (int)heads);

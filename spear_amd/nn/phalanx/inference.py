@@ -331,29 +331,14 @@ def phalanx_step(layer, x_t: torch.Tensor, state: PhalanxStepState, out: torch.T
 @torch.no_grad()
 def phalanx_prefill(layer, x: torch.Tensor) -> tuple[torch.Tensor, PhalanxStepState]:
     """A prompt ``x`` [B, L, dim] (any L >= 1) through ``layer``: returns the layer's output for it and the state
-    after its last token, from which :func:`phalanx_step` continues. The whole blocks go through the fused
-    forward kernel, which also leaves the hand-over state (``spear_phalanx_mix_prefill``: after a whole number of
-    blocks the state is the last block's terminal local state, a zero block-local state and a gate product of
-    one); the at most 15 tokens of a partial last block are projected together and stepped one kernel each."""
+    after its last token, from which :func:`phalanx_step` continues. The whole prompt is one launch of the fused forward
+    kernel, which also leaves the state: after a whole number of blocks the last block's terminal local state, a zero
+    block-local state and a gate product of one, inside a block the block-local state and gate product so far."""
     _need_gpu(x)
-    B, L, _ = x.shape
-    p, bl = layer.param, 16
+    p = layer.param
     if layer.k != 2:
         raise RuntimeError("phalanx_prefill needs a layer with k == 2")
-    full = (L // bl) * bl
-    state = PhalanxStepState.zeros(B, layer.heads, x.device, bl)
     xc = x.to(p.compute_dtype)
-    parts = []
-    if full > 0:
-        a, b, c, v = (proj(xc[:, :full]) for proj in (p.proj_a, p.proj_b, p.proj_c, p.proj_v))
-        mixed = torch.empty_like(v)
-        _btp.mix_forward(a, b, c, v, mixed, layer.heads, layer.kv_heads, c_prev_tail=state.c_prev_loc)
-        parts.append(mixed)
-    if L > full:
-        a, b, c, v = (proj(xc[:, full:]).transpose(0, 1).contiguous() for proj in (p.proj_a, p.proj_b, p.proj_c, p.proj_v))
-        tail = torch.empty_like(v)  # [tokens, B, dim]
-        for t in range(L - full):
-            _btp.mix_step(a[t], b[t], c[t], v[t], tail[t], state.h_loc, state.r_pref, state.c_prev_loc, state.pos, False,
-                          bl, layer.heads, layer.kv_heads)
-        parts.append(tail.transpose(0, 1))
-    return layer.proj_out(parts[0] if len(parts) == 1 else torch.cat(parts, dim=1)), state
+    a, b, c, v = (proj(xc).contiguous() for proj in (p.proj_a, p.proj_b, p.proj_c, p.proj_v))
+    mixed, h, r, c_prev, pos = _btp.load_extension().mix_prefill(a, b, c, v, layer.heads, layer.kv_heads)
+    return layer.proj_out(mixed), PhalanxStepState(h, r, c_prev, pos, 16)

@@ -216,3 +216,29 @@ def test_step_rejects_bad_arguments():
         _btp.mix_step(a, b, c, v, out, h, r[:1], cp, None, False, 16, H, H)
     with pytest.raises(RuntimeError, match="block_len must be positive"):
         _btp.mix_step(a, b, c, v, out, h, r, cp, None, False, 0, H, H)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "f16"])
+@pytest.mark.parametrize("B,H,Hkv,L", [(3, 4, 4, 1), (2, 8, 2, 15), (2, 3, 3, 17), (2, 32, 32, 63), (2, 5, 1, 65), (3, 12, 4, 129),
+                                       (2, 8, 8, 513), (2, 24, 3, 1003), (2, 16, 16, 64)])
+def test_prefill_of_any_length_is_one_launch_with_the_state_that_stepping_reaches(B, H, Hkv, L, dtype):
+    """The prompt kernel at lengths that end inside a block (and, last case, at a block's end): its output is that of the
+    forward kernel on the prompt filled up to a whole block, and its state the one the step kernel reaches, bit for bit."""
+    from spear_amd import _btp
+
+    g = torch.Generator().manual_seed(77 + L)
+    a, b, c, v = (torch.randn(B, L, w, generator=g).to(dtype).to(DEV) for w in (H, Hkv * 16, Hkv * 16, H * 16))
+    print(f"prefill of any length B={B} H={H} Hkv={Hkv} L={L} {dtype}", flush=True)
+    out, h, r, c_prev, pos = _btp.load_extension().mix_prefill(a, b, c, v, H, Hkv)
+    torch.cuda.synchronize()
+    whole = [torch.nn.functional.pad(t, (0, 0, 0, -L % 16)).contiguous() for t in (a, b, c, v)]
+    want = torch.empty_like(whole[3])
+    _btp.mix_forward(*whole, want, H, Hkv)
+    assert torch.equal(out, want[:, :L])
+    sh, sr, sc = torch.zeros(B, H, 16, device=DEV), torch.ones(B, H, device=DEV), torch.zeros(B, H, 16, device=DEV)
+    sp = torch.zeros(B, device=DEV, dtype=torch.int32)
+    y = torch.empty(B, H * 16, device=DEV, dtype=dtype)
+    for t in range(L):
+        _btp.mix_step(*(q[:, t].contiguous() for q in (a, b, c, v)), y, sh, sr, sc, sp, False, 16, H, Hkv)
+    for name, got, ref in (("h", h, sh), ("r", r, sr), ("c_prev", c_prev, sc), ("pos", pos, sp)):
+        assert torch.equal(got, ref), name
