@@ -11,7 +11,8 @@ initialises identical weights).
     y = proj_out( (recurrence(A, X) * C + V)  laid out as [B, L, H*16] )
 
 ``method`` picks who evaluates the recurrence:
-  ``"default"``           the HIP kernels through :func:`spear_amd.ops.btp.btp`
+  ``"default"``           the HIP kernels: :func:`spear_amd.ops.btp.btp` between the gates and ``* C + V``; a plain
+                          eager call in bf16 with ``k == 2`` runs the whole mixing stage in the kernels of ``"fused"``
   ``"pytorch"``           the log-space PyTorch statement of the two-pass algorithm
   ``"pytorch_linspace"``  the linear-space PyTorch statement
   ``"fused"``             (addition) one HIP kernel for gates + recurrence + ``* C + V`` working
@@ -19,8 +20,8 @@ initialises identical weights).
                           needs ``k == 2``
 The choice is explicit; ``"default"`` and ``"fused"`` never degrade to a PyTorch path. Code written
 against the reference says ``method="default"``; with ``SPEAR_PHALANX_DEFAULT=fused`` in the environment
-such a layer runs the fused kernels wherever they apply (``k == 2``, 16-bit output) and
-the stand-alone kernels elsewhere, without a change to the calling code.
+such a layer runs the fused kernels wherever they apply (``k == 2``, 16-bit output), under ``torch.compile`` and
+autocast too, and the stand-alone kernels elsewhere, without a change to the calling code.
 
 On a GPU, from 8192 tokens per call on, the ``"default"`` and ``"fused"`` layers run their five
 projections through :mod:`.projections` (same forward; weight gradients cut along the token axis, one
@@ -35,7 +36,7 @@ import os
 import torch
 import torch.nn as nn
 
-from .projections import input_projections, linear, pays_off, project_and_mix
+from .projections import input_projections, linear, packed_columns, pays_off, project_and_mix
 
 _HEAD_DIM = 16
 _METHODS = ("default", "pytorch", "pytorch_linspace", "fused")
@@ -222,17 +223,48 @@ class Phalanx(nn.Module):
         A, X, C, V = self.param.forward_axcv(x)
         return self._mix_and_project(self.pytorch_block_two_pass(A, X, self.block_size), C, V)
 
+    def _mixes_in_one_kernel(self, x: torch.Tensor) -> bool:
+        """Whether a ``"default"`` call runs gates, recurrence and ``* C + V`` in the fused kernels, on the projections'
+        own layout, instead of the stand-alone recurrence between about twenty elementwise and transposing passes.
+        Forward + backward, us, stand-alone / fused: B=1024 L=128 dim=512 4692 / 1373, B=8 822 / 562; no size was
+        found where the stand-alone kernels win. They keep every call that the fused ones would answer in
+        another way: k = 1, other types than bf16 throughout, autocast, anything that traces or transforms the call
+        (``_plain_eager``), the matrix-core and checkpoint-store switches, a replaced recurrence or class, empty inputs,
+        lengths and ``wpb`` that :func:`btp` refuses, and batch rows past the fused backward's 2 GiB."""
+        if torch.compiler.is_compiling():
+            return False
+        from spear_amd.ops.btp import btp, interface
+
+        p = self.param
+        if not (x.is_cuda and x.dim() == 3 and x.numel() > 0 and self.k == 2 and self.wpb in interface.SUPPORTED_WPB):
+            return False
+        L, weights = x.shape[1], (p.proj_a.weight, p.proj_b.weight, p.proj_c.weight, p.proj_v.weight)
+        return (
+            L % interface.BLK == 0 and 2 * L * packed_columns(self.heads, self.kv_heads)[1] < 1 << 31
+            and interface._FORWARD_FLAGS == 0 and self.btp_module is btp
+            and type(self) is Phalanx and type(p) is SigmoidA and p.token_sliced_backward
+            and self.output_dtype == p.compute_dtype and all(w.dtype == p.compute_dtype for w in weights)
+            and not torch.is_autocast_enabled("cuda") and interface._plain_eager(x, *weights)
+        )
+
     def _forward_default(self, x: torch.Tensor) -> torch.Tensor:
+        if self._mixes_in_one_kernel(x):
+            from spear_amd.ops.btp import phalanx_mix
+
+            return self._forward_on_projections(x, phalanx_mix)
         A, X, C, V = self.param.forward_axcv(x)
         return self._mix_and_project(self.btp_module(A, X, self.k, self.wpb, self.output_dtype), C, V)
 
     def _forward_fused(self, x: torch.Tensor) -> torch.Tensor:
+        return self._forward_on_projections(x, self.mix_module)
+
+    def _forward_on_projections(self, x: torch.Tensor, mix) -> torch.Tensor:
         p = self.param
         xc = x.to(p.compute_dtype)
         if xc.dim() == 3 and pays_off(xc):
             mixed = project_and_mix(xc, p.proj_a, p.proj_b, p.proj_c, p.proj_v, self.heads, self.kv_heads)
         else:
-            mixed = self.mix_module(*p.project(xc), self.heads, self.kv_heads)
+            mixed = mix(*p.project(xc), self.heads, self.kv_heads)
         return self._project_out(mixed)
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:

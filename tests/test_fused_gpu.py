@@ -289,3 +289,51 @@ def test_qkv_form_backward_against_the_oracle(H, Hkv):
     assert_close(f64(outs[1]), rk, BF16_ATOL, BF16_RTOL, "dk")
     assert_close(f64(outs[2]), rq, BF16_ATOL, BF16_RTOL, "dq")
     assert_close(f64(outs[3]), rv, BF16_ATOL, BF16_RTOL, "dv")
+
+
+@pytest.mark.parametrize("B,L,dim,kv_heads", [(1, 16, 16, None), (3, 48, 96, 2), (8, 128, 512, None), (64, 144, 80, 1)])
+def test_default_layer_mixes_in_the_fused_kernels(B, L, dim, kv_heads):
+    """A plain bf16 call of a default layer has the fused layer's bits, below and above the 8192 tokens from which the
+    projections' backward is shared, and lies as close to the stand-alone composition as two bf16 roundings allow."""
+    from spear_amd import Phalanx, btp
+
+    torch.manual_seed(11)
+    layer = Phalanx(dim=dim, length=L, dtype=torch.bfloat16, kv_heads=kv_heads).to(DEV)
+    fused = Phalanx(dim=dim, length=L, method="fused", dtype=torch.bfloat16, kv_heads=kv_heads).to(DEV)
+    fused.load_state_dict(layer.state_dict())
+    x = torch.randn(B, L, dim, generator=torch.Generator().manual_seed(12)).bfloat16().to(DEV)
+    dy = torch.randn(B, L, dim, generator=torch.Generator().manual_seed(13)).bfloat16().to(DEV)
+
+    def run(model):
+        model.zero_grad()
+        xx = x.clone().requires_grad_(True)
+        y = model(xx)
+        y.backward(dy)
+        return [y.detach(), xx.grad] + [p.grad for p in model.parameters()]
+
+    assert layer._mixes_in_one_kernel(x)
+    got = run(layer)
+    for a, b in zip(got, run(fused)):
+        assert torch.equal(a, b)
+    layer.btp_module = lambda *args: btp(*args)  # a replaced recurrence is called: the stand-alone composition
+    assert not layer._mixes_in_one_kernel(x)
+    for i, (a, b) in enumerate(zip(got, run(layer))):
+        # each of the about ten roundings between input and gradient is 2^-9 relative; they are independent
+        assert (a.float() - b.float()).norm() <= 2 ** -9 * 10 * b.float().norm(), i
+
+
+def test_calls_that_stay_with_the_stand_alone_kernels():
+    from spear_amd import Phalanx
+
+    x = torch.randn(2, 32, 64, device=DEV).bfloat16()
+    for kwargs, xx in ((dict(k=1), x), (dict(output_dtype=torch.float32), x), (dict(wpb=3), x), (dict(), x[:, :17]), (dict(), x[:0]),
+                       (dict(), x[0])):
+        assert not Phalanx(dim=64, dtype=torch.bfloat16, **kwargs).to(DEV)._mixes_in_one_kernel(xx)
+    layer = Phalanx(dim=64, dtype=torch.bfloat16).to(DEV)
+    assert layer._mixes_in_one_kernel(x)
+    with torch.autocast("cuda", dtype=torch.bfloat16):
+        assert not layer._mixes_in_one_kernel(x)
+    with torch.device(DEV):  # a function mode
+        assert not layer._mixes_in_one_kernel(x)
+    with pytest.raises(AssertionError, match="multiple"):
+        layer(x[:, :17])
