@@ -18,6 +18,15 @@ extern "C" {
 int spear_layer_prefill(const void* a_logit, const void* b_logit, const void* c, const void* v, void* out, float* h,
                         float* r, float* c_prev, int* pos, int B, int L, int H, int kv_heads, int dtype, void* stream);
 
+/* One token of B sequences through the layer's four input projections and the mixing stage's step (spear_phalanx_mix_step
+ * with positions on the device), bf16 operands, fp32 sums and state:
+ *     x [B, K], rows ldx elements apart   w_a [H, K]   w_b, w_c [kv_heads * 16, K]   w_v [H * 16, K]   b_a, b_b, b_c biases
+ *     out [B, H * 16]    h, c_prev [B, H, 16] fp32    r [B, H] fp32    pos [B] int32       state updated in place
+ * K and ldx multiples of 8; x, weights, out, h and c_prev 16-byte aligned, b_b and b_c 8-byte, b_a 2-byte, r and pos 4-byte. */
+int spear_layer_token(const void* x, long long ldx, const void* w_a, const void* b_a, const void* w_b, const void* b_b,
+                      const void* w_c, const void* b_c, const void* w_v, void* out, float* h, float* r, float* c_prev, int* pos,
+                      int block_len, int B, int K, int H, int kv_heads, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -64,7 +64,7 @@ int check_common(const char* who, int B, int H, int L, int k, int in_dtype, int 
 
 extern "C" {
 
-int spear_btp_abi_version(void) { return 19; }
+int spear_btp_abi_version(void) { return 20; }
 
 const char* spear_btp_last_error(void) { return g_error; }
 
@@ -215,6 +215,36 @@ int spear_layer_prefill(const void* a_logit, const void* b_logit, const void* c,
     return fail(SPEAR_BTP_EINVAL, "%s: r and pos must be 4-byte aligned", who);
   spear_btp::MixArgs a{a_logit, b_logit, c, v, out, B, L, H, H / kv_heads, dtype, false, false, c_prev, h, r, pos};
   const hipError_t err = spear_btp::fused_mix_forward(a, static_cast<hipStream_t>(stream));
+  if (err != hipSuccess) return fail(SPEAR_BTP_ELAUNCH, "%s: launch failed: %s", who, hipGetErrorString(err));
+  return 0;
+}
+
+int spear_layer_token(const void* x, long long ldx, const void* w_a, const void* b_a, const void* w_b, const void* b_b,
+                      const void* w_c, const void* b_c, const void* w_v, void* out, float* h, float* r, float* c_prev, int* pos,
+                      int block_len, int B, int K, int H, int kv_heads, void* stream) {
+  g_error[0] = '\0';
+  const char* who = "spear_layer_token";
+  if (B < 0 || H < 0 || K < 0) return fail(SPEAR_BTP_EINVAL, "%s: negative dimension (B=%d H=%d K=%d)", who, B, H, K);
+  if (block_len <= 0) return fail(SPEAR_BTP_EINVAL, "%s: block_len must be positive (got %d)", who, block_len);
+  if (kv_heads <= 0 || H % kv_heads != 0)
+    return fail(SPEAR_BTP_EINVAL, "%s: heads (%d) must be divisible by kv_heads (%d)", who, H, kv_heads);
+  if (K == 0 || K % 8 != 0 || ldx < K || ldx % 8 != 0)
+    return fail(SPEAR_BTP_EINVAL, "%s: K and ldx must be positive multiples of 8, ldx not below K (got %d and %lld)", who, K, ldx);
+  // as many wavefronts as there are (head, 16 tokens) pairs at most: the grid stays below 2^31 workgroups
+  if ((long long)B * H >= (1ll << 35)) return fail(SPEAR_BTP_EINVAL, "%s: tensor too large", who);
+  if ((long long)B * H == 0) return 0;
+  for (const void* q : {x, w_a, w_b, w_c, w_v, static_cast<const void*>(out), static_cast<const void*>(h), static_cast<const void*>(c_prev)}) {
+    if (!q) return fail(SPEAR_BTP_ENULL, "%s: NULL tensor pointer", who);
+    if (!aligned16(q)) return fail(SPEAR_BTP_EINVAL, "%s: x, the weights, out, h and c_prev must be 16-byte aligned", who);
+  }
+  if (!b_a || !b_b || !b_c || !r || !pos) return fail(SPEAR_BTP_ENULL, "%s: NULL tensor pointer", who);
+  auto off = [](const void* q, unsigned mask) { return (reinterpret_cast<uintptr_t>(q) & mask) != 0; };
+  if (off(b_a, 1u) || off(b_b, 7u) || off(b_c, 7u) || off(r, 3u) || off(pos, 3u))
+    return fail(SPEAR_BTP_EINVAL, "%s: biases, r or pos are not aligned", who);
+  auto u = [](const void* q) { return static_cast<const uint16_t*>(q); };
+  spear_btp::LayerTokenArgs a{u(x), (long)ldx, u(w_a), u(b_a), u(w_b), u(b_b), u(w_c), u(b_c), u(w_v), static_cast<uint16_t*>(out),
+                              h, r, c_prev, pos, block_len, B, K, H, H / kv_heads};
+  const hipError_t err = spear_btp::layer_token(a, static_cast<hipStream_t>(stream));
   if (err != hipSuccess) return fail(SPEAR_BTP_ELAUNCH, "%s: launch failed: %s", who, hipGetErrorString(err));
   return 0;
 }

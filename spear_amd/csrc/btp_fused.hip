@@ -1186,10 +1186,14 @@ hipError_t fused_mix_step(const MixStepArgs& p, hipStream_t s) {
   }
   if (hipError_t err = hipGetLastError(); err != hipSuccess) return err;
   if (p.pos != nullptr && !advance_inside) {  // stream order puts this after every read of pos above
-    hipLaunchKernelGGL(advance_block_positions_kernel, dim3((unsigned)((p.B + 255) / 256)), dim3(256), 0, s, p.pos, p.B, p.block_len);
-    return hipGetLastError();
+    return advance_block_positions(p.pos, p.B, p.block_len, s);
   }
   return hipSuccess;
+}
+
+hipError_t advance_block_positions(int* pos, int B, int block_len, hipStream_t s) {
+  hipLaunchKernelGGL(advance_block_positions_kernel, dim3((unsigned)((B + 255) / 256)), dim3(256), 0, s, pos, B, block_len);
+  return hipGetLastError();
 }
 
 long fused_mix_backward_bias_scratch_floats(long B, int H, int kv_groups, int L) {

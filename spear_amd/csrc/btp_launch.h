@@ -101,6 +101,21 @@ struct MixStepArgs {
   int dtype;
 };
 hipError_t fused_mix_step(const MixStepArgs& p, hipStream_t s);
+// pos[b] <- position of the next token inside its block
+hipError_t advance_block_positions(int* pos, int B, int block_len, hipStream_t s);
+
+// The same step behind the layer's input projections (layer_token.hip), bf16: x [B, K] with rows `ldx` elements apart,
+// weights [features, K] dense, biases [features].
+struct LayerTokenArgs {
+  const uint16_t* x;
+  long ldx;
+  const uint16_t *w_a, *b_a, *w_b, *b_b, *w_c, *b_c, *w_v;
+  uint16_t* out;           // [B, H*16]
+  float *h, *r, *c_prev;   // [B, H, 16], [B, H], [B, H, 16]
+  int* pos;                // [B], advanced
+  int block_len, B, K, H, kv_groups;
+};
+hipError_t layer_token(const LayerTokenArgs& p, hipStream_t s);
 
 // Streaming form (btp_jagged.hip). Tensors [B, H, D, L] / [B, H, L]; state vectors [B, H, D] / [B, H].
 struct JagPrefillArgs {

@@ -396,6 +396,40 @@ std::vector<at::Tensor> mix_prefill(const at::Tensor& a_logit, const at::Tensor&
   return {out, h, r, c_prev, pos};
 }
 
+// One token through the layer's input projections and the step of its mixing stage (the caller applies proj_out): x [B, K]
+// bf16 with unit column stride, weights and biases of the four projections, the state updated in place.
+at::Tensor layer_token(const at::Tensor& x, const at::Tensor& w_a, const at::Tensor& b_a, const at::Tensor& w_b, const at::Tensor& b_b,
+                       const at::Tensor& w_c, const at::Tensor& b_c, const at::Tensor& w_v, at::Tensor h, at::Tensor r,
+                       at::Tensor c_prev, at::Tensor pos, int64_t block_len, int64_t heads, int64_t kv_heads) {
+  TORCH_CHECK(x.is_cuda() && h.is_cuda() && r.is_cuda() && c_prev.is_cuda() && pos.is_cuda(), "All tensors must be CUDA.");
+  TORCH_CHECK(x.dim() == 2 && x.stride(1) == 1, "x must be [B, dim] with dense rows.");
+  TORCH_CHECK(heads > 0 && kv_heads > 0 && heads % kv_heads == 0, "heads must be divisible by kv_heads.");
+  const int64_t B = x.size(0), K = x.size(1);
+  const struct { const char* name; const at::Tensor& t; int64_t rows; } weights[] = {
+      {"w_a", w_a, heads}, {"w_b", w_b, kv_heads * 16}, {"w_c", w_c, kv_heads * 16}, {"w_v", w_v, heads * 16}};
+  for (const auto& w : weights) check_layout(w.name, w.t, {w.rows, K});
+  check_layout("b_a", b_a, {heads});
+  check_layout("b_b", b_b, {kv_heads * 16});
+  check_layout("b_c", b_c, {kv_heads * 16});
+  for (const at::Tensor* t : {&x, &w_a, &b_a, &w_b, &b_b, &w_c, &b_c, &w_v})
+    TORCH_CHECK(t->scalar_type() == at::kBFloat16, "x, weights and biases must be bfloat16.");
+  TORCH_CHECK(h.scalar_type() == at::kFloat && r.scalar_type() == at::kFloat && c_prev.scalar_type() == at::kFloat, "the state must be float32.");
+  TORCH_CHECK(pos.scalar_type() == at::kInt, "pos must be int32.");
+  check_layout("h", h, {B, heads, 16});
+  check_layout("c_prev", c_prev, {B, heads, 16});
+  check_layout("r", r, {B, heads});
+  check_layout("pos", pos, {B});
+  check_same_device({&x, &w_a, &b_a, &w_b, &b_b, &w_c, &b_c, &w_v, &h, &r, &c_prev, &pos});
+  const c10::DeviceGuard guard(x.device());
+  at::Tensor out = at::empty({B, heads * 16}, x.options());
+  const int rc = spear_layer_token(x.data_ptr(), B > 1 ? x.stride(0) : K, w_a.data_ptr(), b_a.data_ptr(), w_b.data_ptr(), b_b.data_ptr(),
+                                   w_c.data_ptr(), b_c.data_ptr(), w_v.data_ptr(), out.data_ptr(), h.data_ptr<float>(),
+                                   r.data_ptr<float>(), c_prev.data_ptr<float>(), pos.data_ptr<int>(), (int)block_len, (int)B, (int)K,
+                                   (int)heads, (int)kv_heads, stream_of(x));
+  if (rc != 0) raise_native(rc);
+  return out;
+}
+
 }  // namespace
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
@@ -422,6 +456,9 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         "out = phalanx_mix(...) (or the q/k/v/gate form) with its autograd node (contiguous plain tensors)");
   m.def("mix_prefill", &mix_prefill, py::arg("a_logit"), py::arg("b_logit"), py::arg("c"), py::arg("v"), py::arg("heads"),
         py::arg("kv_heads"), "[out, h, r, c_prev, pos]: a prompt of any length through the mixing stage, with the state after it");
+  m.def("layer_token", &layer_token, py::arg("x"), py::arg("w_a"), py::arg("b_a"), py::arg("w_b"), py::arg("b_b"), py::arg("w_c"),
+        py::arg("b_c"), py::arg("w_v"), py::arg("h"), py::arg("r"), py::arg("c_prev"), py::arg("pos"), py::arg("block_len"),
+        py::arg("heads"), py::arg("kv_heads"), "one token through the input projections and the step of the mixing stage");
   m.def("abi_version", []() { return spear_btp_abi_version(); });
   m.def("mix_backward_sum_rows", [](int64_t B, int64_t L, int64_t heads) {
     return (int64_t)spear_phalanx_mix_backward_sum_rows((int)B, (int)L, (int)heads);

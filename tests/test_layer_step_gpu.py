@@ -242,3 +242,54 @@ def test_prefill_of_any_length_is_one_launch_with_the_state_that_stepping_reache
         _btp.mix_step(*(q[:, t].contiguous() for q in (a, b, c, v)), y, sh, sr, sc, sp, False, 16, H, Hkv)
     for name, got, ref in (("h", h, sh), ("r", r, sr), ("c_prev", c_prev, sc), ("pos", pos, sp)):
         assert torch.equal(got, ref), name
+
+
+# (B, H, kv heads): one to four token tiles per wavefront, tiles and head groups that are not full, K = 16 H that ends inside
+# a matrix instruction's 32 columns and inside a chunk of loads
+@pytest.mark.parametrize("B,H,Hkv", [(1, 1, 1), (16, 3, 1), (17, 5, 5), (33, 32, 8), (1024, 17, 17), (700, 33, 11), (1000, 72, 9)])
+def test_layer_token_kernel_against_the_oracle(B, H, Hkv):
+    from spear_amd import _btp
+
+    K, g = 16 * H, torch.Generator().manual_seed(31 + B)
+    bf = lambda *s, std=1.0: (std * torch.randn(*s, generator=g)).bfloat16()
+    w = [bf(n, K, std=K ** -0.5) for n in (H, Hkv * 16, Hkv * 16, H * 16)]
+    bias = [bf(n, std=0.3) for n in (H, Hkv * 16, Hkv * 16)]
+    x = bf(B, 2 * K)[:, :K]  # rows of a wider buffer
+    h, cp = torch.randn(B, H, 16, generator=g), torch.randn(B, H, 16, generator=g)
+    r, pos = torch.rand(B, H, generator=g), torch.randint(0, 16, (B,), generator=g, dtype=torch.int32)
+    dev = [t.to(DEV) for t in (h, r, cp, pos)]
+    xd = torch.zeros(B, 2 * K, device=DEV, dtype=torch.bfloat16)[:, :K].copy_(x)
+    wd, bd = [t.to(DEV) for t in w], [t.to(DEV) for t in bias]
+    print(f"layer token B={B} H={H} Hkv={Hkv}", flush=True)
+    out = _btp.load_extension().layer_token(xd, wd[0], bd[0], wd[1], bd[1], wd[2], bd[2], wd[3], *dev, 16, H, Hkv)
+    torch.cuda.synchronize()
+    a, b, c, v = (x.double() @ w_.double().T + (0 if b_ is None else b_.double()) for w_, b_ in zip(w, [*bias, None]))
+    expand = lambda t: t.view(B, Hkv, 16).repeat_interleave(H // Hkv, 1)
+    gate, v = torch.sigmoid(a), v.view(B, H, 16)
+    h2 = gate[..., None] * h.double() + torch.sigmoid(expand(b)) * v
+    r2 = gate * r.double()
+    want = (h2 + r2[..., None] * cp.double()) * expand(c) + v
+    done = (pos == 15)[:, None]
+    # fp32 sums of K products of about unit total: K roundings of 2^-24 at most, and the hardware's exp and reciprocal
+    tol = K * 2.0 ** -24 + 1e-5
+    assert_close(f64(out), want.reshape(B, K).numpy(), 2.0 ** -8, 2.0 ** -8, "out")
+    assert_close(f64(dev[0]), torch.where(done[..., None], 0.0, h2).numpy(), tol, tol, "h")
+    assert_close(f64(dev[1]), torch.where(done, 1.0, r2).numpy(), tol, tol, "r")
+    assert_close(f64(dev[2]), torch.where(done[..., None], h2, cp.double()).numpy(), tol, tol, "c_prev")
+    assert dev[3].tolist() == ((pos + 1) % 16).tolist()
+
+
+def test_hooked_projections_are_called_and_give_the_same_step():
+    from spear_amd.nn.phalanx.inference import PhalanxStepState, phalanx_step
+
+    layer = _layer(dim=256, seed=6)
+    x = torch.randn(5, 256, generator=torch.Generator().manual_seed(8)).bfloat16().to(DEV)
+    one, two = PhalanxStepState.zeros(5, 16, DEV), PhalanxStepState.zeros(5, 16, DEV)
+    y = phalanx_step(layer, x, one)
+    calls = []
+    handle = layer.param.proj_b.register_forward_hook(lambda *a: calls.append(1))
+    y_hooked = phalanx_step(layer, x, two)
+    handle.remove()
+    assert calls == [1]
+    assert_close(f64(y), f64(y_hooked), 2e-2, 2e-2, "y")
+    assert_close(f64(one.h_loc), f64(two.h_loc), 2e-2, 2e-2, "h")
