@@ -27,6 +27,12 @@ int spear_layer_token(const void* x, long long ldx, const void* w_a, const void*
                       const void* w_c, const void* b_c, const void* w_v, void* out, float* h, float* r, float* c_prev, int* pos,
                       int block_len, int B, int K, int H, int kv_heads, void* stream);
 
+/* Column sums of n (1 .. 5) dense fp32 arrays, rounded to `dtype` (16-bit), in one launch:
+ *     out[i][c] = sum over r of in[i][r * cols[i] + c]
+ * in[i] 16-byte and out[i] 8-byte aligned. An array without rows gives zeros. */
+int spear_layer_sums(int n, const float* const* in, void* const* out, const long long* rows, const long long* cols, int dtype,
+                     void* stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -64,7 +64,7 @@ int check_common(const char* who, int B, int H, int L, int k, int in_dtype, int 
 
 extern "C" {
 
-int spear_btp_abi_version(void) { return 20; }
+int spear_btp_abi_version(void) { return 21; }
 
 const char* spear_btp_last_error(void) { return g_error; }
 
@@ -245,6 +245,28 @@ int spear_layer_token(const void* x, long long ldx, const void* w_a, const void*
   spear_btp::LayerTokenArgs a{u(x), (long)ldx, u(w_a), u(b_a), u(w_b), u(b_b), u(w_c), u(b_c), u(w_v), static_cast<uint16_t*>(out),
                               h, r, c_prev, pos, block_len, B, K, H, H / kv_heads};
   const hipError_t err = spear_btp::layer_token(a, static_cast<hipStream_t>(stream));
+  if (err != hipSuccess) return fail(SPEAR_BTP_ELAUNCH, "%s: launch failed: %s", who, hipGetErrorString(err));
+  return 0;
+}
+
+int spear_layer_sums(int n, const float* const* in, void* const* out, const long long* rows, const long long* cols, int dtype,
+                     void* stream) {
+  g_error[0] = '\0';
+  const char* who = "spear_layer_sums";
+  if (n < 1 || n > spear_btp::kLayerSumJobs) return fail(SPEAR_BTP_EINVAL, "%s: 1 to %d arrays (got %d)", who, spear_btp::kLayerSumJobs, n);
+  if (dtype != SPEAR_BTP_BF16 && dtype != SPEAR_BTP_F16) return fail(SPEAR_BTP_EINVAL, "%s: results must be float16 or bfloat16.", who);
+  if (!in || !out || !rows || !cols) return fail(SPEAR_BTP_ENULL, "%s: NULL array", who);
+  spear_btp::LayerSumJob jobs[spear_btp::kLayerSumJobs];
+  for (int i = 0; i < n; ++i) {
+    if (rows[i] < 0 || cols[i] < 0 || rows[i] >= (1ll << 40) || cols[i] >= (1ll << 40))
+      return fail(SPEAR_BTP_EINVAL, "%s: bad shape [%lld, %lld]", who, rows[i], cols[i]);
+    if (cols[i] != 0 && (!out[i] || (rows[i] != 0 && !in[i]))) return fail(SPEAR_BTP_ENULL, "%s: NULL tensor pointer", who);
+    if (!aligned16(in[i]) || (reinterpret_cast<uintptr_t>(out[i]) & 7u))
+      return fail(SPEAR_BTP_EINVAL, "%s: arrays must be 16-byte, results 8-byte aligned", who);
+    jobs[i] = {in[i], static_cast<uint16_t*>(out[i]), (long)rows[i], (long)cols[i]};
+  }
+  if (spear_btp::layer_sums_blocks(jobs, n) >= (1ll << 31)) return fail(SPEAR_BTP_EINVAL, "%s: too many columns for one launch", who);
+  const hipError_t err = spear_btp::layer_sums(jobs, n, dtype, static_cast<hipStream_t>(stream));
   if (err != hipSuccess) return fail(SPEAR_BTP_ELAUNCH, "%s: launch failed: %s", who, hipGetErrorString(err));
   return 0;
 }

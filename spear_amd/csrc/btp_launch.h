@@ -117,6 +117,16 @@ struct LayerTokenArgs {
 };
 hipError_t layer_token(const LayerTokenArgs& p, hipStream_t s);
 
+// out[c] <- sum over the rows of in[rows, cols] (dense fp32), rounded to 16 bits (layer_grad.hip)
+struct LayerSumJob {
+  const float* in;
+  uint16_t* out;
+  long rows, cols;
+};
+constexpr int kLayerSumJobs = 5;  // the most jobs of one launch
+hipError_t layer_sums(const LayerSumJob* jobs, int n, int dtype, hipStream_t s);
+long layer_sums_blocks(const LayerSumJob* jobs, int n);
+
 // Streaming form (btp_jagged.hip). Tensors [B, H, D, L] / [B, H, L]; state vectors [B, H, D] / [B, H].
 struct JagPrefillArgs {
   const void *a, *x, *c, *v;  // c and v both null: no "* C + V" epilogue

@@ -396,6 +396,27 @@ std::vector<at::Tensor> mix_prefill(const at::Tensor& a_logit, const at::Tensor&
   return {out, h, r, c_prev, pos};
 }
 
+// out[i] <- column sums of the dense fp32 matrix in[i], rounded to out[i]'s 16-bit type: one launch for all.
+void layer_sums(const std::vector<at::Tensor>& in, const std::vector<at::Tensor>& out) {
+  TORCH_CHECK(in.size() == out.size() && !in.empty() && in.size() <= 5, "1 to 5 matrices with a result each.");
+  const float* src[5];
+  void* dst[5];
+  long long rows[5], cols[5];
+  for (size_t i = 0; i < in.size(); ++i) {
+    TORCH_CHECK(in[i].is_cuda() && out[i].is_cuda() && in[i].dim() == 2 && in[i].scalar_type() == at::kFloat, "matrices must be float32 CUDA tensors.");
+    TORCH_CHECK(is_16bit(out[i]) && out[i].scalar_type() == out[0].scalar_type(), "results must be float16 or bfloat16, all of one type.");
+    TORCH_CHECK(in[i].is_contiguous() && out[i].is_contiguous() && out[i].numel() == in[i].size(1), "matrices and results must be dense, one result per column.");
+    check_same_device({&in[0], &in[i], &out[i]});
+    src[i] = static_cast<const float*>(in[i].data_ptr());
+    dst[i] = out[i].data_ptr();
+    rows[i] = in[i].size(0);
+    cols[i] = in[i].size(1);
+  }
+  const c10::DeviceGuard guard(in[0].device());
+  const int rc = spear_layer_sums((int)in.size(), src, dst, rows, cols, tag_of(out[0].scalar_type()), stream_of(in[0]));
+  if (rc != 0) raise_native(rc);
+}
+
 // One token through the layer's input projections and the step of its mixing stage (the caller applies proj_out): x [B, K]
 // bf16 with unit column stride, weights and biases of the four projections, the state updated in place.
 at::Tensor layer_token(const at::Tensor& x, const at::Tensor& w_a, const at::Tensor& b_a, const at::Tensor& w_b, const at::Tensor& b_b,
@@ -456,6 +477,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         "out = phalanx_mix(...) (or the q/k/v/gate form) with its autograd node (contiguous plain tensors)");
   m.def("mix_prefill", &mix_prefill, py::arg("a_logit"), py::arg("b_logit"), py::arg("c"), py::arg("v"), py::arg("heads"),
         py::arg("kv_heads"), "[out, h, r, c_prev, pos]: a prompt of any length through the mixing stage, with the state after it");
+  m.def("layer_sums", &layer_sums, py::arg("matrices"), py::arg("results"), "column sums of fp32 matrices, rounded to 16 bits");
   m.def("layer_token", &layer_token, py::arg("x"), py::arg("w_a"), py::arg("b_a"), py::arg("w_b"), py::arg("b_b"), py::arg("w_c"),
         py::arg("b_c"), py::arg("w_v"), py::arg("h"), py::arg("r"), py::arg("c_prev"), py::arg("pos"), py::arg("block_len"),
         py::arg("heads"), py::arg("kv_heads"), "one token through the input projections and the step of the mixing stage");

@@ -1,0 +1,114 @@
+// The small passes around the matrix products of a Phalanx layer's backward on gfx950 (MI355X).
+//
+// layer_sums: column sums of several fp32 arrays, rounded to 16 bits, in one launch. They are the weight gradients' partial
+// products (one per slice of the token axis: few rows, millions of columns) and the bias gradients' partial sums (one per
+// 64 time steps of a batch row: thousands of rows, a few hundred columns). Both are bound by reading the fp32 array once. As
+// library reductions and conversions they were ten launches: at B=1024 L=128 dim=512 101 us of GPU time for 123 MB, most of it in
+// the tall arrays and in passes over results that had just been written; here 37 us.
+//
+// A block of 512 threads takes either 2048 columns, four to a thread, and walks the rows with eight 16-byte loads in flight
+// (few rows), or 16 columns with 32 threads to a column that add up through LDS (many rows: 2048 rows by 512 columns
+// still make 32 blocks). Sums are taken in an order that depends on the shape only: the same bits in every run.
+#include <hip/hip_runtime.h>
+#include <stdint.h>
+
+#include "btp_device.h"
+#include "btp_launch.h"
+
+namespace spear_btp {
+
+namespace {
+
+constexpr int kThreads = 512;
+constexpr int kFlatColumns = 4 * kThreads;
+constexpr int kTallColumns = 16, kTallLanes = kThreads / kTallColumns;
+
+// Four columns to a thread need rows that start on 16 bytes and enough columns to fill the chip; with 64 rows or fewer the
+// weight gradients' arrays all have them. Narrow ones go the tall way at any number of rows.
+__host__ __device__ inline bool is_flat(const LayerSumJob& j) { return j.cols % 4 == 0 && j.rows <= 64; }
+
+inline long job_blocks(const LayerSumJob& j) {
+  return is_flat(j) ? (j.cols + kFlatColumns - 1) / kFlatColumns : (j.cols + kTallColumns - 1) / kTallColumns;
+}
+
+struct Jobs {
+  LayerSumJob job[kLayerSumJobs];
+  long first_block[kLayerSumJobs + 1];
+};
+
+template <class E>
+__global__ __launch_bounds__(kThreads) void layer_sums_kernel(const Jobs jobs, int n) {
+  __shared__ float part[kTallLanes][kTallColumns];
+  int at = 0;
+  while (at + 1 < n && (long)blockIdx.x >= jobs.first_block[at + 1]) ++at;
+  const LayerSumJob j = jobs.job[at];
+  const long block = (long)blockIdx.x - jobs.first_block[at];
+  if (is_flat(j)) {
+    const long col = block * kFlatColumns + 4 * (long)threadIdx.x;
+    if (col >= j.cols) return;
+    const float* p = j.in + col;
+    float4 sum = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    int row = 0;
+    for (; row + 8 <= j.rows; row += 8) {
+      float4 q[8];
+#pragma unroll
+      for (int i = 0; i < 8; ++i) q[i] = *reinterpret_cast<const float4*>(p + (long)(row + i) * j.cols);
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        sum.x += q[i].x; sum.y += q[i].y; sum.z += q[i].z; sum.w += q[i].w;
+      }
+    }
+    for (; row < j.rows; ++row) {
+      const float4 q = *reinterpret_cast<const float4*>(p + (long)row * j.cols);
+      sum.x += q.x; sum.y += q.y; sum.z += q.z; sum.w += q.w;
+    }
+    *reinterpret_cast<uint2*>(j.out + col) = make_uint2(E::pack2(sum.x, sum.y), E::pack2(sum.z, sum.w));
+    return;
+  }
+  const int lane = threadIdx.x / kTallColumns, c = threadIdx.x % kTallColumns;
+  const long col = block * kTallColumns + c;
+  float sum = 0.0f;
+  if (col < j.cols) {
+    const float* p = j.in + col;
+    long row = lane;
+    for (; row + 7 * kTallLanes < j.rows; row += 8 * kTallLanes) {
+      float q[8];
+#pragma unroll
+      for (int i = 0; i < 8; ++i) q[i] = p[(row + i * kTallLanes) * j.cols];
+#pragma unroll
+      for (int i = 0; i < 8; ++i) sum += q[i];
+    }
+    for (; row < j.rows; row += kTallLanes) sum += p[row * j.cols];
+  }
+  part[lane][c] = sum;
+  __syncthreads();
+  if (lane == 0 && col < j.cols) {
+    for (int i = 1; i < kTallLanes; ++i) sum += part[i][c];
+    j.out[col] = (uint16_t)E::pack2(sum, 0.0f);
+  }
+}
+
+}  // namespace
+
+long layer_sums_blocks(const LayerSumJob* jobs, int n) {
+  long blocks = 0;
+  for (int i = 0; i < n; ++i) blocks += job_blocks(jobs[i]);
+  return blocks;
+}
+
+hipError_t layer_sums(const LayerSumJob* jobs, int n, int dtype, hipStream_t s) {
+  Jobs all{};
+  long blocks = 0;
+  for (int i = 0; i < n; ++i) {
+    all.job[i] = jobs[i];
+    all.first_block[i] = blocks;
+    blocks += job_blocks(jobs[i]);
+  }
+  all.first_block[n] = blocks;
+  if (blocks == 0) return hipSuccess;
+  if (dtype == kBf16) hipLaunchKernelGGL(layer_sums_kernel<Bf16>, dim3((unsigned)blocks), dim3(kThreads), 0, s, all, n);
+  else hipLaunchKernelGGL(layer_sums_kernel<Fp16>, dim3((unsigned)blocks), dim3(kThreads), 0, s, all, n);
+  return hipGetLastError();
+}
+
+}  // namespace spear_btp

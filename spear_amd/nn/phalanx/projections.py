@@ -25,6 +25,8 @@ from __future__ import annotations
 import torch
 import torch.nn.functional as F
 
+from spear_amd import _btp
+
 __all__ = ["weight_grad", "input_projections", "linear", "pays_off", "project_and_mix", "packed_columns"]
 
 _TILE = 128           # output tile edge the slice count is sized against
@@ -58,7 +60,10 @@ def weight_grad(dy: torch.Tensor, x: torch.Tensor) -> torch.Tensor:
         return dy.t() @ x
     dy3 = dy.contiguous().view(s, M // s, N)
     x3 = x.contiguous().view(s, M // s, K)
-    return torch.bmm(dy3.transpose(1, 2), x3, out_dtype=torch.float32).sum(0).to(dy.dtype)
+    parts = torch.bmm(dy3.transpose(1, 2), x3, out_dtype=torch.float32)
+    out = dy.new_empty((N, K))
+    _btp.load_extension().layer_sums([parts.view(s, N * K)], [out])
+    return out
 
 
 @weight_grad.register_fake
@@ -127,8 +132,6 @@ def _mix_backward_packed(
     """Backward of the fused mixing stage with its four gradients written side by side into one
     ``[B, L, ld]`` buffer (``packed_columns``; padding columns zero), and the sums over all tokens of the
     ``a``, ``b`` and ``c`` blocks: ``(packed, da.sum, db.sum, dc.sum)``."""
-    from spear_amd import _btp
-
     B, L, _ = v.shape
     cols, ld = packed_columns(heads, kv_heads)
     packed = torch.empty((B, L, ld), device=v.device, dtype=v.dtype)
@@ -139,7 +142,9 @@ def _mix_backward_packed(
     rows = _btp.mix_backward_sum_rows(B, L, heads)
     sums = [torch.empty((rows, t.shape[-1]), device=v.device, dtype=torch.float32) for t in (a_logits, b_logits, c)]
     _btp.mix_backward(a_logits, b_logits, c, v, dout, da, db, dc, dv, heads, kv_heads, sums=tuple(sums))
-    return (packed, *(s.sum(0).to(v.dtype) for s in sums))
+    biases = [v.new_empty(s.shape[1]) for s in sums]
+    _btp.load_extension().layer_sums(sums, biases)
+    return (packed, *biases)
 
 
 @_mix_backward_packed.register_fake

@@ -114,3 +114,23 @@ def test_project_and_mix_matches_the_mixing_op_on_linear_autograd(B, L, dim, hea
         scale = ref.abs().max().item()
         # bf16 results of fp32-accumulated sums; the bias sums are taken before the gradients' rounding
         assert (got - ref).abs().max().item() <= 2 ** -6 * scale, (name, (got - ref).abs().max().item() / scale)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "f16"])
+def test_column_sums_of_every_kind_of_array_in_one_launch(dtype):
+    """Few rows and many columns (four to a thread, with and without a full block and a full run of eight rows), many rows
+    and few columns, column counts that four does not divide, one row, none."""
+    from spear_amd import _btp
+
+    g = torch.Generator().manual_seed(5)
+    for shapes in (((64, 4100), (2048, 32), (300, 513), (1, 7), (0, 20)), ((13, 2048),), ((65, 16), (7, 8196), (33, 1))):
+        mats = [torch.randn(*s, generator=g) for s in shapes]
+        outs = [torch.full((s[1],), float("nan"), device="cuda:0", dtype=dtype) for s in shapes]
+        print(f"column sums {shapes} {dtype}", flush=True)
+        _btp.load_extension().layer_sums([m.to("cuda:0") for m in mats], outs)
+        for m, out in zip(mats, outs):
+            want = m.double().sum(0)
+            # one rounding of the result and at most `rows` fp32 additions of partial sums below sum |m|
+            bound = torch.finfo(dtype).eps / 2 * want.abs() + m.shape[0] * 2.0 ** -24 * m.double().abs().sum(0) + 1e-7
+            assert ((out.cpu().double() - want).abs() <= bound).all(), m.shape
