@@ -33,6 +33,12 @@ int spear_layer_token(const void* x, long long ldx, const void* w_a, const void*
 int spear_layer_sums(int n, const float* const* in, void* const* out, const long long* rows, const long long* cols, int dtype,
                      void* stream);
 
+/* The four projections' weights one under the other in the order b, c, v, a, and the padding of the gradient buffer they meet:
+ *     stacked [ld, K]: w_b [Fkv, K], w_c [Fkv, K], w_v [F, K], w_a [H, K], zero rows       packed [M, ld]: columns 2 Fkv + F + H .. ld <- 0
+ * 16-bit elements, dense, 16-byte aligned; ld and K multiples of 8. */
+int spear_layer_stack(const void* w_a, const void* w_b, const void* w_c, const void* w_v, void* stacked, void* packed, long long M,
+                      int ld, int K, int H, int Fkv, int F, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

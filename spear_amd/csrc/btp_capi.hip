@@ -64,7 +64,7 @@ int check_common(const char* who, int B, int H, int L, int k, int in_dtype, int 
 
 extern "C" {
 
-int spear_btp_abi_version(void) { return 21; }
+int spear_btp_abi_version(void) { return 22; }
 
 const char* spear_btp_last_error(void) { return g_error; }
 
@@ -245,6 +245,25 @@ int spear_layer_token(const void* x, long long ldx, const void* w_a, const void*
   spear_btp::LayerTokenArgs a{u(x), (long)ldx, u(w_a), u(b_a), u(w_b), u(b_b), u(w_c), u(b_c), u(w_v), static_cast<uint16_t*>(out),
                               h, r, c_prev, pos, block_len, B, K, H, H / kv_heads};
   const hipError_t err = spear_btp::layer_token(a, static_cast<hipStream_t>(stream));
+  if (err != hipSuccess) return fail(SPEAR_BTP_ELAUNCH, "%s: launch failed: %s", who, hipGetErrorString(err));
+  return 0;
+}
+
+int spear_layer_stack(const void* w_a, const void* w_b, const void* w_c, const void* w_v, void* stacked, void* packed, long long M,
+                      int ld, int K, int H, int Fkv, int F, void* stream) {
+  g_error[0] = '\0';
+  const char* who = "spear_layer_stack";
+  if (M < 0 || H < 0 || Fkv < 0 || F < 0 || K <= 0 || K % 8 != 0 || ld <= 0 || ld % 8 != 0 || 2ll * Fkv + F + H > ld)
+    return fail(SPEAR_BTP_EINVAL, "%s: bad shape (M=%lld ld=%d K=%d H=%d Fkv=%d F=%d)", who, M, ld, K, H, Fkv, F);
+  if (M * ld >= (1ll << 41) || (long long)ld * K >= (1ll << 41)) return fail(SPEAR_BTP_EINVAL, "%s: tensor too large", who);
+  for (const void* q : {w_a, w_b, w_c, w_v, static_cast<const void*>(stacked), static_cast<const void*>(packed)}) {
+    if (!q) return fail(SPEAR_BTP_ENULL, "%s: NULL tensor pointer", who);
+    if (!aligned16(q)) return fail(SPEAR_BTP_EINVAL, "%s: tensor pointers must be 16-byte aligned", who);
+  }
+  auto u = [](const void* q) { return static_cast<const uint16_t*>(q); };
+  spear_btp::LayerStackArgs a{{u(w_b), u(w_c), u(w_v), u(w_a)}, {Fkv, Fkv, F, H}, static_cast<uint16_t*>(stacked),
+                              static_cast<uint16_t*>(packed), (long)M, 2 * Fkv + F + H, ld, K};
+  const hipError_t err = spear_btp::layer_stack(a, static_cast<hipStream_t>(stream));
   if (err != hipSuccess) return fail(SPEAR_BTP_ELAUNCH, "%s: launch failed: %s", who, hipGetErrorString(err));
   return 0;
 }

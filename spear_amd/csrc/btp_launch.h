@@ -123,6 +123,16 @@ struct LayerSumJob {
   uint16_t* out;
   long rows, cols;
 };
+// The weights of the projections stacked as [ld, K] (b, c, v, a, zero rows), and zeros into the columns used .. ld of packed [M, ld].
+struct LayerStackArgs {
+  const uint16_t* weight[4];
+  int rows[4];
+  uint16_t *stacked, *packed;
+  long M;
+  int used, ld, K;  // ld and K multiples of 8
+};
+hipError_t layer_stack(const LayerStackArgs& p, hipStream_t s);
+
 constexpr int kLayerSumJobs = 5;  // the most jobs of one launch
 hipError_t layer_sums(const LayerSumJob* jobs, int n, int dtype, hipStream_t s);
 long layer_sums_blocks(const LayerSumJob* jobs, int n);

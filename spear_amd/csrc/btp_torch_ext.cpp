@@ -11,6 +11,7 @@
 // the C ABI on torch's current stream of the tensors' device, without synchronising.
 #include <c10/core/DeviceGuard.h>
 #include <c10/hip/HIPStream.h>
+#include <torch/csrc/autograd/functions/basic_ops.h>
 #include <torch/extension.h>
 
 #include <string>
@@ -417,6 +418,121 @@ void layer_sums(const std::vector<at::Tensor>& in, const std::vector<at::Tensor>
   if (rc != 0) raise_native(rc);
 }
 
+// dy [M, N], x [M, K] -> dy^T x [N, K] in dy's type, fp32 sums. With s > 1 the token axis is cut into s slices multiplied as one
+// batched product with fp32 parts, which the caller adds with layer_sums (`parts`, `sums`).
+at::Tensor weight_grad(const at::Tensor& dy, const at::Tensor& x, int64_t s, std::vector<at::Tensor>& parts, std::vector<at::Tensor>& sums) {
+  const int64_t M = dy.size(0), N = dy.size(1), K = x.size(1);
+  if (s <= 1) return at::mm(dy.t(), x);
+  at::Tensor out = at::empty({N, K}, dy.options());
+  parts.push_back(at::bmm(dy.view({s, M / s, N}).transpose(1, 2), x.view({s, M / s, K}), at::kFloat).view({s, N * K}));
+  sums.push_back(out);
+  return out;
+}
+
+// A whole layer call on plain bf16 tensors: the four input projections, the mixing stage and the output projection, with one
+// autograd node. Backward is what spear_amd/nn/phalanx/projections.py does with _ProjectAndMix and _Linear (one product each for the
+// input and weight gradients of the four projections, against the packed gradient buffer), without Python frames and with
+// layer_stack and layer_sums around the products: 13 launches for forward and backward where separate modules had 23.
+// The library's products and the mixing kernels are the same.
+struct LayerNode : public torch::autograd::Function<LayerNode> {
+  static at::Tensor forward(torch::autograd::AutogradContext* ctx, const at::Tensor& x, const at::Tensor& w_a, const at::Tensor& b_a,
+                            const at::Tensor& w_b, const at::Tensor& b_b, const at::Tensor& w_c, const at::Tensor& b_c,
+                            const at::Tensor& w_v, const at::Tensor& w_out, int64_t heads, int64_t kv_heads, int64_t slices_in,
+                            int64_t slices_out) {
+    const at::Tensor a = at::linear(x, w_a, b_a), b = at::linear(x, w_b, b_b), c = at::linear(x, w_c, b_c), v = at::linear(x, w_v);
+    at::Tensor mixed = at::empty(v.sizes(), v.options());
+    mix_forward(a, b, c, v, mixed, heads, kv_heads, false);
+    at::Tensor y = at::linear(mixed, w_out);
+    if (ctx != nullptr) {
+      ctx->save_for_backward({x, w_a, w_b, w_c, w_v, w_out, a, b, c, v, mixed});
+      ctx->saved_data["heads"] = heads;
+      ctx->saved_data["kv_heads"] = kv_heads;
+      ctx->saved_data["slices_in"] = slices_in;
+      ctx->saved_data["slices_out"] = slices_out;
+    }
+    return y;
+  }
+
+  static torch::autograd::variable_list backward(torch::autograd::AutogradContext* ctx, torch::autograd::variable_list grad_outputs) {
+    const bool create_graph = at::GradMode::is_enabled();
+    const at::NoGradGuard no_grad;
+    const auto saved = ctx->get_saved_variables();
+    const at::Tensor &x = saved[0], &w_a = saved[1], &w_b = saved[2], &w_c = saved[3], &w_v = saved[4], &w_out = saved[5], &a = saved[6],
+                     &b = saved[7], &c = saved[8], &v = saved[9], &mixed = saved[10];
+    const int64_t heads = ctx->saved_data["heads"].toInt(), kv_heads = ctx->saved_data["kv_heads"].toInt();
+    const int64_t B = v.size(0), L = v.size(1), F = v.size(2), Fkv = b.size(2), M = B * L, K = x.size(2), dim = w_out.size(0);
+    const c10::DeviceGuard guard(v.device());
+    const at::Tensor dy = grad_outputs[0].contiguous().view({M, dim}), x2 = x.view({M, K}), mixed2 = mixed.view({M, F});
+    torch::autograd::variable_list out(13);  // forward's arguments, of which the first nine are tensors
+    std::vector<at::Tensor> parts, sums;
+    bool front = false, weights = false;
+    for (int i = 0; i < 8; ++i) {
+      front = front || ctx->needs_input_grad(i);
+      weights = weights || ((i == 1 || i == 3 || i == 5 || i == 7) && ctx->needs_input_grad(i));
+    }
+    if (ctx->needs_input_grad(8)) {
+      out[8] = weight_grad(dy, mixed2, ctx->saved_data["slices_out"].toInt(), parts, sums);
+      if (!parts.empty()) layer_sums(parts, sums);  // while the parts are in the memory-side cache
+      parts.clear();
+      sums.clear();
+    }
+    if (front) {
+      const at::Tensor dmixed = at::mm(dy, w_out).view({B, L, F});
+      const int64_t used = 2 * Fkv + F + heads, ld = (used + 63) / 64 * 64;  // [b | c | v | a | padding]
+      const at::Tensor packed = at::empty({B, L, ld}, v.options()), stacked = at::empty({ld, K}, v.options());
+      const int rc = spear_layer_stack(w_a.data_ptr(), w_b.data_ptr(), w_c.data_ptr(), w_v.data_ptr(), stacked.data_ptr(),
+                                       packed.data_ptr(), M, (int)ld, (int)K, (int)heads, (int)Fkv, (int)F, stream_of(v));
+      if (rc != 0) raise_native(rc);
+      const int64_t rows = spear_phalanx_mix_backward_sum_rows((int)B, (int)L, (int)heads);
+      const auto f32 = v.options().dtype(at::kFloat);
+      parts = {at::empty({rows, heads}, f32), at::empty({rows, Fkv}, f32), at::empty({rows, Fkv}, f32)};
+      mix_backward(a, b, c, v, dmixed, packed.narrow(2, 2 * Fkv + F, heads), packed.narrow(2, 0, Fkv), packed.narrow(2, Fkv, Fkv),
+                   packed.narrow(2, 2 * Fkv, F), heads, kv_heads, parts, false);
+      sums = {at::empty({heads}, v.options()), at::empty({Fkv}, v.options()), at::empty({Fkv}, v.options())};
+      out[2] = sums[0];
+      out[4] = sums[1];
+      out[6] = sums[2];
+      const at::Tensor d2 = packed.view({M, ld});
+      if (ctx->needs_input_grad(0)) out[0] = at::mm(d2, stacked).view(x.sizes());
+      if (weights) {
+        const at::Tensor dw = weight_grad(d2, x2, ctx->saved_data["slices_in"].toInt(), parts, sums);
+        out[3] = dw.narrow(0, 0, Fkv);
+        out[5] = dw.narrow(0, Fkv, Fkv);
+        out[7] = dw.narrow(0, 2 * Fkv, F);
+        out[1] = dw.narrow(0, 2 * Fkv + F, heads);
+      }
+      layer_sums(parts, sums);
+    }
+    if (!create_graph) return out;
+    // the mixing kernels have no second derivative: a second differentiation says so
+    torch::autograd::variable_list given;
+    std::vector<size_t> at_;
+    for (size_t i = 0; i < out.size(); ++i) {
+      if (!out[i].defined()) continue;
+      given.push_back(out[i].detach().requires_grad_(true));
+      at_.push_back(i);
+    }
+    const at::AutoGradMode grad(true);
+    const auto error = std::make_shared<torch::autograd::DelayedError>("the gradients of a Phalanx layer cannot be differentiated again", (int64_t)given.size());
+    given = error->apply(std::move(given));
+    for (size_t i = 0; i < at_.size(); ++i) out[at_[i]] = given[i];
+    return out;
+  }
+};
+
+// y = layer(x) for x [B, L, dim]; slices: into how many slices of tokens the weight gradients' products are cut.
+at::Tensor layer(const at::Tensor& x, const at::Tensor& w_a, const at::Tensor& b_a, const at::Tensor& w_b, const at::Tensor& b_b,
+                 const at::Tensor& w_c, const at::Tensor& b_c, const at::Tensor& w_v, const at::Tensor& w_out, int64_t heads,
+                 int64_t kv_heads, int64_t slices_in, int64_t slices_out) {
+  TORCH_CHECK(x.dim() == 3 && x.is_contiguous(), "x must be dense [B, L, dim].");
+  if (at::GradMode::is_enabled()) {
+    for (const at::Tensor* t : {&x, &w_a, &b_a, &w_b, &b_b, &w_c, &b_c, &w_v, &w_out})
+      if (t->requires_grad())
+        return LayerNode::apply(x, w_a, b_a, w_b, b_b, w_c, b_c, w_v, w_out, heads, kv_heads, slices_in, slices_out);
+  }
+  return LayerNode::forward(nullptr, x, w_a, b_a, w_b, b_b, w_c, b_c, w_v, w_out, heads, kv_heads, slices_in, slices_out);
+}
+
 // One token through the layer's input projections and the step of its mixing stage (the caller applies proj_out): x [B, K]
 // bf16 with unit column stride, weights and biases of the four projections, the state updated in place.
 at::Tensor layer_token(const at::Tensor& x, const at::Tensor& w_a, const at::Tensor& b_a, const at::Tensor& w_b, const at::Tensor& b_b,
@@ -477,6 +593,9 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         "out = phalanx_mix(...) (or the q/k/v/gate form) with its autograd node (contiguous plain tensors)");
   m.def("mix_prefill", &mix_prefill, py::arg("a_logit"), py::arg("b_logit"), py::arg("c"), py::arg("v"), py::arg("heads"),
         py::arg("kv_heads"), "[out, h, r, c_prev, pos]: a prompt of any length through the mixing stage, with the state after it");
+  m.def("layer", &layer, py::arg("x"), py::arg("w_a"), py::arg("b_a"), py::arg("w_b"), py::arg("b_b"), py::arg("w_c"), py::arg("b_c"),
+        py::arg("w_v"), py::arg("w_out"), py::arg("heads"), py::arg("kv_heads"), py::arg("slices_in"), py::arg("slices_out"),
+        "a whole layer call with its autograd node (plain bf16 tensors)");
   m.def("layer_sums", &layer_sums, py::arg("matrices"), py::arg("results"), "column sums of fp32 matrices, rounded to 16 bits");
   m.def("layer_token", &layer_token, py::arg("x"), py::arg("w_a"), py::arg("b_a"), py::arg("w_b"), py::arg("b_b"), py::arg("w_c"),
         py::arg("b_c"), py::arg("w_v"), py::arg("h"), py::arg("r"), py::arg("c_prev"), py::arg("pos"), py::arg("block_len"),

@@ -6,7 +6,11 @@
 // library reductions and conversions they were ten launches: at B=1024 L=128 dim=512 101 us of GPU time for 123 MB, most of it in
 // the tall arrays and in passes over results that had just been written; here 37 us.
 //
-// A block of 512 threads takes either 2048 columns, four to a thread, and walks the rows with eight 16-byte loads in flight
+// layer_stack: the projections' weights one under the other in the column order of the packed gradient buffer, zero rows for its
+// padding columns, and zeros in those columns: one launch where a concatenation and two fills were three (and a copy more where a
+// weight's type or layout had to be changed). Bound by the launch at small sizes, by writing [ld, K] else.
+//
+// A block of layer_sums, 512 threads, takes either 2048 columns, four to a thread, and walks the rows with eight 16-byte loads in flight
 // (few rows), or 16 columns with 32 threads to a column that add up through LDS (many rows: 2048 rows by 512 columns
 // still make 32 blocks). Sums are taken in an order that depends on the shape only: the same bits in every run.
 #include <hip/hip_runtime.h>
@@ -88,7 +92,46 @@ __global__ __launch_bounds__(kThreads) void layer_sums_kernel(const Jobs jobs, i
   }
 }
 
+// One 16-byte piece per thread: first the pieces of the stacked weights [ld, K], then those of the buffer's rows that reach
+// past the last used column. Only columns from `used` on are written there.
+__global__ __launch_bounds__(256) void layer_stack_kernel(const LayerStackArgs p, long stack_pieces, long total) {
+  const long i = (long)blockIdx.x * 256 + threadIdx.x;
+  if (i >= total) return;
+  const uint4 zero = make_uint4(0, 0, 0, 0);
+  if (i < stack_pieces) {
+    const int per_row = p.K / 8;
+    long row = i / per_row;
+    const int piece = (int)(i - row * per_row);
+    uint4 q = zero;
+    for (int part = 0; part < 4; ++part) {
+      if (row < p.rows[part]) {
+        q = *reinterpret_cast<const uint4*>(p.weight[part] + row * p.K + 8 * piece);
+        break;
+      }
+      row -= p.rows[part];
+    }
+    *reinterpret_cast<uint4*>(p.stacked + i * 8) = q;
+    return;
+  }
+  const int first = p.used / 8, per_row = p.ld / 8 - first;
+  const long j = i - stack_pieces, row = j / per_row;
+  const int col = 8 * (first + (int)(j - row * per_row));
+  uint16_t* at = p.packed + row * p.ld + col;
+  if (col >= p.used) {
+    *reinterpret_cast<uint4*>(at) = zero;
+  } else {
+    for (int e = p.used - col; e < 8; ++e) at[e] = 0;
+  }
+}
+
 }  // namespace
+
+hipError_t layer_stack(const LayerStackArgs& p, hipStream_t s) {
+  const long stack_pieces = (long)p.ld * (p.K / 8), total = stack_pieces + (p.used < p.ld ? p.M * (p.ld / 8 - p.used / 8) : 0);
+  if (total == 0) return hipSuccess;
+  hipLaunchKernelGGL(layer_stack_kernel, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, s, p, stack_pieces, total);
+  return hipGetLastError();
+}
 
 long layer_sums_blocks(const LayerSumJob* jobs, int n) {
   long blocks = 0;

@@ -42,10 +42,10 @@ from __future__ import annotations
 from dataclasses import dataclass
 
 import torch
-import torch.nn.modules.module as _nn_module
 
 from spear_amd import _btp
-from spear_amd.ops.btp.interface import _plain_eager
+
+from .projections import plain_operands
 
 __all__ = [
     "jagged_band_infer_sequential",
@@ -311,31 +311,16 @@ class PhalanxStepState:
 
 def _token_operands(layer, x: torch.Tensor):
     """Weights and biases for the kernel that runs the input projections and the step in one launch, or None where the
-    call is for the general path: other types than bf16, replaced or hooked projections, autocast, traced or transformed
-    calls, weights that the kernel's 16-byte accesses do not fit, and sizes from which the library's products are
-    faster (on the GPU alone: B=1024 with 64 heads 33.7 against 43.0 us, 700 with 100 heads 61 against 52)."""
+    call is for the general path: what ``plain_operands`` leaves to the modules, rows that 16-byte accesses do not fit, and sizes
+    from which the library's products are faster (on the GPU alone: B=1024 with 64 heads 33.7 against 43.0 us, 700 with
+    100 heads 61 against 52)."""
     if x.dim() != 2 or x.shape[0] == 0 or x.stride(1) != 1 or x.stride(0) % 8 != 0 or x.data_ptr() % 16 != 0:
         return None
+    p = layer.param
     if x.shape[0] * layer.heads * x.shape[1] > 1 << 26:
         return None
-    p = layer.param
-    ops = []
-    for proj, bias in ((p.proj_a, True), (p.proj_b, True), (p.proj_c, True), (p.proj_v, False)):
-        if type(proj) is not torch.nn.Linear or proj._forward_hooks or proj._forward_pre_hooks or "forward" in proj.__dict__:
-            return None
-        w, b = proj._parameters.get("weight"), proj._parameters.get("bias")
-        if w is None or (b is None) == bias or w.shape[1] != x.shape[1] or not w.is_contiguous() or w.data_ptr() % 16 != 0:
-            return None
-        ops.append(w)
-        if bias:
-            if not b.is_contiguous() or b.data_ptr() % 8 != 0:
-                return None
-            ops.append(b)
-    if any(t.dtype != torch.bfloat16 or t.device != x.device for t in (x, *ops)):
-        return None
-    if _nn_module._global_forward_hooks or _nn_module._global_forward_pre_hooks or torch.is_autocast_enabled("cuda"):
-        return None
-    return ops if _plain_eager(x, *ops) else None
+    ops = plain_operands(x, (p.proj_a, True), (p.proj_b, True), (p.proj_c, True), (p.proj_v, False))
+    return ops if ops is not None and ops[-1].shape == (layer.heads * 16, x.shape[1]) else None
 
 
 @torch.no_grad()

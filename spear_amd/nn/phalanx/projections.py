@@ -13,8 +13,9 @@ projection, so input and weight gradients are one GEMM each against the stacked 
 four GEMMs, which measured faster than one wide one); and the kernel leaves the column sums of the gate
 gradients (the three bias gradients) per tile of 64 time steps, so they are not read again to be summed.
 
-Short token axes gain nothing (their step is bound by launch overhead, of which this path has more), so
-the layer uses these functions from 8192 tokens on (``pays_off``).
+Plain eager calls run all of this from one compiled autograd node at every size (``layer_call``). The Python functions are
+for the calls that it leaves: short token axes gain nothing there (their step is bound by launch overhead, of which these
+functions have more), so the layer uses them from 8192 tokens on (``pays_off``).
 
 Forward results are those of ``torch.nn.functional.linear``. Parameters stay in the layer's
 ``nn.Linear`` modules; these functions only take their tensors.
@@ -24,10 +25,11 @@ from __future__ import annotations
 
 import torch
 import torch.nn.functional as F
+import torch.nn.modules.module as _nn_module
 
 from spear_amd import _btp
 
-__all__ = ["weight_grad", "input_projections", "linear", "pays_off", "project_and_mix", "packed_columns"]
+__all__ = ["weight_grad", "input_projections", "linear", "pays_off", "project_and_mix", "packed_columns", "layer_call", "plain_operands"]
 
 _TILE = 128           # output tile edge the slice count is sized against
 _TARGET_TILES = 1024  # about four tiles per compute unit
@@ -204,6 +206,51 @@ class _ProjectAndMix(torch.autograd.Function):
 
         return (dx, rows_of("a", need[1]), s_a if need[2] else None, rows_of("b", need[3]), s_b if need[4] else None,
                 rows_of("c", need[5]), s_c if need[6] else None, rows_of("v", need[7]), None, None)
+
+
+def plain_operands(x: torch.Tensor, *linears) -> list[torch.Tensor] | None:
+    """Weights and biases of ``(module, has_bias)`` pairs for the compiled paths that take them as they lie, or None where
+    a call has to go through the modules: other types than bf16, replaced or hooked modules, autocast, traced or transformed
+    calls (``_plain_eager``), and layouts that 16-byte accesses do not fit."""
+    from spear_amd.ops.btp.interface import _plain_eager
+
+    ops = []
+    for proj, has_bias in linears:
+        if type(proj) is not torch.nn.Linear or proj._forward_hooks or proj._forward_pre_hooks or proj._backward_hooks \
+                or proj._backward_pre_hooks or "forward" in proj.__dict__:
+            return None
+        w, b = proj._parameters.get("weight"), proj._parameters.get("bias")
+        if w is None or (b is None) == has_bias or not w.is_contiguous() or w.data_ptr() % 16 != 0:
+            return None
+        ops.append(w)
+        if has_bias:
+            if not b.is_contiguous() or b.data_ptr() % 8 != 0:
+                return None
+            ops.append(b)
+    device = x.device
+    if x.dtype != torch.bfloat16 or any(t.dtype != torch.bfloat16 or t.device != device for t in ops):
+        return None
+    if _nn_module._has_any_global_hook() or torch.is_autocast_enabled("cuda") or not _plain_eager(x, *ops):
+        return None
+    return ops
+
+
+def layer_call(x: torch.Tensor, proj_a, proj_b, proj_c, proj_v, proj_out, heads: int, kv_heads: int) -> torch.Tensor | None:
+    """The whole layer on ``x[B, L, K]`` as one autograd node compiled into the binding (``LayerNode`` in
+    ``btp_torch_ext.cpp``), or None where the call is for the modules and the Python nodes of this file: what
+    ``plain_operands`` leaves to them, lengths and sizes that the mixing kernels refuse, and a row of gradients of 2 GiB.
+    Forward + backward, us, modules and Python nodes / compiled: B=8 L=128 dim=512 562 / 360, B=1024 1330 / 1307,
+    B=64 L=2048 dim=2048 8152 / 7992."""
+    if not x.is_cuda or x.dim() != 3 or x.numel() == 0 or x.shape[1] % 16 != 0:
+        return None
+    ld, K = packed_columns(heads, kv_heads)[1], x.shape[2]
+    if 2 * x.shape[1] * ld >= 1 << 31 or K % 8 != 0:
+        return None
+    operands = plain_operands(x, (proj_a, True), (proj_b, True), (proj_c, True), (proj_v, False), (proj_out, False))
+    if operands is None or operands[-2].shape != (heads * 16, K) or operands[-1].shape != (K, heads * 16):
+        return None
+    M = x.numel() // K
+    return _btp.load_extension().layer(x.contiguous(), *operands, heads, kv_heads, slice_count(M, ld, K), slice_count(M, K, heads * 16))
 
 
 def project_and_mix(x: torch.Tensor, proj_a, proj_b, proj_c, proj_v, heads: int, kv_heads: int) -> torch.Tensor:

@@ -36,7 +36,7 @@ import os
 import torch
 import torch.nn as nn
 
-from .projections import input_projections, linear, packed_columns, pays_off, project_and_mix
+from .projections import input_projections, layer_call, linear, pays_off, project_and_mix
 
 _HEAD_DIM = 16
 _METHODS = ("default", "pytorch", "pytorch_linspace", "fused")
@@ -223,48 +223,46 @@ class Phalanx(nn.Module):
         A, X, C, V = self.param.forward_axcv(x)
         return self._mix_and_project(self.pytorch_block_two_pass(A, X, self.block_size), C, V)
 
-    def _mixes_in_one_kernel(self, x: torch.Tensor) -> bool:
-        """Whether a ``"default"`` call runs gates, recurrence and ``* C + V`` in the fused kernels, on the projections'
-        own layout, instead of the stand-alone recurrence between about twenty elementwise and transposing passes.
-        Forward + backward, us, stand-alone / fused: B=1024 L=128 dim=512 4692 / 1373, B=8 822 / 562; no size was
-        found where the stand-alone kernels win. They keep every call that the fused ones would answer in
-        another way: k = 1, other types than bf16 throughout, autocast, anything that traces or transforms the call
-        (``_plain_eager``), the matrix-core and checkpoint-store switches, a replaced recurrence or class, empty inputs,
-        lengths and ``wpb`` that :func:`btp` refuses, and batch rows past the fused backward's 2 GiB."""
-        if torch.compiler.is_compiling():
-            return False
-        from spear_amd.ops.btp import btp, interface
+    def _as_one_node(self, x: torch.Tensor) -> torch.Tensor | None:
+        """A plain bf16 call as one compiled autograd node around the fused mixing kernels, or None where the call is for the
+        composition of modules below.
 
+        For ``"default"`` this takes the place of the stand-alone recurrence between about twenty elementwise and transposing
+        passes. Forward + backward, us, stand-alone / one node: B=1024 L=128 dim=512 4692 / 1307, B=8 822 / 360; no size was
+        found where the stand-alone kernels win. They keep every call that the fused ones would answer in another way:
+        k = 1, other types than bf16 throughout, autocast, anything that traces or transforms the call, hooked or replaced
+        projections (``plain_operands``), the matrix-core and checkpoint-store switches, a replaced recurrence or class, empty
+        inputs, lengths and ``wpb`` that :func:`btp` refuses, and batch rows past the fused backward's 2 GiB."""
         p = self.param
-        if not (x.is_cuda and x.dim() == 3 and x.numel() > 0 and self.k == 2 and self.wpb in interface.SUPPORTED_WPB):
-            return False
-        L, weights = x.shape[1], (p.proj_a.weight, p.proj_b.weight, p.proj_c.weight, p.proj_v.weight)
-        return (
-            L % interface.BLK == 0 and 2 * L * packed_columns(self.heads, self.kv_heads)[1] < 1 << 31
-            and interface._FORWARD_FLAGS == 0 and self.btp_module is btp
-            and type(self) is Phalanx and type(p) is SigmoidA and p.token_sliced_backward
-            and self.output_dtype == p.compute_dtype and all(w.dtype == p.compute_dtype for w in weights)
-            and not torch.is_autocast_enabled("cuda") and interface._plain_eager(x, *weights)
-        )
+        if torch.compiler.is_compiling() or type(self) is not Phalanx or type(p) is not SigmoidA or not p.token_sliced_backward:
+            return None
+        from spear_amd.ops.btp import btp, interface, phalanx_mix
+
+        if self._forward_fn == self._forward_default:
+            if not (self.btp_module is btp and self.k == 2 and self.wpb in interface.SUPPORTED_WPB
+                    and self.output_dtype == p.compute_dtype and interface._FORWARD_FLAGS == 0):
+                return None
+        elif self.mix_module is not phalanx_mix:
+            return None
+        return layer_call(x.to(p.compute_dtype), p.proj_a, p.proj_b, p.proj_c, p.proj_v, self.proj_out, self.heads, self.kv_heads)
 
     def _forward_default(self, x: torch.Tensor) -> torch.Tensor:
-        if self._mixes_in_one_kernel(x):
-            from spear_amd.ops.btp import phalanx_mix
-
-            return self._forward_on_projections(x, phalanx_mix)
+        y = self._as_one_node(x)
+        if y is not None:
+            return y
         A, X, C, V = self.param.forward_axcv(x)
         return self._mix_and_project(self.btp_module(A, X, self.k, self.wpb, self.output_dtype), C, V)
 
     def _forward_fused(self, x: torch.Tensor) -> torch.Tensor:
-        return self._forward_on_projections(x, self.mix_module)
-
-    def _forward_on_projections(self, x: torch.Tensor, mix) -> torch.Tensor:
+        y = self._as_one_node(x)
+        if y is not None:
+            return y
         p = self.param
         xc = x.to(p.compute_dtype)
         if xc.dim() == 3 and pays_off(xc):
             mixed = project_and_mix(xc, p.proj_a, p.proj_b, p.proj_c, p.proj_v, self.heads, self.kv_heads)
         else:
-            mixed = mix(*p.project(xc), self.heads, self.kv_heads)
+            mixed = self.mix_module(*p.project(xc), self.heads, self.kv_heads)
         return self._project_out(mixed)
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:

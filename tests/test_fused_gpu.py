@@ -311,12 +311,12 @@ def test_default_layer_mixes_in_the_fused_kernels(B, L, dim, kv_heads):
         y.backward(dy)
         return [y.detach(), xx.grad] + [p.grad for p in model.parameters()]
 
-    assert layer._mixes_in_one_kernel(x)
+    assert layer._as_one_node(x) is not None
     got = run(layer)
     for a, b in zip(got, run(fused)):
         assert torch.equal(a, b)
     layer.btp_module = lambda *args: btp(*args)  # a replaced recurrence is called: the stand-alone composition
-    assert not layer._mixes_in_one_kernel(x)
+    assert layer._as_one_node(x) is None
     for i, (a, b) in enumerate(zip(got, run(layer))):
         # each of the about ten roundings between input and gradient is 2^-9 relative; they are independent
         assert (a.float() - b.float()).norm() <= 2 ** -9 * 10 * b.float().norm(), i
@@ -328,12 +328,61 @@ def test_calls_that_stay_with_the_stand_alone_kernels():
     x = torch.randn(2, 32, 64, device=DEV).bfloat16()
     for kwargs, xx in ((dict(k=1), x), (dict(output_dtype=torch.float32), x), (dict(wpb=3), x), (dict(), x[:, :17]), (dict(), x[:0]),
                        (dict(), x[0])):
-        assert not Phalanx(dim=64, dtype=torch.bfloat16, **kwargs).to(DEV)._mixes_in_one_kernel(xx)
+        assert Phalanx(dim=64, dtype=torch.bfloat16, **kwargs).to(DEV)._as_one_node(xx) is None
     layer = Phalanx(dim=64, dtype=torch.bfloat16).to(DEV)
-    assert layer._mixes_in_one_kernel(x)
+    assert layer._as_one_node(x) is not None
     with torch.autocast("cuda", dtype=torch.bfloat16):
-        assert not layer._mixes_in_one_kernel(x)
+        assert layer._as_one_node(x) is None
     with torch.device(DEV):  # a function mode
-        assert not layer._mixes_in_one_kernel(x)
+        assert layer._as_one_node(x) is None
+    handle = layer.param.proj_c.register_forward_hook(lambda *a: None)
+    assert layer._as_one_node(x) is None
+    handle.remove()
     with pytest.raises(AssertionError, match="multiple"):
         layer(x[:, :17])
+
+
+@pytest.mark.parametrize("B,L,dim,kv_heads", [(2, 16, 16, 1), (3, 48, 80, None), (8, 128, 96, 2), (64, 128, 256, 4)])
+def test_layer_node_against_separate_modules(B, L, dim, kv_heads):
+    """Every gradient of the one-node layer against the modules' own autograd (a hook keeps them separate), for every subset of
+    frozen tensors that changes what backward computes; padding columns of the packed gradients at odd head counts included."""
+    from spear_amd import Phalanx
+
+    torch.manual_seed(21)
+    layer = Phalanx(dim=dim, length=L, method="fused", dtype=torch.bfloat16, kv_heads=kv_heads).to(DEV)
+    x = torch.randn(B, L, dim, generator=torch.Generator().manual_seed(22)).bfloat16().to(DEV)
+    dy = torch.randn(B, dim, L, generator=torch.Generator().manual_seed(23)).bfloat16().to(DEV).transpose(1, 2)  # not dense
+
+    def run():
+        layer.zero_grad()
+        xx = x.clone().requires_grad_(x_grad)
+        y = layer(xx)
+        y.backward(dy)
+        return {"y": y.detach(), "x": xx.grad, **{n: p.grad for n, p in layer.named_parameters()}}
+
+    names = [n for n, _ in layer.named_parameters()]
+    for x_grad, trained in ((True, names), (False, names), (True, []), (False, ["proj_out.weight"]), (False, ["param.proj_b.bias"]),
+                            (True, ["param.proj_a.weight"])):
+        for n, p in layer.named_parameters():
+            p.requires_grad_(n in trained)
+        got = run()
+        handle = layer.param.proj_a.register_forward_hook(lambda *a: None)
+        want = run()
+        handle.remove()
+        for n in want:
+            assert (got[n] is None) == (want[n] is None), n
+            if want[n] is not None:
+                # bf16 roundings of the modules' intermediate gradients, which the node does not make: fewer than ten of 2^-9
+                assert (got[n].float() - want[n].float()).norm() <= 10 * 2 ** -9 * want[n].float().norm() + 1e-6, (n, x_grad, trained)
+
+
+def test_layer_node_is_differentiable_once_and_says_so():
+    from spear_amd import Phalanx
+
+    layer = Phalanx(dim=64, dtype=torch.bfloat16).to(DEV)
+    x = torch.randn(2, 32, 64, device=DEV).bfloat16().requires_grad_(True)
+    plain, = torch.autograd.grad(layer(x).float().sum(), x)
+    again, = torch.autograd.grad(layer(x).float().sum(), x, create_graph=True)
+    assert torch.equal(plain, again.detach())
+    with pytest.raises(RuntimeError, match="differentiated again"):
+        again.float().square().sum().backward()
