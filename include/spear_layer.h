@@ -39,6 +39,11 @@ int spear_layer_sums(int n, const float* const* in, void* const* out, const long
 int spear_layer_stack(const void* w_a, const void* w_b, const void* w_c, const void* w_v, void* stacked, void* packed, long long M,
                       int ld, int K, int H, int Fkv, int F, void* stream);
 
+/* n (1 .. 4) linear layers on the same rows, bf16 with fp32 sums:  out[i] [M, N[i]] = x [M, K] w[i]^T + bias[i] (null: none). x has
+ * rows ldx elements apart, the rest is dense; K and ldx multiples of 8; x and w 16-byte, out 8-byte, bias 2-byte aligned. */
+int spear_layer_linear(int n, const void* x, long long ldx, int M, int K, const void* const* w, const void* const* bias,
+                       void* const* out, const int* N, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

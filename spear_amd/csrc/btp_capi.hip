@@ -64,7 +64,7 @@ int check_common(const char* who, int B, int H, int L, int k, int in_dtype, int 
 
 extern "C" {
 
-int spear_btp_abi_version(void) { return 22; }
+int spear_btp_abi_version(void) { return 23; }
 
 const char* spear_btp_last_error(void) { return g_error; }
 
@@ -264,6 +264,35 @@ int spear_layer_stack(const void* w_a, const void* w_b, const void* w_c, const v
   spear_btp::LayerStackArgs a{{u(w_b), u(w_c), u(w_v), u(w_a)}, {Fkv, Fkv, F, H}, static_cast<uint16_t*>(stacked),
                               static_cast<uint16_t*>(packed), (long)M, 2 * Fkv + F + H, ld, K};
   const hipError_t err = spear_btp::layer_stack(a, static_cast<hipStream_t>(stream));
+  if (err != hipSuccess) return fail(SPEAR_BTP_ELAUNCH, "%s: launch failed: %s", who, hipGetErrorString(err));
+  return 0;
+}
+
+int spear_layer_linear(int n, const void* x, long long ldx, int M, int K, const void* const* w, const void* const* bias,
+                       void* const* out, const int* N, void* stream) {
+  g_error[0] = '\0';
+  const char* who = "spear_layer_linear";
+  if (n < 1 || n > 4 || M < 0 || K <= 0 || K % 8 != 0 || ldx < K || ldx % 8 != 0)
+    return fail(SPEAR_BTP_EINVAL, "%s: bad shape (n=%d M=%d K=%d ldx=%lld)", who, n, M, K, ldx);
+  if (!w || !bias || !out || !N) return fail(SPEAR_BTP_ENULL, "%s: NULL array", who);
+  spear_btp::LayerLinearArgs a{static_cast<const uint16_t*>(x), (long)ldx, M, K, n, {}, {}, {}, {}};
+  long long groups = 0;
+  for (int i = 0; i < n; ++i) {
+    if (N[i] <= 0) return fail(SPEAR_BTP_EINVAL, "%s: a layer needs columns (got %d)", who, N[i]);
+    groups += (N[i] + 63ll) / 64;
+    if (!w[i] || !out[i]) return fail(SPEAR_BTP_ENULL, "%s: NULL tensor pointer", who);
+    if (!aligned16(w[i]) || (reinterpret_cast<uintptr_t>(out[i]) & 7u) || (reinterpret_cast<uintptr_t>(bias[i]) & 1u))
+      return fail(SPEAR_BTP_EINVAL, "%s: weights must be 16-byte, results 8-byte, biases 2-byte aligned", who);
+    a.w[i] = static_cast<const uint16_t*>(w[i]);
+    a.bias[i] = static_cast<const uint16_t*>(bias[i]);
+    a.out[i] = static_cast<uint16_t*>(out[i]);
+    a.N[i] = N[i];
+  }
+  if (groups * ((M + 15ll) / 16) >= (1ll << 31)) return fail(SPEAR_BTP_EINVAL, "%s: too many tiles for one launch", who);
+  if (M == 0) return 0;
+  if (!x) return fail(SPEAR_BTP_ENULL, "%s: NULL tensor pointer", who);
+  if (!aligned16(x)) return fail(SPEAR_BTP_EINVAL, "%s: x must be 16-byte aligned", who);
+  const hipError_t err = spear_btp::layer_linear(a, static_cast<hipStream_t>(stream));
   if (err != hipSuccess) return fail(SPEAR_BTP_ELAUNCH, "%s: launch failed: %s", who, hipGetErrorString(err));
   return 0;
 }

@@ -117,6 +117,18 @@ struct LayerTokenArgs {
 };
 hipError_t layer_token(const LayerTokenArgs& p, hipStream_t s);
 
+// Up to four linear layers on the same rows (layer_linear.hip), bf16: out[j] [M, N[j]] = x [M, K] w[j]^T + bias[j]; dense but for
+// x, whose rows are `ldx` elements apart; K and ldx multiples of 8. A null bias is none.
+struct LayerLinearArgs {
+  const uint16_t* x;
+  long ldx;
+  int M, K, jobs;
+  const uint16_t *w[4], *bias[4];
+  uint16_t* out[4];
+  int N[4];
+};
+hipError_t layer_linear(const LayerLinearArgs& p, hipStream_t s);
+
 // out[c] <- sum over the rows of in[rows, cols] (dense fp32), rounded to 16 bits (layer_grad.hip)
 struct LayerSumJob {
   const float* in;

@@ -418,6 +418,58 @@ void layer_sums(const std::vector<at::Tensor>& in, const std::vector<at::Tensor>
   if (rc != 0) raise_native(rc);
 }
 
+// x [M, K] through up to four linear layers in one launch (bf16; biases may be undefined): [M, N_i] each.
+std::vector<at::Tensor> linears(const at::Tensor& x, const std::vector<at::Tensor>& weights, const std::vector<at::Tensor>& biases) {
+  TORCH_CHECK(x.is_cuda() && x.dim() == 2 && x.stride(1) == 1 && x.scalar_type() == at::kBFloat16, "x must be [M, K] bfloat16 CUDA with dense rows.");
+  TORCH_CHECK(!weights.empty() && weights.size() <= 4 && biases.size() == weights.size(), "1 to 4 layers.");
+  const int64_t M = x.size(0), K = x.size(1);
+  const void *w[4], *b[4];
+  void* o[4];
+  int N[4];
+  std::vector<at::Tensor> out;
+  for (size_t i = 0; i < weights.size(); ++i) {
+    const int64_t n = weights[i].size(0);
+    check_layout("weight", weights[i], {n, K});
+    TORCH_CHECK(weights[i].scalar_type() == at::kBFloat16, "weights must be bfloat16.");
+    if (biases[i].defined()) {
+      check_layout("bias", biases[i], {n});
+      TORCH_CHECK(biases[i].scalar_type() == at::kBFloat16, "biases must be bfloat16.");
+    }
+    check_same_device({&x, &weights[i], &biases[i]});
+    out.push_back(at::empty({M, n}, x.options()));
+    w[i] = weights[i].data_ptr();
+    b[i] = biases[i].defined() ? biases[i].data_ptr() : nullptr;
+    o[i] = out[i].data_ptr();
+    N[i] = (int)n;
+  }
+  const c10::DeviceGuard guard(x.device());
+  const int rc = spear_layer_linear((int)weights.size(), x.data_ptr(), M > 1 ? x.stride(0) : K, (int)M, (int)K, w, b, o, N, stream_of(x));
+  if (rc != 0) raise_native(rc);
+  return out;
+}
+
+// The four input projections (a, b, c, v) of x [..., K], and one projection without bias: through the kernel above where it is
+// the faster one (the sizes measured at layer_linear.hip), through the library's products elsewhere. x dense.
+std::vector<at::Tensor> project(const at::Tensor& x, const std::vector<at::Tensor>& weights, const std::vector<at::Tensor>& biases) {
+  const int64_t K = x.size(-1), M = K > 0 ? x.numel() / K : 0;
+  int64_t columns = 0;
+  for (const at::Tensor& w : weights) columns += w.size(0);
+  const bool small = weights.size() > 1 ? M * columns * K <= 1600000000 : (K <= 512 && M * columns * K <= 300000000);
+  std::vector<at::Tensor> out;
+  const auto aligned = [](const at::Tensor& t) { return (reinterpret_cast<uintptr_t>(t.data_ptr()) & 15u) == 0; };
+  if (small && M > 0 && K % 8 == 0 && aligned(x)) {
+    out = linears(x.view({M, K}), weights, biases);
+    auto sizes = x.sizes().vec();
+    for (at::Tensor& t : out) {
+      sizes.back() = t.size(1);
+      t = t.view(sizes);
+    }
+  } else {
+    for (size_t i = 0; i < weights.size(); ++i) out.push_back(biases[i].defined() ? at::linear(x, weights[i], biases[i]) : at::linear(x, weights[i]));
+  }
+  return out;
+}
+
 // dy [M, N], x [M, K] -> dy^T x [N, K] in dy's type, fp32 sums. With s > 1 the token axis is cut into s slices multiplied as one
 // batched product with fp32 parts, which the caller adds with layer_sums (`parts`, `sums`).
 at::Tensor weight_grad(const at::Tensor& dy, const at::Tensor& x, int64_t s, std::vector<at::Tensor>& parts, std::vector<at::Tensor>& sums) {
@@ -432,17 +484,18 @@ at::Tensor weight_grad(const at::Tensor& dy, const at::Tensor& x, int64_t s, std
 // A whole layer call on plain bf16 tensors: the four input projections, the mixing stage and the output projection, with one
 // autograd node. Backward is what spear_amd/nn/phalanx/projections.py does with _ProjectAndMix and _Linear (one product each for the
 // input and weight gradients of the four projections, against the packed gradient buffer), without Python frames and with
-// layer_stack and layer_sums around the products: 13 launches for forward and backward where separate modules had 23.
-// The library's products and the mixing kernels are the same.
+// layer_stack and layer_sums around the products: 10 launches for forward and backward of a small layer where separate modules had 29.
+// The mixing kernels are the same; the input gradients and weight gradients are the library's products.
 struct LayerNode : public torch::autograd::Function<LayerNode> {
   static at::Tensor forward(torch::autograd::AutogradContext* ctx, const at::Tensor& x, const at::Tensor& w_a, const at::Tensor& b_a,
                             const at::Tensor& w_b, const at::Tensor& b_b, const at::Tensor& w_c, const at::Tensor& b_c,
                             const at::Tensor& w_v, const at::Tensor& w_out, int64_t heads, int64_t kv_heads, int64_t slices_in,
                             int64_t slices_out) {
-    const at::Tensor a = at::linear(x, w_a, b_a), b = at::linear(x, w_b, b_b), c = at::linear(x, w_c, b_c), v = at::linear(x, w_v);
+    const auto front = project(x, {w_a, w_b, w_c, w_v}, {b_a, b_b, b_c, at::Tensor()});
+    const at::Tensor &a = front[0], &b = front[1], &c = front[2], &v = front[3];
     at::Tensor mixed = at::empty(v.sizes(), v.options());
     mix_forward(a, b, c, v, mixed, heads, kv_heads, false);
-    at::Tensor y = at::linear(mixed, w_out);
+    at::Tensor y = project(mixed, {w_out}, {at::Tensor()})[0];
     if (ctx != nullptr) {
       ctx->save_for_backward({x, w_a, w_b, w_c, w_v, w_out, a, b, c, v, mixed});
       ctx->saved_data["heads"] = heads;
@@ -567,6 +620,24 @@ at::Tensor layer_token(const at::Tensor& x, const at::Tensor& w_a, const at::Ten
   return out;
 }
 
+// A prompt through a whole layer (plain bf16 tensors, x dense [B, L, dim], any L >= 1): [y, h, r, c_prev, pos].
+std::vector<at::Tensor> layer_prefill(const at::Tensor& x, const at::Tensor& w_a, const at::Tensor& b_a, const at::Tensor& w_b,
+                                      const at::Tensor& b_b, const at::Tensor& w_c, const at::Tensor& b_c, const at::Tensor& w_v,
+                                      const at::Tensor& w_out, int64_t heads, int64_t kv_heads) {
+  TORCH_CHECK(x.dim() == 3 && x.is_contiguous(), "x must be dense [B, L, dim].");
+  const auto front = project(x, {w_a, w_b, w_c, w_v}, {b_a, b_b, b_c, at::Tensor()});
+  auto out = mix_prefill(front[0], front[1], front[2], front[3], heads, kv_heads);
+  out[0] = project(out[0], {w_out}, {at::Tensor()})[0];
+  return out;
+}
+
+// One token through a whole layer: layer_token and the output projection.
+at::Tensor layer_step(const at::Tensor& x, const at::Tensor& w_a, const at::Tensor& b_a, const at::Tensor& w_b, const at::Tensor& b_b,
+                      const at::Tensor& w_c, const at::Tensor& b_c, const at::Tensor& w_v, const at::Tensor& w_out, at::Tensor h,
+                      at::Tensor r, at::Tensor c_prev, at::Tensor pos, int64_t block_len, int64_t heads, int64_t kv_heads) {
+  return project(layer_token(x, w_a, b_a, w_b, b_b, w_c, b_c, w_v, h, r, c_prev, pos, block_len, heads, kv_heads), {w_out}, {at::Tensor()})[0];
+}
+
 }  // namespace
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
@@ -596,6 +667,13 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("layer", &layer, py::arg("x"), py::arg("w_a"), py::arg("b_a"), py::arg("w_b"), py::arg("b_b"), py::arg("w_c"), py::arg("b_c"),
         py::arg("w_v"), py::arg("w_out"), py::arg("heads"), py::arg("kv_heads"), py::arg("slices_in"), py::arg("slices_out"),
         "a whole layer call with its autograd node (plain bf16 tensors)");
+  m.def("linears", [](const at::Tensor& x, const std::vector<at::Tensor>& w, const std::vector<std::optional<at::Tensor>>& b) {
+    std::vector<at::Tensor> biases;
+    for (const auto& t : b) biases.push_back(t.value_or(at::Tensor()));
+    return linears(x, w, biases);
+  }, py::arg("x"), py::arg("weights"), py::arg("biases"), "up to four linear layers on the same rows in one launch (bf16)");
+  m.def("layer_prefill", &layer_prefill, "[y, h, r, c_prev, pos]: a prompt through a whole layer (plain bf16 tensors)");
+  m.def("layer_step", &layer_step, "one token through a whole layer (plain bf16 tensors), the state updated in place");
   m.def("layer_sums", &layer_sums, py::arg("matrices"), py::arg("results"), "column sums of fp32 matrices, rounded to 16 bits");
   m.def("layer_token", &layer_token, py::arg("x"), py::arg("w_a"), py::arg("b_a"), py::arg("w_b"), py::arg("b_b"), py::arg("w_c"),
         py::arg("b_c"), py::arg("w_v"), py::arg("h"), py::arg("r"), py::arg("c_prev"), py::arg("pos"), py::arg("block_len"),

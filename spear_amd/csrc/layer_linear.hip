@@ -1,0 +1,85 @@
+// The layer's linear projections at sizes where launches count, on gfx950 (MI355X): up to four of them on the same rows in one
+// launch.
+//
+//     out_j[M, N_j] = x[M, K] w_j[N_j, K]^T + bias_j          bf16, fp32 sums, rounded once
+//
+// The four input projections of a thousand tokens are a GFLOP or two. The library serves them one by one, in 5 to 7 us each on
+// the GPU and about 15 us of host time per call, which is what such a layer is bound by. A workgroup makes 64 columns by 16 kNT
+// rows (layer_mfma.h: a quarter of K per wavefront), whatever array the columns belong to, so the narrow arrays share the chip with the
+// wide ones.
+//
+// The four input projections (dim, kv heads = heads) at M rows, us in a HIP graph, this kernel / the library's four: M=128 dim=256
+// 5.7 / 28.0, M=1024 dim=512 13.1 / 21.9, M=512 dim=1024 22.2 / 25.8, M=2048 dim=512 23.2 / 23.3 (1.64 G multiply-adds), M=1024
+// dim=768 25.3 / 24.0 (1.85 G), M=4096 dim=512 38.2 / 28.4: past about 1.6 G the library's larger tiles, which read x and the
+// weights less often, win. One projection (dim x dim): M=1024 dim=512 5.7 / 5.8 (0.27 G), M=2048 dim=512 7.6 / 6.2, M=16 dim=512
+// 4.8 / 3.8, M=128 dim=768 7.2 / 4.7: alone it is taken for the host time it saves, up to 0.3 G and K = 512.
+#include <hip/hip_runtime.h>
+#include <stdint.h>
+
+#include "btp_device.h"
+#include "btp_launch.h"
+#include "layer_mfma.h"
+
+namespace spear_btp {
+
+namespace {
+
+template <int kNT, int kChunk>
+__global__ __launch_bounds__(256) void layer_linear_kernel(const LayerLinearArgs p, int groups) {
+  __shared__ f32x4_t partial[kParts][4][kNT][64];
+  const int lane = threadIdx.x & 63, n = lane & 15, q = lane >> 4, wave = threadIdx.x >> 6;
+  int group = (int)(blockIdx.x % (unsigned)groups), j = 0;
+  const int first = (int)(blockIdx.x / (unsigned)groups) * 16 * kNT;
+  while (group >= (p.N[j] + 63) / 64) group -= (p.N[j++] + 63) / 64;
+  const int N = p.N[j], col = 64 * group, K = p.K;
+  const uint16_t *w[4], *x[kNT];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) w[i] = p.w[j] + (long)min(col + 16 * i + n, N - 1) * K;  // past the last row or column: read it, store nothing
+#pragma unroll
+  for (int t = 0; t < kNT; ++t) x[t] = p.x + (long)min(first + 16 * t + n, p.M - 1) * p.ldx;
+  f32x4_t acc[4][kNT], sum[4];
+  quarter_product<kNT, kChunk>(w, x, K, wave, q, acc);
+  add_quarters<kNT>(partial, acc, wave, lane, sum);
+  const int row = first + 16 * wave + n;
+  if (wave >= kNT || row >= p.M) return;
+  const uint16_t* bias = p.bias[j];
+  uint16_t* out = p.out[j] + (long)row * N;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int c = col + 16 * i + 4 * q;
+    float v[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[e] = sum[i][e] + (bias != nullptr && c + e < N ? Bf16::lo(bias[c + e]) : 0.0f);
+    const uint2 packed = make_uint2(Bf16::pack2(v[0], v[1]), Bf16::pack2(v[2], v[3]));
+    if (N % 4 == 0) {  // rows of the result start on 8 bytes and end with a whole piece
+      if (c < N) *reinterpret_cast<uint2*>(out + c) = packed;
+    } else {
+      if (c < N) out[c] = (uint16_t)packed.x;
+      if (c + 1 < N) out[c + 1] = (uint16_t)(packed.x >> 16);
+      if (c + 2 < N) out[c + 2] = (uint16_t)packed.y;
+      if (c + 3 < N) out[c + 3] = (uint16_t)(packed.y >> 16);
+    }
+  }
+}
+
+template <int kNT, int kChunk>
+void launch(const LayerLinearArgs& p, int groups, hipStream_t s) {
+  const long tiles = (p.M + 16 * kNT - 1) / (16 * kNT);
+  hipLaunchKernelGGL((layer_linear_kernel<kNT, kChunk>), dim3((unsigned)(groups * tiles)), dim3(256), 0, s, p, groups);
+}
+
+}  // namespace
+
+hipError_t layer_linear(const LayerLinearArgs& p, hipStream_t s) {
+  int groups = 0;
+  for (int j = 0; j < p.jobs; ++j) groups += (p.N[j] + 63) / 64;
+  if (groups == 0 || p.M == 0) return hipSuccess;
+  // as layer_token chooses: as many workgroups as there are while they are few
+  const long pairs = (long)groups * ((p.M + 15) / 16);
+  if (pairs <= 256) launch<1, 4>(p, groups, s);
+  else if (pairs <= 512) launch<2, 4>(p, groups, s);
+  else launch<4, 2>(p, groups, s);
+  return hipGetLastError();
+}
+
+}  // namespace spear_btp

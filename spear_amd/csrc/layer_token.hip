@@ -21,34 +21,20 @@
 // Measured in a HIP graph, us, this kernel / four library products and the step kernel: B=1 8 heads 5.5 / 23.8, B=1 128 heads
 // 10.8 / 30.1, B=256 32 heads 7.7 / 25.7, B=1024 32 heads 14.0 / 25.8 (1.7 GFLOP), B=1024 64 heads 33.7 / 43.0, 128 heads 111 / 64:
 // every workgroup reads its weights and tokens through L2 once, which the library's larger tiles do less often, so the caller
-// takes the library from B H K > 2^26 on. The whole step as a call at B=1024, 32 heads: 122 -> 37 us.
+// takes the library from B H K > 2^26 on. The whole step as a call at B=1024, 32 heads: 122 -> 23 us, with
+// the output projection in layer_linear.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
 #include "btp_device.h"
 #include "btp_launch.h"
+#include "layer_mfma.h"
 
 namespace spear_btp {
 
 namespace {
 
-typedef float f32x4_t __attribute__((ext_vector_type(4)));
-typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
-
-__device__ __forceinline__ f32x4_t mfma(uint4 a, uint4 b, f32x4_t acc) {
-  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, a), __builtin_bit_cast(bf16x8_t, b), acc, 0, 0, 0);
-}
-
 __device__ __forceinline__ float sigmoid(float z) { return __builtin_amdgcn_rcpf(1.0f + __expf(-z)); }
-
-constexpr int kStep = 32;  // columns of one matrix instruction
-constexpr int kParts = 4;  // wavefronts of a workgroup: quarters of the columns
-
-template <int kNT, int kChunk>
-struct Operands {
-  uint4 w[kChunk][4];  // v, b, c, a
-  uint4 x[kChunk][kNT];
-};
 
 template <int kNT, int kChunk>
 __global__ __launch_bounds__(256) void layer_token_kernel(const LayerTokenArgs p) {
@@ -61,49 +47,11 @@ __global__ __launch_bounds__(256) void layer_token_kernel(const LayerTokenArgs p
   const uint16_t* w[4] = {p.w_v + ((long)head * 16 + n) * K, p.w_b + ((long)kv * 16 + n) * K, p.w_c + ((long)kv * 16 + n) * K,
                           p.w_a + (long)head * K};
   const uint16_t* x[kNT];
-  f32x4_t acc[4][kNT];
 #pragma unroll
-  for (int t = 0; t < kNT; ++t) {
+  for (int t = 0; t < kNT; ++t)
     x[t] = p.x + (long)min(first + 16 * t + n, p.B - 1) * p.ldx;  // tokens past the batch read its last one and store nothing
-#pragma unroll
-    for (int i = 0; i < 4; ++i) acc[i][t] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
-  }
 
-  const int steps = (K + kStep - 1) / kStep, share = (steps + kParts - 1) / kParts;
-  const int from = wave * share, to = min(from + share, steps);
-  auto load = [&](Operands<kNT, kChunk>& o, int s0) {
-#pragma unroll
-    for (int s = 0; s < kChunk; ++s) {
-      const int k = min((s0 + s) * kStep + 8 * q, K - 8);  // K is a multiple of 8; what lies past it is replaced by zeros below
-#pragma unroll
-      for (int i = 0; i < 4; ++i) o.w[s][i] = *reinterpret_cast<const uint4*>(w[i] + k);
-#pragma unroll
-      for (int t = 0; t < kNT; ++t) o.x[s][t] = *reinterpret_cast<const uint4*>(x[t] + k);
-    }
-  };
-  auto multiply = [&](Operands<kNT, kChunk>& o, int s0) {
-#pragma unroll
-    for (int s = 0; s < kChunk; ++s) {
-      const int k = (s0 + s) * kStep;
-      if (s0 + s >= to) break;
-      if (k + kStep > K && k + 8 * q >= K) {
-        const uint4 zero = make_uint4(0, 0, 0, 0);
-#pragma unroll
-        for (int i = 0; i < 4; ++i) o.w[s][i] = zero;
-#pragma unroll
-        for (int t = 0; t < kNT; ++t) o.x[s][t] = zero;
-      }
-#pragma unroll
-      for (int t = 0; t < kNT; ++t) {
-#pragma unroll
-        for (int i = 0; i < 4; ++i) acc[i][t] = mfma(o.w[s][i], o.x[s][t], acc[i][t]);
-      }
-    }
-  };
-  Operands<kNT, kChunk> even, odd;
-  if (from < to) load(even, from);
-
-  // wavefront t finishes token tile t; the state travels while the products run
+  // wavefront t finishes token tile t; the state travels with the first operands
   const int token = first + 16 * wave + n;
   const bool mine = wave < kNT && token < p.B;
   const long unit = (long)token * p.H + head;
@@ -121,27 +69,10 @@ __global__ __launch_bounds__(256) void layer_token_kernel(const LayerTokenArgs p
     ba = Bf16::lo(p.b_a[head]);
   }
 
-  for (int s = from; s < to; s += 2 * kChunk) {
-    if (s + kChunk < to) load(odd, s + kChunk);
-    multiply(even, s);
-    if (s + 2 * kChunk < to) load(even, s + 2 * kChunk);
-    if (s + kChunk < to) multiply(odd, s + kChunk);
-  }
-
-#pragma unroll
-  for (int t = 0; t < kNT; ++t) {
-#pragma unroll
-    for (int i = 0; i < 4; ++i) partial[wave][i][t][lane] = acc[i][t];
-  }
-  __syncthreads();
+  f32x4_t acc[4][kNT], sum[4];
+  quarter_product<kNT, kChunk>(w, x, K, wave, q, acc);
+  add_quarters<kNT>(partial, acc, wave, lane, sum);
   if (!mine) return;
-  f32x4_t sum[4];
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    sum[i] = partial[0][i][wave][lane];
-#pragma unroll
-    for (int w_ = 1; w_ < kParts; ++w_) sum[i] += partial[w_][i][wave][lane];
-  }
 
   const float bias_b[4] = {Bf16::lo(bb.x), Bf16::hi(bb.x), Bf16::lo(bb.y), Bf16::hi(bb.y)};
   const float bias_c[4] = {Bf16::lo(bc.x), Bf16::hi(bc.x), Bf16::lo(bc.y), Bf16::hi(bc.y)};

@@ -309,8 +309,14 @@ class PhalanxStepState:
         )
 
 
+def _layer_operands(layer, x: torch.Tensor):
+    p, F = layer.param, layer.heads * 16
+    ops = plain_operands(x, (p.proj_a, True), (p.proj_b, True), (p.proj_c, True), (p.proj_v, False), (layer.proj_out, False))
+    return ops if ops is not None and ops[-2].shape == (F, x.shape[-1]) and ops[-1].shape[1] == F else None
+
+
 def _token_operands(layer, x: torch.Tensor):
-    """Weights and biases for the kernel that runs the input projections and the step in one launch, or None where the
+    """Weights and biases for the compiled step, whose first kernel runs the input projections and the step, or None where the
     call is for the general path: what ``plain_operands`` leaves to the modules, rows that 16-byte accesses do not fit, and sizes
     from which the library's products are faster (on the GPU alone: B=1024 with 64 heads 33.7 against 43.0 us, 700 with
     100 heads 61 against 52)."""
@@ -319,8 +325,7 @@ def _token_operands(layer, x: torch.Tensor):
     p = layer.param
     if x.shape[0] * layer.heads * x.shape[1] > 1 << 26:
         return None
-    ops = plain_operands(x, (p.proj_a, True), (p.proj_b, True), (p.proj_c, True), (p.proj_v, False))
-    return ops if ops is not None and ops[-1].shape == (layer.heads * 16, x.shape[1]) else None
+    return _layer_operands(layer, x)
 
 
 @torch.no_grad()
@@ -336,14 +341,14 @@ def phalanx_step(layer, x_t: torch.Tensor, state: PhalanxStepState, out: torch.T
     xc = x_t.to(p.compute_dtype)
     operands = None if state.pos is None else _token_operands(layer, xc)
     if operands is not None:
-        mixed = _btp.load_extension().layer_token(xc, *operands, state.h_loc, state.r_pref, state.c_prev_loc, state.pos,
-                                                  state.block_len, layer.heads, layer.kv_heads)
+        y = _btp.load_extension().layer_step(xc, *operands, state.h_loc, state.r_pref, state.c_prev_loc, state.pos,
+                                             state.block_len, layer.heads, layer.kv_heads)
     else:
         a, b, c, v = p.proj_a(xc), p.proj_b(xc), p.proj_c(xc), p.proj_v(xc)
         mixed = torch.empty_like(v)
         _btp.mix_step(a, b, c, v, mixed, state.h_loc, state.r_pref, state.c_prev_loc, state.pos, False,
                       state.block_len, layer.heads, layer.kv_heads)
-    y = layer.proj_out(mixed)
+        y = layer.proj_out(mixed)
     if out is not None:
         out.copy_(y)
         return out
@@ -361,6 +366,10 @@ def phalanx_prefill(layer, x: torch.Tensor) -> tuple[torch.Tensor, PhalanxStepSt
     if layer.k != 2:
         raise RuntimeError("phalanx_prefill needs a layer with k == 2")
     xc = x.to(p.compute_dtype)
+    operands = _layer_operands(layer, xc) if xc.dim() == 3 and xc.numel() > 0 and xc.shape[2] % 8 == 0 else None
+    if operands is not None:
+        y, h, r, c_prev, pos = _btp.load_extension().layer_prefill(xc.contiguous(), *operands, layer.heads, layer.kv_heads)
+        return y, PhalanxStepState(h, r, c_prev, pos, 16)
     a, b, c, v = (proj(xc).contiguous() for proj in (p.proj_a, p.proj_b, p.proj_c, p.proj_v))
     mixed, h, r, c_prev, pos = _btp.load_extension().mix_prefill(a, b, c, v, layer.heads, layer.kv_heads)
     return layer.proj_out(mixed), PhalanxStepState(h, r, c_prev, pos, 16)

@@ -239,7 +239,7 @@ def layer_call(x: torch.Tensor, proj_a, proj_b, proj_c, proj_v, proj_out, heads:
     """The whole layer on ``x[B, L, K]`` as one autograd node compiled into the binding (``LayerNode`` in
     ``btp_torch_ext.cpp``), or None where the call is for the modules and the Python nodes of this file: what
     ``plain_operands`` leaves to them, lengths and sizes that the mixing kernels refuse, and a row of gradients of 2 GiB.
-    Forward + backward, us, modules and Python nodes / compiled: B=8 L=128 dim=512 562 / 360, B=1024 1330 / 1307,
+    Forward + backward, us, modules and Python nodes / compiled: B=8 L=128 dim=512 562 / 245, B=1024 1330 / 1307,
     B=64 L=2048 dim=2048 8152 / 7992."""
     if not x.is_cuda or x.dim() != 3 or x.numel() == 0 or x.shape[1] % 16 != 0:
         return None

@@ -134,3 +134,23 @@ def test_column_sums_of_every_kind_of_array_in_one_launch(dtype):
             # one rounding of the result and at most `rows` fp32 additions of partial sums below sum |m|
             bound = torch.finfo(dtype).eps / 2 * want.abs() + m.shape[0] * 2.0 ** -24 * m.double().abs().sum(0) + 1e-7
             assert ((out.cpu().double() - want).abs() <= bound).all(), m.shape
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,K,Ns", [(1, 8, (1,)), (17, 16, (64, 3)), (33, 48, (65, 16, 130, 5)), (300, 512, (512, 512, 512, 32)), (1000, 200, (96, 7))])
+def test_linear_layers_of_one_launch(M, K, Ns):
+    """One to four row tiles per wavefront, columns and rows that end inside a tile, result rows of any alignment, K that ends
+    inside a matrix instruction's 32 columns and K too short for every wavefront to have a share."""
+    from spear_amd import _btp
+
+    g = torch.Generator().manual_seed(M)
+    x = torch.randn(M, 2 * K, generator=g).bfloat16()
+    ws = [torch.randn(n, K, generator=g).bfloat16() for n in Ns]
+    bs = [None if i % 2 else torch.randn(n, generator=g).bfloat16() for i, n in enumerate(Ns)]
+    print(f"linears M={M} K={K} N={Ns}", flush=True)
+    outs = _btp.load_extension().linears(x.to("cuda:0")[:, :K], [w.to("cuda:0") for w in ws], [None if b is None else b.to("cuda:0") for b in bs])
+    for w, b, out in zip(ws, bs, outs):
+        want = x[:, :K].double() @ w.double().T + (0 if b is None else b.double())
+        # one bf16 rounding, and K fp32 additions of terms of |x| |w|
+        bound = 2.0 ** -8 * want.abs() + K * 2.0 ** -24 * (x[:, :K].double().abs() @ w.double().abs().T) + 1e-6
+        assert ((out.cpu().double() - want).abs() <= bound).all(), tuple(w.shape)
