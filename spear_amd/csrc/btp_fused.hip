@@ -291,15 +291,34 @@ __device__ __forceinline__ HeadSlot head_slot(int slot, int pass, int H, int gro
 // `batch row * tiles + tile` of the three arrays is written.
 // kWide: head groupings other than 1, 2, 4, 8 heads per kv head (head_slot above).
 // ==========================================================================================
-template <class E, bool kQkv, bool kF32, bool kSums = false, bool kWide = false>
+enum class Sharing { kAlone, kShared, kWide };  // one head per kv head; 2, 4 or 8; any other number
+
+// p and q summed over pairs of lanes 16 (32) apart, each sum in one lane of the pair only: p's where the lane's bit 4 (5) is clear,
+// q's where it is set.
+__device__ __forceinline__ float scatter16(float p, float q) {
+  const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(p), __float_as_uint(q), false, false);
+  return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+__device__ __forceinline__ float scatter32(float p, float q) {
+  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(p), __float_as_uint(q), false, false);
+  return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+// The same over lanes 8 apart.
+__device__ __forceinline__ float scatter8(float p, float q, bool odd) {
+  const float keep = odd ? q : p, send = odd ? p : q;
+  return keep + row_xor<8>(send);
+}
+
+template <class E, bool kQkv, bool kF32, bool kSums, Sharing kSharing>
 __global__ __launch_bounds__(64 * kTileWaves)
-__attribute__((amdgpu_waves_per_eu(kWide ? SPEAR_FUSED_WIDE_WAVES_PER_EU : SPEAR_FUSED_TILE_WAVES_PER_EU)))
+__attribute__((amdgpu_waves_per_eu(kSharing == Sharing::kWide ? SPEAR_FUSED_WIDE_WAVES_PER_EU : SPEAR_FUSED_TILE_WAVES_PER_EU)))
 void phalanx_mix_bwd_tile_kernel(
     const uint16_t* __restrict__ a_logit, const uint16_t* __restrict__ b_logit, const uint16_t* __restrict__ c_in,
     const uint16_t* __restrict__ v_in, const uint16_t* __restrict__ dout, uint16_t* __restrict__ da_logit,
     uint16_t* __restrict__ db_logit, uint16_t* __restrict__ dc, uint16_t* __restrict__ dv, float* __restrict__ sum_da,
     float* __restrict__ sum_db, float* __restrict__ sum_dc, int ld_da, int ld_db, int ld_dc, int ld_dv, int L, int H,
     int kv_groups, int tiles, int slots) {
+  constexpr bool kWide = kSharing == Sharing::kWide, kShared = kSharing == Sharing::kShared;
   // per wavefront: decay of its block, product of the block's other decays per step, decay of the block beyond the edge
   __shared__ __align__(16) float gate_tiles[kTileWaves][3][kHeadsPerWave * kGateRow];
   __shared__ float2 carry_out[kTileWaves][2][64];  // [0] dC_out, [1] c_out of the wavefront's block, per lane
@@ -368,8 +387,14 @@ void phalanx_mix_bwd_tile_kernel(
   const int f_lane = 2 * (head * kChan + d0);
   const int kv_lane = 2 * ((head / kv_groups) * kChan + d0);
   const int o_lane = real ? f_lane * (kGradBytes / 2) : kNowhere;  // and store nowhere
-  // groups of 2, 4 or 8 heads: the sums over a group end up in all its lanes; its first head stores them
-  const int okv_lane = (!kWide && real && (head % kv_groups) == 0) ? kv_lane * (kGradBytes / 2) : kNowhere;
+  const int okv_lane = (!kWide && real) ? kv_lane * (kGradBytes / 2) : kNowhere;
+  // Groups of 2, 4 or 8 heads: the sums over a group of four steps' gradients are dealt to the group's lanes instead of left in
+  // all of them (half the additions, a quarter of the stores, and lane swaps on the VALU in place of 64 LDS exchanges per block).
+  // Which step of the four a lane ends up with; with two heads it has another one two steps later, with eight dc or db only.
+  const bool odd8 = (lane & 8) != 0, odd16 = (lane & 16) != 0, odd32 = (lane & 32) != 0;
+  const int g_step = kv_groups == 2 ? (odd8 ? 1 : 0) : kv_groups == 4 ? 2 * (odd8 ? 1 : 0) + (odd16 ? 1 : 0) : 2 * (odd16 ? 1 : 0) + (odd32 ? 1 : 0);
+  const int g_dc = okv_lane == kNowhere || (kv_groups == 8 && odd8) ? kNowhere : okv_lane + g_step * ld_dc * kGradBytes;
+  const int g_db = okv_lane == kNowhere || (kv_groups == 8 && !odd8) ? kNowhere : okv_lane + g_step * ld_db * kGradBytes;
   const GatePlace gp = gate_place<kQkv>(hs.first, H, lane);
   // da_logit: lane k of a head (k = lane % 8) ends up with steps 2k and 2k+1 of that head
   const int da_lane = real ? kDaBytes * ((2 * (lane & 7)) * ld_da + head) : kNowhere;
@@ -558,6 +583,7 @@ void phalanx_mix_bwd_tile_kernel(
   for (int c4 = 0; c4 < 4; ++c4) {
     const float4 qa = *reinterpret_cast<const float4*>(ta + head_local * kGateRow + 4 * c4);
     const float a4[4] = {qa.x, qa.y, qa.z, qa.w};
+    float tc0[4], tc1[4], tb0[4], tb1[4];  // kShared: the four steps' dc and db before the sum over a group
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const int r = 4 * c4 + i;
@@ -584,31 +610,58 @@ void phalanx_mix_bwd_tile_kernel(
           __builtin_amdgcn_raw_buffer_store_b32(E::pack2(dv0, dv1), rdv, o_lane, (t0 + r) * 2 * ld_dv, kNt);
         }
       } else {
-        if (kv_groups > 1) {  // wave-uniform: sum over the heads that share this kv head
-          dc0 += row_xor<8>(dc0); dc1 += row_xor<8>(dc1); db0 += row_xor<8>(db0); db1 += row_xor<8>(db1);
-          if (kv_groups > 2) {
-            dc0 += lane_xor(dc0, lane, 16); dc1 += lane_xor(dc1, lane, 16);
-            db0 += lane_xor(db0, lane, 16); db1 += lane_xor(db1, lane, 16);
-          }
-          if (kv_groups > 4) {
-            dc0 += lane_xor(dc0, lane, 32); dc1 += lane_xor(dc1, lane, 32);
-            db0 += lane_xor(db0, lane, 32); db1 += lane_xor(db1, lane, 32);
-          }
-        }
-        if constexpr (kSums) {
+        if constexpr (kSums && !kShared) {
           acc_b0 += db0; acc_b1 += db1; acc_c0 += dc0; acc_c1 += dc1;
         }
-        if constexpr (kF32) {
-          const u32x2_t wdc = {__float_as_uint(dc0), __float_as_uint(dc1)}, wdv = {__float_as_uint(dv0), __float_as_uint(dv1)},
-                        wdb = {__float_as_uint(db0), __float_as_uint(db1)};
-          __builtin_amdgcn_raw_buffer_store_b64(wdc, rdc, okv_lane, (t0 + r) * 4 * ld_dc, kNt);
-          __builtin_amdgcn_raw_buffer_store_b64(wdv, rdv, o_lane, (t0 + r) * 4 * ld_dv, kNt);
-          __builtin_amdgcn_raw_buffer_store_b64(wdb, rdb, okv_lane, (t0 + r) * 4 * ld_db, kNt);
-        } else {
-          __builtin_amdgcn_raw_buffer_store_b32(E::pack2(dc0, dc1), rdc, okv_lane, (t0 + r) * 2 * ld_dc, kNt);
-          __builtin_amdgcn_raw_buffer_store_b32(E::pack2(dv0, dv1), rdv, o_lane, (t0 + r) * 2 * ld_dv, kNt);
-          __builtin_amdgcn_raw_buffer_store_b32(E::pack2(db0, db1), rdb, okv_lane, (t0 + r) * 2 * ld_db, kNt);
+        if constexpr (kShared) {
+          tc0[i] = dc0; tc1[i] = dc1; tb0[i] = db0; tb1[i] = db1;
         }
+        if constexpr (kF32) {
+          const u32x2_t wdv = {__float_as_uint(dv0), __float_as_uint(dv1)};
+          if constexpr (!kShared) {
+            const u32x2_t wdc = {__float_as_uint(dc0), __float_as_uint(dc1)}, wdb = {__float_as_uint(db0), __float_as_uint(db1)};
+            __builtin_amdgcn_raw_buffer_store_b64(wdc, rdc, okv_lane, (t0 + r) * 4 * ld_dc, kNt);
+            __builtin_amdgcn_raw_buffer_store_b64(wdb, rdb, okv_lane, (t0 + r) * 4 * ld_db, kNt);
+          }
+          __builtin_amdgcn_raw_buffer_store_b64(wdv, rdv, o_lane, (t0 + r) * 4 * ld_dv, kNt);
+        } else {
+          if constexpr (!kShared) __builtin_amdgcn_raw_buffer_store_b32(E::pack2(dc0, dc1), rdc, okv_lane, (t0 + r) * 2 * ld_dc, kNt);
+          __builtin_amdgcn_raw_buffer_store_b32(E::pack2(dv0, dv1), rdv, o_lane, (t0 + r) * 2 * ld_dv, kNt);
+          if constexpr (!kShared) __builtin_amdgcn_raw_buffer_store_b32(E::pack2(db0, db1), rdb, okv_lane, (t0 + r) * 2 * ld_db, kNt);
+        }
+      }
+    }
+    if constexpr (kShared) {
+      auto store = [&](float x0, float x1, __amdgpu_buffer_rsrc_t to, int lane_off, int row, int ld) {
+        if constexpr (kF32) {
+          const u32x2_t w = {__float_as_uint(x0), __float_as_uint(x1)};
+          __builtin_amdgcn_raw_buffer_store_b64(w, to, lane_off, row * 4 * ld, kNt);
+        } else {
+          __builtin_amdgcn_raw_buffer_store_b32(E::pack2(x0, x1), to, lane_off, row * 2 * ld, kNt);
+        }
+      };
+      const int row = t0 + 4 * c4;
+      if (kv_groups == 2) {  // wave-uniform, as the two below
+#pragma unroll
+        for (int half = 0; half < 4; half += 2) {
+          const float c0 = scatter8(tc0[half], tc0[half + 1], odd8), c1 = scatter8(tc1[half], tc1[half + 1], odd8);
+          const float b0 = scatter8(tb0[half], tb0[half + 1], odd8), b1 = scatter8(tb1[half], tb1[half + 1], odd8);
+          if constexpr (kSums) { acc_c0 += c0; acc_c1 += c1; acc_b0 += b0; acc_b1 += b1; }
+          store(c0, c1, rdc, g_dc, row + half, ld_dc);
+          store(b0, b1, rdb, g_db, row + half, ld_db);
+        }
+      } else if (kv_groups == 4) {
+        auto one = [&](const float (&x)[4]) { return scatter8(scatter16(x[0], x[1]), scatter16(x[2], x[3]), odd8); };
+        const float c0 = one(tc0), c1 = one(tc1), b0 = one(tb0), b1 = one(tb1);
+        if constexpr (kSums) { acc_c0 += c0; acc_c1 += c1; acc_b0 += b0; acc_b1 += b1; }
+        store(c0, c1, rdc, g_dc, row, ld_dc);
+        store(b0, b1, rdb, g_db, row, ld_db);
+      } else {
+        auto one = [&](const float (&x)[4]) { return scatter16(scatter32(x[0], x[1]), scatter32(x[2], x[3])); };
+        const float x0 = scatter8(one(tc0), one(tb0), odd8), x1 = scatter8(one(tc1), one(tb1), odd8);
+        if constexpr (kSums) { acc_c0 += x0; acc_c1 += x1; }  // of dc in even lanes of the pair, of db in odd ones
+        store(x0, x1, rdc, g_dc, row, ld_dc);
+        store(x0, x1, rdb, g_db, row, ld_db);
       }
     }
     if constexpr (kWide) {
@@ -693,6 +746,26 @@ void phalanx_mix_bwd_tile_kernel(
     acc_a += row_xor<1>(acc_a);
     acc_a += row_xor<2>(acc_a);
     acc_a += row_xor<4>(acc_a);  // now every lane of the head has the block's sum
+    if constexpr (kShared) {  // the steps dealt to the group's lanes, together again
+      auto group_sum = [&](float x) {
+        if (kv_groups < 8) x += row_xor<8>(x);
+        if (kv_groups > 2) x += lane_xor(x, lane, 16);
+        if (kv_groups > 4) x += lane_xor(x, lane, 32);
+        return x;
+      };
+      acc_c0 = group_sum(acc_c0);
+      acc_c1 = group_sum(acc_c1);
+      if (kv_groups == 8) {
+        const float o0 = row_xor<8>(acc_c0), o1 = row_xor<8>(acc_c1);
+        acc_b0 = odd8 ? acc_c0 : o0;
+        acc_b1 = odd8 ? acc_c1 : o1;
+        acc_c0 = odd8 ? o0 : acc_c0;
+        acc_c1 = odd8 ? o1 : acc_c1;
+      } else {
+        acc_b0 = group_sum(acc_b0);
+        acc_b1 = group_sum(acc_b1);
+      }
+    }
     block_sums[wave][0][lane] = acc_b0;
     block_sums[wave][1][lane] = acc_b1;
     block_sums[wave][2][lane] = acc_c0;
@@ -1027,14 +1100,14 @@ int backward_slots(int H, int kv_groups) {
   return (kv_heads + per_slot - 1) / per_slot;
 }
 
-template <class E, bool kQkv, bool kF32, bool kSums, bool kWide>
+template <class E, bool kQkv, bool kF32, bool kSums, Sharing kSharing>
 void launch_mix_bwd_tile(const MixBwdArgs& p, hipStream_t s) {
   const int slots = backward_slots(p.H, p.kv_groups);
   const TileGrid g = tile_grid(p.B, slots, p.L, kTileWaves);
   auto u = [](const void* q) { return static_cast<const uint16_t*>(q); };
   auto w = [](void* q) { return static_cast<uint16_t*>(q); };
   const int Fkv = (p.H / p.kv_groups) * kChan;
-  hipLaunchKernelGGL((phalanx_mix_bwd_tile_kernel<E, kQkv, kF32, kSums, kWide>), dim3((unsigned)g.wgs),
+  hipLaunchKernelGGL((phalanx_mix_bwd_tile_kernel<E, kQkv, kF32, kSums, kSharing>), dim3((unsigned)g.wgs),
                      dim3(64 * kTileWaves), 0, s, u(p.a_logit), u(p.b_logit), u(p.c), u(p.v), u(p.dout), w(p.da_logit),
                      w(p.db_logit), w(p.dc), w(p.dv), p.sum_da, p.sum_db, p.sum_dc, p.ld_da ? p.ld_da : p.H,
                      p.ld_db ? p.ld_db : Fkv, p.ld_dc ? p.ld_dc : Fkv, p.ld_dv ? p.ld_dv : p.H * kChan, p.L, p.H,
@@ -1082,23 +1155,22 @@ long fused_mix_backward_sum_rows(long B, int H, int L) {
 hipError_t fused_mix_backward(const MixBwdArgs& p, hipStream_t s) {
   const bool sums = p.sum_da != nullptr;
   if (sums && (p.qkv || p.f32_grads)) return hipErrorInvalidValue;  // the caller has checked: layer form, 16-bit results
-  const bool wide = wide_grouping(p.kv_groups);
-  auto by_options = [&](auto e, auto wd) {
+  auto by_options = [&](auto e, auto sharing) {
     using E = decltype(e);
-    constexpr bool kWide = decltype(wd)::value;
-    if (sums) launch_mix_bwd_tile<E, false, false, true, kWide>(p, s);
-    else if (p.f32_grads && p.qkv) launch_mix_bwd_tile<E, true, true, false, kWide>(p, s);
-    else if (p.f32_grads) launch_mix_bwd_tile<E, false, true, false, kWide>(p, s);
-    else if (p.qkv) launch_mix_bwd_tile<E, true, false, false, kWide>(p, s);
-    else launch_mix_bwd_tile<E, false, false, false, kWide>(p, s);
+    constexpr Sharing kSharing = decltype(sharing)::value;
+    if (sums) launch_mix_bwd_tile<E, false, false, true, kSharing>(p, s);
+    else if (p.f32_grads && p.qkv) launch_mix_bwd_tile<E, true, true, false, kSharing>(p, s);
+    else if (p.f32_grads) launch_mix_bwd_tile<E, false, true, false, kSharing>(p, s);
+    else if (p.qkv) launch_mix_bwd_tile<E, true, false, false, kSharing>(p, s);
+    else launch_mix_bwd_tile<E, false, false, false, kSharing>(p, s);
   };
-  if (p.dtype == kBf16) {
-    if (wide) by_options(Bf16{}, std::true_type{});
-    else by_options(Bf16{}, std::false_type{});
-  } else {
-    if (wide) by_options(Fp16{}, std::true_type{});
-    else by_options(Fp16{}, std::false_type{});
-  }
+  auto by_type = [&](auto sharing) {
+    if (p.dtype == kBf16) by_options(Bf16{}, sharing);
+    else by_options(Fp16{}, sharing);
+  };
+  if (p.kv_groups == 1) by_type(std::integral_constant<Sharing, Sharing::kAlone>{});
+  else if (wide_grouping(p.kv_groups)) by_type(std::integral_constant<Sharing, Sharing::kWide>{});
+  else by_type(std::integral_constant<Sharing, Sharing::kShared>{});
   return hipGetLastError();
 }
 
