@@ -145,10 +145,10 @@ __device__ __forceinline__ GateWords load_gate_words(__amdgpu_buffer_rsrc_t ra, 
 // ==========================================================================================
 // Shared by the forward and the backward kernel: which tile a workgroup is.
 // ==========================================================================================
-// Wavefronts per workgroup and per SIMD of the backward kernel. 4 and 3 (168 registers: nothing spills, 12
-// wavefronts per CU) beat 8 and 4 (128 registers, three or four spilled values per lane that show up as 2.5 %
-// more HBM writes, 16 wavefronts per CU) by 1 % at B=1024 L=128 H=32, 3 % at B=16 L=8192 H=64 and 5 % at B=64
-// L=2048 H=128.
+// Wavefronts per workgroup and per SIMD of the backward kernel: 4 and 4. With the number of heads per kv head a compile-time
+// constant every instance fits 114 to 119 registers and nothing spills. As a run-time value it took 133 to 168, that is
+// 3 per SIMD (forced to 128, five to eleven values spill): B=16 H=64 L=8192 groups of 4 232.8 -> 213.8 us. Workgroups of 8 wavefronts
+// were slower by 1 to 5 % at 3 per SIMD (B=1024 L=128 H=32, B=16 L=8192 H=64, B=64 L=2048 H=128).
 #ifndef SPEAR_FUSED_TILE_WAVES
 #define SPEAR_FUSED_TILE_WAVES 4
 #endif
@@ -172,7 +172,7 @@ __device__ __forceinline__ float product_of_the_others(float a) {
 #define SPEAR_FUSED_TILE_XCD_GROUP 64
 #endif
 #ifndef SPEAR_FUSED_TILE_WAVES_PER_EU
-#define SPEAR_FUSED_TILE_WAVES_PER_EU 3
+#define SPEAR_FUSED_TILE_WAVES_PER_EU 4
 #endif
 // The kWide backward (head groups summed through LDS) at 2 per SIMD: 220-250 registers, nothing spills. At 3 it
 // spills 204 bytes per lane and takes 1.8-2.3 times as long (B=1024 L=128 H=32 in groups of 16: 171 -> 301 us).
@@ -291,7 +291,7 @@ __device__ __forceinline__ HeadSlot head_slot(int slot, int pass, int H, int gro
 // `batch row * tiles + tile` of the three arrays is written.
 // kWide: head groupings other than 1, 2, 4, 8 heads per kv head (head_slot above).
 // ==========================================================================================
-enum class Sharing { kAlone, kShared, kWide };  // one head per kv head; 2, 4 or 8; any other number
+enum class Sharing { kWide = 0, kAlone = 1, kTwo = 2, kFour = 4, kEight = 8 };  // heads per kv head, kWide: any other number
 
 // p and q summed over pairs of lanes 16 (32) apart, each sum in one lane of the pair only: p's where the lane's bit 4 (5) is clear,
 // q's where it is set.
@@ -318,7 +318,8 @@ void phalanx_mix_bwd_tile_kernel(
     uint16_t* __restrict__ db_logit, uint16_t* __restrict__ dc, uint16_t* __restrict__ dv, float* __restrict__ sum_da,
     float* __restrict__ sum_db, float* __restrict__ sum_dc, int ld_da, int ld_db, int ld_dc, int ld_dv, int L, int H,
     int kv_groups, int tiles, int slots) {
-  constexpr bool kWide = kSharing == Sharing::kWide, kShared = kSharing == Sharing::kShared;
+  constexpr bool kWide = kSharing == Sharing::kWide, kShared = !kWide && kSharing != Sharing::kAlone;
+  constexpr int kGroup = (int)kSharing;  // kShared: heads per kv head
   // per wavefront: decay of its block, product of the block's other decays per step, decay of the block beyond the edge
   __shared__ __align__(16) float gate_tiles[kTileWaves][3][kHeadsPerWave * kGateRow];
   __shared__ float2 carry_out[kTileWaves][2][64];  // [0] dC_out, [1] c_out of the wavefront's block, per lane
@@ -392,9 +393,9 @@ void phalanx_mix_bwd_tile_kernel(
   // all of them (half the additions, a quarter of the stores, and lane swaps on the VALU in place of 64 LDS exchanges per block).
   // Which step of the four a lane ends up with; with two heads it has another one two steps later, with eight dc or db only.
   const bool odd8 = (lane & 8) != 0, odd16 = (lane & 16) != 0, odd32 = (lane & 32) != 0;
-  const int g_step = kv_groups == 2 ? (odd8 ? 1 : 0) : kv_groups == 4 ? 2 * (odd8 ? 1 : 0) + (odd16 ? 1 : 0) : 2 * (odd16 ? 1 : 0) + (odd32 ? 1 : 0);
-  const int g_dc = okv_lane == kNowhere || (kv_groups == 8 && odd8) ? kNowhere : okv_lane + g_step * ld_dc * kGradBytes;
-  const int g_db = okv_lane == kNowhere || (kv_groups == 8 && !odd8) ? kNowhere : okv_lane + g_step * ld_db * kGradBytes;
+  const int g_step = kGroup == 2 ? (odd8 ? 1 : 0) : kGroup == 4 ? 2 * (odd8 ? 1 : 0) + (odd16 ? 1 : 0) : 2 * (odd16 ? 1 : 0) + (odd32 ? 1 : 0);
+  const int g_dc = okv_lane == kNowhere || (kGroup == 8 && odd8) ? kNowhere : okv_lane + g_step * ld_dc * kGradBytes;
+  const int g_db = okv_lane == kNowhere || (kGroup == 8 && !odd8) ? kNowhere : okv_lane + g_step * ld_db * kGradBytes;
   const GatePlace gp = gate_place<kQkv>(hs.first, H, lane);
   // da_logit: lane k of a head (k = lane % 8) ends up with steps 2k and 2k+1 of that head
   const int da_lane = real ? kDaBytes * ((2 * (lane & 7)) * ld_da + head) : kNowhere;
@@ -641,7 +642,7 @@ void phalanx_mix_bwd_tile_kernel(
         }
       };
       const int row = t0 + 4 * c4;
-      if (kv_groups == 2) {  // wave-uniform, as the two below
+      if constexpr (kGroup == 2) {
 #pragma unroll
         for (int half = 0; half < 4; half += 2) {
           const float c0 = scatter8(tc0[half], tc0[half + 1], odd8), c1 = scatter8(tc1[half], tc1[half + 1], odd8);
@@ -650,7 +651,7 @@ void phalanx_mix_bwd_tile_kernel(
           store(c0, c1, rdc, g_dc, row + half, ld_dc);
           store(b0, b1, rdb, g_db, row + half, ld_db);
         }
-      } else if (kv_groups == 4) {
+      } else if constexpr (kGroup == 4) {
         auto one = [&](const float (&x)[4]) { return scatter8(scatter16(x[0], x[1]), scatter16(x[2], x[3]), odd8); };
         const float c0 = one(tc0), c1 = one(tc1), b0 = one(tb0), b1 = one(tb1);
         if constexpr (kSums) { acc_c0 += c0; acc_c1 += c1; acc_b0 += b0; acc_b1 += b1; }
@@ -748,14 +749,14 @@ void phalanx_mix_bwd_tile_kernel(
     acc_a += row_xor<4>(acc_a);  // now every lane of the head has the block's sum
     if constexpr (kShared) {  // the steps dealt to the group's lanes, together again
       auto group_sum = [&](float x) {
-        if (kv_groups < 8) x += row_xor<8>(x);
-        if (kv_groups > 2) x += lane_xor(x, lane, 16);
-        if (kv_groups > 4) x += lane_xor(x, lane, 32);
+        if constexpr (kGroup < 8) x += row_xor<8>(x);
+        if constexpr (kGroup > 2) x += lane_xor(x, lane, 16);
+        if constexpr (kGroup > 4) x += lane_xor(x, lane, 32);
         return x;
       };
       acc_c0 = group_sum(acc_c0);
       acc_c1 = group_sum(acc_c1);
-      if (kv_groups == 8) {
+      if constexpr (kGroup == 8) {
         const float o0 = row_xor<8>(acc_c0), o1 = row_xor<8>(acc_c1);
         acc_b0 = odd8 ? acc_c0 : o0;
         acc_b1 = odd8 ? acc_c1 : o1;
@@ -1170,7 +1171,9 @@ hipError_t fused_mix_backward(const MixBwdArgs& p, hipStream_t s) {
   };
   if (p.kv_groups == 1) by_type(std::integral_constant<Sharing, Sharing::kAlone>{});
   else if (wide_grouping(p.kv_groups)) by_type(std::integral_constant<Sharing, Sharing::kWide>{});
-  else by_type(std::integral_constant<Sharing, Sharing::kShared>{});
+  else if (p.kv_groups == 2) by_type(std::integral_constant<Sharing, Sharing::kTwo>{});
+  else if (p.kv_groups == 4) by_type(std::integral_constant<Sharing, Sharing::kFour>{});
+  else by_type(std::integral_constant<Sharing, Sharing::kEight>{});
   return hipGetLastError();
 }
 
