@@ -22,10 +22,11 @@ int spear_layer_prefill(const void* a_logit, const void* b_logit, const void* c,
  * with positions on the device), bf16 operands, fp32 sums and state:
  *     x [B, K], rows ldx elements apart   w_a [H, K]   w_b, w_c [kv_heads * 16, K]   w_v [H * 16, K]   b_a, b_b, b_c biases
  *     out [B, H * 16]    h, c_prev [B, H, 16] fp32    r [B, H] fp32    pos [B] int32       state updated in place
+ * With advance == 0 pos is read only, and is to be moved by spear_layer_linear on the results.
  * K and ldx multiples of 8; x, weights, out, h and c_prev 16-byte aligned, b_b and b_c 8-byte, b_a 2-byte, r and pos 4-byte. */
 int spear_layer_token(const void* x, long long ldx, const void* w_a, const void* b_a, const void* w_b, const void* b_b,
                       const void* w_c, const void* b_c, const void* w_v, void* out, float* h, float* r, float* c_prev, int* pos,
-                      int block_len, int B, int K, int H, int kv_heads, void* stream);
+                      int block_len, int advance, int B, int K, int H, int kv_heads, void* stream);
 
 /* Column sums of n (1 .. 5) dense fp32 arrays, rounded to `dtype` (16-bit), in one launch:
  *     out[i][c] = sum over r of in[i][r * cols[i] + c]
@@ -40,9 +41,10 @@ int spear_layer_stack(const void* w_a, const void* w_b, const void* w_c, const v
                       int ld, int K, int H, int Fkv, int F, void* stream);
 
 /* n (1 .. 4) linear layers on the same rows, bf16 with fp32 sums:  out[i] [M, N[i]] = x [M, K] w[i]^T + bias[i] (null: none). x has
- * rows ldx elements apart, the rest is dense; K and ldx multiples of 8; x and w 16-byte, out 8-byte, bias 2-byte aligned. */
+ * rows ldx elements apart, the rest is dense; K and ldx multiples of 8; x and w 16-byte, out 8-byte, bias 2-byte aligned.
+ * pos: NULL, or int32 [M] block positions that are moved on by one, to 0 from block_len - 1. */
 int spear_layer_linear(int n, const void* x, long long ldx, int M, int K, const void* const* w, const void* const* bias,
-                       void* const* out, const int* N, void* stream);
+                       void* const* out, const int* N, int* pos, int block_len, void* stream);
 
 #ifdef __cplusplus
 }

@@ -64,7 +64,7 @@ int check_common(const char* who, int B, int H, int L, int k, int in_dtype, int 
 
 extern "C" {
 
-int spear_btp_abi_version(void) { return 23; }
+int spear_btp_abi_version(void) { return 24; }
 
 const char* spear_btp_last_error(void) { return g_error; }
 
@@ -221,7 +221,7 @@ int spear_layer_prefill(const void* a_logit, const void* b_logit, const void* c,
 
 int spear_layer_token(const void* x, long long ldx, const void* w_a, const void* b_a, const void* w_b, const void* b_b,
                       const void* w_c, const void* b_c, const void* w_v, void* out, float* h, float* r, float* c_prev, int* pos,
-                      int block_len, int B, int K, int H, int kv_heads, void* stream) {
+                      int block_len, int advance, int B, int K, int H, int kv_heads, void* stream) {
   g_error[0] = '\0';
   const char* who = "spear_layer_token";
   if (B < 0 || H < 0 || K < 0) return fail(SPEAR_BTP_EINVAL, "%s: negative dimension (B=%d H=%d K=%d)", who, B, H, K);
@@ -243,7 +243,7 @@ int spear_layer_token(const void* x, long long ldx, const void* w_a, const void*
     return fail(SPEAR_BTP_EINVAL, "%s: biases, r or pos are not aligned", who);
   auto u = [](const void* q) { return static_cast<const uint16_t*>(q); };
   spear_btp::LayerTokenArgs a{u(x), (long)ldx, u(w_a), u(b_a), u(w_b), u(b_b), u(w_c), u(b_c), u(w_v), static_cast<uint16_t*>(out),
-                              h, r, c_prev, pos, block_len, B, K, H, H / kv_heads};
+                              h, r, c_prev, pos, block_len, B, K, H, H / kv_heads, advance != 0};
   const hipError_t err = spear_btp::layer_token(a, static_cast<hipStream_t>(stream));
   if (err != hipSuccess) return fail(SPEAR_BTP_ELAUNCH, "%s: launch failed: %s", who, hipGetErrorString(err));
   return 0;
@@ -269,13 +269,15 @@ int spear_layer_stack(const void* w_a, const void* w_b, const void* w_c, const v
 }
 
 int spear_layer_linear(int n, const void* x, long long ldx, int M, int K, const void* const* w, const void* const* bias,
-                       void* const* out, const int* N, void* stream) {
+                       void* const* out, const int* N, int* pos, int block_len, void* stream) {
   g_error[0] = '\0';
   const char* who = "spear_layer_linear";
   if (n < 1 || n > 4 || M < 0 || K <= 0 || K % 8 != 0 || ldx < K || ldx % 8 != 0)
     return fail(SPEAR_BTP_EINVAL, "%s: bad shape (n=%d M=%d K=%d ldx=%lld)", who, n, M, K, ldx);
   if (!w || !bias || !out || !N) return fail(SPEAR_BTP_ENULL, "%s: NULL array", who);
-  spear_btp::LayerLinearArgs a{static_cast<const uint16_t*>(x), (long)ldx, M, K, n, {}, {}, {}, {}};
+  spear_btp::LayerLinearArgs a{static_cast<const uint16_t*>(x), (long)ldx, M, K, n, {}, {}, {}, {}, pos, block_len};
+  if (pos && (block_len <= 0 || (reinterpret_cast<uintptr_t>(pos) & 3u)))
+    return fail(SPEAR_BTP_EINVAL, "%s: pos must be 4-byte aligned and block_len positive (got %d)", who, block_len);
   long long groups = 0;
   for (int i = 0; i < n; ++i) {
     if (N[i] <= 0) return fail(SPEAR_BTP_EINVAL, "%s: a layer needs columns (got %d)", who, N[i]);

@@ -112,8 +112,9 @@ struct LayerTokenArgs {
   const uint16_t *w_a, *b_a, *w_b, *b_b, *w_c, *b_c, *w_v;
   uint16_t* out;           // [B, H*16]
   float *h, *r, *c_prev;   // [B, H, 16], [B, H], [B, H, 16]
-  int* pos;                // [B], advanced
+  int* pos;                // [B], advanced if `advance` is set
   int block_len, B, K, H, kv_groups;
+  bool advance;
 };
 hipError_t layer_token(const LayerTokenArgs& p, hipStream_t s);
 
@@ -126,6 +127,9 @@ struct LayerLinearArgs {
   const uint16_t *w[4], *bias[4];
   uint16_t* out[4];
   int N[4];
+  // null, or int32 [M]: moved to the next token's position inside its block (what layer_token leaves when it doesn't advance)
+  int* pos;
+  int block_len;
 };
 hipError_t layer_linear(const LayerLinearArgs& p, hipStream_t s);
 

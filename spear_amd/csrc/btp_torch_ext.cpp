@@ -419,7 +419,8 @@ void layer_sums(const std::vector<at::Tensor>& in, const std::vector<at::Tensor>
 }
 
 // x [M, K] through up to four linear layers in one launch (bf16; biases may be undefined): [M, N_i] each.
-std::vector<at::Tensor> linears(const at::Tensor& x, const std::vector<at::Tensor>& weights, const std::vector<at::Tensor>& biases) {
+std::vector<at::Tensor> linears(const at::Tensor& x, const std::vector<at::Tensor>& weights, const std::vector<at::Tensor>& biases,
+                                int* pos = nullptr, int64_t block_len = 0) {
   TORCH_CHECK(x.is_cuda() && x.dim() == 2 && x.stride(1) == 1 && x.scalar_type() == at::kBFloat16, "x must be [M, K] bfloat16 CUDA with dense rows.");
   TORCH_CHECK(!weights.empty() && weights.size() <= 4 && biases.size() == weights.size(), "1 to 4 layers.");
   const int64_t M = x.size(0), K = x.size(1);
@@ -443,21 +444,25 @@ std::vector<at::Tensor> linears(const at::Tensor& x, const std::vector<at::Tenso
     N[i] = (int)n;
   }
   const c10::DeviceGuard guard(x.device());
-  const int rc = spear_layer_linear((int)weights.size(), x.data_ptr(), M > 1 ? x.stride(0) : K, (int)M, (int)K, w, b, o, N, stream_of(x));
+  const int rc = spear_layer_linear((int)weights.size(), x.data_ptr(), M > 1 ? x.stride(0) : K, (int)M, (int)K, w, b, o, N, pos, (int)block_len,
+                                    stream_of(x));
   if (rc != 0) raise_native(rc);
   return out;
 }
 
-// The four input projections (a, b, c, v) of x [..., K], and one projection without bias: through the kernel above where it is
-// the faster one (the sizes measured at layer_linear.hip), through the library's products elsewhere. x dense.
+// Whether `layers` projections of M rows, `columns` columns together, are faster in the kernel above than as the library's
+// products (the sizes measured at layer_linear.hip).
+bool small_products(int64_t M, int64_t columns, int64_t K, size_t layers) {
+  return M > 0 && K > 0 && K % 8 == 0 && (layers > 1 ? M * columns * K <= 1600000000 : K <= 512 && M * columns * K <= 300000000);
+}
+
+// The four input projections (a, b, c, v) of x [..., K], or one projection without bias, by either. x dense.
 std::vector<at::Tensor> project(const at::Tensor& x, const std::vector<at::Tensor>& weights, const std::vector<at::Tensor>& biases) {
   const int64_t K = x.size(-1), M = K > 0 ? x.numel() / K : 0;
   int64_t columns = 0;
   for (const at::Tensor& w : weights) columns += w.size(0);
-  const bool small = weights.size() > 1 ? M * columns * K <= 1600000000 : (K <= 512 && M * columns * K <= 300000000);
   std::vector<at::Tensor> out;
-  const auto aligned = [](const at::Tensor& t) { return (reinterpret_cast<uintptr_t>(t.data_ptr()) & 15u) == 0; };
-  if (small && M > 0 && K % 8 == 0 && aligned(x)) {
+  if (small_products(M, columns, K, weights.size()) && (reinterpret_cast<uintptr_t>(x.data_ptr()) & 15u) == 0) {
     out = linears(x.view({M, K}), weights, biases);
     auto sizes = x.sizes().vec();
     for (at::Tensor& t : out) {
@@ -590,7 +595,7 @@ at::Tensor layer(const at::Tensor& x, const at::Tensor& w_a, const at::Tensor& b
 // bf16 with unit column stride, weights and biases of the four projections, the state updated in place.
 at::Tensor layer_token(const at::Tensor& x, const at::Tensor& w_a, const at::Tensor& b_a, const at::Tensor& w_b, const at::Tensor& b_b,
                        const at::Tensor& w_c, const at::Tensor& b_c, const at::Tensor& w_v, at::Tensor h, at::Tensor r,
-                       at::Tensor c_prev, at::Tensor pos, int64_t block_len, int64_t heads, int64_t kv_heads) {
+                       at::Tensor c_prev, at::Tensor pos, int64_t block_len, int64_t heads, int64_t kv_heads, bool advance) {
   TORCH_CHECK(x.is_cuda() && h.is_cuda() && r.is_cuda() && c_prev.is_cuda() && pos.is_cuda(), "All tensors must be CUDA.");
   TORCH_CHECK(x.dim() == 2 && x.stride(1) == 1, "x must be [B, dim] with dense rows.");
   TORCH_CHECK(heads > 0 && kv_heads > 0 && heads % kv_heads == 0, "heads must be divisible by kv_heads.");
@@ -614,7 +619,7 @@ at::Tensor layer_token(const at::Tensor& x, const at::Tensor& w_a, const at::Ten
   at::Tensor out = at::empty({B, heads * 16}, x.options());
   const int rc = spear_layer_token(x.data_ptr(), B > 1 ? x.stride(0) : K, w_a.data_ptr(), b_a.data_ptr(), w_b.data_ptr(), b_b.data_ptr(),
                                    w_c.data_ptr(), b_c.data_ptr(), w_v.data_ptr(), out.data_ptr(), h.data_ptr<float>(),
-                                   r.data_ptr<float>(), c_prev.data_ptr<float>(), pos.data_ptr<int>(), (int)block_len, (int)B, (int)K,
+                                   r.data_ptr<float>(), c_prev.data_ptr<float>(), pos.data_ptr<int>(), (int)block_len, advance ? 1 : 0, (int)B, (int)K,
                                    (int)heads, (int)kv_heads, stream_of(x));
   if (rc != 0) raise_native(rc);
   return out;
@@ -635,7 +640,11 @@ std::vector<at::Tensor> layer_prefill(const at::Tensor& x, const at::Tensor& w_a
 at::Tensor layer_step(const at::Tensor& x, const at::Tensor& w_a, const at::Tensor& b_a, const at::Tensor& w_b, const at::Tensor& b_b,
                       const at::Tensor& w_c, const at::Tensor& b_c, const at::Tensor& w_v, const at::Tensor& w_out, at::Tensor h,
                       at::Tensor r, at::Tensor c_prev, at::Tensor pos, int64_t block_len, int64_t heads, int64_t kv_heads) {
-  return project(layer_token(x, w_a, b_a, w_b, b_b, w_c, b_c, w_v, h, r, c_prev, pos, block_len, heads, kv_heads), {w_out}, {at::Tensor()})[0];
+  // the positions move on with the output projection where that is a kernel of this library
+  const auto in = [&](bool advance) { return layer_token(x, w_a, b_a, w_b, b_b, w_c, b_c, w_v, h, r, c_prev, pos, block_len, heads, kv_heads, advance); };
+  if (small_products(x.size(0), w_out.size(0), w_out.size(1), 1))
+    return linears(in(false), {w_out}, {at::Tensor()}, pos.data_ptr<int>(), block_len)[0];
+  return at::linear(in(true), w_out);
 }
 
 }  // namespace
@@ -677,7 +686,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("layer_sums", &layer_sums, py::arg("matrices"), py::arg("results"), "column sums of fp32 matrices, rounded to 16 bits");
   m.def("layer_token", &layer_token, py::arg("x"), py::arg("w_a"), py::arg("b_a"), py::arg("w_b"), py::arg("b_b"), py::arg("w_c"),
         py::arg("b_c"), py::arg("w_v"), py::arg("h"), py::arg("r"), py::arg("c_prev"), py::arg("pos"), py::arg("block_len"),
-        py::arg("heads"), py::arg("kv_heads"), "one token through the input projections and the step of the mixing stage");
+        py::arg("heads"), py::arg("kv_heads"), py::arg("advance") = true, "one token through the input projections and the step of the mixing stage");
   m.def("abi_version", []() { return spear_btp_abi_version(); });
   m.def("mix_backward_sum_rows", [](int64_t B, int64_t L, int64_t heads) {
     return (int64_t)spear_phalanx_mix_backward_sum_rows((int)B, (int)L, (int)heads);

@@ -42,6 +42,10 @@ __global__ __launch_bounds__(256) void layer_linear_kernel(const LayerLinearArgs
   add_quarters<kNT>(partial, acc, wave, lane, sum);
   const int row = first + 16 * wave + n;
   if (wave >= kNT || row >= p.M) return;
+  if (p.pos != nullptr && blockIdx.x % (unsigned)groups == 0 && q == 0) {  // one lane of the grid per row
+    const int next = p.pos[row] + 1;
+    p.pos[row] = next >= p.block_len ? 0 : next;
+  }
   const uint16_t* bias = p.bias[j];
   uint16_t* out = p.out[j] + (long)row * N;
 #pragma unroll

@@ -114,7 +114,8 @@ hipError_t layer_token(const LayerTokenArgs& p, hipStream_t s) {
   else if (nt == 2) launch<2, 4>(p, s);
   else launch<4, 2>(p, s);
   if (const hipError_t err = hipGetLastError(); err != hipSuccess) return err;
-  return advance_block_positions(p.pos, p.B, p.block_len, s);  // every wavefront of a row has to have read it
+  // every wavefront of a row has to have read pos: a launch of its own (4.4 us), or with the next kernel on the stream
+  return p.advance ? advance_block_positions(p.pos, p.B, p.block_len, s) : hipSuccess;
 }
 
 }  // namespace spear_btp
