@@ -145,10 +145,12 @@ __device__ __forceinline__ GateWords load_gate_words(__amdgpu_buffer_rsrc_t ra, 
 // ==========================================================================================
 // Shared by the forward and the backward kernel: which tile a workgroup is.
 // ==========================================================================================
-// Wavefronts per workgroup and per SIMD of the backward kernel: 4 and 4. With the number of heads per kv head a compile-time
-// constant every instance fits 114 to 119 registers and nothing spills. As a run-time value it took 133 to 168, that is
-// 3 per SIMD (forced to 128, five to eleven values spill): B=16 H=64 L=8192 groups of 4 232.8 -> 213.8 us. Workgroups of 8 wavefronts
-// were slower by 1 to 5 % at 3 per SIMD (B=1024 L=128 H=32, B=16 L=8192 H=64, B=64 L=2048 H=128).
+// Wavefronts per workgroup of the backward kernel (8 were slower by 1 to 5 %), and per SIMD. With the number of heads per kv head a
+// compile-time constant every instance fits 114 to 119 registers and nothing spills. Shared heads run 4 to a SIMD: as a run-time
+// value the grouping took 133 to 168 registers, 3 per SIMD (B=16 H=64 L=8192 groups of 4: 232.8 -> 213.8 us). Without sharing
+// the kernel moves 5.9 TB/s and more wavefronts only get in each other's way, so those instances are held to 3: 3 / 4 per SIMD, us,
+// q/k/v form B=1024 H=32 L=128 160 / 164, B=16 H=64 L=8192 326 / 333, B=64 H=128 L=2048 657 / 674; layer form 155 / 158, 319 / 325,
+// 642 / 652.
 #ifndef SPEAR_FUSED_TILE_WAVES
 #define SPEAR_FUSED_TILE_WAVES 4
 #endif
@@ -172,7 +174,10 @@ __device__ __forceinline__ float product_of_the_others(float a) {
 #define SPEAR_FUSED_TILE_XCD_GROUP 64
 #endif
 #ifndef SPEAR_FUSED_TILE_WAVES_PER_EU
-#define SPEAR_FUSED_TILE_WAVES_PER_EU 4
+#define SPEAR_FUSED_TILE_WAVES_PER_EU 3  // without shared heads: exactly so many
+#endif
+#ifndef SPEAR_FUSED_SHARED_WAVES_PER_EU
+#define SPEAR_FUSED_SHARED_WAVES_PER_EU 4
 #endif
 // The kWide backward (head groups summed through LDS) at 2 per SIMD: 220-250 registers, nothing spills. At 3 it
 // spills 204 bytes per lane and takes 1.8-2.3 times as long (B=1024 L=128 H=32 in groups of 16: 171 -> 301 us).
@@ -230,7 +235,7 @@ __device__ __forceinline__ unsigned tile_workgroup() {
 // Which heads a wavefront of the backward kernel owns. A head slot is normally 8 consecutive heads (the last
 // slot of a row may hold fewer). The gradients of b and c are sums over the heads that share a kv head; with
 // groups of 1, 2, 4 or 8 heads a group lies inside one slot on lanes a power of two apart, and the sum is a few
-// DPP / permute exchanges. Every other grouping (kWide) gets slots cut at group borders instead:
+// DPP / lane-swap exchanges. Every other grouping (kWide) gets slots cut at group borders instead:
 //   groups of 3, 5, 6, 7 heads:   a slot = as many whole groups as fit into 8 heads (2, 1, 1, 1)
 //   groups of more than 8 heads:  a slot = one kv head; the wavefront works through the group's heads 8 at a
 //                                 time (a loop around the whole tile computation) and adds up as it goes
@@ -311,7 +316,10 @@ __device__ __forceinline__ float scatter8(float p, float q, bool odd) {
 
 template <class E, bool kQkv, bool kF32, bool kSums, Sharing kSharing>
 __global__ __launch_bounds__(64 * kTileWaves)
-__attribute__((amdgpu_waves_per_eu(kSharing == Sharing::kWide ? SPEAR_FUSED_WIDE_WAVES_PER_EU : SPEAR_FUSED_TILE_WAVES_PER_EU)))
+__attribute__((amdgpu_waves_per_eu(kSharing == Sharing::kWide    ? SPEAR_FUSED_WIDE_WAVES_PER_EU
+                                   : kSharing == Sharing::kAlone ? SPEAR_FUSED_TILE_WAVES_PER_EU
+                                                                 : SPEAR_FUSED_SHARED_WAVES_PER_EU,
+                                   kSharing == Sharing::kAlone ? SPEAR_FUSED_TILE_WAVES_PER_EU : 8)))
 void phalanx_mix_bwd_tile_kernel(
     const uint16_t* __restrict__ a_logit, const uint16_t* __restrict__ b_logit, const uint16_t* __restrict__ c_in,
     const uint16_t* __restrict__ v_in, const uint16_t* __restrict__ dout, uint16_t* __restrict__ da_logit,
