@@ -124,6 +124,10 @@ int spear_phalanx_mix_forward(const void* a_logit, const void* b_logit, const vo
  * tolerances: forward `out`; backward `da_logit`, `db_logit`, `dc`, `dv` (row strides then count fp32
  * elements). Inputs keep their types. Not combinable with the column sums of _backward_ex. */
 #define SPEAR_MIX_F32_RESULTS 0x2u
+/* Layer form with 16-bit results (backward: with the three sum arrays): the decay, the input gate, the gated input and the
+ * recurrence's upstream gradient are rounded to the operands' 16-bit type on the way, as in a layer that forms them in tensors of
+ * their own for the stand-alone operator. Without the flag they stay in fp32. Give it to forward and backward alike. */
+#define SPEAR_MIX_ROUND 0x100u
 
 /* Backward of spear_phalanx_mix_forward: reads a_logit, b_logit, c, v and the upstream gradient
  * dout [B, L, H * 16]; writes da_logit [B, L, H], db_logit and dc [B, L, kv_heads * 16] (summed over

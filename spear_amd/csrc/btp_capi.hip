@@ -64,7 +64,7 @@ int check_common(const char* who, int B, int H, int L, int k, int in_dtype, int 
 
 extern "C" {
 
-int spear_btp_abi_version(void) { return 24; }
+int spear_btp_abi_version(void) { return 25; }
 
 const char* spear_btp_last_error(void) { return g_error; }
 
@@ -188,9 +188,10 @@ int spear_phalanx_mix_prefill(const void* a_logit, const void* b_logit, const vo
   g_error[0] = '\0';
   const char* who = c_prev_tail ? "spear_phalanx_mix_prefill" : "spear_phalanx_mix_forward";
   if (L % 16 != 0) return fail(SPEAR_BTP_EINVAL, "%s: Length L must be multiple of 16 (got %d)", who, L);
-  const unsigned known = SPEAR_MIX_QKV_GATE | SPEAR_MIX_F32_RESULTS;
+  const unsigned known = SPEAR_MIX_QKV_GATE | SPEAR_MIX_F32_RESULTS | SPEAR_MIX_ROUND;
   if (flags & ~known) return fail(SPEAR_BTP_EINVAL, "%s: unknown flag bits 0x%x", who, flags & ~known);
   const bool f32 = (flags & SPEAR_MIX_F32_RESULTS) != 0;
+  if ((flags & SPEAR_MIX_ROUND) && flags != SPEAR_MIX_ROUND) return fail(SPEAR_BTP_EINVAL, "%s: SPEAR_MIX_ROUND is for the layer form with 16-bit results", who);
   const void* const ptrs[5] = {a_logit, b_logit, c, v, out};
   if (int rc = check_mix_forward(who, ptrs, B, L, H, kv_heads, dtype, f32)) return rc < 0 ? rc : 0;
   if (c_prev_tail && !aligned16(c_prev_tail)) return fail(SPEAR_BTP_EINVAL, "%s: tensor pointers must be 16-byte aligned", who);
@@ -198,6 +199,7 @@ int spear_phalanx_mix_prefill(const void* a_logit, const void* b_logit, const vo
     return fail(SPEAR_BTP_EINVAL, "%s: the hand-over state belongs to the layer form, not SPEAR_MIX_QKV_GATE", who);
   spear_btp::MixArgs a{a_logit, b_logit, c, v, out, B, L, H, H / kv_heads, dtype, (flags & SPEAR_MIX_QKV_GATE) != 0, f32,
                        c_prev_tail};
+  a.round = (flags & SPEAR_MIX_ROUND) != 0;
   const hipError_t err = spear_btp::fused_mix_forward(a, static_cast<hipStream_t>(stream));
   if (err != hipSuccess) return fail(SPEAR_BTP_ELAUNCH, "%s: launch failed: %s", who, hipGetErrorString(err));
   return 0;
@@ -376,11 +378,13 @@ int spear_phalanx_mix_backward_ex(const void* a_logit, const void* b_logit, cons
   const char* who = "spear_phalanx_mix_backward";
   const void* const ptrs[9] = {a_logit, b_logit, c, v, dout, da_logit, db_logit, dc, dv};
   const int lds[4] = {ld_da, ld_db, ld_dc, ld_dv};
-  if (int rc = check_mix_backward(who, ptrs, lds, B, L, H, kv_heads, dtype, flags, SPEAR_MIX_QKV_GATE | SPEAR_MIX_F32_RESULTS))
+  if (int rc = check_mix_backward(who, ptrs, lds, B, L, H, kv_heads, dtype, flags, SPEAR_MIX_QKV_GATE | SPEAR_MIX_F32_RESULTS | SPEAR_MIX_ROUND))
     return rc < 0 ? rc : 0;
   const bool qkv = (flags & SPEAR_MIX_QKV_GATE) != 0, f32 = (flags & SPEAR_MIX_F32_RESULTS) != 0;
   const bool sums = sum_da || sum_db || sum_dc;
   if (sums && qkv) return fail(SPEAR_BTP_EINVAL, "%s: column sums are for the layer form, not SPEAR_MIX_QKV_GATE", who);
+  if ((flags & SPEAR_MIX_ROUND) && (!sums || qkv || f32))
+    return fail(SPEAR_BTP_EINVAL, "%s: SPEAR_MIX_ROUND is for the layer form with 16-bit results and column sums", who);
   if (sums && f32) return fail(SPEAR_BTP_EINVAL, "%s: column sums are not available with SPEAR_MIX_F32_RESULTS", who);
   if (sums) {
     if (!sum_da || !sum_db || !sum_dc) return fail(SPEAR_BTP_ENULL, "%s: the three sum arrays must be given together", who);
@@ -392,6 +396,7 @@ int spear_phalanx_mix_backward_ex(const void* a_logit, const void* b_logit, cons
   }
   spear_btp::MixBwdArgs a{a_logit, b_logit, c, v, dout, da_logit, db_logit, dc, dv, B, L, H, H / kv_heads, dtype,
                           sum_da, sum_db, sum_dc, ld_da, ld_db, ld_dc, ld_dv, qkv, f32};
+  a.round = (flags & SPEAR_MIX_ROUND) != 0;
   const hipError_t err = spear_btp::fused_mix_backward(a, static_cast<hipStream_t>(stream));
   if (err != hipSuccess) return fail(SPEAR_BTP_ELAUNCH, "%s: launch failed: %s", who, hipGetErrorString(err));
   return 0;

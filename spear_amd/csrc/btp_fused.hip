@@ -72,13 +72,23 @@ struct GateWords {
   uint32_t lo, hi;  // layer form: lo = two 16-bit logits; q/k/v form: two fp32 log-decays
 };
 
-template <class E, bool kQkv>
+// kRound (layer form): what a layer that forms its gates and products in tensors of their own has rounded to the operands' 16-bit
+// type on the way -- the decay, the input gate, the gated input and the upstream gradient of the recurrence -- is rounded here too.
+template <class E, bool kRound>
+__device__ __forceinline__ float2 as_tensor(float a, float b) {
+  if constexpr (!kRound) return make_float2(a, b);
+  const uint32_t word = E::pack2(a, b);
+  return make_float2(E::lo(word), E::hi(word));
+}
+
+template <class E, bool kQkv, bool kRound>
 __device__ __forceinline__ float2 decay_pair(GateWords w) {
   if constexpr (kQkv) {
     const float a0 = __expf(__uint_as_float(w.lo)), a1 = __expf(__uint_as_float(w.hi));
     return make_float2(clamp_coeff<E>(a0), clamp_coeff<E>(a1));
   } else {
-    return make_float2(clamp_coeff<E>(fast_sigmoid(E::lo(w.lo))), clamp_coeff<E>(fast_sigmoid(E::hi(w.lo))));
+    const float2 q = as_tensor<E, kRound>(fast_sigmoid(E::lo(w.lo)), fast_sigmoid(E::hi(w.lo)));
+    return make_float2(clamp_coeff<E>(q.x), clamp_coeff<E>(q.y));
   }
 }
 
@@ -86,6 +96,22 @@ template <bool kQkv>
 __device__ __forceinline__ float input_gate(float b) {
   if constexpr (kQkv) return b;
   else return fast_sigmoid(b);
+}
+
+// Input gates of a feature pair, and the gated inputs.
+template <class E, bool kQkv, bool kRound>
+__device__ __forceinline__ float2 input_gates(uint32_t b) {
+  return as_tensor<E, kRound>(input_gate<kQkv>(E::lo(b)), input_gate<kQkv>(E::hi(b)));
+}
+template <class E, bool kQkv, bool kRound>
+__device__ __forceinline__ float2 gated_input(uint32_t b, uint32_t v) {
+  const float2 g = input_gates<E, kQkv, kRound>(b);
+  return as_tensor<E, kRound>(g.x * E::lo(v), g.y * E::hi(v));
+}
+// The recurrence's upstream gradient of a feature pair.
+template <class E, bool kRound>
+__device__ __forceinline__ float2 upstream(uint32_t dout, uint32_t c) {
+  return as_tensor<E, kRound>(E::lo(dout) * E::lo(c), E::hi(dout) * E::hi(c));
 }
 
 constexpr int kHeadsPerWave = 8;
@@ -314,7 +340,7 @@ __device__ __forceinline__ float scatter8(float p, float q, bool odd) {
   return keep + row_xor<8>(send);
 }
 
-template <class E, bool kQkv, bool kF32, bool kSums, Sharing kSharing>
+template <class E, bool kQkv, bool kF32, bool kSums, Sharing kSharing, bool kRound>
 __global__ __launch_bounds__(64 * kTileWaves)
 __attribute__((amdgpu_waves_per_eu(kSharing == Sharing::kWide    ? SPEAR_FUSED_WIDE_WAVES_PER_EU
                                    : kSharing == Sharing::kAlone ? SPEAR_FUSED_TILE_WAVES_PER_EU
@@ -450,11 +476,11 @@ void phalanx_mix_bwd_tile_kernel(
   float cin0 = 0.0f, cin1 = 0.0f, dC0 = 0.0f, dC1 = 0.0f;
   float R[32];  // local reverse states, later dX, channel pair interleaved: R[2 r], R[2 r + 1]
   if (valid) {
-    const float2 a01 = decay_pair<E, kQkv>(araw);
+    const float2 a01 = decay_pair<E, kQkv, kRound>(araw);
     write_tile(ta, a01.x, a01.y);
     write_tile(te, product_of_the_others(a01.x), product_of_the_others(a01.y));
     if (halo) {
-      const float2 n01 = decay_pair<E, kQkv>(haraw);
+      const float2 n01 = decay_pair<E, kQkv, kRound>(haraw);
       write_tile(tn, n01.x, n01.y);
     }
     wave_lds_handover();
@@ -468,8 +494,9 @@ void phalanx_mix_bwd_tile_kernel(
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
           const int r = 4 * c4 + i;
-          cin0 = fmaf(a4[i], cin0, input_gate<kQkv>(E::lo(h0[r])) * E::lo(h1[r]));
-          cin1 = fmaf(a4[i], cin1, input_gate<kQkv>(E::hi(h0[r])) * E::hi(h1[r]));
+          const float2 x = gated_input<E, kQkv, kRound>(h0[r], h1[r]);
+          cin0 = fmaf(a4[i], cin0, x.x);
+          cin1 = fmaf(a4[i], cin1, x.y);
         }
         asm volatile("" ::: "memory");
       }
@@ -482,8 +509,9 @@ void phalanx_mix_bwd_tile_kernel(
 #pragma unroll
         for (int i = 3; i >= 0; --i) {
           const int r = 4 * c4 + i;
-          r0 = fmaf(up, r0, E::lo(h0[r]) * E::lo(h1[r]));
-          r1 = fmaf(up, r1, E::hi(h0[r]) * E::hi(h1[r]));
+          const float2 u = upstream<E, kRound>(h0[r], h1[r]);
+          r0 = fmaf(up, r0, u.x);
+          r1 = fmaf(up, r1, u.y);
           up = a4[i];
         }
         asm volatile("" ::: "memory");
@@ -508,8 +536,9 @@ void phalanx_mix_bwd_tile_kernel(
 #pragma unroll
         for (int i = 3; i >= 0; --i) {
           const int r = 4 * c4 + i;
-          r0 = fmaf(up, r0, E::lo(g[r]) * E::lo(c[r]));
-          r1 = fmaf(up, r1, E::hi(g[r]) * E::hi(c[r]));
+          const float2 u = upstream<E, kRound>(g[r], c[r]);
+          r0 = fmaf(up, r0, u.x);
+          r1 = fmaf(up, r1, u.y);
           R[2 * r] = r0;
           R[2 * r + 1] = r1;
           up = a4[i];
@@ -528,8 +557,9 @@ void phalanx_mix_bwd_tile_kernel(
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
           const int r = 4 * c4 + i;
-          l0 = fmaf(a4[i], l0, input_gate<kQkv>(E::lo(b[r])) * E::lo(v[r]));
-          l1 = fmaf(a4[i], l1, input_gate<kQkv>(E::hi(b[r])) * E::hi(v[r]));
+          const float2 x = gated_input<E, kQkv, kRound>(b[r], v[r]);
+          l0 = fmaf(a4[i], l0, x.x);
+          l1 = fmaf(a4[i], l1, x.y);
         }
         asm volatile("" ::: "memory");
       }
@@ -596,13 +626,15 @@ void phalanx_mix_bwd_tile_kernel(
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const int r = 4 * c4 + i;
-      const float G0 = input_gate<kQkv>(E::lo(b[r])), G1 = input_gate<kQkv>(E::hi(b[r]));
+      const float2 G = input_gates<E, kQkv, kRound>(b[r]);
+      const float G0 = G.x, G1 = G.y;
       const float v0 = E::lo(v[r]), v1 = E::hi(v[r]);
       const float go0 = E::lo(g[r]), go1 = E::hi(g[r]);
       const float dX0 = R[2 * r], dX1 = R[2 * r + 1];
       e[r] = fmaf(dX0, hs0, dX1 * hs1);
-      hs0 = fmaf(a4[i], hs0, G0 * v0);
-      hs1 = fmaf(a4[i], hs1, G1 * v1);
+      const float2 x = as_tensor<E, kRound>(G0 * v0, G1 * v1);
+      hs0 = fmaf(a4[i], hs0, x.x);
+      hs1 = fmaf(a4[i], hs1, x.y);
       float dc0 = go0 * hs0, dc1 = go1 * hs1;
       float db0 = dX0 * v0, db1 = dX1 * v1;  // dX * v: the gradient of k in the q/k/v form
       if constexpr (!kQkv) {
@@ -828,7 +860,7 @@ void phalanx_mix_bwd_tile_kernel(
 //   512 128 64: 91.6 / 90.2     16 8192 64: 167.5 / 170.6  64 2048 128: 336.1 / 338.3
 //   256 128 128: 87.7 / 90.1    4096 128 8: 92.9 / 88.1    1024 128 48: 132.9 / 125.3
 // ==========================================================================================
-template <class E, int kW, bool kQkv, bool kF32, bool kRagged>
+template <class E, int kW, bool kQkv, bool kF32, bool kRagged, bool kRound>
 __global__ __launch_bounds__(64 * kW) __attribute__((amdgpu_waves_per_eu(SPEAR_FUSED_TILE_WAVES_PER_EU)))
 void phalanx_mix_fwd_tile_kernel(const uint16_t* __restrict__ a_logit, const uint16_t* __restrict__ b_logit,
                                  const uint16_t* __restrict__ c_in, const uint16_t* __restrict__ v_in,
@@ -919,10 +951,10 @@ void phalanx_mix_fwd_tile_kernel(const uint16_t* __restrict__ a_logit, const uin
   float a[16], x0[16], x1[16];
   float cin0 = 0.0f, cin1 = 0.0f;
   if (valid) {
-    const float2 a01 = decay_pair<E, kQkv>(araw);
+    const float2 a01 = decay_pair<E, kQkv, kRound>(araw);
     write_tile(ta, a01.x, a01.y);
     if (halo) {
-      const float2 n01 = decay_pair<E, kQkv>(haraw);
+      const float2 n01 = decay_pair<E, kQkv, kRound>(haraw);
       write_tile(tn, n01.x, n01.y);
     }
     wave_lds_handover();
@@ -931,8 +963,9 @@ void phalanx_mix_fwd_tile_kernel(const uint16_t* __restrict__ a_logit, const uin
       read_decays(tn, an);
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
-        cin0 = fmaf(an[r], cin0, input_gate<kQkv>(E::lo(hb[r])) * E::lo(hv[r]));
-        cin1 = fmaf(an[r], cin1, input_gate<kQkv>(E::hi(hb[r])) * E::hi(hv[r]));
+        const float2 x = gated_input<E, kQkv, kRound>(hb[r], hv[r]);
+        cin0 = fmaf(an[r], cin0, x.x);
+        cin1 = fmaf(an[r], cin1, x.y);
       }
     }
     __builtin_amdgcn_sched_barrier(0);
@@ -941,8 +974,9 @@ void phalanx_mix_fwd_tile_kernel(const uint16_t* __restrict__ a_logit, const uin
     float l0 = 0.0f, l1 = 0.0f;
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
-      x0[r] = input_gate<kQkv>(E::lo(b[r])) * E::lo(v[r]);
-      x1[r] = input_gate<kQkv>(E::hi(b[r])) * E::hi(v[r]);
+      const float2 x = gated_input<E, kQkv, kRound>(b[r], v[r]);
+      x0[r] = x.x;
+      x1[r] = x.y;
       if (!kRagged || r < steps) {  // wave-uniform: a block that ends early keeps the state after its last step
         l0 = fmaf(a[r], l0, x0[r]);
         l1 = fmaf(a[r], l1, x1[r]);
@@ -1088,10 +1122,10 @@ TileGrid tile_grid(long B, int slots, int L, int waves) {
 // (table at the forward kernel).
 bool forward_takes_eight_waves(int H, int L) { return H < 16 || (L >= 512 && H <= 32); }
 
-template <class E, int kW, bool kQkv, bool kF32 = false, bool kRagged = false>
+template <class E, int kW, bool kQkv, bool kF32 = false, bool kRagged = false, bool kRound = false>
 void launch_mix_fwd_tile(const MixArgs& p, hipStream_t s) {
   const TileGrid g = tile_grid(p.B, (p.H + kHeadsPerWave - 1) / kHeadsPerWave, p.L, kW);
-  hipLaunchKernelGGL((phalanx_mix_fwd_tile_kernel<E, kW, kQkv, kF32, kRagged>), dim3((unsigned)g.wgs), dim3(64 * kW), 0, s,
+  hipLaunchKernelGGL((phalanx_mix_fwd_tile_kernel<E, kW, kQkv, kF32, kRagged, kRound>), dim3((unsigned)g.wgs), dim3(64 * kW), 0, s,
                      static_cast<const uint16_t*>(p.a_logit), static_cast<const uint16_t*>(p.b_logit),
                      static_cast<const uint16_t*>(p.c), static_cast<const uint16_t*>(p.v), static_cast<uint16_t*>(p.out),
                      p.c_prev_tail, p.h_tail, p.r_tail, p.pos_tail, p.L, p.H, p.kv_groups, g.tiles);
@@ -1109,14 +1143,14 @@ int backward_slots(int H, int kv_groups) {
   return (kv_heads + per_slot - 1) / per_slot;
 }
 
-template <class E, bool kQkv, bool kF32, bool kSums, Sharing kSharing>
+template <class E, bool kQkv, bool kF32, bool kSums, Sharing kSharing, bool kRound = false>
 void launch_mix_bwd_tile(const MixBwdArgs& p, hipStream_t s) {
   const int slots = backward_slots(p.H, p.kv_groups);
   const TileGrid g = tile_grid(p.B, slots, p.L, kTileWaves);
   auto u = [](const void* q) { return static_cast<const uint16_t*>(q); };
   auto w = [](void* q) { return static_cast<uint16_t*>(q); };
   const int Fkv = (p.H / p.kv_groups) * kChan;
-  hipLaunchKernelGGL((phalanx_mix_bwd_tile_kernel<E, kQkv, kF32, kSums, kSharing>), dim3((unsigned)g.wgs),
+  hipLaunchKernelGGL((phalanx_mix_bwd_tile_kernel<E, kQkv, kF32, kSums, kSharing, kRound>), dim3((unsigned)g.wgs),
                      dim3(64 * kTileWaves), 0, s, u(p.a_logit), u(p.b_logit), u(p.c), u(p.v), u(p.dout), w(p.da_logit),
                      w(p.db_logit), w(p.dc), w(p.dv), p.sum_da, p.sum_db, p.sum_dc, p.ld_da ? p.ld_da : p.H,
                      p.ld_db ? p.ld_db : Fkv, p.ld_dc ? p.ld_dc : Fkv, p.ld_dv ? p.ld_dv : p.H * kChan, p.L, p.H,
@@ -1139,6 +1173,11 @@ hipError_t fused_mix_forward(const MixArgs& p, hipStream_t s) {
       if (p.L % kTile != 0) {  // prompts, layer form with 16-bit results only (the caller has checked)
         if (eight) launch_mix_fwd_tile<E, 8, false, false, true>(p, s);
         else launch_mix_fwd_tile<E, 4, false, false, true>(p, s);
+        return;
+      }
+      if (p.round) {
+        if (eight) launch_mix_fwd_tile<E, 8, false, false, false, true>(p, s);
+        else launch_mix_fwd_tile<E, 4, false, false, false, true>(p, s);
         return;
       }
     }
@@ -1167,7 +1206,8 @@ hipError_t fused_mix_backward(const MixBwdArgs& p, hipStream_t s) {
   auto by_options = [&](auto e, auto sharing) {
     using E = decltype(e);
     constexpr Sharing kSharing = decltype(sharing)::value;
-    if (sums) launch_mix_bwd_tile<E, false, false, true, kSharing>(p, s);
+    if (sums && p.round) launch_mix_bwd_tile<E, false, false, true, kSharing, true>(p, s);
+    else if (sums) launch_mix_bwd_tile<E, false, false, true, kSharing>(p, s);
     else if (p.f32_grads && p.qkv) launch_mix_bwd_tile<E, true, true, false, kSharing>(p, s);
     else if (p.f32_grads) launch_mix_bwd_tile<E, false, true, false, kSharing>(p, s);
     else if (p.qkv) launch_mix_bwd_tile<E, true, false, false, kSharing>(p, s);

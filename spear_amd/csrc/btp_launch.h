@@ -61,6 +61,7 @@ struct MixArgs {
   // state, fp32 [B, H] gate product, int32 [B] position inside the block. L % 16 != 0 is for these calls.
   float *h_tail = nullptr, *r_tail = nullptr;
   int* pos_tail = nullptr;
+  bool round = false;  // layer form, whole blocks, 16-bit results: gates and gated inputs rounded to the operands' type on the way
 };
 hipError_t fused_mix_forward(const MixArgs& p, hipStream_t s);
 // Workgroups the forward / backward kernel launches for a shape (must fit a 31-bit grid).
@@ -79,6 +80,7 @@ struct MixBwdArgs {
   int ld_da = 0, ld_db = 0, ld_dc = 0, ld_dv = 0;
   bool qkv = false;  // as in MixArgs; da_logit is then the fp32 gradient of the gate
   bool f32_grads = false;  // check mode: da_logit, db_logit, dc, dv are fp32
+  bool round = false;  // as in MixArgs, the upstream gradient too; with sums only
 };
 hipError_t fused_mix_backward(const MixBwdArgs& p, hipStream_t s);
 long fused_mix_backward_sum_rows(long B, int H, int L);

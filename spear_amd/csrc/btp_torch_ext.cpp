@@ -249,7 +249,7 @@ MixShape check_mix_inputs(const at::Tensor& a_logit, const at::Tensor& b_logit, 
 // out <- btp(sigmoid(a_logit), sigmoid(b_logit) * v) * c + v on [B, L, features] tensors, or with
 // qkv_gate out <- c * btp(exp(a_logit), b_logit * v) + v. A float32 `out` selects the fp32 check mode.
 void mix_forward(const at::Tensor& a_logit, const at::Tensor& b_logit, const at::Tensor& c, const at::Tensor& v,
-                 at::Tensor out, int64_t heads, int64_t kv_heads, bool qkv_gate) {
+                 at::Tensor out, int64_t heads, int64_t kv_heads, bool qkv_gate, bool round_products = false) {
   const MixShape s = check_mix_inputs(a_logit, b_logit, c, v, heads, kv_heads, qkv_gate);
   TORCH_CHECK(out.is_cuda(), "All tensors must be CUDA.");
   TORCH_CHECK(out.scalar_type() == v.scalar_type() || out.scalar_type() == at::kFloat,
@@ -257,7 +257,8 @@ void mix_forward(const at::Tensor& a_logit, const at::Tensor& b_logit, const at:
   check_layout("out", out, {s.B, s.L, s.F});
   check_same_device({&a_logit, &b_logit, &c, &v, &out});
   const c10::DeviceGuard guard(v.device());
-  const unsigned flags = (qkv_gate ? SPEAR_MIX_QKV_GATE : 0u) | (out.scalar_type() == at::kFloat ? SPEAR_MIX_F32_RESULTS : 0u);
+  const unsigned flags = (qkv_gate ? SPEAR_MIX_QKV_GATE : 0u) | (out.scalar_type() == at::kFloat ? SPEAR_MIX_F32_RESULTS : 0u) |
+                         (round_products ? SPEAR_MIX_ROUND : 0u);
   const int rc = spear_phalanx_mix_forward(a_logit.data_ptr(), b_logit.data_ptr(), c.data_ptr(), v.data_ptr(), out.data_ptr(),
                                            (int)s.B, (int)s.L, (int)heads, (int)kv_heads, tag_of(v.scalar_type()), flags,
                                            stream_of(v));
@@ -279,7 +280,7 @@ int64_t row_stride(const char* name, const at::Tensor& t, int64_t B, int64_t L, 
 // tile of 64 time steps).
 void mix_backward(const at::Tensor& a_logit, const at::Tensor& b_logit, const at::Tensor& c, const at::Tensor& v,
                   const at::Tensor& dout, at::Tensor da_logit, at::Tensor db_logit, at::Tensor dc, at::Tensor dv,
-                  int64_t heads, int64_t kv_heads, const std::vector<at::Tensor>& sums, bool qkv_gate) {
+                  int64_t heads, int64_t kv_heads, const std::vector<at::Tensor>& sums, bool qkv_gate, bool round_products = false) {
   const MixShape s = check_mix_inputs(a_logit, b_logit, c, v, heads, kv_heads, qkv_gate);
   TORCH_CHECK(dout.is_cuda() && da_logit.is_cuda() && db_logit.is_cuda() && dc.is_cuda() && dv.is_cuda(), "All tensors must be CUDA.");
   TORCH_CHECK(dout.scalar_type() == v.scalar_type(), "all tensors must share one dtype.");
@@ -313,7 +314,7 @@ void mix_backward(const at::Tensor& a_logit, const at::Tensor& b_logit, const at
     }
   }
   const c10::DeviceGuard guard(v.device());
-  const unsigned flags = (qkv_gate ? SPEAR_MIX_QKV_GATE : 0u) | (f32 ? SPEAR_MIX_F32_RESULTS : 0u);
+  const unsigned flags = (qkv_gate ? SPEAR_MIX_QKV_GATE : 0u) | (f32 ? SPEAR_MIX_F32_RESULTS : 0u) | (round_products ? SPEAR_MIX_ROUND : 0u);
   const int rc = spear_phalanx_mix_backward_ex(
       a_logit.data_ptr(), b_logit.data_ptr(), c.data_ptr(), v.data_ptr(), dout.data_ptr(), da_logit.data_ptr(),
       db_logit.data_ptr(), dc.data_ptr(), dv.data_ptr(), (int)ld_da, (int)ld_db, (int)ld_dc, (int)ld_dv, sp[0], sp[1], sp[2],
@@ -495,11 +496,11 @@ struct LayerNode : public torch::autograd::Function<LayerNode> {
   static at::Tensor forward(torch::autograd::AutogradContext* ctx, const at::Tensor& x, const at::Tensor& w_a, const at::Tensor& b_a,
                             const at::Tensor& w_b, const at::Tensor& b_b, const at::Tensor& w_c, const at::Tensor& b_c,
                             const at::Tensor& w_v, const at::Tensor& w_out, int64_t heads, int64_t kv_heads, int64_t slices_in,
-                            int64_t slices_out) {
+                            int64_t slices_out, bool round_products) {
     const auto front = project(x, {w_a, w_b, w_c, w_v}, {b_a, b_b, b_c, at::Tensor()});
     const at::Tensor &a = front[0], &b = front[1], &c = front[2], &v = front[3];
     at::Tensor mixed = at::empty(v.sizes(), v.options());
-    mix_forward(a, b, c, v, mixed, heads, kv_heads, false);
+    mix_forward(a, b, c, v, mixed, heads, kv_heads, false, round_products);
     at::Tensor y = project(mixed, {w_out}, {at::Tensor()})[0];
     if (ctx != nullptr) {
       ctx->save_for_backward({x, w_a, w_b, w_c, w_v, w_out, a, b, c, v, mixed});
@@ -507,6 +508,7 @@ struct LayerNode : public torch::autograd::Function<LayerNode> {
       ctx->saved_data["kv_heads"] = kv_heads;
       ctx->saved_data["slices_in"] = slices_in;
       ctx->saved_data["slices_out"] = slices_out;
+      ctx->saved_data["round_products"] = round_products;
     }
     return y;
   }
@@ -521,7 +523,7 @@ struct LayerNode : public torch::autograd::Function<LayerNode> {
     const int64_t B = v.size(0), L = v.size(1), F = v.size(2), Fkv = b.size(2), M = B * L, K = x.size(2), dim = w_out.size(0);
     const c10::DeviceGuard guard(v.device());
     const at::Tensor dy = grad_outputs[0].contiguous().view({M, dim}), x2 = x.view({M, K}), mixed2 = mixed.view({M, F});
-    torch::autograd::variable_list out(13);  // forward's arguments, of which the first nine are tensors
+    torch::autograd::variable_list out(14);  // forward's arguments, of which the first nine are tensors
     std::vector<at::Tensor> parts, sums;
     bool front = false, weights = false;
     for (int i = 0; i < 8; ++i) {
@@ -545,7 +547,7 @@ struct LayerNode : public torch::autograd::Function<LayerNode> {
       const auto f32 = v.options().dtype(at::kFloat);
       parts = {at::empty({rows, heads}, f32), at::empty({rows, Fkv}, f32), at::empty({rows, Fkv}, f32)};
       mix_backward(a, b, c, v, dmixed, packed.narrow(2, 2 * Fkv + F, heads), packed.narrow(2, 0, Fkv), packed.narrow(2, Fkv, Fkv),
-                   packed.narrow(2, 2 * Fkv, F), heads, kv_heads, parts, false);
+                   packed.narrow(2, 2 * Fkv, F), heads, kv_heads, parts, false, ctx->saved_data["round_products"].toBool());
       sums = {at::empty({heads}, v.options()), at::empty({Fkv}, v.options()), at::empty({Fkv}, v.options())};
       out[2] = sums[0];
       out[4] = sums[1];
@@ -578,17 +580,17 @@ struct LayerNode : public torch::autograd::Function<LayerNode> {
   }
 };
 
-// y = layer(x) for x [B, L, dim]; slices: into how many slices of tokens the weight gradients' products are cut.
+// y = layer(x) for x [B, L, dim]; round_products: gates and products of the mixing stage in 16 bits, as in tensors of their own; slices: into how many slices of tokens the weight gradients' products are cut.
 at::Tensor layer(const at::Tensor& x, const at::Tensor& w_a, const at::Tensor& b_a, const at::Tensor& w_b, const at::Tensor& b_b,
                  const at::Tensor& w_c, const at::Tensor& b_c, const at::Tensor& w_v, const at::Tensor& w_out, int64_t heads,
-                 int64_t kv_heads, int64_t slices_in, int64_t slices_out) {
+                 int64_t kv_heads, int64_t slices_in, int64_t slices_out, bool round_products) {
   TORCH_CHECK(x.dim() == 3 && x.is_contiguous(), "x must be dense [B, L, dim].");
   if (at::GradMode::is_enabled()) {
     for (const at::Tensor* t : {&x, &w_a, &b_a, &w_b, &b_b, &w_c, &b_c, &w_v, &w_out})
       if (t->requires_grad())
-        return LayerNode::apply(x, w_a, b_a, w_b, b_b, w_c, b_c, w_v, w_out, heads, kv_heads, slices_in, slices_out);
+        return LayerNode::apply(x, w_a, b_a, w_b, b_b, w_c, b_c, w_v, w_out, heads, kv_heads, slices_in, slices_out, round_products);
   }
-  return LayerNode::forward(nullptr, x, w_a, b_a, w_b, b_b, w_c, b_c, w_v, w_out, heads, kv_heads, slices_in, slices_out);
+  return LayerNode::forward(nullptr, x, w_a, b_a, w_b, b_b, w_c, b_c, w_v, w_out, heads, kv_heads, slices_in, slices_out, round_products);
 }
 
 // One token through the layer's input projections and the step of its mixing stage (the caller applies proj_out): x [B, K]
@@ -662,10 +664,10 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("forward_log", &forward_log, py::arg("gate"), py::arg("x"), py::arg("y"), py::arg("k"));
   m.def("backward_log", &backward_log, py::arg("gate"), py::arg("x"), py::arg("dy"), py::arg("dx"), py::arg("dgate"), py::arg("k"));
   m.def("mix_forward", &mix_forward, py::arg("a_logit"), py::arg("b_logit"), py::arg("c"), py::arg("v"), py::arg("out"),
-        py::arg("heads"), py::arg("kv_heads"), py::arg("qkv_gate") = false);
+        py::arg("heads"), py::arg("kv_heads"), py::arg("qkv_gate") = false, py::arg("round_products") = false);
   m.def("mix_backward", &mix_backward, py::arg("a_logit"), py::arg("b_logit"), py::arg("c"), py::arg("v"), py::arg("dout"),
         py::arg("da_logit"), py::arg("db_logit"), py::arg("dc"), py::arg("dv"), py::arg("heads"), py::arg("kv_heads"),
-        py::arg("sums") = std::vector<at::Tensor>(), py::arg("qkv_gate") = false);
+        py::arg("sums") = std::vector<at::Tensor>(), py::arg("qkv_gate") = false, py::arg("round_products") = false);
   m.def("btp_log_autograd", &btp_log_autograd, py::arg("gate"), py::arg("x"), py::arg("k"), py::arg("y_f32"),
         "y = btp(exp(gate), x) with its autograd node (contiguous plain tensors; gradients: dgate float32, dx in x's dtype)");
   m.def("mix_autograd", &mix_autograd, py::arg("a_logit"), py::arg("b_logit"), py::arg("c"), py::arg("v"), py::arg("heads"),
@@ -674,7 +676,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("mix_prefill", &mix_prefill, py::arg("a_logit"), py::arg("b_logit"), py::arg("c"), py::arg("v"), py::arg("heads"),
         py::arg("kv_heads"), "[out, h, r, c_prev, pos]: a prompt of any length through the mixing stage, with the state after it");
   m.def("layer", &layer, py::arg("x"), py::arg("w_a"), py::arg("b_a"), py::arg("w_b"), py::arg("b_b"), py::arg("w_c"), py::arg("b_c"),
-        py::arg("w_v"), py::arg("w_out"), py::arg("heads"), py::arg("kv_heads"), py::arg("slices_in"), py::arg("slices_out"),
+        py::arg("w_v"), py::arg("w_out"), py::arg("heads"), py::arg("kv_heads"), py::arg("slices_in"), py::arg("slices_out"), py::arg("round_products"),
         "a whole layer call with its autograd node (plain bf16 tensors)");
   m.def("linears", [](const at::Tensor& x, const std::vector<at::Tensor>& w, const std::vector<std::optional<at::Tensor>>& b) {
     std::vector<at::Tensor> biases;

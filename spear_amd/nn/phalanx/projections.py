@@ -214,6 +214,8 @@ def plain_operands(x: torch.Tensor, *linears) -> list[torch.Tensor] | None:
     calls (``_plain_eager``), and layouts that 16-byte accesses do not fit."""
     from spear_amd.ops.btp.interface import _plain_eager
 
+    if torch._C._get_tracing_state() is not None or torch.autograd.forward_ad._current_level >= 0:
+        return None  # torch.jit.trace has to see the ops; tangents have to meet the nodes that refuse or carry them
     ops = []
     for proj, has_bias in linears:
         if type(proj) is not torch.nn.Linear or proj._forward_hooks or proj._forward_pre_hooks or proj._backward_hooks \
@@ -235,9 +237,11 @@ def plain_operands(x: torch.Tensor, *linears) -> list[torch.Tensor] | None:
     return ops
 
 
-def layer_call(x: torch.Tensor, proj_a, proj_b, proj_c, proj_v, proj_out, heads: int, kv_heads: int) -> torch.Tensor | None:
+def layer_call(x: torch.Tensor, proj_a, proj_b, proj_c, proj_v, proj_out, heads: int, kv_heads: int,
+               round_products: bool) -> torch.Tensor | None:
     """The whole layer on ``x[B, L, K]`` as one autograd node compiled into the binding (``LayerNode`` in
-    ``btp_torch_ext.cpp``), or None where the call is for the modules and the Python nodes of this file: what
+    ``btp_torch_ext.cpp``; ``round_products``: gates and gated inputs
+    rounded to 16 bits as the tensors that :func:`btp` takes), or None where the call is for the modules and the Python nodes of this file: what
     ``plain_operands`` leaves to them, lengths and sizes that the mixing kernels refuse, and a row of gradients of 2 GiB.
     Forward + backward, us, modules and Python nodes / compiled: B=8 L=128 dim=512 562 / 245, B=1024 1330 / 1307,
     B=64 L=2048 dim=2048 8152 / 7992."""
@@ -250,7 +254,8 @@ def layer_call(x: torch.Tensor, proj_a, proj_b, proj_c, proj_v, proj_out, heads:
     if operands is None or operands[-2].shape != (heads * 16, K) or operands[-1].shape != (K, heads * 16):
         return None
     M = x.numel() // K
-    return _btp.load_extension().layer(x.contiguous(), *operands, heads, kv_heads, slice_count(M, ld, K), slice_count(M, K, heads * 16))
+    return _btp.load_extension().layer(x.contiguous(), *operands, heads, kv_heads, slice_count(M, ld, K),
+                                       slice_count(M, K, heads * 16), round_products)
 
 
 def project_and_mix(x: torch.Tensor, proj_a, proj_b, proj_c, proj_v, heads: int, kv_heads: int) -> torch.Tensor:

@@ -227,7 +227,7 @@ class Phalanx(nn.Module):
         """A plain bf16 call as one compiled autograd node around the fused mixing kernels, or None where the call is for the
         composition of modules below.
 
-        For ``"default"`` this takes the place of the stand-alone recurrence between about twenty elementwise and transposing
+        For ``"default"``, whose gates and gated inputs keep the 16 bits in which :func:`btp` takes them, this takes the place of the stand-alone recurrence between about twenty elementwise and transposing
         passes. Forward + backward, us, stand-alone / one node: B=1024 L=128 dim=512 4692 / 1307, B=8 822 / 245; no size was
         found where the stand-alone kernels win. They keep every call that the fused ones would answer in another way:
         k = 1, other types than bf16 throughout, autocast, anything that traces or transforms the call, hooked or replaced
@@ -238,13 +238,15 @@ class Phalanx(nn.Module):
             return None
         from spear_amd.ops.btp import btp, interface, phalanx_mix
 
-        if self._forward_fn == self._forward_default:
+        default = self._forward_fn == self._forward_default
+        if default:
             if not (self.btp_module is btp and self.k == 2 and self.wpb in interface.SUPPORTED_WPB
                     and self.output_dtype == p.compute_dtype and interface._FORWARD_FLAGS == 0):
                 return None
         elif self.mix_module is not phalanx_mix:
             return None
-        return layer_call(x.to(p.compute_dtype), p.proj_a, p.proj_b, p.proj_c, p.proj_v, self.proj_out, self.heads, self.kv_heads)
+        return layer_call(x.to(p.compute_dtype), p.proj_a, p.proj_b, p.proj_c, p.proj_v, self.proj_out, self.heads, self.kv_heads,
+                          round_products=default)
 
     def _forward_default(self, x: torch.Tensor) -> torch.Tensor:
         y = self._as_one_node(x)

@@ -293,8 +293,8 @@ def test_qkv_form_backward_against_the_oracle(H, Hkv):
 
 @pytest.mark.parametrize("B,L,dim,kv_heads", [(1, 16, 16, None), (3, 48, 96, 2), (8, 128, 512, None), (64, 144, 80, 1)])
 def test_default_layer_mixes_in_the_fused_kernels(B, L, dim, kv_heads):
-    """A plain bf16 call of a default layer has the fused layer's bits, below and above the 8192 tokens from which the
-    projections' backward is shared, and lies as close to the stand-alone composition as two bf16 roundings allow."""
+    """A plain bf16 call of a default layer lies as close to the fused layer and to the stand-alone composition as their bf16
+    roundings allow, below and above the 8192 tokens from which the weight gradients are cut into slices."""
     from spear_amd import Phalanx, btp
 
     torch.manual_seed(11)
@@ -313,8 +313,8 @@ def test_default_layer_mixes_in_the_fused_kernels(B, L, dim, kv_heads):
 
     assert layer._as_one_node(x) is not None
     got = run(layer)
-    for a, b in zip(got, run(fused)):
-        assert torch.equal(a, b)
+    for i, (a, b) in enumerate(zip(got, run(fused))):  # they differ in roundings to 16 bits on the way
+        assert (a.float() - b.float()).norm() <= 2 ** -9 * 10 * b.float().norm(), i
     layer.btp_module = lambda *args: btp(*args)  # a replaced recurrence is called: the stand-alone composition
     assert layer._as_one_node(x) is None
     for i, (a, b) in enumerate(zip(got, run(layer))):
@@ -335,6 +335,11 @@ def test_calls_that_stay_with_the_stand_alone_kernels():
         assert layer._as_one_node(x) is None
     with torch.device(DEV):  # a function mode
         assert layer._as_one_node(x) is None
+    with torch.autograd.forward_ad.dual_level():
+        assert layer._as_one_node(x) is None
+    with torch.no_grad():  # a trace records the ops and not one call's result
+        traced, other = torch.jit.trace(layer, x, check_trace=False), x.flip(0, 1)
+        assert (traced(other).float() - layer(other).float()).norm() <= 10 * 2 ** -9 * layer(other).float().norm()
     handle = layer.param.proj_c.register_forward_hook(lambda *a: None)
     assert layer._as_one_node(x) is None
     handle.remove()
