@@ -237,7 +237,8 @@ int spear_phalanx_mix_step(const void* a_logit, const void* b_logit, const void*
  * block_len = 16 and a in x_dtype (a_t or log a_t) or fp32 log(a_t) run the tiled kernel (HBM-bound; rows
  * whose length is not a multiple of 8 or that are not 16-byte aligned are realigned in registers, at
  * 0.5-0.65 of peak instead of 0.75); everything else (fp32 tensors, other D / block_len, fp32 linear a_t)
- * runs a tile kernel of any element type, alignment, D and block_len up to 256 (beyond that one thread per block). */
+ * runs a tile kernel of any element type, alignment and D, or one thread per block where rows or blocks have too few
+ * steps for tiles to pay off and where min(block_len, L) is above 256. Both take the same steps in the same order. */
 int spear_jagged_prefill(const void* a, const void* x, const void* c, const void* v, const void* carry_init, void* y,
                          void* h_tail, void* r_tail, void* c_prev_tail, int B, int H, int D, int L, int block_len,
                          int a_dtype, int x_dtype, int state_dtype, int r_dtype, unsigned flags, void* stream);

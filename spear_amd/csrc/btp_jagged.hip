@@ -272,7 +272,9 @@ struct TileArgs {
   void *y, *h_tail, *r_tail, *c_prev_tail;
   long rd_total;     // channel rows: B * H * D
   long tensor_bytes;
-  int D, L, block_len, nblk;
+  int D, L, nblk;
+  int block_len;  // of the tiles: the streaming form's, or L where that is longer than the rows
+  int whole;      // steps of a complete block
   int a_dtype, log_a, state_dtype, r_dtype;
   int lanes, per_lane;    // lane groups in use, blocks per lane group
   int spans;              // tiles per channel row
@@ -528,8 +530,8 @@ __global__ __launch_bounds__(64 * kTileWaves) void jagged_prefill_tile_kernel(co
       }
       const long o = rd0 + d;
       store_scalar(p.h_tail, o, p.state_dtype, h);
-      store_scalar(p.c_prev_tail, o, p.state_dtype, len == bl ? h : prev);
-      if (o % p.D == 0) store_scalar(p.r_tail, o / p.D, p.r_dtype, len == bl ? 1.0f : r);
+      store_scalar(p.c_prev_tail, o, p.state_dtype, len == p.whole ? h : prev);
+      if (o % p.D == 0) store_scalar(p.r_tail, o / p.D, p.r_dtype, len == p.whole ? 1.0f : r);
     }
   }
 
@@ -621,8 +623,8 @@ __global__ __launch_bounds__(64 * kTileWaves) void jagged_prefill_tile_kernel(co
 }
 
 // ==========================================================================================
-// Prefill, element-granular: blocks too long for a tile in LDS (block_len above kMaxTileBlock), or rows too long for the tile
-// kernel's 32-bit offsets. One thread per (row, channel, block); lanes run over blocks.
+// Prefill, element-granular: rows and blocks of few steps (tiles_pay_off), blocks too long for a tile in LDS (above
+// kMaxTileBlock), or rows too long for the tile kernel's 32-bit offsets. One thread per (row, channel, block); lanes run over blocks.
 // ==========================================================================================
 template <class T>
 __global__ __launch_bounds__(256) void jagged_prefill_any_kernel(
@@ -852,9 +854,25 @@ void launch_prefill_any(const JagPrefillArgs& p, hipStream_t s) {
 }
 
 
-// Longest block the tile kernel takes: its image holds two blocks of 16 channel rows in fp32 per wavefront, 33 KiB at
-// 256 steps, and four wavefronts' images have to fit the 160 KiB of a compute unit.
+// Longest block the tile kernel takes: its image holds two blocks of 16 channel rows in fp32 and their gates per wavefront, 34.25 KiB
+// at 256 steps, and four wavefronts' images have to fit the 160 KiB of a compute unit.
 constexpr int kMaxTileBlock = 256;
+
+// How blocks of `block_len` <= L steps make a tile: about 64 steps, as at most four lane groups of whole blocks. Tiles of 128 steps measured
+// the same or slower: 177 -> 184 us in fp32 at B=1024 H=32 L=128, 78 us either way in bf16 at B=16 H=16 D=64 L=2048 in blocks of 64.
+struct TileShape {
+  int per_lane, lanes, width, spans;  // blocks per lane group, lane groups, steps of a tile, tiles per row
+};
+TileShape tile_shape(int block_len, int L) {
+  constexpr int steps = 64;
+  TileShape t;
+  t.per_lane = block_len < steps / 4 ? steps / 4 / block_len : 1;
+  const int chunk = t.per_lane * block_len;
+  t.lanes = chunk > steps ? 1 : steps / chunk > 4 ? 4 : steps / chunk;
+  t.width = t.lanes * chunk;
+  t.spans = (L + t.width - 1) / t.width;
+  return t;
+}
 
 template <class T, int kG, int kN>
 hipError_t launch_tile_as(const TileArgs& t, bool shared, hipStream_t s) {
@@ -881,8 +899,9 @@ hipError_t launch_prefill_tile(const JagPrefillArgs& p, hipStream_t s) {
   t.y = p.y; t.h_tail = p.h_tail; t.r_tail = p.r_tail; t.c_prev_tail = p.c_prev_tail;
   t.rd_total = (long)p.B * p.H * p.D;
   t.tensor_bytes = t.rd_total * p.L * kBytes;
-  t.D = p.D; t.L = p.L; t.block_len = p.block_len;
-  t.nblk = (p.L + p.block_len - 1) / p.block_len;
+  t.D = p.D; t.L = p.L; t.whole = p.block_len;
+  const int block_len = t.block_len = p.block_len < p.L ? p.block_len : p.L;
+  t.nblk = (p.L + block_len - 1) / block_len;
   t.a_dtype = p.a_dtype; t.log_a = p.log_a ? 1 : 0; t.state_dtype = p.state_dtype; t.r_dtype = p.r_dtype;
   // The widest granule whose grid every row of every tensor (and, with block lengths on that grid, every tile of a row)
   // starts on.
@@ -890,17 +909,14 @@ hipError_t launch_prefill_tile(const JagPrefillArgs& p, hipStream_t s) {
     auto on = [&](const void* q) { return (reinterpret_cast<uintptr_t>(q) % bytes) == 0; };
     return on(p.x) && on(p.c) && on(p.v) && on(p.y);
   };
-  const bool wide = all_on(16) && ((long)p.L * kBytes) % 16 == 0 && (p.block_len * kBytes) % 16 == 0;
+  const bool wide = all_on(16) && ((long)p.L * kBytes) % 16 == 0 && (block_len * kBytes) % 16 == 0;
   const int granule = wide ? 16 : all_on(4) ? 4 : 2;
   const int per_granule = granule / kBytes;
-  // About 64 steps per tile, as at most four lane groups of whole blocks. Tiles of 128 steps measured the same or slower: 177 -> 184 us
-  // in fp32 at B=1024 H=32 L=128, 78 us either way in bf16 at B=16 H=16 D=64 L=2048 in blocks of 64.
-  constexpr int steps = 64;
-  t.per_lane = p.block_len < steps / 4 ? steps / 4 / p.block_len : 1;
-  const int chunk = t.per_lane * p.block_len;
-  t.lanes = chunk > steps ? 1 : steps / chunk > 4 ? 4 : steps / chunk;
-  const int W = t.lanes * chunk, pad = (p.block_len + 3) & ~3;
-  t.spans = (t.nblk + t.lanes * t.per_lane - 1) / (t.lanes * t.per_lane);
+  const TileShape shape = tile_shape(block_len, p.L);
+  t.per_lane = shape.per_lane;
+  t.lanes = shape.lanes;
+  t.spans = shape.spans;
+  const int W = shape.width, pad = (block_len + 3) & ~3;
   t.tiles = (t.rd_total + kTileRows - 1) / kTileRows * t.spans;
   const int chunks = (pad + W + 3) / 4;
   t.stride = 4 * (chunks | 1);  // an odd number of 16-byte chunks: 16 rows' reads of one column spread over the banks
@@ -908,7 +924,7 @@ hipError_t launch_prefill_tile(const JagPrefillArgs& p, hipStream_t s) {
   // a 16-bit row that starts on a word's second half covers one word more
   const int extra = kBytes == 2 && granule == 4 ? 1 : 0;
   t.main_gpr = (W + per_granule - 1) / per_granule + extra;
-  t.halo_gpr = (p.block_len + per_granule - 1) / per_granule + extra;
+  t.halo_gpr = (block_len + per_granule - 1) / per_granule + extra;
   t.main_magic = ((1u << 20) + t.main_gpr - 1) / t.main_gpr;
   t.halo_magic = ((1u << 20) + t.halo_gpr - 1) / t.halo_gpr;
   const bool shared = p.D % kTileRows == 0;  // a tile's channel rows then share one gate row
@@ -921,12 +937,33 @@ hipError_t launch_prefill_tile(const JagPrefillArgs& p, hipStream_t s) {
   }
 }
 
-// 32-bit offsets inside the 16 rows of a tile, and a grid of 31 bits
+// Which kernel a prompt takes. A tile has room for about 64 steps of a row and its lanes walk whole blocks, so rows and blocks of few steps
+// leave much of it idle; one thread per block is wasteful where its neighbours' words lie far apart (long blocks) and the tensors
+// are larger than the L2 caches. Tile kernel / one thread per block, us, D=16 (16 channel rows share a gate row) and D=5 (they don't):
+//   fp32, 128 MiB per tensor: L=96 in blocks of 16 85 / 1446, 197 / 1518; of 8 86 / 481, 166 / 504; of 4 86 / 238, 142 / 248; of 2
+//     130 / 169, 209 / 171; L=9 in blocks of 9 or more 507 / 650, 877 / 672 (bf16 2.3 and 2.7 times as long in tiles)
+//   fp32, 2 MiB: L=96 in blocks of 16 5.1 / 14.8, 11.1 / 15.4; of 8 5.5 / 8.5, 10.2 / 8.7; of 4 5.7 / 6.1, 9.2 / 6.1
+//   bf16, 8 MiB: L=96 in blocks of 8 10.5 / 31.8, 17.7 / 38.6; of 4 18.1 / 18.0, 24.3 / 18.6
+// Over 9960 forms (L 5 to 1000, blocks of 1 to 200, D 1, 5, 16, 1 to 128 MiB, fp32 and bf16) the rule takes the slower kernel by more than
+// 3 % in 12, by 20 % at most (D=5, rows of 19), and 0.72 of the time of one thread per block in the geometric mean; the faster
+// one of the two each time would be 0.66, tiles throughout 0.93.
+bool tiles_pay_off(const JagPrefillArgs& p, int block_len, long row_bytes) {
+  const TileShape t = tile_shape(block_len, p.L);
+  const bool shared = p.D % kTileRows == 0, big = (long)p.B * p.H * p.D * row_bytes >= (8L << 20);
+  const double used = (double)p.L / ((double)t.spans * t.width);  // of the tiles' columns
+  if (block_len >= 16) return big || (shared && used >= 0.45);
+  if (block_len >= 8) return big && used >= 0.6;
+  return block_len >= 4 && big && shared && used >= 0.8;
+}
+
+// The tile kernel's limits: 32-bit offsets inside the 16 rows of a tile, and a grid of 31 bits
 template <class T>
 hipError_t launch_prefill_general(const JagPrefillArgs& p, hipStream_t s) {
   const long row_bytes = (long)p.L * (long)sizeof(typename Scalar<T>::type);
-  const long tiles_at_most = ((long)p.B * p.H * p.D / kTileRows + 1) * ((p.L + p.block_len - 1) / p.block_len);
-  if (p.block_len <= kMaxTileBlock && row_bytes * (kTileRows + 1) < 0x70000000L && tiles_at_most < (1L << 31))
+  const int block_len = p.block_len < p.L ? p.block_len : p.L;  // of a lane's work: rows shorter than a block end before it does
+  const long tiles_at_most = ((long)p.B * p.H * p.D / kTileRows + 1) * ((p.L + block_len - 1) / block_len);
+  if (block_len <= kMaxTileBlock && row_bytes * (kTileRows + 1) < 0x70000000L && tiles_at_most < (1L << 31) &&
+      tiles_pay_off(p, block_len, row_bytes))
     return launch_prefill_tile<T>(p, s);
   launch_prefill_any<T>(p, s);
   return hipGetLastError();

@@ -385,6 +385,74 @@ def test_prefill_tiles_of_any_type_block_length_and_head_size(D, L, bl, dtype, a
     assert_close(f64(y), want, *tol(dtype), "sequential form")
 
 
+# D, L, block_len, dtype, elements before the tensors: tensors of at least 8 MiB, which these forms need for tiles
+BIG_TILES = [(24, 131, 24, torch.float32, 0), (5, 97, 8, torch.bfloat16, 0), (1, 300, 200, torch.bfloat16, 1), (16, 96, 4, torch.float32, 0),
+             (48, 101, 5, torch.float32, 1), (48, 120, 12, torch.bfloat16, 0), (16, 77, 9, torch.float16, 1), (5, 19, 20, torch.float32, 0),
+             (16, 100, 300, torch.bfloat16, 0)]
+
+
+@pytest.mark.parametrize("D,L,bl,dtype,offset", BIG_TILES)
+def test_tiles_and_one_thread_per_block_give_the_same_bits(D, L, bl, dtype, offset):
+    """What a prompt of many rows gets is what each of its sequences gets alone, where too few rows for tiles go through
+    the kernel of one thread per block: both take the same steps in the same order."""
+    from spear_amd import _btp
+
+    H = 3
+    B = -(-(8 << 20) // (H * D * L * dtype.itemsize))
+    g = torch.Generator(device=DEV).manual_seed(L + bl)
+
+    def tensor(*shape, like=dtype):
+        return torch.randn(shape[0] * int(np.prod(shape[1:])) + offset, device=DEV, generator=g).to(like)[offset:].view(shape)
+
+    A = tensor(B, H, L).sigmoid_()
+    X, C, V = (tensor(B, H, D, L) for _ in range(3))
+    carry = tensor(B, H, D, like=torch.float32)
+
+    def run(rows, with_carry):
+        y = torch.full_like(X[rows], float("nan"))
+        if with_carry:
+            _btp.jagged_prefill(A[rows], X[rows], None, None, carry[rows], y, None, None, None, bl, False)
+            return [y]
+        n = y.shape[0]
+        h, cp = (torch.full((n, H, D), float("nan"), device=DEV) for _ in range(2))
+        r = torch.full((n, H), float("nan"), device=DEV)
+        _btp.jagged_prefill(A[rows], X[rows], C[rows], V[rows], None, y, h, r, cp, bl, False)
+        return [y, h, r, cp]
+
+    print(f"big tiles D={D} L={L} bl={bl} {dtype} offset={offset} B={B}", flush=True)
+    for with_carry in (False, True):
+        whole = run(slice(0, B), with_carry)
+        for b in (0, 1, B // 2, B - 1):
+            for name, all_rows, one in zip(("y", "h", "r", "c_prev"), whole, run(slice(b, b + 1), with_carry)):
+                assert torch.equal(all_rows[b:b + 1], one), (name, b, with_carry)
+
+
+def test_rows_shorter_than_a_block_cost_what_their_steps_cost():
+    """Nine steps are nine steps, however long the block that they begin is: the same results in about the same time (a kernel that
+    walks the whole block takes 15 times as long here)."""
+    from spear_amd import _btp
+
+    B, H, D, L = 2427, 8, 24, 9
+    A, X, C, V = (t.to(DEV) for t in make(B, H, D, L, seed=3, dtype=torch.float32))
+    ys, times = [], []
+    for bl in (16, 256):
+        y = torch.empty_like(X)
+        h, cp, r = torch.empty(B, H, D, device=DEV), torch.empty(B, H, D, device=DEV), torch.empty(B, H, device=DEV)
+        spans = []
+        for _ in range(6):
+            begin, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            begin.record()
+            for _ in range(20):
+                _btp.jagged_prefill(A, X, C, V, None, y, h, r, cp, bl, False)
+            end.record()
+            end.synchronize()
+            spans.append(begin.elapsed_time(end))
+        times.append(min(spans))
+        ys.append([y, h, r, cp])
+    assert all(torch.equal(a, b) for a, b in zip(*ys))
+    assert times[1] < 3 * times[0], times
+
+
 @pytest.mark.parametrize("case", ["full", "ragged", "short", "one_block", "bl4"])
 def test_kernels_match_the_reference_vectors(case):
     """The HIP prefill and decode kernels against vectors computed by the reference's own
