@@ -209,6 +209,7 @@ int spear_layer_prefill(const void* a_logit, const void* b_logit, const void* c,
                         float* c_prev, int* pos, int B, int L, int H, int kv_heads, int dtype, void* stream) {
   g_error[0] = '\0';
   const char* who = "spear_layer_prefill";
+  if (L < 1) return fail(SPEAR_BTP_EINVAL, "%s: a prompt has at least one step (got L=%d)", who, L);
   const void* const ptrs[5] = {a_logit, b_logit, c, v, out};
   if (int rc = check_mix_forward(who, ptrs, B, L, H, kv_heads, dtype, false)) return rc < 0 ? rc : 0;
   if (!h || !r || !c_prev || !pos) return fail(SPEAR_BTP_ENULL, "%s: NULL tensor pointer", who);

@@ -176,3 +176,13 @@ def test_streaming_entry_points_validate_on_the_host():
     assert step(p, p, None, None, p, p, p, p, p, p, p, 1, 1, 16, 0, 0, 0, 7, 0, 0, 0.0, None) == -1
     assert step(p, p, None, None, p, p, p, p, p, p, p, 0, 1, 16, 0, 0, 0, 0, 0, 0, 0.0, None) == 0
     assert lib.spear_btp_last_error() == b""
+
+
+def test_a_prompt_without_steps_is_refused():
+    """There is no state to hand over after it; the arrays would come back unwritten."""
+    from spear_amd import _btp
+
+    lib = _btp.load_library()
+    for B in (0, 2):
+        assert lib.spear_layer_prefill(*[None] * 9, B, 0, 4, 4, 0, None) == -1
+        assert b"at least one step" in lib.spear_btp_last_error()

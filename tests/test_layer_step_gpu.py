@@ -293,3 +293,14 @@ def test_hooked_projections_are_called_and_give_the_same_step():
     assert calls == [1]
     assert_close(f64(y), f64(y_hooked), 2e-2, 2e-2, "y")
     assert_close(f64(one.h_loc), f64(two.h_loc), 2e-2, 2e-2, "h")
+
+
+def test_prefill_refuses_an_empty_prompt_and_takes_an_empty_batch():
+    from spear_amd.nn.phalanx.inference import phalanx_prefill
+
+    layer = _layer(dim=64, seed=7)
+    x = torch.zeros(2, 3, 64, device=DEV, dtype=torch.bfloat16)
+    with pytest.raises(ValueError, match="at least one token"):
+        phalanx_prefill(layer, x[:, :0])
+    y, st = phalanx_prefill(layer, x[:0])
+    assert y.shape == (0, 3, 64) and st.h_loc.shape == (0, 4, 16) and st.pos.shape == (0,)
