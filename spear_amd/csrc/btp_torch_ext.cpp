@@ -419,16 +419,20 @@ void layer_sums(const std::vector<at::Tensor>& in, const std::vector<at::Tensor>
   if (rc != 0) raise_native(rc);
 }
 
-// x [M, K] through up to four linear layers in one launch (bf16; biases may be undefined): [M, N_i] each.
+// x [..., K] through up to four linear layers in one launch (bf16; biases may be undefined): [..., N_i] each, allocated in that shape (a
+// view of a matrix would leave an autograd node as a view, on which callers could not work in place). x dense, or [M, K] with dense rows.
 std::vector<at::Tensor> linears(const at::Tensor& x, const std::vector<at::Tensor>& weights, const std::vector<at::Tensor>& biases,
                                 int* pos = nullptr, int64_t block_len = 0) {
-  TORCH_CHECK(x.is_cuda() && x.dim() == 2 && x.stride(1) == 1 && x.scalar_type() == at::kBFloat16, "x must be [M, K] bfloat16 CUDA with dense rows.");
+  TORCH_CHECK(x.is_cuda() && x.dim() >= 2 && x.scalar_type() == at::kBFloat16, "x must be a bfloat16 CUDA tensor of two dimensions or more.");
+  const bool rows = x.dim() == 2;
+  TORCH_CHECK(rows ? x.stride(1) == 1 : x.is_contiguous(), "x must have dense rows, and be dense where it has more than two dimensions.");
   TORCH_CHECK(!weights.empty() && weights.size() <= 4 && biases.size() == weights.size(), "1 to 4 layers.");
-  const int64_t M = x.size(0), K = x.size(1);
+  const int64_t K = x.size(-1), M = K > 0 ? x.numel() / K : 0;
   const void *w[4], *b[4];
   void* o[4];
   int N[4];
   std::vector<at::Tensor> out;
+  std::vector<int64_t> sizes = x.sizes().vec();
   for (size_t i = 0; i < weights.size(); ++i) {
     const int64_t n = weights[i].size(0);
     check_layout("weight", weights[i], {n, K});
@@ -438,14 +442,15 @@ std::vector<at::Tensor> linears(const at::Tensor& x, const std::vector<at::Tenso
       TORCH_CHECK(biases[i].scalar_type() == at::kBFloat16, "biases must be bfloat16.");
     }
     check_same_device({&x, &weights[i], &biases[i]});
-    out.push_back(at::empty({M, n}, x.options()));
+    sizes.back() = n;
+    out.push_back(at::empty(sizes, x.options()));
     w[i] = weights[i].data_ptr();
     b[i] = biases[i].defined() ? biases[i].data_ptr() : nullptr;
     o[i] = out[i].data_ptr();
     N[i] = (int)n;
   }
   const c10::DeviceGuard guard(x.device());
-  const int rc = spear_layer_linear((int)weights.size(), x.data_ptr(), M > 1 ? x.stride(0) : K, (int)M, (int)K, w, b, o, N, pos, (int)block_len,
+  const int rc = spear_layer_linear((int)weights.size(), x.data_ptr(), rows && M > 1 ? x.stride(0) : K, (int)M, (int)K, w, b, o, N, pos, (int)block_len,
                                     stream_of(x));
   if (rc != 0) raise_native(rc);
   return out;
@@ -462,17 +467,9 @@ std::vector<at::Tensor> project(const at::Tensor& x, const std::vector<at::Tenso
   const int64_t K = x.size(-1), M = K > 0 ? x.numel() / K : 0;
   int64_t columns = 0;
   for (const at::Tensor& w : weights) columns += w.size(0);
+  if (small_products(M, columns, K, weights.size()) && (reinterpret_cast<uintptr_t>(x.data_ptr()) & 15u) == 0) return linears(x, weights, biases);
   std::vector<at::Tensor> out;
-  if (small_products(M, columns, K, weights.size()) && (reinterpret_cast<uintptr_t>(x.data_ptr()) & 15u) == 0) {
-    out = linears(x.view({M, K}), weights, biases);
-    auto sizes = x.sizes().vec();
-    for (at::Tensor& t : out) {
-      sizes.back() = t.size(1);
-      t = t.view(sizes);
-    }
-  } else {
-    for (size_t i = 0; i < weights.size(); ++i) out.push_back(biases[i].defined() ? at::linear(x, weights[i], biases[i]) : at::linear(x, weights[i]));
-  }
+  for (size_t i = 0; i < weights.size(); ++i) out.push_back(biases[i].defined() ? at::linear(x, weights[i], biases[i]) : at::linear(x, weights[i]));
   return out;
 }
 
@@ -553,7 +550,11 @@ struct LayerNode : public torch::autograd::Function<LayerNode> {
       out[4] = sums[1];
       out[6] = sums[2];
       const at::Tensor d2 = packed.view({M, ld});
-      if (ctx->needs_input_grad(0)) out[0] = at::mm(d2, stacked).view(x.sizes());
+      if (ctx->needs_input_grad(0)) {
+        out[0] = at::empty(x.sizes(), x.options());  // not a view of the product, for callers that work on it in place
+        at::Tensor dx = out[0].view({M, K});
+        at::mm_out(dx, d2, stacked);
+      }
       if (weights) {
         const at::Tensor dw = weight_grad(d2, x2, ctx->saved_data["slices_in"].toInt(), parts, sums);
         out[3] = dw.narrow(0, 0, Fkv);

@@ -391,3 +391,33 @@ def test_layer_node_is_differentiable_once_and_says_so():
     assert torch.equal(plain, again.detach())
     with pytest.raises(RuntimeError, match="differentiated again"):
         again.float().square().sum().backward()
+
+
+@pytest.mark.parametrize("method", ["default", "fused"])
+@pytest.mark.parametrize("B,L,dim", [(2, 16, 16), (8, 128, 512), (4, 32, 1024), (64, 144, 80)])
+def test_a_layers_results_can_be_worked_on_in_place(B, L, dim, method):
+    """Residual connections, scales and masks written into a layer's output, under autograd and after no_grad, and trainable terms
+    added to the input's gradient: with the output projection in a kernel of this library and in the library's product."""
+    from spear_amd import Phalanx
+    from spear_amd.nn.phalanx.inference import phalanx_prefill
+
+    torch.manual_seed(31)
+    layer = Phalanx(dim=dim, length=L, method=method, dtype=torch.bfloat16).to(DEV)
+    x = torch.randn(B, L, dim, device=DEV).bfloat16().requires_grad_(True)
+    dy = torch.randn(B, L, dim, device=DEV).bfloat16()
+
+    def grads(y):
+        return torch.autograd.grad(y, [x, *layer.parameters()], dy)
+
+    y = layer(x)
+    y += x
+    y *= 2
+    want = grads((layer(x) + x) * 2)
+    assert all(torch.equal(a, b) for a, b in zip(grads(y), want))
+    scale = torch.full((dim,), 2.0, device=DEV, dtype=torch.bfloat16, requires_grad=True)
+    with torch.no_grad():
+        plain = [layer(x), phalanx_prefill(layer, x)[0]]
+    for t in plain + [torch.autograd.grad(layer(x), x, dy)[0]]:
+        before = t.clone()
+        t *= scale
+        assert torch.equal(t, before * 2) and t.requires_grad
