@@ -304,3 +304,27 @@ def test_prefill_refuses_an_empty_prompt_and_takes_an_empty_batch():
         phalanx_prefill(layer, x[:, :0])
     y, st = phalanx_prefill(layer, x[:0])
     assert y.shape == (0, 3, 64) and st.h_loc.shape == (0, 4, 16) and st.pos.shape == (0,)
+
+
+@pytest.mark.parametrize("B", [1, 5, 64])
+@pytest.mark.parametrize("layout", ["expanded", "overlapping", "wide_rows", "unaligned", "columns", "odd_stride"])
+def test_step_takes_tokens_in_any_layout(layout, B):
+    """Rows that are one row, that overlap, that lie apart, that start off the 16-byte grid, that are columns: the step of the same
+    values laid out densely, up to the roundings of the projections to 16 bits that the general path makes."""
+    from spear_amd.nn.phalanx.inference import PhalanxStepState, phalanx_step
+
+    dim, layer = 128, _layer(dim=128, seed=9)
+    g = torch.Generator().manual_seed(10)
+    base = torch.randn(B + 1, 2 * dim, generator=g).bfloat16().to(DEV)
+    x = {"expanded": lambda: base[0, :dim].expand(B, dim),
+         "overlapping": lambda: base.view(-1).as_strided((B, dim), (8, 1)),
+         "wide_rows": lambda: base[:B, dim:],
+         "unaligned": lambda: base.view(-1)[1:1 + B * dim].view(B, dim),
+         "columns": lambda: base.view(-1)[:B * dim].view(dim, B).t(),
+         "odd_stride": lambda: base.view(-1).as_strided((B, dim), (dim + 1, 1))}[layout]()
+    one, two = PhalanxStepState.zeros(B, dim // 16, DEV), PhalanxStepState.zeros(B, dim // 16, DEV)
+    for _ in range(2):
+        y, want = phalanx_step(layer, x, one), phalanx_step(layer, x.contiguous(), two)
+    assert_close(f64(y), f64(want), 2e-2, 2e-2, "y")
+    assert_close(f64(one.h_loc), f64(two.h_loc), 2e-2, 2e-2, "h")
+    assert one.pos.tolist() == [2] * B
