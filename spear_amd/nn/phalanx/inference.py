@@ -311,7 +311,7 @@ class PhalanxStepState:
 
 def _layer_operands(layer, x: torch.Tensor):
     p, F = layer.param, layer.heads * 16
-    ops = plain_operands(x, (p.proj_a, True), (p.proj_b, True), (p.proj_c, True), (p.proj_v, False), (layer.proj_out, False))
+    ops = plain_operands(x, x.dtype, (p.proj_a, True), (p.proj_b, True), (p.proj_c, True), (p.proj_v, False), (layer.proj_out, False))
     return ops if ops is not None and ops[-2].shape == (F, x.shape[-1]) and ops[-1].shape[1] == F else None
 
 

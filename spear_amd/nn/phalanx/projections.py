@@ -208,13 +208,15 @@ class _ProjectAndMix(torch.autograd.Function):
                 rows_of("c", need[5]), s_c if need[6] else None, rows_of("v", need[7]), None, None)
 
 
-def plain_operands(x: torch.Tensor, *linears) -> list[torch.Tensor] | None:
+def plain_operands(x: torch.Tensor, dtype: torch.dtype, *linears) -> list[torch.Tensor] | None:
     """Weights and biases of ``(module, has_bias)`` pairs for the compiled paths that take them as they lie, or None where
-    a call has to go through the modules: other types than bf16, replaced or hooked modules, autocast, traced or transformed
+    a call has to go through the modules: other types than bf16 (``dtype`` is the one in which ``x`` goes through them; it need not be
+    cast yet), replaced or hooked modules, autocast, traced or transformed
     calls (``_plain_eager``), and layouts that 16-byte accesses do not fit."""
     from spear_amd.ops.btp.interface import _plain_eager
 
-    if torch._C._get_tracing_state() is not None or torch.autograd.forward_ad._current_level >= 0:
+    if dtype != torch.bfloat16 or torch.is_autocast_enabled("cuda") or torch._C._get_tracing_state() is not None \
+            or torch.autograd.forward_ad._current_level >= 0:
         return None  # torch.jit.trace has to see the ops; tangents have to meet the nodes that refuse or carry them
     ops = []
     for proj, has_bias in linears:
@@ -230,16 +232,16 @@ def plain_operands(x: torch.Tensor, *linears) -> list[torch.Tensor] | None:
                 return None
             ops.append(b)
     device = x.device
-    if x.dtype != torch.bfloat16 or any(t.dtype != torch.bfloat16 or t.device != device for t in ops):
+    if any(t.dtype != torch.bfloat16 or t.device != device for t in ops):
         return None
-    if _nn_module._has_any_global_hook() or torch.is_autocast_enabled("cuda") or not _plain_eager(x, *ops):
+    if _nn_module._has_any_global_hook() or not _plain_eager(x, *ops):
         return None
     return ops
 
 
-def layer_call(x: torch.Tensor, proj_a, proj_b, proj_c, proj_v, proj_out, heads: int, kv_heads: int,
+def layer_call(x: torch.Tensor, dtype: torch.dtype, proj_a, proj_b, proj_c, proj_v, proj_out, heads: int, kv_heads: int,
                round_products: bool) -> torch.Tensor | None:
-    """The whole layer on ``x[B, L, K]`` as one autograd node compiled into the binding (``LayerNode`` in
+    """The whole layer on ``x[B, L, K]``, cast to ``dtype`` once the call is taken, as one autograd node compiled into the binding (``LayerNode`` in
     ``btp_torch_ext.cpp``; ``round_products``: gates and gated inputs
     rounded to 16 bits as the tensors that :func:`btp` takes), or None where the call is for the modules and the Python nodes of this file: what
     ``plain_operands`` leaves to them, lengths and sizes that the mixing kernels refuse, and a row of gradients of 2 GiB.
@@ -250,11 +252,11 @@ def layer_call(x: torch.Tensor, proj_a, proj_b, proj_c, proj_v, proj_out, heads:
     ld, K = packed_columns(heads, kv_heads)[1], x.shape[2]
     if 2 * x.shape[1] * ld >= 1 << 31 or K % 8 != 0:
         return None
-    operands = plain_operands(x, (proj_a, True), (proj_b, True), (proj_c, True), (proj_v, False), (proj_out, False))
+    operands = plain_operands(x, dtype, (proj_a, True), (proj_b, True), (proj_c, True), (proj_v, False), (proj_out, False))
     if operands is None or operands[-2].shape != (heads * 16, K) or operands[-1].shape != (K, heads * 16):
         return None
     M = x.numel() // K
-    return _btp.load_extension().layer(x.contiguous(), *operands, heads, kv_heads, slice_count(M, ld, K),
+    return _btp.load_extension().layer(x.to(dtype).contiguous(), *operands, heads, kv_heads, slice_count(M, ld, K),
                                        slice_count(M, K, heads * 16), round_products)
 
 

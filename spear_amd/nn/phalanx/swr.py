@@ -245,7 +245,7 @@ class Phalanx(nn.Module):
                 return None
         elif self.mix_module is not phalanx_mix:
             return None
-        return layer_call(x.to(p.compute_dtype), p.proj_a, p.proj_b, p.proj_c, p.proj_v, self.proj_out, self.heads, self.kv_heads,
+        return layer_call(x, p.compute_dtype, p.proj_a, p.proj_b, p.proj_c, p.proj_v, self.proj_out, self.heads, self.kv_heads,
                           round_products=default)
 
     def _forward_default(self, x: torch.Tensor) -> torch.Tensor:

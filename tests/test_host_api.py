@@ -371,6 +371,26 @@ def test_the_compiled_autograd_node_is_for_plain_eager_tensors_only():
     assert _plain_eager(t)
 
 
+@pytest.mark.parametrize("method", ["default", "fused"])
+def test_a_call_that_the_compiled_layer_leaves_is_not_cast_for_it(method):
+    """The decision comes before the cast to 16 bits, which the composition then makes itself: not twice."""
+    from torch.utils._python_dispatch import TorchDispatchMode
+
+    class Ops(TorchDispatchMode):
+        def __init__(self):
+            super().__init__()
+            self.names = []
+
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            self.names.append(str(func))
+            return func(*args, **(kwargs or {}))
+
+    layer = Phalanx(dim=32, method=method, dtype=torch.bfloat16)
+    with Ops() as ops:
+        assert layer._as_one_node(torch.randn(2, 16, 32)) is None
+    assert not any("_to_copy" in name for name in ops.names), ops.names
+
+
 def test_streaming_module_surface_and_state_dataclass():
     from spear_amd.nn.phalanx import inference as inf
 
