@@ -231,7 +231,7 @@ class Phalanx(nn.Module):
         passes. Forward + backward, us, stand-alone / one node: B=1024 L=128 dim=512 4692 / 1307, B=8 822 / 245; no size was
         found where the stand-alone kernels win. They keep every call that the fused ones would answer in another way:
         k = 1, other types than bf16 throughout, autocast, anything that traces or transforms the call, hooked or replaced
-        projections (``plain_operands``), the matrix-core and checkpoint-store switches, a replaced recurrence or class, empty
+        projections (``plain_operands``), the matrix-core and checkpoint-store switches, a replaced recurrence, class or method, empty
         inputs, lengths and ``wpb`` that :func:`btp` refuses, and batch rows past the fused backward's 2 GiB."""
         p = self.param
         if torch.compiler.is_compiling() or type(self) is not Phalanx or type(p) is not SigmoidA or not p.token_sliced_backward:
@@ -245,6 +245,8 @@ class Phalanx(nn.Module):
                 return None
         elif self.mix_module is not phalanx_mix:
             return None
+        if not (_is_own(self, _LAYER_METHODS) and _is_own(p, _PROJECTION_METHODS)) or type(p.kv_repeat) is not KVRepeat:
+            return None  # a method of the composition replaced on the instance or the class is called
         return layer_call(x, p.compute_dtype, p.proj_a, p.proj_b, p.proj_c, p.proj_v, self.proj_out, self.heads, self.kv_heads,
                           round_products=default)
 
@@ -269,3 +271,12 @@ class Phalanx(nn.Module):
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         return self._forward_fn(x)
+
+
+# What the composition calls on its way: _as_one_node leaves a call to it where one of these is not the method defined here.
+_LAYER_METHODS = {n: getattr(Phalanx, n) for n in ("_mix_and_project", "_project_out")}
+_PROJECTION_METHODS = {n: getattr(SigmoidA, n) for n in ("forward_axcv", "_compute_base_projections", "project")}
+
+
+def _is_own(module: nn.Module, methods: dict) -> bool:
+    return all(getattr(getattr(module, n), "__func__", None) is f for n, f in methods.items())

@@ -421,3 +421,25 @@ def test_a_layers_results_can_be_worked_on_in_place(B, L, dim, method):
         before = t.clone()
         t *= scale
         assert torch.equal(t, before * 2) and t.requires_grad
+
+
+@pytest.mark.parametrize("method,owner,name", [
+    ("default", "layer", "_mix_and_project"), ("default", "layer", "_project_out"), ("default", "param", "forward_axcv"),
+    ("default", "param", "_compute_base_projections"), ("default", "param", "project"), ("fused", "layer", "_project_out"),
+    ("fused", "param", "project")])
+@pytest.mark.parametrize("where", ["instance", "class"])
+def test_a_replaced_method_is_called(method, owner, name, where, monkeypatch):
+    from spear_amd import Phalanx
+
+    layer = Phalanx(dim=32, method=method, dtype=torch.bfloat16).to(DEV)
+    x = torch.randn(2, 32, 32, device=DEV).bfloat16()
+    obj, calls = (layer if owner == "layer" else layer.param), []
+    own = getattr(type(obj), name)
+
+    def replacement(*args):
+        calls.append(name)
+        return own(*(args if where == "class" else (obj, *args)))
+
+    monkeypatch.setattr(type(obj) if where == "class" else obj, name, replacement)
+    layer(x)
+    assert calls == [name]
