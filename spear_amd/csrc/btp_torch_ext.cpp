@@ -514,12 +514,22 @@ struct LayerNode : public torch::autograd::Function<LayerNode> {
     const bool create_graph = at::GradMode::is_enabled();
     const at::NoGradGuard no_grad;
     const auto saved = ctx->get_saved_variables();
-    const at::Tensor &x = saved[0], &w_a = saved[1], &w_b = saved[2], &w_c = saved[3], &w_v = saved[4], &w_out = saved[5], &a = saved[6],
-                     &b = saved[7], &c = saved[8], &v = saved[9], &mixed = saved[10];
     const int64_t heads = ctx->saved_data["heads"].toInt(), kv_heads = ctx->saved_data["kv_heads"].toInt();
-    const int64_t B = v.size(0), L = v.size(1), F = v.size(2), Fkv = b.size(2), M = B * L, K = x.size(2), dim = w_out.size(0);
-    const c10::DeviceGuard guard(v.device());
-    const at::Tensor dy = grad_outputs[0].contiguous().view({M, dim}), x2 = x.view({M, K}), mixed2 = mixed.view({M, F});
+    const int64_t B = grad_outputs[0].size(0), L = grad_outputs[0].size(1), K = grad_outputs[0].size(2);  // the layer's input is as wide
+    const int64_t F = heads * 16, Fkv = kv_heads * 16, M = B * L;
+    const c10::DeviceGuard guard(grad_outputs[0].device());
+    // Saved-tensor hooks may hand back other tensors than were saved: the kernels below take these as they lie.
+    auto dense = [&](size_t i, at::IntArrayRef sizes) {
+      const at::Tensor& t = saved[i];
+      TORCH_CHECK(t.scalar_type() == at::kBFloat16 && t.device() == grad_outputs[0].device() && t.sizes() == sizes,
+                  "a saved tensor of a Phalanx layer came back with another type, device or shape.");
+      const at::Tensor d = t.contiguous();
+      return (reinterpret_cast<uintptr_t>(d.data_ptr()) & 15u) == 0 ? d : d.clone();
+    };
+    const at::Tensor x2 = dense(0, {B, L, K}).view({M, K}), w_a = dense(1, {heads, K}), w_b = dense(2, {Fkv, K}), w_c = dense(3, {Fkv, K}),
+                     w_v = dense(4, {F, K}), w_out = dense(5, {K, F}), a = dense(6, {B, L, heads}), b = dense(7, {B, L, Fkv}),
+                     c = dense(8, {B, L, Fkv}), v = dense(9, {B, L, F}), mixed2 = dense(10, {B, L, F}).view({M, F});
+    const at::Tensor dy = grad_outputs[0].contiguous().view({M, K});
     torch::autograd::variable_list out(14);  // forward's arguments, of which the first nine are tensors
     std::vector<at::Tensor> parts, sums;
     bool front = false, weights = false;
@@ -551,7 +561,7 @@ struct LayerNode : public torch::autograd::Function<LayerNode> {
       out[6] = sums[2];
       const at::Tensor d2 = packed.view({M, ld});
       if (ctx->needs_input_grad(0)) {
-        out[0] = at::empty(x.sizes(), x.options());  // not a view of the product, for callers that work on it in place
+        out[0] = at::empty({B, L, K}, v.options());  // not a view of the product, for callers that work on it in place
         at::Tensor dx = out[0].view({M, K});
         at::mm_out(dx, d2, stacked);
       }

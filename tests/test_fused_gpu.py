@@ -443,3 +443,32 @@ def test_a_replaced_method_is_called(method, owner, name, where, monkeypatch):
     monkeypatch.setattr(type(obj) if where == "class" else obj, name, replacement)
     layer(x)
     assert calls == [name]
+
+
+@pytest.mark.parametrize("B,L,dim,kv_heads", [(2, 32, 48, 1), (64, 128, 64, 2)])
+def test_layer_node_with_saved_tensor_hooks(B, L, dim, kv_heads):
+    """Tensors that come back in another layout or off the 16-byte grid give the same gradients; another type, shape or device raises."""
+    from spear_amd import Phalanx
+
+    layer = Phalanx(dim=dim, length=L, dtype=torch.bfloat16, kv_heads=kv_heads).to(DEV)
+    x = torch.randn(B, L, dim, device=DEV).bfloat16().requires_grad_(True)
+    dy = torch.randn(B, L, dim, device=DEV).bfloat16()
+
+    def run(pack, unpack):
+        with torch.autograd.graph.saved_tensors_hooks(pack, unpack):
+            y = layer(x)
+        return torch.autograd.grad(y, [x, *layer.parameters()], dy)
+
+    def shifted(t):
+        return torch.cat([t.new_zeros(1), t.reshape(-1)])[1:].view(t.shape)
+
+    want = run(lambda t: t, lambda t: t)
+    with torch.autograd.graph.save_on_cpu():
+        y = layer(x)
+    other = [torch.autograd.grad(y, [x, *layer.parameters()], dy),
+             run(lambda t: t.transpose(0, -1).contiguous(), lambda t: t.transpose(0, -1)), run(lambda t: t, shifted)]
+    for got in other:
+        assert all(torch.equal(a, b) for a, b in zip(got, want))
+    for unpack in (torch.Tensor.float, torch.Tensor.half, torch.Tensor.cpu, lambda t: t[..., :-1].contiguous(), lambda t: t.flatten()):
+        with pytest.raises(RuntimeError, match="came back with another"):
+            run(lambda t: t, unpack)
