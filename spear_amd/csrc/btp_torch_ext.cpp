@@ -500,7 +500,7 @@ struct LayerNode : public torch::autograd::Function<LayerNode> {
     mix_forward(a, b, c, v, mixed, heads, kv_heads, false, round_products);
     at::Tensor y = project(mixed, {w_out}, {at::Tensor()})[0];
     if (ctx != nullptr) {
-      ctx->save_for_backward({x, w_a, w_b, w_c, w_v, w_out, a, b, c, v, mixed});
+      ctx->save_for_backward({x, w_a, w_b, w_c, w_v, w_out, a, b, c, v, mixed, b_a, b_b, b_c});
       ctx->saved_data["heads"] = heads;
       ctx->saved_data["kv_heads"] = kv_heads;
       ctx->saved_data["slices_in"] = slices_in;
@@ -575,18 +575,55 @@ struct LayerNode : public torch::autograd::Function<LayerNode> {
       layer_sums(parts, sums);
     }
     if (!create_graph) return out;
-    // the mixing kernels have no second derivative: a second differentiation says so
+    const at::AutoGradMode grad(true);
+    // The mixing kernels have no second derivative: a second differentiation of what their backward has a part in says so.
+    const auto twice = twice_differentiable(ctx, saved, grad_outputs[0]);
     torch::autograd::variable_list given;
     std::vector<size_t> at_;
     for (size_t i = 0; i < out.size(); ++i) {
       if (!out[i].defined()) continue;
+      if (twice[i].defined()) {
+        out[i] = twice[i];
+        continue;
+      }
       given.push_back(out[i].detach().requires_grad_(true));
       at_.push_back(i);
     }
-    const at::AutoGradMode grad(true);
     const auto error = std::make_shared<torch::autograd::DelayedError>("the gradients of a Phalanx layer cannot be differentiated again", (int64_t)given.size());
     given = error->apply(std::move(given));
     for (size_t i = 0; i < at_.size(); ++i) out[at_[i]] = given[i];
+    return out;
+  }
+
+  // The gradients that need no backward of the mixing kernels, as functions of the layer's input, its weights and the gradient that
+  // arrived: those of proj_out, and of proj_c where the recurrence's result has a tensor of its own (the composition of a default layer).
+  static torch::autograd::variable_list twice_differentiable(torch::autograd::AutogradContext* ctx, const torch::autograd::variable_list& saved,
+                                                             const at::Tensor& grad_output) {
+    torch::autograd::variable_list out(14);
+    const bool with_c = ctx->saved_data["round_products"].toBool();
+    const bool c_wanted = with_c && (ctx->needs_input_grad(5) || ctx->needs_input_grad(6));
+    if (!ctx->needs_input_grad(8) && !c_wanted) return out;
+    const at::Tensor &x = saved[0], &w_out = saved[5];
+    const int64_t heads = ctx->saved_data["heads"].toInt(), kv_heads = ctx->saved_data["kv_heads"].toInt();
+    const int64_t B = x.size(0), L = x.size(1), K = x.size(2), M = B * L, F = heads * 16, Fkv = kv_heads * 16;
+    const at::Tensor a = at::linear(x, saved[1], saved[11]), b = at::linear(x, saved[2], saved[12]), c = at::linear(x, saved[3], saved[13]),
+                     v = at::linear(x, saved[4]), dy = grad_output.reshape({M, K});
+    at::Tensor h, mixed;
+    if (with_c) {
+      auto expand = [&](const at::Tensor& t) { return t.view({B, L, kv_heads, 1, 16}).expand({B, L, kv_heads, heads / kv_heads, 16}).reshape({B, L, F}); };
+      const at::Tensor gated = (expand(at::sigmoid(b)) * v).view({B, L, heads, 16}).permute({0, 2, 3, 1}).contiguous();
+      h = BtpNode::apply(at::sigmoid(a).transpose(1, 2).contiguous(), gated, (int64_t)2, (int64_t)32, false, (int64_t)0, (int64_t)0)
+              .permute({0, 3, 1, 2}).reshape({B, L, F}).contiguous();
+      mixed = h * expand(c) + v;
+    } else {
+      mixed = MixNode::apply(a, b, c, v, heads, kv_heads, false);
+    }
+    if (ctx->needs_input_grad(8)) out[8] = at::mm(dy.t(), mixed.view({M, F}));
+    if (c_wanted) {
+      const at::Tensor dc = (at::mm(dy, w_out).view({B, L, F}) * h).view({M, kv_heads, heads / kv_heads, 16}).sum(2).view({M, Fkv});
+      if (ctx->needs_input_grad(5)) out[5] = at::mm(dc.t(), x.reshape({M, K}));
+      if (ctx->needs_input_grad(6)) out[6] = dc.sum(0);
+    }
     return out;
   }
 };

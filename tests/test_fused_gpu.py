@@ -472,3 +472,38 @@ def test_layer_node_with_saved_tensor_hooks(B, L, dim, kv_heads):
     for unpack in (torch.Tensor.float, torch.Tensor.half, torch.Tensor.cpu, lambda t: t[..., :-1].contiguous(), lambda t: t.flatten()):
         with pytest.raises(RuntimeError, match="came back with another"):
             run(lambda t: t, unpack)
+
+
+@pytest.mark.parametrize("method,names", [("default", ["proj_out.weight", "param.proj_c.weight", "param.proj_c.bias"]),
+                                          ("fused", ["proj_out.weight"])])
+@pytest.mark.parametrize("B,L,kv_heads", [(2, 32, 4), (3, 48, 2)])
+def test_gradients_without_a_part_of_the_mixing_kernels_can_be_differentiated_again(method, names, B, L, kv_heads):
+    """Hessian-vector products of what enters the layer after the recurrence, against the PyTorch statement of the layer in 64 bits."""
+    from spear_amd import Phalanx
+    from spear_amd.ops.btp import reference
+
+    torch.manual_seed(41)
+    layer = Phalanx(dim=64, method=method, dtype=torch.bfloat16, kv_heads=kv_heads).to(DEV)
+    x = torch.randn(B, L, 64, device=DEV).bfloat16()
+    params = dict(layer.named_parameters())
+    vectors = {n: torch.randn_like(params[n]) for n in names}
+
+    def products(forward, ps, cast):
+        y = forward()
+        gs = torch.autograd.grad((y * y).sum(), [ps[n] for n in names], create_graph=True)
+        return torch.autograd.grad(sum((g * cast(vectors[n])).sum() for g, n in zip(gs, names)), list(ps.values()), allow_unused=True)
+
+    ps = {n: p.detach().double().requires_grad_(True) for n, p in params.items()}
+
+    def exact():
+        lin = lambda n: torch.nn.functional.linear(x.double(), ps[f"param.proj_{n}.weight"], ps.get(f"param.proj_{n}.bias")).transpose(1, 2)
+        heads = lambda t: t.view(B, -1, 16, L).repeat_interleave(4 * 16 // t.shape[1], 1)
+        v = heads(lin("v"))
+        h = reference.block_two_pass_linspace(torch.sigmoid(lin("a")), torch.sigmoid(heads(lin("b"))) * v, 16)
+        return (h * heads(lin("c")) + v).permute(0, 3, 1, 2).reshape(B, L, 64) @ ps["proj_out.weight"].T
+
+    want = products(exact, ps, torch.Tensor.double)
+    got = products(lambda: layer(x).float(), params, torch.Tensor.float)
+    for n, a, b in zip(params, got, want):
+        # two layer passes and two backward ones, about ten bf16 roundings each
+        assert (a.double() - b).norm() <= 40 * 2 ** -9 * b.norm(), (n, ((a.double() - b).norm() / b.norm()).item())
