@@ -507,3 +507,85 @@ def test_gradients_without_a_part_of_the_mixing_kernels_can_be_differentiated_ag
     for n, a, b in zip(params, got, want):
         # two layer passes and two backward ones, about ten bf16 roundings each
         assert (a.double() - b).norm() <= 40 * 2 ** -9 * b.norm(), (n, ((a.double() - b).norm() / b.norm()).item())
+
+
+def _rounding_layer_in_64_bits(a, b, c, v, dout, H, Hkv):
+    """The mixing stage with the decay, the input gate, the gated input and the recurrence's upstream gradient rounded to the operands'
+    type, everything else in 64 bits: out and the gradients of a, b, c and v."""
+    B, L, _ = v.shape
+    to_type = lambda t: t.to(a.dtype).double()
+
+    class Gate(torch.autograd.Function):
+        @staticmethod
+        def forward(ctx, z):
+            y = to_type(torch.sigmoid(z))
+            ctx.save_for_backward(y)
+            return y
+
+        @staticmethod
+        def backward(ctx, g):
+            y, = ctx.saved_tensors
+            return g * y * (1 - y)
+
+    leaves = [t.double().requires_grad_(True) for t in (a, b, c, v)]
+    aa, bb, cc, vv = leaves
+    expand = lambda t: t.view(B, L, Hkv, 16).repeat_interleave(H // Hkv, 2)
+    A, V = Gate.apply(aa), vv.view(B, L, H, 16)
+    product = expand(Gate.apply(bb)) * V
+    X = product + (to_type(product) - product).detach()
+    ys, h, last = [], torch.zeros_like(X[:, 0]), None
+    for t in range(L):
+        if t % 16 == 0:
+            last, h, r = h, torch.zeros_like(h), torch.ones_like(A[:, 0])
+        h, r = A[:, t, :, None] * h + X[:, t], r * A[:, t]
+        ys.append(h + r[..., None] * last)
+    Y = torch.stack(ys, 1)
+    Y.register_hook(to_type)
+    out = (Y * expand(cc) + V).reshape(B, L, H * 16)
+    return [out.detach(), *torch.autograd.grad(out, leaves, dout.double())]
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "f16"])
+@pytest.mark.parametrize("H,Hkv", [(8, 8), (5, 5), (16, 8), (6, 3), (16, 4), (12, 3), (16, 2), (24, 3), (6, 2), (16, 1)])
+def test_mixing_kernels_round_gates_and_products_on_request(H, Hkv, dtype):
+    """SPEAR_MIX_ROUND in every instance of the backward kernel (one, two, four, eight and other numbers of heads per kv head) and both
+    widths of the forward one, against the same roundings in 64 bits. The fp32 column sums tell the rounded kernel from the plain one."""
+    from spear_amd import _btp
+
+    ext = _btp.load_extension()
+    for B, L in ((2, 80), (1, 528)):
+        g = torch.Generator(device=DEV).manual_seed(H + Hkv + L)
+        a, b, c, v, dout = (torch.randn(B, L, w, device=DEV, generator=g).to(dtype) for w in (H, Hkv * 16, Hkv * 16, H * 16, H * 16))
+        want = _rounding_layer_in_64_bits(a, b, c, v, dout, H, Hkv)
+        worst = {}
+        print(f"rounding kernels B={B} L={L} H={H} Hkv={Hkv} {dtype}", flush=True)
+        for rounds in (True, False):
+            got = [torch.full_like(t, float("nan")) for t in (v, a, b, c, v)]
+            sums = [torch.full((_btp.mix_backward_sum_rows(B, L, H), t.shape[2]), float("nan"), device=DEV) for t in (a, b, c)]
+            ext.mix_forward(a, b, c, v, got[0], H, Hkv, False, rounds)
+            ext.mix_backward(a, b, c, v, dout, *got[1:], H, Hkv, sums, False, rounds)
+            far = lambda x, y: ((x.double() - y).norm() / y.norm()).item()
+            totals = [t.double().sum(0) for t in sums]
+            worst[rounds] = (max(map(far, got, want)), max(map(far, totals, (w.sum((0, 1)) for w in want[1:4]))))
+        # results: one rounding, below eps / 2 each; sums: fp32 additions, and here and there a gate whose fp32 value rounds the other
+        # way (plain kernels: every gate and product lies up to eps / 2 away)
+        assert worst[True][0] <= torch.finfo(dtype).eps / 2, worst
+        assert worst[True][1] <= torch.finfo(dtype).eps / 32 and worst[False][1] >= 2 * worst[True][1], worst
+
+
+@pytest.mark.parametrize("dim,kv_heads", [(64, 2), (64, 1), (128, 1), (256, 2), (192, 4)])
+def test_default_layer_gradients_with_shared_kv_heads(dim, kv_heads):
+    """Groups of 2, 4, 8, 8 and 3 heads per kv head, the instances that a default layer's backward runs, against its composition."""
+    from spear_amd import Phalanx, btp
+
+    torch.manual_seed(13)
+    layer = Phalanx(dim=dim, dtype=torch.bfloat16, kv_heads=kv_heads).to(DEV)
+    x = torch.randn(4, 80, dim, device=DEV).bfloat16().requires_grad_(True)
+    dy = torch.randn(4, 80, dim, device=DEV).bfloat16()
+    run = lambda: [y := layer(x), *torch.autograd.grad(y, [x, *layer.parameters()], dy)]
+    assert layer._as_one_node(x) is not None
+    got = run()
+    layer.btp_module = lambda *args: btp(*args)  # the stand-alone composition
+    for i, (a, b) in enumerate(zip(got, run())):
+        # each of the about ten roundings between input and gradient is 2^-9 relative; they are independent
+        assert (a.float() - b.float()).norm() <= 2 ** -9 * 10 * b.float().norm(), i
