@@ -589,3 +589,33 @@ def test_default_layer_gradients_with_shared_kv_heads(dim, kv_heads):
     for i, (a, b) in enumerate(zip(got, run())):
         # each of the about ten roundings between input and gradient is 2^-9 relative; they are independent
         assert (a.float() - b.float()).norm() <= 2 ** -9 * 10 * b.float().norm(), i
+
+
+@pytest.mark.parametrize("method", ["default", "fused"])
+@pytest.mark.parametrize("B,L,dim", [(2, 48, 64), (1, 32, 1040), (64, 144, 80)])
+def test_layer_node_off_the_16_byte_grid_and_on_another_stream(B, L, dim, method):
+    from spear_amd import Phalanx
+
+    torch.manual_seed(51)
+    layer = Phalanx(dim=dim, length=L, method=method, dtype=torch.bfloat16).to(DEV)
+    x = torch.randn(B, L, dim, device=DEV).bfloat16()
+    dy = torch.randn(B, L, dim, device=DEV).bfloat16()
+
+    def run(x, dy):
+        xx = x.requires_grad_(True)
+        assert layer._as_one_node(xx) is not None
+        y = layer(xx)
+        return [y.detach(), *torch.autograd.grad(y, [xx, *layer.parameters()], dy)]
+
+    def shifted(t):
+        return torch.cat([t.new_zeros(1), t.detach().view(-1)])[1:].view(t.shape)
+
+    want = run(x, dy)
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        got = run(x, dy)
+    torch.cuda.current_stream().wait_stream(side)
+    assert all(torch.equal(a, b) for a, b in zip(got, want))
+    for i, (a, b) in enumerate(zip(run(shifted(x), shifted(dy)), want)):  # the library's products for the input projections
+        assert (a.float() - b.float()).norm() <= 2 ** -9 * 10 * b.float().norm(), i

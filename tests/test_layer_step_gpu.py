@@ -328,3 +328,42 @@ def test_step_takes_tokens_in_any_layout(layout, B):
     assert_close(f64(y), f64(want), 2e-2, 2e-2, "y")
     assert_close(f64(one.h_loc), f64(two.h_loc), 2e-2, 2e-2, "h")
     assert one.pos.tolist() == [2] * B
+
+
+def test_step_with_the_output_projection_of_the_library():
+    """Wider than the output projection's kernel takes: the token kernel moves the block positions on itself, also past a block's end."""
+    from spear_amd.nn.phalanx.inference import PhalanxStepState, phalanx_step
+
+    B, dim = 17, 528
+    layer = _layer(dim=dim, seed=12)
+    x = torch.randn(20, B, dim, generator=torch.Generator().manual_seed(13)).bfloat16().to(DEV)
+    one, two = PhalanxStepState.zeros(B, dim // 16, DEV), PhalanxStepState.zeros(B, dim // 16, DEV)
+    one.pos += torch.arange(B, device=DEV, dtype=torch.int32) % 16
+    two.pos += one.pos
+    for t in range(20):
+        y = phalanx_step(layer, x[t], one)
+        handle = layer.param.proj_a.register_forward_hook(lambda *a: None)  # the projections as modules
+        want = phalanx_step(layer, x[t], two)
+        handle.remove()
+        assert_close(f64(y), f64(want), 2e-2, 2e-2, f"y[{t}]")
+        assert one.pos.tolist() == two.pos.tolist() == [(b + t + 1) % 16 for b in range(B)]
+
+
+@pytest.mark.parametrize("B,L,dim", [(2, 48, 64), (1, 33, 1040)])
+def test_prompts_off_the_16_byte_grid_and_on_another_stream(B, L, dim):
+    from spear_amd.nn.phalanx.inference import phalanx_prefill
+
+    layer = _layer(dim=dim, seed=14)
+    x = torch.randn(B, L, dim, generator=torch.Generator().manual_seed(15)).bfloat16().to(DEV)
+    shifted = torch.cat([x.new_zeros(1), x.view(-1)])[1:].view(x.shape)
+    y, st = phalanx_prefill(layer, x)
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        ys, sts = phalanx_prefill(layer, x)
+    torch.cuda.current_stream().wait_stream(side)
+    assert torch.equal(y, ys) and all(torch.equal(getattr(st, n), getattr(sts, n)) for n in ("h_loc", "r_pref", "c_prev_loc", "pos"))
+    yu, stu = phalanx_prefill(layer, shifted)  # the library's products for the projections
+    assert_close(f64(yu), f64(y), 2e-2, 2e-2, "y")
+    assert_close(f64(stu.h_loc), f64(st.h_loc), 2e-2, 2e-2, "h")
+    assert torch.equal(stu.pos, st.pos)
