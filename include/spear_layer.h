@@ -14,7 +14,7 @@ extern "C" {
  * (spear_phalanx_mix_step): what spear_phalanx_mix_prefill does, for lengths that end inside a block too.
  *     a_logit [B, L, H]   b_logit, c [B, L, kv_heads * 16]   v, out [B, L, H * 16]      16-bit, `dtype`
  *     h, c_prev [B, H, 16] fp32    r [B, H] fp32    pos [B] int32      every element is written
- * Tensor pointers 16-byte aligned; r and pos 4-byte. */
+ * L < 1 is refused. Tensor pointers 16-byte aligned; r and pos 4-byte. */
 int spear_layer_prefill(const void* a_logit, const void* b_logit, const void* c, const void* v, void* out, float* h,
                         float* r, float* c_prev, int* pos, int B, int L, int H, int kv_heads, int dtype, void* stream);
 

@@ -353,7 +353,8 @@ def mix_forward(
     ``qkv_gate``: ``a_logit`` is an fp32 log-decay gate, ``b_logit`` is k, ``c`` is q:
     ``out <- c * btp(exp(a_logit), b_logit * v) + v`` (``SPEAR_MIX_QKV_GATE``). ``c_prev_tail``: fp32
     ``[B, heads, 16]`` that receives the terminal local state of every row's last block, the hand-over state
-    for decoding after this prompt (``spear_phalanx_mix_prefill``)."""
+    for decoding after this prompt (``spear_phalanx_mix_prefill``: kept for callers of the C ABI and this view of it; the
+    package's own prompts of any length go through ``spear_layer_prefill``)."""
     _check(all(t.is_cuda for t in (a_logit, b_logit, c, v, out)), "All tensors must be CUDA.")
     _check(v.dim() == 3, "v must be [B, L, heads * 16].")
     B, L, F = v.shape

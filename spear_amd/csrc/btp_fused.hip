@@ -171,9 +171,9 @@ __device__ __forceinline__ GateWords load_gate_words(__amdgpu_buffer_rsrc_t ra, 
 // ==========================================================================================
 // Shared by the forward and the backward kernel: which tile a workgroup is.
 // ==========================================================================================
-// Wavefronts per workgroup of the backward kernel (8 were slower by 1 to 5 %), and per SIMD. With the number of heads per kv head a
-// compile-time constant every instance fits 114 to 119 registers and nothing spills. Shared heads run 4 to a SIMD: as a run-time
-// value the grouping took 133 to 168 registers, 3 per SIMD (B=16 H=64 L=8192 groups of 4: 232.8 -> 213.8 us). Without sharing
+// Wavefronts per workgroup of the backward kernel (8 were slower by 1 to 5 %), and per SIMD. With 1, 2, 4 or 8 heads per kv head as
+// a compile-time constant the kernel fits 114 to 119 registers and nothing spills (kWide is below). Shared heads run 4 to a SIMD: as a
+// run-time value the grouping took 133 to 168 registers, 3 per SIMD (B=16 H=64 L=8192 groups of 4: 232.8 -> 213.8 us). Without sharing
 // the kernel moves 5.9 TB/s and more wavefronts only get in each other's way, so those instances are held to 3: 3 / 4 per SIMD, us,
 // q/k/v form B=1024 H=32 L=128 160 / 164, B=16 H=64 L=8192 326 / 333, B=64 H=128 L=2048 657 / 674; layer form 155 / 158, 319 / 325,
 // 642 / 652.
@@ -853,7 +853,7 @@ void phalanx_mix_bwd_tile_kernel(
 // kRagged: rows whose last block is not whole (prompts of any length). That block's steps past the end read the row's last step
 // and are not stored, and its state is the one after the row's last step: one launch for the whole prompt where the steps of
 // the last block used to go through the decode kernel one launch each, between transposes and a concatenation of the two parts
-// (B=64 L=1003 dim=512: 45 us for the whole prompt; the 11 steps and the copies around them took 350 us more).
+// (B=64 L=1003 dim=512: 52 us for the whole prompt; the 11 steps and the copies around them took 350 us more).
 // kW wavefronts per workgroup, one head slot x kW consecutive blocks (2 head slots x kW / 2 blocks measured
 // slower at every shape): 4 or 8. Microseconds for 4 / 8, B L H:
 //   1024 128 32: 87.3 / 91.5    256 512 32: 89.8 / 86.0    16 8192 32: 89.4 / 87.1

@@ -12,7 +12,9 @@
 // 5.7 / 28.0, M=1024 dim=512 13.1 / 21.9, M=512 dim=1024 22.2 / 25.8, M=2048 dim=512 23.2 / 23.3 (1.64 G multiply-adds), M=1024
 // dim=768 25.3 / 24.0 (1.85 G), M=4096 dim=512 38.2 / 28.4: past about 1.6 G the library's larger tiles, which read x and the
 // weights less often, win. One projection (dim x dim): M=1024 dim=512 5.7 / 5.8 (0.27 G), M=2048 dim=512 7.6 / 6.2, M=16 dim=512
-// 4.8 / 3.8, M=128 dim=768 7.2 / 4.7: alone it is taken for the host time it saves, up to 0.3 G and K = 512.
+// 4.8 / 3.8, M=128 dim=768 7.2 / 4.7: alone it is the slower one on the GPU and is taken for the host time it saves (a decode step of 16
+// sequences 19.7 us as a call at K = 512 with it, 38.5 at K = 1024 with the library's product), up to 0.3 G and K = 512. The line at K is
+// the GPU's, for steps in a graph; between 512 and 768 nothing was timed.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 

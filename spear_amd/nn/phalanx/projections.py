@@ -50,9 +50,10 @@ def slice_count(M: int, N: int, K: int) -> int:
     while s < _MAX_SLICES and tiles * s < _TARGET_TILES and M % (2 * s) == 0 and M // (2 * s) >= _MIN_SLICE_ROWS:
         s *= 2
     # The library's kernel for these products makes 256 x 256 tiles, two at a time on each of the 256 compute units. A neighbouring
-    # slice count is taken where that model gives it 13 % less time (times per product and sum of the parts at 131072
+    # slice count is taken where that model gives it 13 % less time: at 12 % one of 72 shapes was 8 % slower, at 15 % [3200 x 2048]
+    # (17 % faster, modelled 14.9 %) stays out (times per product and sum of the parts at 131072
     # tokens, us): [6272 x 2048] 2 -> 4 slices 3957 -> 3325, [3200 x 2048] 4 -> 8 2139 -> 1772, [2304 x 2048] 4 -> 8 1485 -> 1114,
-    # [1536 x 1536] 8 -> 16 939 -> 593; at 16384 [2368 x 768] 16 -> 8 103 -> 84. Over 70 shapes of 8192 to 131072 tokens it made
+    # [1536 x 1536] 8 -> 16 939 -> 593; at 16384 [2368 x 768] 16 -> 8 103 -> 84. Over 72 shapes of 8192 to 131072 tokens it made
     # none slower; with every slice count open to it, some by 20 %.
     near = [n for n in (s // 2, 2 * s) if 1 <= n <= _MAX_SLICES and M % n == 0 and (n < s or M // n >= _MIN_SLICE_ROWS)]
     cost = {n: _slices_cost(M, N, K, n) for n in (s, *near)}
@@ -210,9 +211,9 @@ class _ProjectAndMix(torch.autograd.Function):
 
 def plain_operands(x: torch.Tensor, dtype: torch.dtype, *linears) -> list[torch.Tensor] | None:
     """Weights and biases of ``(module, has_bias)`` pairs for the compiled paths that take them as they lie, or None where
-    a call has to go through the modules: other types than bf16 (``dtype`` is the one in which ``x`` goes through them; it need not be
-    cast yet), replaced or hooked modules, autocast, traced or transformed
-    calls (``_plain_eager``), and layouts that 16-byte accesses do not fit."""
+    a call has to go through the modules: other types than bf16 (``dtype`` is the one in which ``x`` goes through them; it
+    need not be cast yet), replaced or hooked modules, autocast, traced or transformed calls (``_plain_eager``), and layouts that
+    16-byte accesses do not fit."""
     from spear_amd.ops.btp.interface import _plain_eager
 
     if dtype != torch.bfloat16 or torch.is_autocast_enabled("cuda") or torch._C._get_tracing_state() is not None \
@@ -241,9 +242,9 @@ def plain_operands(x: torch.Tensor, dtype: torch.dtype, *linears) -> list[torch.
 
 def layer_call(x: torch.Tensor, dtype: torch.dtype, proj_a, proj_b, proj_c, proj_v, proj_out, heads: int, kv_heads: int,
                round_products: bool) -> torch.Tensor | None:
-    """The whole layer on ``x[B, L, K]``, cast to ``dtype`` once the call is taken, as one autograd node compiled into the binding (``LayerNode`` in
-    ``btp_torch_ext.cpp``; ``round_products``: gates and gated inputs
-    rounded to 16 bits as the tensors that :func:`btp` takes), or None where the call is for the modules and the Python nodes of this file: what
+    """The whole layer on ``x[B, L, K]``, cast to ``dtype`` once the call is taken, as one autograd node compiled into the
+    binding (``LayerNode`` in ``btp_torch_ext.cpp``; ``round_products``: gates and gated inputs rounded to 16 bits as the tensors
+    that :func:`btp` takes), or None where the call is for the modules and the Python nodes of this file: what
     ``plain_operands`` leaves to them, lengths and sizes that the mixing kernels refuse, and a row of gradients of 2 GiB.
     Forward + backward, us, modules and Python nodes / compiled: B=8 L=128 dim=512 562 / 245, B=1024 1330 / 1307,
     B=64 L=2048 dim=2048 8152 / 7992."""

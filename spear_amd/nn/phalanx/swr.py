@@ -23,8 +23,9 @@ against the reference says ``method="default"``; with ``SPEAR_PHALANX_DEFAULT=fu
 such a layer runs the fused kernels wherever they apply (``k == 2``, 16-bit output), under ``torch.compile`` and
 autocast too, and the stand-alone kernels elsewhere, without a change to the calling code.
 
-On a GPU, from 8192 tokens per call on, the ``"default"`` and ``"fused"`` layers run their five
-projections through :mod:`.projections` (same forward; weight gradients cut along the token axis, one
+On a GPU a plain eager bf16 call of a ``"default"`` or ``"fused"`` layer is one compiled autograd node at every size
+(``Phalanx._as_one_node``). The calls that it leaves (traced, hooked, under autocast, k = 1) run the modules, and from 8192 tokens
+on their five projections through :mod:`.projections` (same forward; weight gradients cut along the token axis, one
 shared input gradient). The two ``"pytorch*"`` methods keep plain ``nn.Linear`` autograd, which is what the
 other two are compared with.
 """
@@ -227,8 +228,8 @@ class Phalanx(nn.Module):
         """A plain bf16 call as one compiled autograd node around the fused mixing kernels, or None where the call is for the
         composition of modules below.
 
-        For ``"default"``, whose gates and gated inputs keep the 16 bits in which :func:`btp` takes them, this takes the place of the stand-alone recurrence between about twenty elementwise and transposing
-        passes. Forward + backward, us, stand-alone / one node: B=1024 L=128 dim=512 4692 / 1307, B=8 822 / 245; no size was
+        For ``"default"``, whose gates and gated inputs keep the 16 bits in which :func:`btp` takes them, this takes the place of
+        the stand-alone recurrence between about twenty elementwise and transposing passes. Forward + backward, us, stand-alone / one node: B=1024 L=128 dim=512 4692 / 1307, B=8 822 / 245; no size was
         found where the stand-alone kernels win. They keep every call that the fused ones would answer in another way:
         k = 1, other types than bf16 throughout, autocast, anything that traces or transforms the call, hooked or replaced
         projections (``plain_operands``), the matrix-core and checkpoint-store switches, a replaced recurrence, class or method, empty
