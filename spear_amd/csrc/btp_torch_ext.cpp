@@ -500,7 +500,8 @@ struct LayerNode : public torch::autograd::Function<LayerNode> {
     mix_forward(a, b, c, v, mixed, heads, kv_heads, false, round_products);
     at::Tensor y = project(mixed, {w_out}, {at::Tensor()})[0];
     if (ctx != nullptr) {
-      ctx->save_for_backward({x, w_a, w_b, w_c, w_v, w_out, a, b, c, v, mixed, b_a, b_b, b_c});
+      ctx->save_for_backward({x, w_a, w_b, w_c, w_v, w_out, a, b, c, v, mixed});
+      ctx->saved_data["biases"] = std::vector<at::Tensor>{b_a, b_b, b_c};  // for their graphs: their values may change before backward
       ctx->saved_data["heads"] = heads;
       ctx->saved_data["kv_heads"] = kv_heads;
       ctx->saved_data["slices_in"] = slices_in;
@@ -606,8 +607,14 @@ struct LayerNode : public torch::autograd::Function<LayerNode> {
     const at::Tensor &x = saved[0], &w_out = saved[5];
     const int64_t heads = ctx->saved_data["heads"].toInt(), kv_heads = ctx->saved_data["kv_heads"].toInt();
     const int64_t B = x.size(0), L = x.size(1), K = x.size(2), M = B * L, F = heads * 16, Fkv = kv_heads * 16;
-    const at::Tensor a = at::linear(x, saved[1], saved[11]), b = at::linear(x, saved[2], saved[12]), c = at::linear(x, saved[3], saved[13]),
-                     v = at::linear(x, saved[4]), dy = grad_output.reshape({M, K});
+    const auto biases = ctx->saved_data["biases"].toTensorVector();
+    // the values that forward had, as functions of the input and the weights
+    auto projection = [&](const at::Tensor& value, const at::Tensor& w, const at::Tensor& bias) {
+      const at::Tensor again = at::linear(x, w, bias);
+      return value.detach() + (again - again.detach());
+    };
+    const at::Tensor a = projection(saved[6], saved[1], biases[0]), b = projection(saved[7], saved[2], biases[1]),
+                     c = projection(saved[8], saved[3], biases[2]), v = projection(saved[9], saved[4], at::Tensor()), dy = grad_output.reshape({M, K});
     at::Tensor h, mixed;
     if (with_c) {
       auto expand = [&](const at::Tensor& t) { return t.view({B, L, kv_heads, 1, 16}).expand({B, L, kv_heads, heads / kv_heads, 16}).reshape({B, L, F}); };

@@ -504,6 +504,9 @@ def test_gradients_without_a_part_of_the_mixing_kernels_can_be_differentiated_ag
 
     want = products(exact, ps, torch.Tensor.double)
     got = products(lambda: layer(x).float(), params, torch.Tensor.float)
+    with pytest.raises(RuntimeError, match="differentiated again"):
+        g, = torch.autograd.grad(layer(x).float().square().sum(), params["param.proj_a.weight"], create_graph=True)
+        g.float().sum().backward()
     for n, a, b in zip(params, got, want):
         # two layer passes and two backward ones, about ten bf16 roundings each
         assert (a.double() - b).norm() <= 40 * 2 ** -9 * b.norm(), (n, ((a.double() - b).norm() / b.norm()).item())
@@ -619,3 +622,28 @@ def test_layer_node_off_the_16_byte_grid_and_on_another_stream(B, L, dim, method
     assert all(torch.equal(a, b) for a, b in zip(got, want))
     for i, (a, b) in enumerate(zip(run(shifted(x), shifted(dy)), want)):  # the library's products for the input projections
         assert (a.float() - b.float()).norm() <= 2 ** -9 * 10 * b.float().norm(), i
+
+
+@pytest.mark.parametrize("method", ["default", "fused"])
+def test_biases_may_change_between_forward_and_backward(method):
+    """No gradient depends on a bias' value, so nothing keeps one from being updated before backward, create_graph included."""
+    from spear_amd import Phalanx
+
+    torch.manual_seed(61)
+    layer = Phalanx(dim=64, method=method, dtype=torch.bfloat16).to(DEV)
+    x = torch.randn(2, 32, 64, device=DEV).bfloat16().requires_grad_(True)
+
+    def run(change, create_graph):
+        biases = [p.detach().clone() for n, p in layer.named_parameters() if n.endswith("bias")]
+        y = layer(x)
+        with torch.no_grad():
+            for p in (p for n, p in layer.named_parameters() if n.endswith("bias") and change):
+                p.mul_(3)
+        got = torch.autograd.grad(y, [x, *layer.parameters()], torch.ones_like(y), create_graph=create_graph)
+        with torch.no_grad():
+            for p, old in zip((p for n, p in layer.named_parameters() if n.endswith("bias")), biases):
+                p.copy_(old)
+        return got
+
+    for create_graph in (False, True):
+        assert all(torch.equal(a, b) for a, b in zip(run(True, create_graph), run(False, create_graph)))
