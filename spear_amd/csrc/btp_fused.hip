@@ -92,6 +92,14 @@ __device__ __forceinline__ float2 decay_pair(GateWords w) {
   }
 }
 
+// d sigmoid / d logit of a pair of rounded decays as the layer's own sigmoid has it: from the decay before the floor of the recurrences, so
+// that a decay at or below the floor keeps its gradient and a NaN logit gives a NaN one.
+template <class E>
+__device__ __forceinline__ float2 rounded_decay_slopes(GateWords w) {
+  const float2 q = as_tensor<E, true>(fast_sigmoid(E::lo(w.lo)), fast_sigmoid(E::hi(w.lo)));
+  return make_float2(q.x * (1.0f - q.x), q.y * (1.0f - q.y));
+}
+
 template <bool kQkv>
 __device__ __forceinline__ float input_gate(float b) {
   if constexpr (kQkv) return b;
@@ -767,12 +775,21 @@ void phalanx_mix_bwd_tile_kernel(
   two_hop += row_xor<1>(two_hop);
   two_hop += row_xor<2>(two_hop);
   two_hop += row_xor<4>(two_hop);
-  const float2 aa = *reinterpret_cast<const float2*>(ta + head_local * kGateRow + 2 * kk);
+  if constexpr (kRound) {  // into the tile of the block beyond the edge, which has been read long since
+    const float2 slopes = rounded_decay_slopes<E>(araw);
+    write_tile(tn, slopes.x, slopes.y);
+    wave_lds_handover();
+  }
+  const float2 aa = *reinterpret_cast<const float2*>((kRound ? tn : ta) + head_local * kGateRow + 2 * kk);
   const float2 ee = *reinterpret_cast<const float2*>(te + head_local * kGateRow + 2 * kk);
   s0 = fmaf(-ee.x, two_hop, s0);
   s1 = fmaf(-ee.y, two_hop, s1);
   // d/d a_logit = dA a (1 - a);  d/d gate = dA a  (gate = log a)
-  const float da0 = kQkv ? s0 * aa.x : s0 * aa.x * (1.0f - aa.x), da1 = kQkv ? s1 * aa.y : s1 * aa.y * (1.0f - aa.y);
+  float da0 = s0 * aa.x, da1 = s1 * aa.y;
+  if constexpr (!kQkv && !kRound) {
+    da0 *= 1.0f - aa.x;
+    da1 *= 1.0f - aa.y;
+  }
   if constexpr (kDaBytes == 4) {
     __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(da0), rda, da_lane, t0 * ld_da * 4, 0);
     __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(da1), rda, da_lane1, t0 * ld_da * 4, 0);

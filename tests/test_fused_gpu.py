@@ -647,3 +647,30 @@ def test_biases_may_change_between_forward_and_backward(method):
 
     for create_graph in (False, True):
         assert all(torch.equal(a, b) for a, b in zip(run(True, create_graph), run(False, create_graph)))
+
+
+@pytest.mark.parametrize("kv_heads", [4, 2, 1])
+@pytest.mark.parametrize("bias", [float("nan"), float("inf"), float("-inf"), -30.0, -80.0, 30.0])
+def test_default_layer_gradients_at_the_ends_of_the_decay(bias, kv_heads):
+    """A NaN decay logit reaches the gradients that it reaches through the layer's own sigmoid; decays below the recurrences' floor keep
+    the gradient of their logit."""
+    from spear_amd import Phalanx, btp
+
+    torch.manual_seed(71)
+    layer = Phalanx(dim=64, dtype=torch.bfloat16, kv_heads=kv_heads).to(DEV)
+    with torch.no_grad():
+        layer.param.proj_a.bias[1] = bias
+    x = torch.randn(2, 80, 64, device=DEV).bfloat16().requires_grad_(True)
+    dy = torch.randn(2, 80, 64, device=DEV).bfloat16()
+    run = lambda: [y := layer(x), *torch.autograd.grad(y, [x, *layer.parameters()], dy)]
+    assert layer._as_one_node(x) is not None
+    got = run()
+    layer.btp_module = lambda *args: btp(*args)  # the stand-alone composition
+    want = run()
+    assert torch.isnan(want[1]).all() if bias != bias else not torch.isnan(want[1]).any()
+    for i, (a, b) in enumerate(zip(got, want)):
+        assert torch.equal(torch.isnan(a), torch.isnan(b)), i
+        a, b = a.double().nan_to_num(), b.double().nan_to_num()
+        assert (a - b).norm() <= 2 ** -9 * 10 * b.norm(), i
+    a, b = got[3][1].double(), want[3][1].double()  # the bias of that head alone
+    assert bias != bias or abs(a - b) <= 0.1 * abs(b), (a, b)
