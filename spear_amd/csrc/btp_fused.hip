@@ -180,7 +180,8 @@ __device__ __forceinline__ GateWords load_gate_words(__amdgpu_buffer_rsrc_t ra, 
 // Shared by the forward and the backward kernel: which tile a workgroup is.
 // ==========================================================================================
 // Wavefronts per workgroup of the backward kernel (8 were slower by 1 to 5 %), and per SIMD. With 1, 2, 4 or 8 heads per kv head as
-// a compile-time constant the kernel fits 114 to 119 registers and nothing spills (kWide is below). Shared heads run 4 to a SIMD: as a
+// a compile-time constant the kernel takes 115 to 128 registers; nothing spills, but one to three values per lane in three instances
+// with groups of eight (kWide is below). Shared heads run 4 to a SIMD: as a
 // run-time value the grouping took 133 to 168 registers, 3 per SIMD (B=16 H=64 L=8192 groups of 4: 232.8 -> 213.8 us). Without sharing
 // the kernel moves 5.9 TB/s and more wavefronts only get in each other's way, so those instances are held to 3: 3 / 4 per SIMD, us,
 // q/k/v form B=1024 H=32 L=128 160 / 164, B=16 H=64 L=8192 326 / 333, B=64 H=128 L=2048 657 / 674; layer form 155 / 158, 319 / 325,

@@ -368,7 +368,8 @@ def phalanx_prefill(layer, x: torch.Tensor) -> tuple[torch.Tensor, PhalanxStepSt
     p = layer.param
     if layer.k != 2:
         raise RuntimeError("phalanx_prefill needs a layer with k == 2")
-    if x.dim() == 3 and x.shape[1] == 0:
+    _, L, _ = x.shape
+    if L == 0:
         raise ValueError("phalanx_prefill needs a prompt of at least one token")
     xc = x.to(p.compute_dtype)
     operands = _layer_operands(layer, xc) if xc.dim() == 3 and xc.numel() > 0 and xc.shape[2] % 8 == 0 else None
