@@ -11,7 +11,8 @@
 // decoder continues from (block-local state, in-block gate product, previous block's terminal
 // state) written by the 16 lanes that own the row's last step. Prompts have any length, so rows
 // that are not 16-byte aligned are handled too, by realigning 32-bit words in registers. A second
-// tile kernel covers what the first does not (fp32 tensors, other block lengths and head sizes).
+// tile kernel covers what the first does not (fp32 tensors, other block lengths and head sizes), and a kernel of one thread per
+// block the rows and blocks that are too short or too long for it.
 //
 // The step kernel is element-wise over [B, H, D]: a thread owns 8 consecutive channels of one head
 // (one 16-byte access per 16-bit operand), the per-head scalars are read by every thread of the
