@@ -456,18 +456,28 @@ std::vector<at::Tensor> linears(const at::Tensor& x, const std::vector<at::Tenso
   return out;
 }
 
-// Whether `layers` projections of M rows, `columns` columns together, are faster in the kernel above than as the library's
-// products (the sizes measured at layer_linear.hip).
-bool small_products(int64_t M, int64_t columns, int64_t K, size_t layers) {
-  return M > 0 && K > 0 && K % 8 == 0 && (layers > 1 ? M * columns * K <= 1600000000 : K <= 512 && M * columns * K <= 300000000);
+// Whether one projection is taken by spear_layer_linear's kernel for few rows although the library's product is no slower on the GPU (the
+// sizes measured at layer_linear.hip).
+bool small_product(int64_t M, int64_t columns, int64_t K) { return M > 0 && K > 0 && K % 8 == 0 && K <= 512 && M * columns * K <= 300000000; }
+
+// Whether projections of M rows are faster through spear_layer_linear than as the library's products. Measured in HIP graphs, us, dim = K,
+// spear_layer_linear / the library. The four input projections: K=128 131072 rows 52 / 67, K=512 16384 rows 32 / 54, 131072 rows 229 / 284,
+// K=768 65536 rows 230 / 239, K=1024 8192 rows 52 / 74, 131072 rows 729 / 717 (with kv heads shared by four 401 / 405), K=1536 16384 rows
+// 203 / 238, 65536 rows 772 / 742, K=2048 4096 rows 95 / 114, 8192 rows 193 / 174: all below K = 1024, and few tiles from there on.
+// One: K=512 65536 rows 40 / 43, 16384 rows 17.2 / 15.3, K=768 131072 rows 147 / 140.
+bool own_products(int64_t M, const std::vector<at::Tensor>& weights, int64_t K) {
+  if (M <= 0 || K <= 0 || K % 8 != 0) return false;
+  int64_t tiles = 0;
+  for (const at::Tensor& w : weights) tiles += (w.size(0) + 255) / 256;
+  tiles *= (M + 255) / 256;
+  if (weights.size() > 1) return K < 1024 || tiles <= 600;
+  return small_product(M, weights[0].size(0), K) || (K <= 512 && tiles >= 512);
 }
 
 // The four input projections (a, b, c, v) of x [..., K], or one projection without bias, by either. x dense.
 std::vector<at::Tensor> project(const at::Tensor& x, const std::vector<at::Tensor>& weights, const std::vector<at::Tensor>& biases) {
   const int64_t K = x.size(-1), M = K > 0 ? x.numel() / K : 0;
-  int64_t columns = 0;
-  for (const at::Tensor& w : weights) columns += w.size(0);
-  if (small_products(M, columns, K, weights.size()) && (reinterpret_cast<uintptr_t>(x.data_ptr()) & 15u) == 0) return linears(x, weights, biases);
+  if (own_products(M, weights, K) && (reinterpret_cast<uintptr_t>(x.data_ptr()) & 15u) == 0) return linears(x, weights, biases);
   std::vector<at::Tensor> out;
   for (size_t i = 0; i < weights.size(); ++i) out.push_back(biases[i].defined() ? at::linear(x, weights[i], biases[i]) : at::linear(x, weights[i]));
   return out;
@@ -699,7 +709,7 @@ at::Tensor layer_step(const at::Tensor& x, const at::Tensor& w_a, const at::Tens
                       at::Tensor r, at::Tensor c_prev, at::Tensor pos, int64_t block_len, int64_t heads, int64_t kv_heads) {
   // the positions move on with the output projection where that is a kernel of this library
   const auto in = [&](bool advance) { return layer_token(x, w_a, b_a, w_b, b_b, w_c, b_c, w_v, h, r, c_prev, pos, block_len, heads, kv_heads, advance); };
-  if (small_products(x.size(0), w_out.size(0), w_out.size(1), 1))
+  if (small_product(x.size(0), w_out.size(0), w_out.size(1)))
     return linears(in(false), {w_out}, {at::Tensor()}, pos.data_ptr<int>(), block_len)[0];
   return at::linear(in(true), w_out);
 }

@@ -1,0 +1,266 @@
+// The layer's linear projections at sizes where the matrix units are the limit, on gfx950 (MI355X): up to four of them on the same
+// rows in one launch.
+//
+//     out_j[M, N_j] = x[M, K] w_j[N_j, K]^T + bias_j          bf16, fp32 sums, rounded once
+//
+// One workgroup of eight wavefronts per compute unit makes 256 x 256 tiles of the results, one after the other, in steps of 64 columns of K on
+// v_mfma_f32_16x16x32_bf16 (2048 cycles of the matrix units per step). A wavefront owns 128 rows by 64 columns: 128 accumulators.
+//   - Operands go from memory to LDS without registers (buffer_load ... lds, 16 bytes per lane, rows of 128 bytes): three stages of x
+//     and two of the weights, 32 KiB each, all 160 KiB. x comes from memory and is asked for two steps ahead, the weights
+//     come from L2 and are asked for when the stage before is free. Requests run on over the end of a tile into the next one, so
+//     only the first tile waits for memory.
+//   - 16-byte pieces are exchanged inside their row by the row's index ((row >> 1) & 7), on the way in by the lane that asks for them:
+//     the reads of a fragment then touch every bank once (SQ_LDS_BANK_CONFLICT 0; a swizzle over 64-byte rows that ignored which
+//     lanes share a cycle had one conflict per read and cost a fifth of the whole).
+//   - The two wavefronts of a SIMD (wm = 0, 1) are half a phase apart, held there by the barriers: one reads fragments (12 reads)
+//     while the other multiplies (32 instructions, 512 cycles), so neither needs a second set of fragment registers. Phases of
+//     16 instructions gave 0.68 of the matrix units' cycles on an 8192^3 product, of 32 0.77.
+//   - What lies past a row's end, the last row or the last column reads as zero: the descriptors of the buffer loads end with the tile's
+//     last valid row, and the lanes whose piece lies past K ask past that end. K, M and N need no padding.
+//   - Results are rounded, exchanged between lane rows (v_permlane16_swap) to 16 bytes per lane and stored while the next tile's
+//     requests are under way; the waits count the stores, so the next tile doesn't wait for them before its second step.
+//   - A tile with 128 columns or fewer spreads them over all wavefronts and skips half of the matrix instructions.
+//   - Workgroups of one XCD take consecutive tiles of groups of four row panels by all columns: the panels of x and the weights
+//     that are used at one time fit its L2.
+//
+// Measured, TFLOP/s, this kernel / the library's products: 131072 rows, K=512, N=512+512+512+32 950 / 775; N=512 960 / 850; K=1024
+// N=1024 1180 / 1270; K=2048 N=2048+512+512+128 1310 / 1270. Without the stores of the results K=512 would run at 1150: they
+// are what is left there (402 MB for 206 GFLOP). Long K is bound by the hand-over between the two groups of wavefronts and the chip's power:
+// 8192^3 at 1470, where the library's kernel reaches 1630.
+#include <hip/hip_runtime.h>
+#include <stdint.h>
+
+#include "btp_device.h"
+#include "btp_launch.h"
+#include "layer_tile.h"
+
+namespace spear_btp {
+
+namespace {
+
+constexpr int kTileRows = 256, kTileCols = 256, kStepK = 64;
+constexpr int kStage = kTileRows * kStepK * 2;  // bytes of a stage of either operand
+constexpr int kPanels = 4;                      // row panels of a group of tiles
+
+struct Tile {
+  int panel, job, col;  // 256 rows from 256 panel on, columns of out[job] from col on
+};
+
+__device__ __forceinline__ Tile tile_at(const LayerLinearArgs& p, int tiles_n, int id) {
+  const int panels = (p.M + kTileRows - 1) / kTileRows, group = id / (kPanels * tiles_n), at = id - group * kPanels * tiles_n;
+  const int in_group = min(kPanels, panels - group * kPanels);
+  int n = at / in_group;
+  Tile t{group * kPanels + at - n * in_group, 0, 0};
+  while (n >= (p.N[t.job] + kTileCols - 1) / kTileCols) n -= (p.N[t.job++] + kTileCols - 1) / kTileCols;
+  t.col = kTileCols * n;
+  return t;
+}
+
+// The fragments of 32 columns: 8 row tiles of x, 4 column tiles of the weights, 2 KiB apart. The wait is part of the block: the
+// registers are written when it ends.
+__device__ __forceinline__ void read_fragments(uint32_t x, uint32_t w, i32x4_t (&fx)[8], i32x4_t (&fw)[4]) {
+  asm volatile(
+      "ds_read_b128 %8, %13\n ds_read_b128 %9, %13 offset:2048\n ds_read_b128 %10, %13 offset:4096\n ds_read_b128 %11, %13 offset:6144\n"
+      "ds_read_b128 %0, %12\n ds_read_b128 %1, %12 offset:2048\n ds_read_b128 %2, %12 offset:4096\n ds_read_b128 %3, %12 offset:6144\n"
+      "ds_read_b128 %4, %12 offset:8192\n ds_read_b128 %5, %12 offset:10240\n ds_read_b128 %6, %12 offset:12288\n"
+      "ds_read_b128 %7, %12 offset:14336\n"
+      "s_waitcnt lgkmcnt(0)"
+      : "=&v"(fx[0]), "=&v"(fx[1]), "=&v"(fx[2]), "=&v"(fx[3]), "=&v"(fx[4]), "=&v"(fx[5]), "=&v"(fx[6]), "=&v"(fx[7]),
+        "=&v"(fw[0]), "=&v"(fw[1]), "=&v"(fw[2]), "=&v"(fw[3])
+      : "v"(x), "v"(w)
+      : "memory");
+}
+
+// kStreamed: results are stored with the non-temporal hint, so that L2 writes them back at once and not when the next tile's
+// stores need the room. K=512: 223 against 236 us for the four projections of 131072 rows; K=1600: 192 against 184.
+template <bool kStreamed>
+__global__ __launch_bounds__(512) void layer_gemm_kernel(const LayerLinearArgs p, int tiles_n, int tiles) {
+  __shared__ __attribute__((aligned(1024))) char lds[5 * kStage];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  const int n = lane & 15, q = lane >> 4, wm = wave >> 2, wn = wave & 3;
+  const int K = p.K, ldx = (int)p.ldx, steps = (K + kStepK - 1) / kStepK;
+  const int xcd = blockIdx.x & 7, slots = gridDim.x >> 3;
+  const int last = (int)((long)tiles * (xcd + 1) / 8);
+  int id = (int)((long)tiles * xcd / 8) + (int)(blockIdx.x >> 3);
+  if (id >= last) return;
+
+  // Requests: number i (0 .. 3) of wavefront w moves rows 32 w + 8 i .. + 7 of a stage, 16 bytes per lane
+  const int row = 32 * wave + (lane >> 3);
+  const uint32_t piece = ((lane & 7) ^ (lane >> 4)) * 16;  // rows 8 further have it 64 bytes across
+  const uint32_t x0 = row * ldx * 2 + piece, x1 = (row + 8) * ldx * 2 + (piece ^ 64), x16 = 32 * ldx, w16 = 32 * K;
+  uint32_t w0 = 0, w1 = 0;
+  const char *px = nullptr, *pw = nullptr;  // next step's columns of the tile, and what is left from there: bytes to the end of
+  int nx = 0, nw = 0, kx = 0, kw = 0;       // the last row, bytes of a row
+  auto aim_x = [&](const Tile& t) {
+    const int rows = min(kTileRows, p.M - t.panel * kTileRows);
+    px = reinterpret_cast<const char*>(p.x + (long)t.panel * kTileRows * ldx);
+    nx = ((rows - 1) * ldx + K) * 2;
+    kx = 2 * K;
+  };
+  auto aim_w = [&](const Tile& t) {
+    const int cols = min(kTileCols, p.N[t.job] - t.col);
+    pw = reinterpret_cast<const char*>(p.w[t.job] + (long)t.col * K);
+    nw = cols * K * 2;
+    kw = 2 * K;
+    // wavefront wn has the rows 64 wn .. of a stage: the tile's columns in order, or 32 wn .. + 31 and these + 128 where there are
+    // no more than 128 columns
+    const int col = cols > 128 ? row : (row & 31) + (row >> 6) * 32 + (row & 32) * 4;
+    w0 = col * K * 2 + piece;
+    w1 = (col + 8) * K * 2 + (piece ^ 64);
+  };
+  auto request = [&](char* to, const char* from, int bytes, int left, uint32_t v0, uint32_t v1, uint32_t step) {
+    const auto desc = buffer_of(from, bytes);
+    const uint32_t u0 = (int)piece < left ? v0 : kNowhere, u1 = (int)(piece ^ 64) < left ? v1 : kNowhere;
+    load_to_lds(desc, to, u0);
+    load_to_lds(desc, to + 1024, u1);
+    load_to_lds(desc, to + 2048, u0 + step);
+    load_to_lds(desc, to + 3072, u1 + step);
+  };
+  auto request_x = [&](int stage) {
+    request(lds + stage * kStage + wave * 4096, px, nx, kx, x0, x1, x16);
+    px += 2 * kStepK; nx -= 2 * kStepK; kx -= 2 * kStepK;
+  };
+  auto request_w = [&](int stage) {
+    request(lds + (3 + stage) * kStage + wave * 4096, pw, nw, kw, w0, w1, w16);
+    pw += 2 * kStepK; nw -= 2 * kStepK; kw -= 2 * kStepK;
+  };
+
+  const uint32_t base = lds_address(lds), fragment = n * 128 + (q ^ (n >> 1)) * 16;
+  const uint32_t x_at = base + wm * 128 * 128 + fragment, w_at = base + 3 * kStage + wn * 64 * 128 + fragment;
+  f32x4_t acc[8][4];  // [row tile][column tile]; lane 16 q + n: columns 4 q .. 4 q + 3 of row n
+  i32x4_t fx[8], fw[4];
+
+  Tile cur = tile_at(p, tiles_n, id);
+  aim_x(cur);
+  aim_w(cur);
+  request_x(0); request_w(0); request_x(1); request_w(1);
+  wait_vm<8>();
+  phase_barrier();
+  if (wm == 1) phase_barrier();
+  uint16_t bias_of[4][4];
+  auto load_bias = [&](const Tile& t) {
+    const uint16_t* bias = p.bias[t.job];
+    const int N = p.N[t.job];
+    const bool full = N - t.col > 128;
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int c = t.col + (full ? 64 : 32) * wn + (full ? 32 : 128) * (j >> 1) + 16 * (j & 1) + 4 * q + e;
+        bias_of[j][e] = bias != nullptr ? bias[min(c, N - 1)] : 0;
+      }
+  };
+  load_bias(cur);
+  int sx = 0, sw = 0;
+  bool stored = false;  // 16 stores are among the requests that a wait counts
+  while (true) {
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) acc[i][j] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+    const int N = p.N[cur.job], left = N - cur.col;
+    const bool full = left > 128;
+    const int span = full ? 64 : 32, across = full ? 32 : 128;  // first column of column tile j: span wn + across (j / 2) + 16 (j % 2)
+    const bool more = id + slots < last;
+    const Tile next = more ? tile_at(p, tiles_n, id + slots) : cur;  // past the last tile its first steps are asked for again, for nothing
+    auto multiply = [&]() {
+      __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+#pragma unroll
+        for (int i = 0; i < 8; ++i) acc[i][j] = mfma(fw[j], fx[i], acc[i][j]);
+      if (full) {
+#pragma unroll
+        for (int j = 2; j < 4; ++j)
+#pragma unroll
+          for (int i = 0; i < 8; ++i) acc[i][j] = mfma(fw[j], fx[i], acc[i][j]);
+      }
+      __builtin_amdgcn_s_setprio(0);
+      phase_barrier();
+    };
+    int t = 0;
+    do {
+      read_fragments(x_at + sx * kStage, w_at + sw * kStage, fx, fw);
+      phase_barrier();
+      multiply();
+      if (t == steps - 2) aim_x(next);
+      request_x(sx == 0 ? 2 : sx - 1);  // step t + 2, where step t - 1 was
+      read_fragments((x_at ^ 64) + sx * kStage, (w_at ^ 64) + sw * kStage, fx, fw);
+      // step t + 1 has landed: all but the request just made, and the stores if they came after step t + 1 was asked for
+      if (stored) wait_vm<20>();
+      else wait_vm<4>();
+      stored = false;
+      phase_barrier();
+      multiply();
+      if (t == steps - 2) aim_w(next);
+      request_w(sw);  // step t + 2: both groups of wavefronts have read the stage
+      sx = sx == 2 ? 0 : sx + 1;
+      sw ^= 1;
+    } while (++t < steps);
+
+    if (p.bias[cur.job] != nullptr) {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const f32x4_t add = {Bf16::lo(bias_of[j][0]), Bf16::lo(bias_of[j][1]), Bf16::lo(bias_of[j][2]), Bf16::lo(bias_of[j][3])};
+#pragma unroll
+        for (int i = 0; i < 8; ++i) acc[i][j] += add;
+      }
+    }
+    load_bias(next);  // before the stores: the waits of the next tile don't count these loads
+    const int rows = min(kTileRows, p.M - cur.panel * kTileRows);
+    uint16_t* out = p.out[cur.job] + (long)cur.panel * kTileRows * N + cur.col;
+    const auto desc = buffer_of(out, ((rows - 1) * N + min(kTileCols, left)) * 2);
+    const bool wide = N % 8 == 0 && (reinterpret_cast<uintptr_t>(p.out[cur.job]) & 15u) == 0;
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const int c = span * wn + across * h + (q & 1) * 16 + (q >> 1) * 8, r = wm * 128 + n;
+      const uint32_t to = c < left && (h == 0 || full) ? (uint32_t)(r * N + c) * 2 : kNowhere;
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        // lane row q gets columns 8 (q >> 1) .. + 7 of column tile 2 h + (q & 1)
+        const f32x4_t v0 = acc[i][2 * h], v1 = acc[i][2 * h + 1];
+        const u32x2_t lo = __builtin_amdgcn_permlane16_swap(Bf16::pack2(v0[0], v0[1]), Bf16::pack2(v1[0], v1[1]), false, false);
+        const u32x2_t hi = __builtin_amdgcn_permlane16_swap(Bf16::pack2(v0[2], v0[3]), Bf16::pack2(v1[2], v1[3]), false, false);
+        const u32x4_t d = {lo[0], hi[0], lo[1], hi[1]};
+        if (wide) {
+          __builtin_amdgcn_raw_buffer_store_b128(d, desc, to + (uint32_t)(16 * i * N * 2), 0, kStreamed ? 2 : 0);
+        } else if (to != kNowhere && r + 16 * i < rows) {
+#pragma unroll
+          for (int e = 0; e < 8; ++e)
+            if (c + e < left) out[(long)(r + 16 * i) * N + c + e] = (uint16_t)(d[e >> 1] >> (16 * (e & 1)));
+        }
+      }
+    }
+    if (!more) break;
+    cur = next;
+    id += slots;
+    stored = wide;
+  }
+  if (wm == 0) phase_barrier();
+  wait_vm<0>();  // the requests past the last tile write LDS
+}
+
+}  // namespace
+
+bool layer_gemm_takes(const LayerLinearArgs& p) {
+  if (p.K <= kStepK || p.K % 8 != 0 || p.ldx % 8 != 0 || p.pos != nullptr || p.K >= 1 << 21 || p.ldx >= 1 << 21) return false;
+  long tiles = 0;
+  for (int j = 0; j < p.jobs; ++j) {
+    if (p.N[j] >= 1 << 21) return false;
+    tiles += (p.N[j] + kTileCols - 1) / kTileCols;
+  }
+  return tiles * ((p.M + kTileRows - 1) / kTileRows) < 1l << 30;
+}
+
+hipError_t layer_gemm(const LayerLinearArgs& p, hipStream_t s) {
+  int tiles_n = 0;
+  for (int j = 0; j < p.jobs; ++j) tiles_n += (p.N[j] + kTileCols - 1) / kTileCols;
+  const int tiles = tiles_n * ((p.M + kTileRows - 1) / kTileRows);
+  if (tiles == 0) return hipSuccess;
+  const dim3 grid(256), block(512);  // a workgroup for every compute unit
+  if (p.K <= 1024) hipLaunchKernelGGL(layer_gemm_kernel<true>, grid, block, 0, s, p, tiles_n, tiles);
+  else hipLaunchKernelGGL(layer_gemm_kernel<false>, grid, block, 0, s, p, tiles_n, tiles);
+  return hipGetLastError();
+}
+
+}  // namespace spear_btp

@@ -8,12 +8,10 @@
 // rows (layer_mfma.h: a quarter of K per wavefront), whatever array the columns belong to, so the narrow arrays share the chip with the
 // wide ones.
 //
-// The four input projections (dim, kv heads = heads) at M rows, us in a HIP graph, this kernel / the library's four: M=128 dim=256
-// 5.7 / 28.0, M=1024 dim=512 13.1 / 21.9, M=512 dim=1024 22.2 / 25.8, M=2048 dim=512 23.2 / 23.3 (1.64 G multiply-adds), M=1024
-// dim=768 25.3 / 24.0 (1.85 G), M=4096 dim=512 38.2 / 28.4: past about 1.6 G the library's larger tiles, which read x and the
-// weights less often, win. One projection (dim x dim): M=1024 dim=512 5.7 / 5.8 (0.27 G), M=2048 dim=512 7.6 / 6.2, M=16 dim=512
-// 4.8 / 3.8, M=128 dim=768 7.2 / 4.7: alone it is the slower one on the GPU and is taken for the host time it saves (a decode step of 16
-// sequences 19.7 us as a call at K = 512 with it, 38.5 at K = 1024 with the library's product), up to 0.3 G and K = 512. The line at K is
+// Longer inputs are for the 256 x 256 tiles of layer_gemm.hip (takes_large_tiles). One projection (dim x dim) here / as the library's
+// product, us in a HIP graph: M=1024 dim=512 5.7 / 5.8 (0.27 G multiply-adds), M=2048 dim=512 7.6 / 6.2, M=16 dim=512 4.8 / 3.8, M=128
+// dim=768 7.2 / 4.7: alone it is the slower one on the GPU and is taken for the host time it saves (a decode step of 16 sequences 19.7 us
+// as a call at K = 512 with it, 38.5 at K = 1024 with the library's product), up to 0.3 G and K = 512. The line at K is
 // the GPU's, for steps in a graph; between 512 and 768 nothing was timed.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
@@ -76,10 +74,25 @@ void launch(const LayerLinearArgs& p, int groups, hipStream_t s) {
 
 }  // namespace
 
+// Whether layer_gemm's large tiles are the faster ones. Both kernels' times in us as fitted to 70 shapes (K and dim 128 to 2048, 256 to
+// 131072 rows): here rounds of 256 workgroups, growing with K; there rounds of 256 tiles of 256 x 256, 1 us per 64 columns of K. Four
+// projections, dim = K, this kernel / the other: K=128 4096 rows 7.6 / 9.6, 16384 rows 21 / 10; K=512 1024 rows 11.9 / 16.7, 2048 rows
+// 19.8 / 16.8; K=1024 256 rows 11.8 / 24, 1024 rows 37 / 26; K=2048 256 rows 36 / 41, 1024 rows 112 / 44.
+static bool takes_large_tiles(const LayerLinearArgs& p, int groups) {
+  if (!layer_gemm_takes(p)) return false;
+  long tiles = 0;
+  for (int j = 0; j < p.jobs; ++j) tiles += (p.N[j] + 255) / 256;
+  tiles *= (p.M + 255) / 256;
+  const double here = 4.0 + (0.7 + 0.0098 * p.K) * (double)groups * ((p.M + 63) / 64) / 256;
+  const double there = 8.0 + (double)((tiles + 255) / 256) * (1.0 + (p.K + 63) / 64);
+  return there < here;
+}
+
 hipError_t layer_linear(const LayerLinearArgs& p, hipStream_t s) {
   int groups = 0;
   for (int j = 0; j < p.jobs; ++j) groups += (p.N[j] + 63) / 64;
   if (groups == 0 || p.M == 0) return hipSuccess;
+  if (takes_large_tiles(p, groups)) return layer_gemm(p, s);
   // as layer_token chooses: as many workgroups as there are while they are few
   const long pairs = (long)groups * ((p.M + 15) / 16);
   if (pairs <= 256) launch<1, 4>(p, groups, s);

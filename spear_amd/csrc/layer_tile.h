@@ -1,0 +1,54 @@
+// What the layer's large matrix kernels share: 16-byte loads from memory to LDS, waits and barriers that the compiler leaves where they
+// are, and the matrix instruction.
+#pragma once
+
+#include <hip/hip_runtime.h>
+#include <stdint.h>
+
+namespace spear_btp {
+
+namespace {
+
+typedef float f32x4_t __attribute__((ext_vector_type(4)));
+typedef int i32x4_t __attribute__((ext_vector_type(4)));
+typedef unsigned u32x2_t __attribute__((ext_vector_type(2)));
+typedef unsigned u32x4_t __attribute__((ext_vector_type(4)));
+typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
+typedef __attribute__((address_space(3))) void lds_void_t;
+
+// An offset past the end of every buffer: loads give zero there and stores are dropped. Offsets of up to 2^30 may be added to it.
+constexpr uint32_t kNowhere = 0x80000000u;
+
+__device__ __forceinline__ f32x4_t mfma(i32x4_t a, i32x4_t b, f32x4_t acc) {
+  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, a), __builtin_bit_cast(bf16x8_t, b), acc, 0, 0, 0);
+}
+
+// A buffer of `bytes` bytes (none if negative), which the hardware checks every access against.
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t buffer_of(const void* p, int bytes) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, max(bytes, 0), 0x00020000);
+}
+
+// 16 bytes per lane from `offset` (the lane's own) to `to` + 16 lane; `to` is the same in all lanes. Counted by wait_vm.
+__device__ __forceinline__ void load_to_lds(__amdgpu_buffer_rsrc_t from, char* to, uint32_t offset) {
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(from, (lds_void_t*)to, 16, offset, 0, 0, 0);
+}
+
+__device__ __forceinline__ uint32_t lds_address(char* p) { return (uint32_t)(uintptr_t)(lds_void_t*)p; }
+
+// Until no more than kOutstanding of this wavefront's loads and stores are under way.
+template <int kOutstanding>
+__device__ __forceinline__ void wait_vm() {
+  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kOutstanding) : "memory");
+}
+
+// A barrier that no instruction is moved over. It orders LDS only with the waits that the caller has made: fragment reads end with
+// theirs, loads to LDS with wait_vm.
+__device__ __forceinline__ void phase_barrier() {
+  __builtin_amdgcn_sched_barrier(0);
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_sched_barrier(0);
+}
+
+}  // namespace
+
+}  // namespace spear_btp

@@ -1,0 +1,86 @@
+"""The layer's projections at sizes of the large-tile kernel (spear_layer_linear on many rows): up to four of them on the same rows,
+against float64 products of the same bf16 operands, at the edges of its 256 x 256 x 64 tiles."""
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+def assert_product(got, x, w, bias, label):
+    """|got - x w^T - b| <= half a step of the result (bf16 has 8 significant bits: up to 2^-8 of it) and the fp32 sum's error, K 2^-24 of the terms' sum."""
+    x, w = x.double(), w.double()
+    want = x @ w.t()
+    terms = x.abs() @ w.abs().t()
+    if bias is not None:
+        want = want + bias.double()
+        terms = terms + bias.double().abs()
+    bound = want.abs() * 2.0**-8 + terms * (x.shape[1] + 1) * 2.0**-24 * (1 + 2.0**-8)
+    over = (got.double() - want).abs() - bound
+    assert over.max().item() <= 0, f"{label}: {over.max().item():.3e} over the bound"
+
+
+# M, K, columns of the projections (bias on all but every third). The rows make the large tiles the faster choice: remainders of 256 rows and
+# columns, of 64 columns of K, widths of 128 and less (half tiles), not a multiple of 8 (element stores), several tiles per workgroup and
+# more than one group of row panels, two steps of K.
+SHAPES = [
+    (4099, 520, (592, 592, 257, 37)),
+    (4096, 512, (512, 512, 512, 32)),
+    (2305, 1032, (1040, 129, 128, 127)),
+    (16400, 136, (256, 272, 16, 5)),
+    (20000, 72, (1024, 130)),
+    (9000, 1000, (640,)),
+    (1024, 2048, (2048, 512, 512, 128)),
+]
+
+
+@pytest.mark.parametrize("M,K,columns", SHAPES)
+@pytest.mark.parametrize("extra", [0, 24], ids=["dense", "strided"])
+def test_large_projections_against_float64(M, K, columns, extra):
+    from spear_amd import _btp
+
+    g = torch.Generator(device=DEV).manual_seed(M + K + extra)
+
+    def normal(*shape):
+        return torch.randn(*shape, generator=g, device=DEV).bfloat16()
+
+    x = normal(M, K + extra)[:, :K]
+    weights = [(normal(n, K) * K**-0.5).bfloat16() for n in columns]
+    biases = [None if i % 3 == 2 else normal(n) for i, n in enumerate(columns)]
+    print(f"projections M={M} K={K} columns={columns} row stride {K + extra}", flush=True)
+    out = _btp.load_extension().linears(x, weights, biases)
+    for i, (y, w, b) in enumerate(zip(out, weights, biases)):
+        assert_product(y, x, w, b, f"M={M} K={K} projection {i} of {len(columns)}")
+
+
+def test_large_projections_keep_rows_apart():
+    """What lies beside a row (the next row's first columns, read with a step that K does not fill) must not reach its result."""
+    from spear_amd import _btp
+
+    M, K, N = 4096, 520, 1040
+    x = torch.randn(M, K, device=DEV).bfloat16()
+    x[1::2] = float("nan")
+    w = torch.randn(N, K, device=DEV).bfloat16()
+    y, = _btp.load_extension().linears(x, [w], [None])
+    torch.cuda.synchronize()
+    assert torch.isfinite(y[::2]).all() and torch.isnan(y[1::2]).all()
+
+
+def test_large_projections_in_a_graph_follow_their_inputs():
+    from spear_amd import _btp
+
+    M, K, N = 4096, 512, 1024
+    x, w = torch.randn(M, K, device=DEV).bfloat16(), torch.randn(N, K, device=DEV).bfloat16()
+    run = lambda: _btp.load_extension().linears(x, [w, w], [None, None])
+    run()
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        y = run()
+    for seed in range(3):
+        x.copy_(torch.randn(M, K, generator=torch.Generator().manual_seed(seed)).to(DEV))
+        graph.replay()
+        torch.cuda.synchronize()
+        for got, want in zip(y, run()):
+            assert torch.equal(got, want)
