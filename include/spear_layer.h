@@ -40,6 +40,13 @@ int spear_layer_sums(int n, const float* const* in, void* const* out, const long
 int spear_layer_stack(const void* w_a, const void* w_b, const void* w_c, const void* w_v, void* stacked, void* packed, long long M,
                       int ld, int K, int H, int Fkv, int F, void* stream);
 
+/* The same weights transposed, as spear_layer_linear takes them for the input gradients, and proj_out's, and the same padding:
+ *     stacked [K, ld]: columns w_b^T, w_c^T, w_v^T, w_a^T, zeros       out_t [F, K]: w_out^T, w_out [K, F]
+ *     packed [M, ld]: columns 2 Fkv + F + H .. ld <- 0
+ * 16-bit elements, dense, 16-byte aligned; ld, K, Fkv and F multiples of 8. */
+int spear_layer_transpose(const void* w_a, const void* w_b, const void* w_c, const void* w_v, const void* w_out, void* stacked, void* out_t,
+                          void* packed, long long M, int ld, int K, int H, int Fkv, int F, void* stream);
+
 /* n (1 .. 4) linear layers on the same rows, bf16 with fp32 sums:  out[i] [M, N[i]] = x [M, K] w[i]^T + bias[i] (null: none). x has
  * rows ldx elements apart, the rest is dense; K and ldx multiples of 8; x and w 16-byte, out 8-byte, bias 2-byte aligned.
  * pos: NULL, or int32 [M] block positions that are moved on by one, to 0 from block_len - 1. */

@@ -64,7 +64,7 @@ int check_common(const char* who, int B, int H, int L, int k, int in_dtype, int 
 
 extern "C" {
 
-int spear_btp_abi_version(void) { return 25; }
+int spear_btp_abi_version(void) { return 26; }
 
 const char* spear_btp_last_error(void) { return g_error; }
 
@@ -267,6 +267,29 @@ int spear_layer_stack(const void* w_a, const void* w_b, const void* w_c, const v
   spear_btp::LayerStackArgs a{{u(w_b), u(w_c), u(w_v), u(w_a)}, {Fkv, Fkv, F, H}, static_cast<uint16_t*>(stacked),
                               static_cast<uint16_t*>(packed), (long)M, 2 * Fkv + F + H, ld, K};
   const hipError_t err = spear_btp::layer_stack(a, static_cast<hipStream_t>(stream));
+  if (err != hipSuccess) return fail(SPEAR_BTP_ELAUNCH, "%s: launch failed: %s", who, hipGetErrorString(err));
+  return 0;
+}
+
+int spear_layer_transpose(const void* w_a, const void* w_b, const void* w_c, const void* w_v, const void* w_out, void* stacked, void* out_t,
+                          void* packed, long long M, int ld, int K, int H, int Fkv, int F, void* stream) {
+  g_error[0] = '\0';
+  const char* who = "spear_layer_transpose";
+  if (M < 0 || H < 0 || Fkv < 0 || F < 0 || K <= 0 || ld <= 0 || 2ll * Fkv + F + H > ld)
+    return fail(SPEAR_BTP_EINVAL, "%s: bad shape (M=%lld ld=%d K=%d H=%d Fkv=%d F=%d)", who, M, ld, K, H, Fkv, F);
+  if (K % 8 != 0 || ld % 8 != 0 || Fkv % 8 != 0 || F % 8 != 0)
+    return fail(SPEAR_BTP_EINVAL, "%s: K, ld, Fkv and F must be multiples of 8 (K=%d ld=%d Fkv=%d F=%d)", who, K, ld, Fkv, F);
+  if (M * ld >= (1ll << 41) || ((long long)ld + F) * K >= (1ll << 41)) return fail(SPEAR_BTP_EINVAL, "%s: tensor too large", who);
+  for (const void* q : {w_a, w_b, w_c, w_v, w_out, static_cast<const void*>(stacked), static_cast<const void*>(out_t), static_cast<const void*>(packed)}) {
+    if (!q) return fail(SPEAR_BTP_ENULL, "%s: NULL tensor pointer", who);
+    if (!aligned16(q)) return fail(SPEAR_BTP_EINVAL, "%s: tensor pointers must be 16-byte aligned", who);
+  }
+  auto u = [](const void* q) { return static_cast<const uint16_t*>(q); };
+  uint16_t* const to = static_cast<uint16_t*>(stacked);
+  const int a_at = 2 * Fkv + F;  // the columns of a reach to the end of a row, padding included
+  const spear_btp::LayerTransposeJob jobs[] = {{u(w_b), to, Fkv, K, Fkv, ld}, {u(w_c), to + Fkv, Fkv, K, Fkv, ld}, {u(w_v), to + 2 * Fkv, F, K, F, ld},
+                                               {u(w_a), to + a_at, H, K, ld - a_at, ld}, {u(w_out), static_cast<uint16_t*>(out_t), K, F, K, K}};
+  const hipError_t err = spear_btp::layer_transpose(jobs, 5, static_cast<uint16_t*>(packed), (long)M, a_at + H, ld, static_cast<hipStream_t>(stream));
   if (err != hipSuccess) return fail(SPEAR_BTP_ELAUNCH, "%s: launch failed: %s", who, hipGetErrorString(err));
   return 0;
 }

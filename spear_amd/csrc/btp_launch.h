@@ -154,6 +154,16 @@ struct LayerStackArgs {
 };
 hipError_t layer_stack(const LayerStackArgs& p, hipStream_t s);
 
+// in [rows, cols] (dense, cols a multiple of 8) as out[c * ld + r], zeros for r = rows .. width - 1 (width and ld multiples of 8; 16-byte
+// aligned), and zeros into the columns used .. ld of packed [M, ld] as layer_stack leaves them (none if used == ld).
+struct LayerTransposeJob {
+  const uint16_t* in;
+  uint16_t* out;
+  int rows, cols, width, ld;
+};
+constexpr int kLayerTransposeJobs = 5;
+hipError_t layer_transpose(const LayerTransposeJob* jobs, int n, uint16_t* packed, long M, int used, int ld, hipStream_t s);
+
 constexpr int kLayerSumJobs = 5;  // the most jobs of one launch
 hipError_t layer_sums(const LayerSumJob* jobs, int n, int dtype, hipStream_t s);
 long layer_sums_blocks(const LayerSumJob* jobs, int n);

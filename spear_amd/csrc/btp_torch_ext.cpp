@@ -474,6 +474,17 @@ bool own_products(int64_t M, const std::vector<at::Tensor>& weights, int64_t K) 
   return small_product(M, weights[0].size(0), K) || (K <= 512 && tiles >= 512);
 }
 
+// Whether an input gradient of M rows by K columns is faster through spear_layer_linear with the weights transposed first than as the
+// library's product with them as they lie: where its tiles fill the chip. Measured, us, spear_layer_linear / the library, K the layer's
+// width: proj_out's input gradient at K=512 131072 rows 75 / 91, 16384 rows (128 tiles) 17.2 / 16.8, K=768 16384 rows (192 tiles) 23.4 /
+// 26.5, K=1024 8192 rows (128) 26.2 / 23.8, K=2048 65536 rows 453 / 470, 8192 rows (256) 58 / 59; that of the four input projections at K=512
+// 131072 rows 198 / 208, 16384 rows (128) 37 / 30, K=768 16384 rows (192) 55 / 57, K=1024 131072 rows 663 / 697, K=2048 65536 rows 1213 /
+// 1299. A round of the chip that is three quarters full still gains; at 20000 rows of K=1024, 316 tiles, it would not be.
+bool own_input_grads(int64_t M, int64_t K) {
+  const int64_t tiles = (M + 255) / 256 * ((K + 255) / 256), rounds = (tiles + 255) / 256;
+  return K % 8 == 0 && 4 * tiles >= 3 * 256 * rounds;
+}
+
 // The four input projections (a, b, c, v) of x [..., K], or one projection without bias, by either. x dense.
 std::vector<at::Tensor> project(const at::Tensor& x, const std::vector<at::Tensor>& weights, const std::vector<at::Tensor>& biases) {
   const int64_t K = x.size(-1), M = K > 0 ? x.numel() / K : 0;
@@ -498,7 +509,7 @@ at::Tensor weight_grad(const at::Tensor& dy, const at::Tensor& x, int64_t s, std
 // autograd node. Backward is what spear_amd/nn/phalanx/projections.py does with _ProjectAndMix and _Linear (one product each for the
 // input and weight gradients of the four projections, against the packed gradient buffer), without Python frames and with
 // layer_stack and layer_sums around the products: 10 launches for forward and backward of a small layer where separate modules had 29.
-// The mixing kernels are the same; the input gradients and weight gradients are the library's products.
+// The mixing kernels are the same; the weight gradients are the library's products, and so are the input gradients of few rows.
 struct LayerNode : public torch::autograd::Function<LayerNode> {
   static at::Tensor forward(torch::autograd::AutogradContext* ctx, const at::Tensor& x, const at::Tensor& w_a, const at::Tensor& b_a,
                             const at::Tensor& w_b, const at::Tensor& b_b, const at::Tensor& w_c, const at::Tensor& b_c,
@@ -555,12 +566,24 @@ struct LayerNode : public torch::autograd::Function<LayerNode> {
       sums.clear();
     }
     if (front) {
-      const at::Tensor dmixed = at::mm(dy, w_out).view({B, L, F});
       const int64_t used = 2 * Fkv + F + heads, ld = (used + 63) / 64 * 64;  // [b | c | v | a | padding]
-      const at::Tensor packed = at::empty({B, L, ld}, v.options()), stacked = at::empty({ld, K}, v.options());
-      const int rc = spear_layer_stack(w_a.data_ptr(), w_b.data_ptr(), w_c.data_ptr(), w_v.data_ptr(), stacked.data_ptr(),
-                                       packed.data_ptr(), M, (int)ld, (int)K, (int)heads, (int)Fkv, (int)F, stream_of(v));
-      if (rc != 0) raise_native(rc);
+      // input gradients against the stacked weights: [ld, K] as the library takes them, or transposed for the kernel here
+      const bool own = own_input_grads(M, K) && (reinterpret_cast<uintptr_t>(dy.data_ptr()) & 15u) == 0;
+      const at::Tensor packed = at::empty({B, L, ld}, v.options());
+      const at::Tensor stacked = own ? at::empty({K, ld}, v.options()) : at::empty({ld, K}, v.options());
+      at::Tensor dmixed;
+      if (own) {
+        const at::Tensor out_t = at::empty({F, K}, v.options());
+        const int rc = spear_layer_transpose(w_a.data_ptr(), w_b.data_ptr(), w_c.data_ptr(), w_v.data_ptr(), w_out.data_ptr(), stacked.data_ptr(),
+                                             out_t.data_ptr(), packed.data_ptr(), M, (int)ld, (int)K, (int)heads, (int)Fkv, (int)F, stream_of(v));
+        if (rc != 0) raise_native(rc);
+        dmixed = linears(dy, {out_t}, {at::Tensor()})[0].view({B, L, F});
+      } else {
+        const int rc = spear_layer_stack(w_a.data_ptr(), w_b.data_ptr(), w_c.data_ptr(), w_v.data_ptr(), stacked.data_ptr(),
+                                         packed.data_ptr(), M, (int)ld, (int)K, (int)heads, (int)Fkv, (int)F, stream_of(v));
+        if (rc != 0) raise_native(rc);
+        dmixed = at::mm(dy, w_out).view({B, L, F});
+      }
       const int64_t rows = spear_phalanx_mix_backward_sum_rows((int)B, (int)L, (int)heads);
       const auto f32 = v.options().dtype(at::kFloat);
       parts = {at::empty({rows, heads}, f32), at::empty({rows, Fkv}, f32), at::empty({rows, Fkv}, f32)};
@@ -572,9 +595,13 @@ struct LayerNode : public torch::autograd::Function<LayerNode> {
       out[6] = sums[2];
       const at::Tensor d2 = packed.view({M, ld});
       if (ctx->needs_input_grad(0)) {
-        out[0] = at::empty({B, L, K}, v.options());  // not a view of the product, for callers that work on it in place
-        at::Tensor dx = out[0].view({M, K});
-        at::mm_out(dx, d2, stacked);
+        if (own) {
+          out[0] = linears(packed, {stacked}, {at::Tensor()})[0];
+        } else {
+          out[0] = at::empty({B, L, K}, v.options());  // not a view of the product, for callers that work on it in place
+          at::Tensor dx = out[0].view({M, K});
+          at::mm_out(dx, d2, stacked);
+        }
       }
       if (weights) {
         const at::Tensor dw = weight_grad(d2, x2, ctx->saved_data["slices_in"].toInt(), parts, sums);

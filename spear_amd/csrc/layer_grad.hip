@@ -10,6 +10,10 @@
 // padding columns, and zeros in those columns: one launch where a concatenation and two fills were three (and a copy more where a
 // weight's type or layout had to be changed). Bound by the launch at small sizes, by writing [ld, K] else.
 //
+// layer_transpose: the same weights and proj_out's as the large-tile kernel (layer_gemm.hip) wants them for the input gradients, rows of the
+// reduction's columns, and the same zeros. 64 x 64 tiles through LDS, 16 bytes per access on both sides; bound by the launch at small
+// sizes (6 us for 2.6 MB at dim 512), by reading and writing each weight once else.
+//
 // A block of layer_sums, 512 threads, takes either 2048 columns, four to a thread, and walks the rows with eight 16-byte loads in flight
 // (few rows), or 16 columns with 32 threads to a column that add up through LDS (many rows: 2048 rows by 512 columns
 // still make 32 blocks). Sums are taken in an order that depends on the shape only: the same bits in every run.
@@ -92,6 +96,19 @@ __global__ __launch_bounds__(kThreads) void layer_sums_kernel(const Jobs jobs, i
   }
 }
 
+// The 16-byte pieces of packed's rows that reach past its last used column <- zeros from that column on. i: which of them.
+__device__ __forceinline__ void clear_padding(uint16_t* packed, int used, int ld, long i) {
+  const int first = used / 8, per_row = ld / 8 - first;
+  const long row = i / per_row;
+  const int col = 8 * (first + (int)(i - row * per_row));
+  uint16_t* at = packed + row * ld + col;
+  if (col >= used) {
+    *reinterpret_cast<uint4*>(at) = make_uint4(0, 0, 0, 0);
+  } else {
+    for (int e = used - col; e < 8; ++e) at[e] = 0;
+  }
+}
+
 // One 16-byte piece per thread: first the pieces of the stacked weights [ld, K], then those of the buffer's rows that reach
 // past the last used column. Only columns from `used` on are written there.
 __global__ __launch_bounds__(256) void layer_stack_kernel(const LayerStackArgs p, long stack_pieces, long total) {
@@ -113,18 +130,64 @@ __global__ __launch_bounds__(256) void layer_stack_kernel(const LayerStackArgs p
     *reinterpret_cast<uint4*>(p.stacked + i * 8) = q;
     return;
   }
-  const int first = p.used / 8, per_row = p.ld / 8 - first;
-  const long j = i - stack_pieces, row = j / per_row;
-  const int col = 8 * (first + (int)(j - row * per_row));
-  uint16_t* at = p.packed + row * p.ld + col;
-  if (col >= p.used) {
-    *reinterpret_cast<uint4*>(at) = zero;
-  } else {
-    for (int e = p.used - col; e < 8; ++e) at[e] = 0;
+  clear_padding(p.packed, p.used, p.ld, i - stack_pieces);
+}
+
+struct Transposes {
+  LayerTransposeJob job[kLayerTransposeJobs];
+  int first_block[kLayerTransposeJobs + 1];
+};
+
+constexpr int kSide = 64;
+
+__global__ __launch_bounds__(256) void layer_transpose_kernel(const Transposes jobs, int n, uint16_t* packed, int used, int ld, long pieces) {
+  __shared__ __attribute__((aligned(16))) uint16_t tile[kSide][kSide + 8];
+  if ((int)blockIdx.x >= jobs.first_block[n]) {
+    const long i = (long)((int)blockIdx.x - jobs.first_block[n]) * 256 + threadIdx.x;
+    if (i < pieces) clear_padding(packed, used, ld, i);
+    return;
+  }
+  int at = 0;
+  while ((int)blockIdx.x >= jobs.first_block[at + 1]) ++at;
+  const LayerTransposeJob j = jobs.job[at];
+  const int block = (int)blockIdx.x - jobs.first_block[at], across = (j.cols + kSide - 1) / kSide;
+  const int r0 = block / across * kSide, c0 = block % across * kSide;
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const int r = (int)threadIdx.x / 8 + 32 * i, c = (int)threadIdx.x % 8 * 8;
+    uint4 q = make_uint4(0, 0, 0, 0);
+    if (r0 + r < j.rows && c0 + c < j.cols) q = *reinterpret_cast<const uint4*>(j.in + (long)(r0 + r) * j.cols + c0 + c);
+    *reinterpret_cast<uint4*>(&tile[r][c]) = q;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const int c = (int)threadIdx.x / 8 + 32 * i, r = (int)threadIdx.x % 8 * 8;
+    if (c0 + c >= j.cols || r0 + r >= j.width) continue;
+    uint32_t w[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) w[e] = tile[r + 2 * e][c] | (uint32_t)tile[r + 2 * e + 1][c] << 16;
+    *reinterpret_cast<uint4*>(j.out + (long)(c0 + c) * j.ld + r0 + r) = make_uint4(w[0], w[1], w[2], w[3]);
   }
 }
 
 }  // namespace
+
+hipError_t layer_transpose(const LayerTransposeJob* jobs, int n, uint16_t* packed, long M, int used, int ld, hipStream_t s) {
+  Transposes all{};
+  long blocks = 0;
+  for (int i = 0; i < n; ++i) {
+    all.job[i] = jobs[i];
+    all.first_block[i] = (int)blocks;
+    blocks += (long)((jobs[i].width + kSide - 1) / kSide) * ((jobs[i].cols + kSide - 1) / kSide);
+  }
+  all.first_block[n] = (int)blocks;
+  const long pieces = used < ld ? M * (ld / 8 - used / 8) : 0;
+  blocks += (pieces + 255) / 256;
+  if (blocks == 0) return hipSuccess;
+  hipLaunchKernelGGL(layer_transpose_kernel, dim3((unsigned)blocks), dim3(256), 0, s, all, n, packed, used, ld, pieces);
+  return hipGetLastError();
+}
 
 hipError_t layer_stack(const LayerStackArgs& p, hipStream_t s) {
   const long stack_pieces = (long)p.ld * (p.K / 8), total = stack_pieces + (p.used < p.ld ? p.M * (p.ld / 8 - p.used / 8) : 0);

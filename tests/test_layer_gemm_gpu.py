@@ -84,3 +84,28 @@ def test_large_projections_in_a_graph_follow_their_inputs():
         torch.cuda.synchronize()
         for got, want in zip(y, run()):
             assert torch.equal(got, want)
+
+
+@pytest.mark.parametrize("M,dim,heads,kv_heads", [(33, 592, 37, 37), (5, 128, 8, 2), (1, 2048, 128, 32), (70, 1040, 65, 5)])
+def test_transposed_weights_and_padding(M, dim, heads, kv_heads):
+    import ctypes
+
+    from spear_amd import _btp
+
+    lib = _btp.load_library()
+    lib.spear_layer_transpose.argtypes = [ctypes.c_void_p] * 8 + [ctypes.c_longlong] + [ctypes.c_int] * 5 + [ctypes.c_void_p]
+    F, Fkv = 16 * heads, 16 * kv_heads
+    used = 2 * Fkv + F + heads
+    ld = -(-used // 64) * 64
+    w_a, w_b, w_c, w_v = (torch.randn(n, dim, device=DEV).bfloat16() for n in (heads, Fkv, Fkv, F))
+    w_out = torch.randn(dim, F, device=DEV).bfloat16()
+    stacked, out_t = torch.full((dim, ld), 7.0, device=DEV).bfloat16(), torch.full((F, dim), 7.0, device=DEV).bfloat16()
+    packed = torch.full((M, ld), 7.0, device=DEV).bfloat16()
+    print(f"transpose M={M} dim={dim} heads={heads} kv_heads={kv_heads} ld={ld}", flush=True)
+    rc = lib.spear_layer_transpose(*(t.data_ptr() for t in (w_a, w_b, w_c, w_v, w_out, stacked, out_t, packed)), M, ld, dim, heads, Fkv, F,
+                                   torch.cuda.current_stream().cuda_stream)
+    assert rc == 0
+    torch.cuda.synchronize()
+    assert torch.equal(stacked[:, :used], torch.cat([w_b, w_c, w_v, w_a]).t()) and (stacked[:, used:] == 0).all()
+    assert torch.equal(out_t, w_out.t())
+    assert (packed[:, :used] == 7).all() and (packed[:, used:] == 0).all()
