@@ -53,6 +53,22 @@ int spear_layer_transpose(const void* w_a, const void* w_b, const void* w_c, con
 int spear_layer_linear(int n, const void* x, long long ldx, int M, int K, const void* const* w, const void* const* bias,
                        void* const* out, const int* N, int* pos, int block_len, void* stream);
 
+/* n (1 .. 2) products over M tokens, bf16, as fp32 parts:  dy[i]^T x[i], [N[i], K[i]], cut into splits[i] runs of tokens.
+ *     dy[i] [M, N[i]], rows ld_dy[i] elements apart, cols_dy[i] >= N[i] of which may be read       x[i] [M, K[i]] dense
+ *     parts  fp32, 65536 * sum of splits[i] ceil(N[i] / 256) ceil(K[i] / 256) elements; written in the order that
+ *            spear_layer_wgrad_sums reads
+ * ld_dy, cols_dy and K multiples of 8; pointers 16-byte aligned; 1 <= splits[i] <= ceil(M / 32). */
+int spear_layer_wgrad(int n, const void* const* dy, const int* ld_dy, const int* cols_dy, const int* N, const void* const* x, const int* K,
+                      const int* splits, long long M, float* parts, void* stream);
+
+/* The number of splits for one of these products that the library's model of it expects to be fastest. */
+int spear_layer_wgrad_splits(long long M, int N, int K);
+
+/* The parts added up and rounded to `dtype` (16-bit), dw[i] [N[i], K[i]] dense, and m (0 .. 3) column sums of dense fp32 arrays as
+ * spear_layer_sums makes them, in one launch. dw[i] 8-byte aligned. */
+int spear_layer_wgrad_sums(int n, const float* parts, const int* N, const int* K, const int* splits, void* const* dw, int m,
+                           const float* const* in, void* const* out, const long long* rows, const long long* cols, int dtype, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

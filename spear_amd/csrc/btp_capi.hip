@@ -325,6 +325,63 @@ int spear_layer_linear(int n, const void* x, long long ldx, int M, int K, const 
   return 0;
 }
 
+static long long wgrad_units(int N, int K, int splits) { return (long long)((N + 255) / 256) * ((K + 255) / 256) * splits; }
+
+int spear_layer_wgrad(int n, const void* const* dy, const int* ld_dy, const int* cols_dy, const int* N, const void* const* x, const int* K,
+                      const int* splits, long long M, float* parts, void* stream) {
+  g_error[0] = '\0';
+  const char* who = "spear_layer_wgrad";
+  if (n < 1 || n > 2 || M < 1 || M >= (1ll << 31)) return fail(SPEAR_BTP_EINVAL, "%s: bad shape (n=%d M=%lld)", who, n, M);
+  if (!dy || !ld_dy || !cols_dy || !N || !x || !K || !splits || !parts) return fail(SPEAR_BTP_ENULL, "%s: NULL array", who);
+  spear_btp::LayerWgradArgs a{{}, (long)M, parts};
+  long long units = 0;
+  for (int i = 0; i < n; ++i) {
+    if (N[i] <= 0 || K[i] <= 0 || cols_dy[i] < N[i] || ld_dy[i] < cols_dy[i] || ld_dy[i] % 8 != 0 || cols_dy[i] % 8 != 0 || K[i] % 8 != 0 ||
+        ld_dy[i] >= (1 << 23) || K[i] >= (1 << 23))
+      return fail(SPEAR_BTP_EINVAL, "%s: bad columns (N=%d of %d in rows of %d, K=%d)", who, N[i], cols_dy[i], ld_dy[i], K[i]);
+    if (splits[i] < 1 || splits[i] > (M + 31) / 32) return fail(SPEAR_BTP_EINVAL, "%s: bad number of splits (%d)", who, splits[i]);
+    if (!dy[i] || !x[i]) return fail(SPEAR_BTP_ENULL, "%s: NULL tensor pointer", who);
+    if (!aligned16(dy[i]) || !aligned16(x[i]) || !aligned16(parts)) return fail(SPEAR_BTP_EINVAL, "%s: tensor pointers must be 16-byte aligned", who);
+    const long long u = wgrad_units(N[i], K[i], splits[i]);
+    units += u;
+    if (units >= (1ll << 28)) return fail(SPEAR_BTP_EINVAL, "%s: too many tiles for one launch", who);
+    a.job[i] = {static_cast<const uint16_t*>(dy[i]), static_cast<const uint16_t*>(x[i]), ld_dy[i], cols_dy[i], N[i], K[i], splits[i], (int)u};
+  }
+  const hipError_t err = spear_btp::layer_wgrad(a, static_cast<hipStream_t>(stream));
+  if (err != hipSuccess) return fail(SPEAR_BTP_ELAUNCH, "%s: launch failed: %s", who, hipGetErrorString(err));
+  return 0;
+}
+
+int spear_layer_wgrad_splits(long long M, int N, int K) { return M > 0 && N > 0 && K > 0 ? spear_btp::layer_wgrad_splits((long)M, N, K) : 1; }
+
+int spear_layer_wgrad_sums(int n, const float* parts, const int* N, const int* K, const int* splits, void* const* dw, int m,
+                           const float* const* in, void* const* out, const long long* rows, const long long* cols, int dtype, void* stream) {
+  g_error[0] = '\0';
+  const char* who = "spear_layer_wgrad_sums";
+  if (n < 1 || n > 2 || m < 0 || m > 3) return fail(SPEAR_BTP_EINVAL, "%s: bad number of results (n=%d m=%d)", who, n, m);
+  if (dtype != SPEAR_BTP_BF16 && dtype != SPEAR_BTP_F16) return fail(SPEAR_BTP_EINVAL, "%s: results must be float16 or bfloat16.", who);
+  if (!parts || !N || !K || !splits || !dw || (m > 0 && (!in || !out || !rows || !cols))) return fail(SPEAR_BTP_ENULL, "%s: NULL array", who);
+  spear_btp::LayerSumJob jobs[5];
+  long long unit = 0;
+  for (int i = 0; i < n; ++i) {
+    if (N[i] <= 0 || K[i] <= 0 || K[i] % 8 != 0 || splits[i] < 1) return fail(SPEAR_BTP_EINVAL, "%s: bad shape (N=%d K=%d splits=%d)", who, N[i], K[i], splits[i]);
+    if (!dw[i]) return fail(SPEAR_BTP_ENULL, "%s: NULL tensor pointer", who);
+    if (!aligned16(parts) || (reinterpret_cast<uintptr_t>(dw[i]) & 7u)) return fail(SPEAR_BTP_EINVAL, "%s: parts must be 16-byte and results 8-byte aligned", who);
+    jobs[i] = {parts + unit * 65536, static_cast<uint16_t*>(dw[i]), N[i], K[i], splits[i]};
+    unit += wgrad_units(N[i], K[i], splits[i]);
+  }
+  for (int i = 0; i < m; ++i) {
+    if (rows[i] < 0 || cols[i] < 0) return fail(SPEAR_BTP_EINVAL, "%s: negative dimension", who);
+    if (cols[i] > 0 && (!in[i] || !out[i])) return fail(SPEAR_BTP_ENULL, "%s: NULL tensor pointer", who);
+    if (!aligned16(in[i]) || (reinterpret_cast<uintptr_t>(out[i]) & 7u)) return fail(SPEAR_BTP_EINVAL, "%s: arrays must be 16-byte and results 8-byte aligned", who);
+    jobs[n + i] = {in[i], static_cast<uint16_t*>(out[i]), (long)rows[i], (long)cols[i]};
+  }
+  if (spear_btp::layer_sums_blocks(jobs, n + m) >= (1l << 31)) return fail(SPEAR_BTP_EINVAL, "%s: too many columns for one launch", who);
+  const hipError_t err = spear_btp::layer_sums(jobs, n + m, dtype, static_cast<hipStream_t>(stream));
+  if (err != hipSuccess) return fail(SPEAR_BTP_ELAUNCH, "%s: launch failed: %s", who, hipGetErrorString(err));
+  return 0;
+}
+
 int spear_layer_sums(int n, const float* const* in, void* const* out, const long long* rows, const long long* cols, int dtype,
                      void* stream) {
   g_error[0] = '\0';

@@ -143,6 +143,7 @@ struct LayerSumJob {
   const float* in;
   uint16_t* out;
   long rows, cols;
+  int splits = 0;  // not 0: `in` holds layer_wgrad's parts of out [rows, cols], this many to add
 };
 // The weights of the projections stacked as [ld, K] (b, c, v, a, zero rows), and zeros into the columns used .. ld of packed [M, ld].
 struct LayerStackArgs {
@@ -153,6 +154,23 @@ struct LayerStackArgs {
   int used, ld, K;  // ld and K multiples of 8
 };
 hipError_t layer_stack(const LayerStackArgs& p, hipStream_t s);
+
+// Products over the tokens in 256 x 256 tiles and splits of the tokens (layer_wgrad.hip), bf16: dy [M, N] with rows ld_dy elements apart, of
+// which cols_dy may be read, and x [M, K] dense; ld_dy, cols_dy and K multiples of 8, 16-byte aligned. parts: fp32, one dense block of 256 x
+// 256 per unit (split-major, then x's tiles, then dy's), of the first job and then the second, in the order that layer_sums reads.
+constexpr int kWgradSide = 256;
+struct LayerWgradJob {
+  const uint16_t *dy, *x;
+  int ld_dy, cols_dy, N, K, splits;
+  int units;  // splits * ceil(N / 256) * ceil(K / 256); 0: no job
+};
+struct LayerWgradArgs {
+  LayerWgradJob job[2];
+  long M;
+  float* parts;
+};
+hipError_t layer_wgrad(const LayerWgradArgs& p, hipStream_t s);
+int layer_wgrad_splits(long M, int N, int K);  // the fastest number of splits as modelled
 
 // in [rows, cols] (dense, cols a multiple of 8) as out[c * ld + r], zeros for r = rows .. width - 1 (width and ld multiples of 8; 16-byte
 // aligned), and zeros into the columns used .. ld of packed [M, ld] as layer_stack leaves them (none if used == ld).

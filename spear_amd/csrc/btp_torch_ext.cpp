@@ -505,11 +505,61 @@ at::Tensor weight_grad(const at::Tensor& dy, const at::Tensor& x, int64_t s, std
   return out;
 }
 
+// Weight gradients of one backward pass through spear_layer_wgrad: products dy^T x in one launch, their sums and the bias gradients' in another.
+struct WeightGrads {
+  std::vector<at::Tensor> dy, x, dw;  // dy [M, N or more], x [M, K], dw [N, K]
+
+  void add(const at::Tensor& grad, const at::Tensor& operand, int64_t columns) {
+    dy.push_back(grad);
+    x.push_back(operand);
+    dw.push_back(at::empty({columns, operand.size(1)}, operand.options()));
+  }
+
+  void run(const std::vector<at::Tensor>& sums_of, const std::vector<at::Tensor>& sums) {
+    const int n = (int)dy.size();
+    const void *g[2], *o[2];
+    void* w[2];
+    int ld[2], N[2], K[2], splits[2];
+    const int64_t M = x[0].size(0);
+    int64_t blocks = 0;
+    for (int i = 0; i < n; ++i) {
+      g[i] = dy[i].data_ptr();
+      o[i] = x[i].data_ptr();
+      w[i] = dw[i].data_ptr();
+      ld[i] = (int)dy[i].size(1);
+      N[i] = (int)dw[i].size(0);
+      K[i] = (int)dw[i].size(1);
+      splits[i] = spear_layer_wgrad_splits(M, N[i], K[i]);
+      blocks += (int64_t)((N[i] + 255) / 256) * ((K[i] + 255) / 256) * splits[i];
+    }
+    const at::Tensor parts = at::empty({blocks * 65536}, x[0].options().dtype(at::kFloat));
+    float* const to = static_cast<float*>(parts.data_ptr());
+    int rc = spear_layer_wgrad(n, g, ld, ld, N, o, K, splits, M, to, stream_of(x[0]));
+    if (rc != 0) raise_native(rc);
+    const float* in[3];
+    void* out[3];
+    long long rows[3], cols[3];
+    for (size_t i = 0; i < sums.size(); ++i) {
+      in[i] = static_cast<const float*>(sums_of[i].data_ptr());
+      out[i] = sums[i].data_ptr();
+      rows[i] = sums_of[i].size(0);
+      cols[i] = sums_of[i].size(1);
+    }
+    rc = spear_layer_wgrad_sums(n, to, N, K, splits, w, (int)sums.size(), in, out, rows, cols, SPEAR_BTP_BF16, stream_of(x[0]));
+    if (rc != 0) raise_native(rc);
+  }
+};
+
+// Whether the weight gradients of a layer's backward are faster through spear_layer_wgrad than as the library's (sliced) products: from
+// 12 G multiply-adds on. Times of single products at layer_wgrad.hip; 16384 tokens [1568, 512] (13 G) 52 / 60, 8192 tokens [1024, 1024] (8.6
+// G) 42 / 34, [1568, 512] (6.6 G) 37 / 37, 131072 tokens [392, 128] (6.6 G) 47 / 37.
+bool own_weight_grads(int64_t M, int64_t multiply_adds_per_token) { return M * multiply_adds_per_token >= 12000000000; }
+
 // A whole layer call on plain bf16 tensors: the four input projections, the mixing stage and the output projection, with one
 // autograd node. Backward is what spear_amd/nn/phalanx/projections.py does with _ProjectAndMix and _Linear (one product each for the
 // input and weight gradients of the four projections, against the packed gradient buffer), without Python frames and with
 // layer_stack and layer_sums around the products: 10 launches for forward and backward of a small layer where separate modules had 29.
-// The mixing kernels are the same; the weight gradients are the library's products, and so are the input gradients of few rows.
+// The mixing kernels are the same; the weight and input gradients of few tokens are the library's products.
 struct LayerNode : public torch::autograd::Function<LayerNode> {
   static at::Tensor forward(torch::autograd::AutogradContext* ctx, const at::Tensor& x, const at::Tensor& w_a, const at::Tensor& b_a,
                             const at::Tensor& w_b, const at::Tensor& b_b, const at::Tensor& w_c, const at::Tensor& b_c,
@@ -559,11 +609,18 @@ struct LayerNode : public torch::autograd::Function<LayerNode> {
       front = front || ctx->needs_input_grad(i);
       weights = weights || ((i == 1 || i == 3 || i == 5 || i == 7) && ctx->needs_input_grad(i));
     }
+    const bool own_weights = own_weight_grads(M, (ctx->needs_input_grad(8) ? K * F : 0) + (weights ? (2 * Fkv + F + heads) * K : 0));
+    WeightGrads grads;
     if (ctx->needs_input_grad(8)) {
-      out[8] = weight_grad(dy, mixed2, ctx->saved_data["slices_out"].toInt(), parts, sums);
-      if (!parts.empty()) layer_sums(parts, sums);  // while the parts are in the memory-side cache
-      parts.clear();
-      sums.clear();
+      if (own_weights && (reinterpret_cast<uintptr_t>(dy.data_ptr()) & 15u) == 0) {
+        grads.add(dy, mixed2, K);
+        out[8] = grads.dw[0];
+      } else {
+        out[8] = weight_grad(dy, mixed2, ctx->saved_data["slices_out"].toInt(), parts, sums);
+        if (!parts.empty()) layer_sums(parts, sums);  // while the parts are in the memory-side cache
+        parts.clear();
+        sums.clear();
+      }
     }
     if (front) {
       const int64_t used = 2 * Fkv + F + heads, ld = (used + 63) / 64 * 64;  // [b | c | v | a | padding]
@@ -604,14 +661,21 @@ struct LayerNode : public torch::autograd::Function<LayerNode> {
         }
       }
       if (weights) {
-        const at::Tensor dw = weight_grad(d2, x2, ctx->saved_data["slices_in"].toInt(), parts, sums);
+        at::Tensor dw;
+        if (own_weights) {
+          grads.add(d2, x2, used);
+          dw = grads.dw.back();
+        } else {
+          dw = weight_grad(d2, x2, ctx->saved_data["slices_in"].toInt(), parts, sums);
+        }
         out[3] = dw.narrow(0, 0, Fkv);
         out[5] = dw.narrow(0, Fkv, Fkv);
         out[7] = dw.narrow(0, 2 * Fkv, F);
         out[1] = dw.narrow(0, 2 * Fkv + F, heads);
       }
-      layer_sums(parts, sums);
+      if (grads.dy.empty()) layer_sums(parts, sums);
     }
+    if (!grads.dy.empty()) grads.run(parts, sums);
     if (!create_graph) return out;
     const at::AutoGradMode grad(true);
     // The mixing kernels have no second derivative: a second differentiation of what their backward has a part in says so.

@@ -18,7 +18,7 @@ from concurrent.futures import ThreadPoolExecutor
 HERE = os.path.dirname(os.path.abspath(__file__))
 PKG = os.path.dirname(HERE)
 LIB_NAME = "libspear_btp.so"
-SOURCES = ["btp_scan.hip", "btp_mfma.hip", "btp_fused.hip", "btp_jagged.hip", "layer_token.hip", "layer_linear.hip", "layer_gemm.hip", "layer_grad.hip", "btp_capi.hip", "btp_probe.hip"]
+SOURCES = ["btp_scan.hip", "btp_mfma.hip", "btp_fused.hip", "btp_jagged.hip", "layer_token.hip", "layer_linear.hip", "layer_gemm.hip", "layer_wgrad.hip", "layer_grad.hip", "btp_capi.hip", "btp_probe.hip"]
 HEADERS = ["btp_device.h", "btp_launch.h", "btp_staging.h", "layer_mfma.h", "layer_tile.h", os.path.join("..", "..", "include", "spear_btp.h"),
            os.path.join("..", "..", "include", "spear_btp_probe.h"), os.path.join("..", "..", "include", "spear_layer.h")]
 

@@ -14,6 +14,8 @@
 // reduction's columns, and the same zeros. 64 x 64 tiles through LDS, 16 bytes per access on both sides; bound by the launch at small
 // sizes (6 us for 2.6 MB at dim 512), by reading and writing each weight once else.
 //
+// The parts of layer_wgrad come as its accumulators lie and are put in order on the way out (8-byte stores, 32 bytes in a row).
+//
 // A block of layer_sums, 512 threads, takes either 2048 columns, four to a thread, and walks the rows with eight 16-byte loads in flight
 // (few rows), or 16 columns with 32 threads to a column that add up through LDS (many rows: 2048 rows by 512 columns
 // still make 32 blocks). Sums are taken in an order that depends on the shape only: the same bits in every run.
@@ -35,7 +37,11 @@ constexpr int kTallColumns = 16, kTallLanes = kThreads / kTallColumns;
 // weight gradients' arrays all have them. Narrow ones go the tall way at any number of rows.
 __host__ __device__ inline bool is_flat(const LayerSumJob& j) { return j.cols % 4 == 0 && j.rows <= 64; }
 
+// A job over the parts of layer_wgrad: four consecutive columns of one row of the result to a thread.
+constexpr int kTileQuads = kWgradSide * kWgradSide / 4;
+
 inline long job_blocks(const LayerSumJob& j) {
+  if (j.splits > 0) return (long)((j.rows + kWgradSide - 1) / kWgradSide) * ((j.cols + kWgradSide - 1) / kWgradSide) * (kTileQuads / kThreads);
   return is_flat(j) ? (j.cols + kFlatColumns - 1) / kFlatColumns : (j.cols + kTallColumns - 1) / kTallColumns;
 }
 
@@ -51,6 +57,36 @@ __global__ __launch_bounds__(kThreads) void layer_sums_kernel(const Jobs jobs, i
   while (at + 1 < n && (long)blockIdx.x >= jobs.first_block[at + 1]) ++at;
   const LayerSumJob j = jobs.job[at];
   const long block = (long)blockIdx.x - jobs.first_block[at];
+  if (j.splits > 0) {
+    constexpr int kBlocks = kTileQuads / kThreads;
+    const int tile = (int)(block / kBlocks), e = (int)(block % kBlocks) * kThreads + (int)threadIdx.x;
+    const int tiles_n = (int)((j.rows + kWgradSide - 1) / kWgradSide), tiles = tiles_n * (int)((j.cols + kWgradSide - 1) / kWgradSide);
+    const int k0 = tile / tiles_n * kWgradSide, n0 = tile % tiles_n * kWgradSide;
+    // where layer_wgrad's accumulators lie: wavefront, tile of dy's columns, tile of x's columns, lane
+    const int wave = e >> 11, i = (e >> 8) & 7, jt = (e >> 6) & 3, lane = e & 63, wn = wave & 3;
+    const bool full = j.cols - k0 > 128;
+    const int n = n0 + 128 * (wave >> 2) + 16 * i + (lane & 15), k = k0 + 16 * ((full ? 4 : 2) * wn + jt) + 4 * (lane >> 4);
+    if ((!full && jt >= 2) || n >= j.rows || k >= j.cols) return;
+    const float* p = j.in + ((long)tile * kTileQuads + e) * 4;
+    const long split = (long)tiles * kTileQuads * 4;
+    float4 sum = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    int row = 0;
+    for (; row + 8 <= j.splits; row += 8) {
+      float4 q[8];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) q[u] = *reinterpret_cast<const float4*>(p + (row + u) * split);
+#pragma unroll
+      for (int u = 0; u < 8; ++u) {
+        sum.x += q[u].x; sum.y += q[u].y; sum.z += q[u].z; sum.w += q[u].w;
+      }
+    }
+    for (; row < j.splits; ++row) {
+      const float4 q = *reinterpret_cast<const float4*>(p + row * split);
+      sum.x += q.x; sum.y += q.y; sum.z += q.z; sum.w += q.w;
+    }
+    *reinterpret_cast<uint2*>(j.out + (long)n * j.cols + k) = make_uint2(E::pack2(sum.x, sum.y), E::pack2(sum.z, sum.w));
+    return;
+  }
   if (is_flat(j)) {
     const long col = block * kFlatColumns + 4 * (long)threadIdx.x;
     if (col >= j.cols) return;

@@ -109,3 +109,49 @@ def test_transposed_weights_and_padding(M, dim, heads, kv_heads):
     assert torch.equal(stacked[:, :used], torch.cat([w_b, w_c, w_v, w_a]).t()) and (stacked[:, used:] == 0).all()
     assert torch.equal(out_t, w_out.t())
     assert (packed[:, :used] == 7).all() and (packed[:, used:] == 0).all()
+
+
+# tokens, (columns of dy, its row length, columns of x) per product, splits (0: as modelled). Remainders of 32 tokens, of 256 and 128 columns;
+# one step per split and fewer steps than stages; units of both products on one workgroup; splits that differ by a step.
+WGRADS = [
+    (1, [(8, 8, 8)], [1]),
+    (33, [(40, 64, 72), (300, 304, 136)], [2, 1]),
+    (1000, [(1813, 1856, 592), (592, 592, 592)], [0, 0]),
+    (4099, [(257, 264, 264), (129, 136, 520)], [7, 128]),
+    (16384, [(1568, 1600, 512), (512, 512, 512)], [0, 0]),
+    (9000, [(3136, 3136, 1024)], [3]),
+]
+
+
+@pytest.mark.parametrize("M,products,splits", WGRADS)
+def test_weight_gradients_over_splits_against_float64(M, products, splits):
+    import ctypes
+
+    from spear_amd import _btp
+
+    lib, n = _btp.load_library(), len(products)
+    g = torch.Generator(device=DEV).manual_seed(M)
+    dys = [torch.randn(M, ld, generator=g, device=DEV).bfloat16() for _, ld, _ in products]
+    xs = [torch.randn(M, K, generator=g, device=DEV).bfloat16() for _, _, K in products]
+    splits = [s or lib.spear_layer_wgrad_splits(ctypes.c_longlong(M), N, K) for s, (N, _, K) in zip(splits, products)]
+    units = sum(-(-N // 256) * -(-K // 256) * s for (N, _, K), s in zip(products, splits))
+    parts = torch.full((units * 65536,), float("nan"), device=DEV)
+    dws = [torch.full((N + 1, K), 7.0, device=DEV).bfloat16() for N, _, K in products]
+    tall = torch.randn(70, 24, generator=g, device=DEV)
+    sums = torch.empty(24, device=DEV).bfloat16()
+    print(f"weight gradients M={M} {products} splits={splits}", flush=True)
+    ints, pointers = ctypes.c_int * n, ctypes.c_void_p * n
+    of = lambda ts: pointers(*(t.data_ptr() for t in ts))
+    lds, Ns, Ks, sp = (ints(*v) for v in ([p[1] for p in products], [p[0] for p in products], [p[2] for p in products], splits))
+    stream = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    assert lib.spear_layer_wgrad(n, of(dys), lds, lds, Ns, of(xs), Ks, sp, ctypes.c_longlong(M), ctypes.c_void_p(parts.data_ptr()), stream) == 0
+    one = lambda t: (ctypes.c_void_p * 1)(t.data_ptr())
+    assert lib.spear_layer_wgrad_sums(n, ctypes.c_void_p(parts.data_ptr()), Ns, Ks, sp, of(dws), 1, one(tall), one(sums), (ctypes.c_longlong * 1)(70),
+                                      (ctypes.c_longlong * 1)(24), _btp._BF16, stream) == 0
+    torch.cuda.synchronize()
+    for dy, x, dw, (N, _, K) in zip(dys, xs, dws, products):
+        assert_product(dw[:N], dy[:, :N].t(), x.t(), None, f"M={M} [{N}, {K}]")
+        assert (dw[N] == 7).all()
+    # 70 fp32 additions, then half a step of the result
+    want = tall.double().sum(0)
+    assert ((sums.double() - want).abs() <= want.abs() * 2.0**-8 + tall.double().abs().sum(0) * 71 * 2.0**-24).all()
