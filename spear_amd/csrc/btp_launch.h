@@ -136,7 +136,8 @@ struct LayerLinearArgs {
 hipError_t layer_linear(const LayerLinearArgs& p, hipStream_t s);
 // The same at large sizes (layer_gemm.hip), for the operands that layer_gemm_takes: K past 64, no positions.
 bool layer_gemm_takes(const LayerLinearArgs& p);
-hipError_t layer_gemm(const LayerLinearArgs& p, hipStream_t s);
+enum class LayerTiles { kMid, kLarge };  // 128 x 128, 256 x 256
+hipError_t layer_gemm(const LayerLinearArgs& p, LayerTiles size, hipStream_t s);
 
 // out[c] <- sum over the rows of in[rows, cols] (dense fp32), rounded to 16 bits (layer_grad.hip)
 struct LayerSumJob {

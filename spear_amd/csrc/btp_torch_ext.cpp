@@ -461,28 +461,19 @@ std::vector<at::Tensor> linears(const at::Tensor& x, const std::vector<at::Tenso
 bool small_product(int64_t M, int64_t columns, int64_t K) { return M > 0 && K > 0 && K % 8 == 0 && K <= 512 && M * columns * K <= 300000000; }
 
 // Whether projections of M rows are faster through spear_layer_linear than as the library's products. Measured in HIP graphs, us, dim = K,
-// spear_layer_linear / the library. The four input projections: K=128 131072 rows 52 / 67, K=512 16384 rows 32 / 54, 131072 rows 229 / 284,
-// K=768 65536 rows 230 / 239, K=1024 8192 rows 52 / 74, 131072 rows 729 / 717 (with kv heads shared by four 401 / 405), K=1536 16384 rows
+// spear_layer_linear / the library. The four input projections: K=128 131072 rows 49 / 67, K=512 1024 rows 8 / 22, 131072 rows 229 / 284,
+// K=768 65536 rows 230 / 239, K=1024 8192 rows 54 / 72, 131072 rows 729 / 717 (with kv heads shared by four 401 / 405), K=1536 16384 rows
 // 203 / 238, 65536 rows 772 / 742, K=2048 4096 rows 95 / 114, 8192 rows 193 / 174: all below K = 1024, and few tiles from there on.
-// One: K=512 65536 rows 40 / 43, 16384 rows 17.2 / 15.3, K=768 131072 rows 147 / 140.
+// One: K=512 65536 rows 40 / 43, 16384 rows 13.7 / 15.5, K=1024 1024 rows 11.2 / 8.2, 4096 rows 13.5 / 13.5, 16384 rows 34 / 30, K=2048 1024 rows
+// 20 / 16. On the GPU it is up to 4 us slower up to 9 G multiply-adds, and saves the 15 us that a library product costs the host, which is
+// what bounds calls of that size.
 bool own_products(int64_t M, const std::vector<at::Tensor>& weights, int64_t K) {
   if (M <= 0 || K <= 0 || K % 8 != 0) return false;
+  if (weights.size() == 1) return K <= 512 || M * weights[0].size(0) * K <= 9000000000;
   int64_t tiles = 0;
   for (const at::Tensor& w : weights) tiles += (w.size(0) + 255) / 256;
   tiles *= (M + 255) / 256;
-  if (weights.size() > 1) return K < 1024 || tiles <= 600;
-  return small_product(M, weights[0].size(0), K) || (K <= 512 && tiles >= 512);
-}
-
-// Whether an input gradient of M rows by K columns is faster through spear_layer_linear with the weights transposed first than as the
-// library's product with them as they lie: where its tiles fill the chip. Measured, us, spear_layer_linear / the library, K the layer's
-// width: proj_out's input gradient at K=512 131072 rows 75 / 91, 16384 rows (128 tiles) 17.2 / 16.8, K=768 16384 rows (192 tiles) 23.4 /
-// 26.5, K=1024 8192 rows (128) 26.2 / 23.8, K=2048 65536 rows 453 / 470, 8192 rows (256) 58 / 59; that of the four input projections at K=512
-// 131072 rows 198 / 208, 16384 rows (128) 37 / 30, K=768 16384 rows (192) 55 / 57, K=1024 131072 rows 663 / 697, K=2048 65536 rows 1213 /
-// 1299. A round of the chip that is three quarters full still gains; at 20000 rows of K=1024, 316 tiles, it would not be.
-bool own_input_grads(int64_t M, int64_t K) {
-  const int64_t tiles = (M + 255) / 256 * ((K + 255) / 256), rounds = (tiles + 255) / 256;
-  return K % 8 == 0 && 4 * tiles >= 3 * 256 * rounds;
+  return K < 1024 || tiles <= 600;
 }
 
 // The four input projections (a, b, c, v) of x [..., K], or one projection without bias, by either. x dense.
@@ -550,16 +541,17 @@ struct WeightGrads {
   }
 };
 
-// Whether the weight gradients of a layer's backward are faster through spear_layer_wgrad than as the library's (sliced) products: from
-// 12 G multiply-adds on. Times of single products at layer_wgrad.hip; 16384 tokens [1568, 512] (13 G) 52 / 60, 8192 tokens [1024, 1024] (8.6
-// G) 42 / 34, [1568, 512] (6.6 G) 37 / 37, 131072 tokens [392, 128] (6.6 G) 47 / 37.
-bool own_weight_grads(int64_t M, int64_t multiply_adds_per_token) { return M * multiply_adds_per_token >= 12000000000; }
+// Whether the weight gradients of a layer's backward are faster through spear_layer_wgrad than as the library's (sliced) products: up to
+// 32768 tokens, and above from 12 G multiply-adds on. Times of single products at layer_wgrad.hip. A whole step, us (and on the GPU alone),
+// with them here / the library's: 1024 tokens, width 512 124 (86) / 169 (86), 4096 tokens 257 (116) / 291 (134), 1024 tokens, width 1024 259
+// (129) / 298 (130), 131072 tokens, width 128 287 / 280.
+bool own_weight_grads(int64_t M, int64_t multiply_adds_per_token) { return M <= 32768 || M * multiply_adds_per_token >= 12000000000; }
 
 // A whole layer call on plain bf16 tensors: the four input projections, the mixing stage and the output projection, with one
 // autograd node. Backward is what spear_amd/nn/phalanx/projections.py does with _ProjectAndMix and _Linear (one product each for the
 // input and weight gradients of the four projections, against the packed gradient buffer), without Python frames and with
 // layer_stack and layer_sums around the products: 10 launches for forward and backward of a small layer where separate modules had 29.
-// The mixing kernels are the same; the weight and input gradients of few tokens are the library's products.
+// The mixing kernels are the same.
 struct LayerNode : public torch::autograd::Function<LayerNode> {
   static at::Tensor forward(torch::autograd::AutogradContext* ctx, const at::Tensor& x, const at::Tensor& w_a, const at::Tensor& b_a,
                             const at::Tensor& w_b, const at::Tensor& b_b, const at::Tensor& w_c, const at::Tensor& b_c,
@@ -624,8 +616,13 @@ struct LayerNode : public torch::autograd::Function<LayerNode> {
     }
     if (front) {
       const int64_t used = 2 * Fkv + F + heads, ld = (used + 63) / 64 * 64;  // [b | c | v | a | padding]
-      // input gradients against the stacked weights: [ld, K] as the library takes them, or transposed for the kernel here
-      const bool own = own_input_grads(M, K) && (reinterpret_cast<uintptr_t>(dy.data_ptr()) & 15u) == 0;
+      // Input gradients against the weights transposed, through spear_layer_linear; as the library's products with the weights as they lie
+      // only for a gradient off the 16-byte grid. Measured, us, spear_layer_linear / the library: proj_out's at K=512 131072 rows 75 / 91,
+      // 8192 rows 9 / 12, 1024 rows 6.1 / 7.2, K=1024 131072 rows 251 / 268, 1024 rows 11.2 / 9.7, K=2048 65536 rows 453 / 470, 2048 rows 22 /
+      // 26; that of the four input projections at K=512 131072 rows 198 / 208, 1024 rows 14 / 11, K=1024 131072 rows 663 / 697, 4096 rows 30 /
+      // 35, 1024 rows 27 / 22, K=2048 65536 rows 1213 / 1299, 1024 rows 51 / 49. The transposing launch takes 3 to 6 us, half of
+      // which layer_stack took too. Where it is the slower one on the GPU the host's 15 us per library product count for more.
+      const bool own = K % 8 == 0 && (reinterpret_cast<uintptr_t>(dy.data_ptr()) & 15u) == 0;
       const at::Tensor packed = at::empty({B, L, ld}, v.options());
       const at::Tensor stacked = own ? at::empty({K, ld}, v.options()) : at::empty({ld, K}, v.options());
       at::Tensor dmixed;
@@ -802,7 +799,7 @@ at::Tensor layer_step(const at::Tensor& x, const at::Tensor& w_a, const at::Tens
   const auto in = [&](bool advance) { return layer_token(x, w_a, b_a, w_b, b_b, w_c, b_c, w_v, h, r, c_prev, pos, block_len, heads, kv_heads, advance); };
   if (small_product(x.size(0), w_out.size(0), w_out.size(1)))
     return linears(in(false), {w_out}, {at::Tensor()}, pos.data_ptr<int>(), block_len)[0];
-  return at::linear(in(true), w_out);
+  return project(in(true), {w_out}, {at::Tensor()})[0];
 }
 
 }  // namespace

@@ -56,6 +56,43 @@ __device__ __forceinline__ Tile tile_at(const LayerLinearArgs& p, int tiles_n, i
   return t;
 }
 
+// One operand's rows of a tile, asked for 64 columns of K at a time: the lane's offsets of four requests (rows 8 apart; a row's pieces are
+// exchanged, see the top), and what is left of K.
+struct Rows {
+  i32x4_t of;             // descriptor, ends with the tile's last row
+  uint32_t at[4], piece;
+  int further, left;      // bytes of a row asked for, and left
+  uint32_t now[4];        // offsets of the step being asked for: `at`, or nowhere past the end of K
+};
+
+__device__ __forceinline__ void aim(Rows& r, const uint16_t* first, int rows, int ld, int K) {
+  r.of = words_of(first, ((rows - 1) * ld + K) * 2);
+  r.further = 0;
+  r.left = 2 * K;
+}
+
+__device__ __forceinline__ void prepare(Rows& r) {
+#pragma unroll
+  for (int i = 0; i < 4; ++i) r.now[i] = r.at[i];
+  if (r.left < 2 * kStepK) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) r.now[i] = (int)(i & 1 ? r.piece ^ 64 : r.piece) < r.left ? r.at[i] : kNowhere;
+  }
+}
+
+__device__ __forceinline__ void advance(Rows& r) {
+  r.further += 2 * kStepK;
+  r.left -= 2 * kStepK;
+}
+
+// The next 64 columns into LDS from address `to` on.
+__device__ __forceinline__ void request(Rows& r, uint32_t to) {
+  prepare(r);
+  asm volatile(SPEAR_REQUEST4("%4", "%0", "%1", "%2", "%3", "%5", "%6")
+               :: "v"(r.now[0]), "v"(r.now[1]), "v"(r.now[2]), "v"(r.now[3]), "s"(to), "s"(r.of), "s"(r.further) : "memory", "m0", "scc");
+  advance(r);
+}
+
 // The fragments of 32 columns: 8 row tiles of x, 4 column tiles of the weights, 2 KiB apart. The wait is part of the block: the
 // registers are written when it ends.
 __device__ __forceinline__ void read_fragments(uint32_t x, uint32_t w, i32x4_t (&fx)[8], i32x4_t (&fw)[4]) {
@@ -69,6 +106,25 @@ __device__ __forceinline__ void read_fragments(uint32_t x, uint32_t w, i32x4_t (
         "=&v"(fw[0]), "=&v"(fw[1]), "=&v"(fw[2]), "=&v"(fw[3])
       : "v"(x), "v"(w)
       : "memory");
+}
+
+// The same with a request between the reads and their wait: the address unit takes 16 cycles per request, 256 for a group's, and the
+// reads of all four wavefronts 192 and their latency. One after the other they take longer than the 512 cycles in which the other group
+// multiplies.
+__device__ __forceinline__ void read_fragments(uint32_t x, uint32_t w, i32x4_t (&fx)[8], i32x4_t (&fw)[4], Rows& r, uint32_t to) {
+  prepare(r);
+  asm volatile(
+      "ds_read_b128 %8, %13\n ds_read_b128 %9, %13 offset:2048\n ds_read_b128 %10, %13 offset:4096\n ds_read_b128 %11, %13 offset:6144\n"
+      "ds_read_b128 %0, %12\n ds_read_b128 %1, %12 offset:2048\n ds_read_b128 %2, %12 offset:4096\n ds_read_b128 %3, %12 offset:6144\n"
+      "ds_read_b128 %4, %12 offset:8192\n ds_read_b128 %5, %12 offset:10240\n ds_read_b128 %6, %12 offset:12288\n"
+      "ds_read_b128 %7, %12 offset:14336\n"
+      SPEAR_REQUEST4("%18", "%14", "%15", "%16", "%17", "%19", "%20")
+      "s_waitcnt lgkmcnt(0)"
+      : "=&v"(fx[0]), "=&v"(fx[1]), "=&v"(fx[2]), "=&v"(fx[3]), "=&v"(fx[4]), "=&v"(fx[5]), "=&v"(fx[6]), "=&v"(fx[7]),
+        "=&v"(fw[0]), "=&v"(fw[1]), "=&v"(fw[2]), "=&v"(fw[3])
+      : "v"(x), "v"(w), "v"(r.now[0]), "v"(r.now[1]), "v"(r.now[2]), "v"(r.now[3]), "s"(to), "s"(r.of), "s"(r.further)
+      : "memory", "m0", "scc");
+  advance(r);
 }
 
 // kStreamed: results are stored with the non-temporal hint, so that L2 writes them back at once and not when the next tile's
@@ -86,46 +142,25 @@ __global__ __launch_bounds__(512) void layer_gemm_kernel(const LayerLinearArgs p
 
   // Requests: number i (0 .. 3) of wavefront w moves rows 32 w + 8 i .. + 7 of a stage, 16 bytes per lane
   const int row = 32 * wave + (lane >> 3);
-  const uint32_t piece = ((lane & 7) ^ (lane >> 4)) * 16;  // rows 8 further have it 64 bytes across
-  const uint32_t x0 = row * ldx * 2 + piece, x1 = (row + 8) * ldx * 2 + (piece ^ 64), x16 = 32 * ldx, w16 = 32 * K;
-  uint32_t w0 = 0, w1 = 0;
-  const char *px = nullptr, *pw = nullptr;  // next step's columns of the tile, and what is left from there: bytes to the end of
-  int nx = 0, nw = 0, kx = 0, kw = 0;       // the last row, bytes of a row
+  Rows rx, rw;
+  rx.piece = rw.piece = ((lane & 7) ^ (lane >> 4)) * 16;  // rows 8 further have it 64 bytes across
+#pragma unroll
+  for (int i = 0; i < 4; ++i) rx.at[i] = (row + 8 * i) * ldx * 2 + (i & 1 ? rx.piece ^ 64 : rx.piece);
   auto aim_x = [&](const Tile& t) {
-    const int rows = min(kTileRows, p.M - t.panel * kTileRows);
-    px = reinterpret_cast<const char*>(p.x + (long)t.panel * kTileRows * ldx);
-    nx = ((rows - 1) * ldx + K) * 2;
-    kx = 2 * K;
+    aim(rx, p.x + (long)t.panel * kTileRows * ldx, min(kTileRows, p.M - t.panel * kTileRows), ldx, K);
   };
   auto aim_w = [&](const Tile& t) {
     const int cols = min(kTileCols, p.N[t.job] - t.col);
-    pw = reinterpret_cast<const char*>(p.w[t.job] + (long)t.col * K);
-    nw = cols * K * 2;
-    kw = 2 * K;
+    aim(rw, p.w[t.job] + (long)t.col * K, cols, K, K);
     // wavefront wn has the rows 64 wn .. of a stage: the tile's columns in order, or 32 wn .. + 31 and these + 128 where there are
     // no more than 128 columns
     const int col = cols > 128 ? row : (row & 31) + (row >> 6) * 32 + (row & 32) * 4;
-    w0 = col * K * 2 + piece;
-    w1 = (col + 8) * K * 2 + (piece ^ 64);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) rw.at[i] = (col + 8 * i) * K * 2 + (i & 1 ? rw.piece ^ 64 : rw.piece);
   };
-  auto request = [&](char* to, const char* from, int bytes, int left, uint32_t v0, uint32_t v1, uint32_t step) {
-    const auto desc = buffer_of(from, bytes);
-    const uint32_t u0 = (int)piece < left ? v0 : kNowhere, u1 = (int)(piece ^ 64) < left ? v1 : kNowhere;
-    load_to_lds(desc, to, u0);
-    load_to_lds(desc, to + 1024, u1);
-    load_to_lds(desc, to + 2048, u0 + step);
-    load_to_lds(desc, to + 3072, u1 + step);
-  };
-  auto request_x = [&](int stage) {
-    request(lds + stage * kStage + wave * 4096, px, nx, kx, x0, x1, x16);
-    px += 2 * kStepK; nx -= 2 * kStepK; kx -= 2 * kStepK;
-  };
-  auto request_w = [&](int stage) {
-    request(lds + (3 + stage) * kStage + wave * 4096, pw, nw, kw, w0, w1, w16);
-    pw += 2 * kStepK; nw -= 2 * kStepK; kw -= 2 * kStepK;
-  };
+  const uint32_t base = lds_address(lds), x_to = base + wave * 4096, w_to = x_to + 3 * kStage;
 
-  const uint32_t base = lds_address(lds), fragment = n * 128 + (q ^ (n >> 1)) * 16;
+  const uint32_t fragment = n * 128 + (q ^ (n >> 1)) * 16;
   const uint32_t x_at = base + wm * 128 * 128 + fragment, w_at = base + 3 * kStage + wn * 64 * 128 + fragment;
   f32x4_t acc[8][4];  // [row tile][column tile]; lane 16 q + n: columns 4 q .. 4 q + 3 of row n
   i32x4_t fx[8], fw[4];
@@ -133,7 +168,7 @@ __global__ __launch_bounds__(512) void layer_gemm_kernel(const LayerLinearArgs p
   Tile cur = tile_at(p, tiles_n, id);
   aim_x(cur);
   aim_w(cur);
-  request_x(0); request_w(0); request_x(1); request_w(1);
+  request(rx, x_to); request(rw, w_to); request(rx, x_to + kStage); request(rw, w_to + kStage);
   wait_vm<8>();
   phase_barrier();
   if (wm == 1) phase_barrier();
@@ -180,23 +215,28 @@ __global__ __launch_bounds__(512) void layer_gemm_kernel(const LayerLinearArgs p
     };
     int t = 0;
     do {
-      read_fragments(x_at + sx * kStage, w_at + sw * kStage, fx, fw);
+      // The weights of step t + 1 (the first ones of a tile have been asked for already) go where those of step t - 1 were, x of step
+      // t + 2 where that of step t - 1 was: both groups of wavefronts have read them.
+      if (t > 0) {
+        if (t == steps - 1) aim_w(next);
+        read_fragments(x_at + sx * kStage, w_at + sw * kStage, fx, fw, rw, w_to + (sw ^ 1) * kStage);
+      } else {
+        read_fragments(x_at + sx * kStage, w_at + sw * kStage, fx, fw);
+      }
       phase_barrier();
       multiply();
       if (t == steps - 2) aim_x(next);
-      request_x(sx == 0 ? 2 : sx - 1);  // step t + 2, where step t - 1 was
-      read_fragments((x_at ^ 64) + sx * kStage, (w_at ^ 64) + sw * kStage, fx, fw);
+      read_fragments((x_at ^ 64) + sx * kStage, (w_at ^ 64) + sw * kStage, fx, fw, rx, x_to + (sx == 0 ? 2 : sx - 1) * kStage);
       // step t + 1 has landed: all but the request just made, and the stores if they came after step t + 1 was asked for
       if (stored) wait_vm<20>();
       else wait_vm<4>();
       stored = false;
       phase_barrier();
       multiply();
-      if (t == steps - 2) aim_w(next);
-      request_w(sw);  // step t + 2: both groups of wavefronts have read the stage
       sx = sx == 2 ? 0 : sx + 1;
       sw ^= 1;
     } while (++t < steps);
+    request(rw, w_to + (sw ^ 1) * kStage);  // the next tile's second step, ahead of the stores
 
     if (p.bias[cur.job] != nullptr) {
 #pragma unroll
@@ -240,6 +280,120 @@ __global__ __launch_bounds__(512) void layer_gemm_kernel(const LayerLinearArgs p
   wait_vm<0>();  // the requests past the last tile write LDS
 }
 
+// ---- products that would not fill the chip with tiles of 256 x 256 --------------------------------------------------------------------
+// 128 x 128 tiles, one to a workgroup of four wavefronts (64 x 64 each). Where there are more tiles than compute units, two stages of 64
+// columns of K (64 KiB): two workgroups share a compute unit and one multiplies while the other waits. Else four stages (128 KiB), three
+// of them under way. Requests, exchange of pieces, bounds and results are those above.
+constexpr int kMidSide = 128, kMidStage = kMidSide * kStepK * 2;
+
+// The fragments of 32 columns, four tiles of either operand, with a request as above.
+__device__ __forceinline__ void read_fragments(uint32_t x, uint32_t w, i32x4_t (&fx)[4], i32x4_t (&fw)[4], Rows& r, uint32_t to) {
+  prepare(r);
+  asm volatile(
+      "ds_read_b128 %4, %9\n ds_read_b128 %5, %9 offset:2048\n ds_read_b128 %6, %9 offset:4096\n ds_read_b128 %7, %9 offset:6144\n"
+      "ds_read_b128 %0, %8\n ds_read_b128 %1, %8 offset:2048\n ds_read_b128 %2, %8 offset:4096\n ds_read_b128 %3, %8 offset:6144\n"
+      SPEAR_REQUEST4("%14", "%10", "%11", "%12", "%13", "%15", "%16")
+      "s_waitcnt lgkmcnt(0)"
+      : "=&v"(fx[0]), "=&v"(fx[1]), "=&v"(fx[2]), "=&v"(fx[3]), "=&v"(fw[0]), "=&v"(fw[1]), "=&v"(fw[2]), "=&v"(fw[3])
+      : "v"(x), "v"(w), "v"(r.now[0]), "v"(r.now[1]), "v"(r.now[2]), "v"(r.now[3]), "s"(to), "s"(r.of), "s"(r.further)
+      : "memory", "m0", "scc");
+  advance(r);
+}
+
+template <int kStages>
+__global__ __launch_bounds__(256, 2) void layer_gemm_mid_kernel(const LayerLinearArgs p, int tiles_n, int tiles) {
+  __shared__ __attribute__((aligned(1024))) char lds[2 * kStages * kMidStage];  // the stages of x, then those of the weights
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  const int n = lane & 15, q = lane >> 4, wm = wave >> 1, wn = wave & 1;
+  const int K = p.K, ldx = (int)p.ldx, steps = (K + kStepK - 1) / kStepK;
+  // an XCD takes consecutive tiles, the columns of a row panel after another
+  const int xcd = blockIdx.x & 7, first = (int)((long)tiles * xcd / 8), id = first + (int)(blockIdx.x >> 3);
+  if (id >= (int)((long)tiles * (xcd + 1) / 8)) return;
+  const int panel = id / tiles_n;
+  int job = 0, col = id - panel * tiles_n;
+  while (col >= (p.N[job] + kMidSide - 1) / kMidSide) col -= (p.N[job++] + kMidSide - 1) / kMidSide;
+  col *= kMidSide;
+  const int N = p.N[job], rows = min(kMidSide, p.M - panel * kMidSide), cols = min(kMidSide, N - col);
+
+  const int row = 32 * wave + (lane >> 3);
+  Rows rx, rw;
+  rx.piece = rw.piece = ((lane & 7) ^ (lane >> 4)) * 16;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int piece = i & 1 ? rx.piece ^ 64 : rx.piece;
+    rx.at[i] = (row + 8 * i) * ldx * 2 + piece;
+    rw.at[i] = (row + 8 * i) * K * 2 + piece;
+  }
+  aim(rx, p.x + (long)panel * kMidSide * ldx, rows, ldx, K);
+  aim(rw, p.w[job] + (long)col * K, cols, K, K);
+
+  const uint32_t fragment = lds_address(lds) + n * 128 + (q ^ (n >> 1)) * 16;
+  const uint32_t x_at = fragment + wm * 64 * 128, w_at = fragment + kStages * kMidStage + wn * 64 * 128;
+  f32x4_t acc[4][4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) acc[i][j] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+  i32x4_t fx[2][4], fw[2][4];
+  const uint32_t x_to = lds_address(lds) + wave * 4096, w_to = x_to + kStages * kMidStage;
+#pragma unroll
+  for (int t = 0; t < kStages - 1; ++t) {
+    request(rx, x_to + t * kMidStage);
+    request(rw, w_to + t * kMidStage);
+  }
+  int stage = 0;
+  for (int t = 0; t < steps; ++t) {
+    wait_vm<8 * (kStages - 2)>();  // step t has landed, the ones after it may be under way
+    phase_barrier();               // in all wavefronts, and all have read step t - 1
+    // Step t + kStages - 1 goes where step t - 1 was. Past the last step nothing is asked for (nowhere), so that the waits' counts hold.
+    const uint32_t at = stage * kMidStage, to = (stage == 0 ? kStages - 1 : stage - 1) * kMidStage;
+    read_fragments(x_at + at, w_at + at, fx[0], fw[0], rx, x_to + to);
+    read_fragments((x_at ^ 64) + at, (w_at ^ 64) + at, fx[1], fw[1], rw, w_to + to);
+#pragma unroll
+    for (int kk = 0; kk < 2; ++kk)
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) acc[i][j] = mfma(fw[kk][j], fx[kk][i], acc[i][j]);
+    stage = stage == kStages - 1 ? 0 : stage + 1;
+  }
+
+  if (const uint16_t* bias = p.bias[job]; bias != nullptr) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      f32x4_t add;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) add[e] = Bf16::lo(bias[min(col + 64 * wn + 16 * j + 4 * q + e, N - 1)]);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) acc[i][j] += add;
+    }
+  }
+  uint16_t* out = p.out[job] + (long)panel * kMidSide * N + col;
+  const bool wide = N % 8 == 0 && (reinterpret_cast<uintptr_t>(p.out[job]) & 15u) == 0;
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    const int c = 64 * wn + 32 * h + (q & 1) * 16 + (q >> 1) * 8;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const f32x4_t v0 = acc[i][2 * h], v1 = acc[i][2 * h + 1];
+      const u32x2_t lo = __builtin_amdgcn_permlane16_swap(Bf16::pack2(v0[0], v0[1]), Bf16::pack2(v1[0], v1[1]), false, false);
+      const u32x2_t hi = __builtin_amdgcn_permlane16_swap(Bf16::pack2(v0[2], v0[3]), Bf16::pack2(v1[2], v1[3]), false, false);
+      const u32x4_t d = {lo[0], hi[0], lo[1], hi[1]};
+      const int r = 64 * wm + 16 * i + n;
+      if (r >= rows || c >= cols) continue;
+      uint16_t* const to = out + (long)r * N + c;
+      if (wide) {
+        *reinterpret_cast<u32x4_t*>(to) = d;
+      } else {
+#pragma unroll
+        for (int e = 0; e < 8; ++e)
+          if (c + e < cols) to[e] = (uint16_t)(d[e >> 1] >> (16 * (e & 1)));
+      }
+    }
+  }
+  wait_vm<0>();  // the requests past the last step write LDS
+}
+
 }  // namespace
 
 bool layer_gemm_takes(const LayerLinearArgs& p) {
@@ -247,16 +401,23 @@ bool layer_gemm_takes(const LayerLinearArgs& p) {
   long tiles = 0;
   for (int j = 0; j < p.jobs; ++j) {
     if (p.N[j] >= 1 << 21) return false;
-    tiles += (p.N[j] + kTileCols - 1) / kTileCols;
+    tiles += (p.N[j] + kMidSide - 1) / kMidSide;
   }
-  return tiles * ((p.M + kTileRows - 1) / kTileRows) < 1l << 30;
+  return tiles * ((p.M + kMidSide - 1) / kMidSide) < 1l << 28;
 }
 
-hipError_t layer_gemm(const LayerLinearArgs& p, hipStream_t s) {
+hipError_t layer_gemm(const LayerLinearArgs& p, LayerTiles size, hipStream_t s) {
+  const int side = size == LayerTiles::kMid ? kMidSide : kTileRows;
   int tiles_n = 0;
-  for (int j = 0; j < p.jobs; ++j) tiles_n += (p.N[j] + kTileCols - 1) / kTileCols;
-  const int tiles = tiles_n * ((p.M + kTileRows - 1) / kTileRows);
+  for (int j = 0; j < p.jobs; ++j) tiles_n += (p.N[j] + side - 1) / side;
+  const int tiles = tiles_n * ((p.M + side - 1) / side);
   if (tiles == 0) return hipSuccess;
+  if (size == LayerTiles::kMid) {
+    const dim3 grid((unsigned)((tiles + 7) / 8 * 8)), block(256);
+    if (tiles <= 256) hipLaunchKernelGGL(layer_gemm_mid_kernel<4>, grid, block, 0, s, p, tiles_n, tiles);
+    else hipLaunchKernelGGL(layer_gemm_mid_kernel<2>, grid, block, 0, s, p, tiles_n, tiles);
+    return hipGetLastError();
+  }
   const dim3 grid(256), block(512);  // a workgroup for every compute unit
   if (p.K <= 1024) hipLaunchKernelGGL(layer_gemm_kernel<true>, grid, block, 0, s, p, tiles_n, tiles);
   else hipLaunchKernelGGL(layer_gemm_kernel<false>, grid, block, 0, s, p, tiles_n, tiles);

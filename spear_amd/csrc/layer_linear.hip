@@ -8,7 +8,7 @@
 // rows (layer_mfma.h: a quarter of K per wavefront), whatever array the columns belong to, so the narrow arrays share the chip with the
 // wide ones.
 //
-// Longer inputs are for the 256 x 256 tiles of layer_gemm.hip (takes_large_tiles). One projection (dim x dim) here / as the library's
+// Longer inputs are for the tiles of layer_gemm.hip (`fastest`). One projection (dim x dim) here / as the library's
 // product, us in a HIP graph: M=1024 dim=512 5.7 / 5.8 (0.27 G multiply-adds), M=2048 dim=512 7.6 / 6.2, M=16 dim=512 4.8 / 3.8, M=128
 // dim=768 7.2 / 4.7: alone it is the slower one on the GPU and is taken for the host time it saves (a decode step of 16 sequences 19.7 us
 // as a call at K = 512 with it, 38.5 at K = 1024 with the library's product), up to 0.3 G and K = 512. The line at K is
@@ -74,25 +74,33 @@ void launch(const LayerLinearArgs& p, int groups, hipStream_t s) {
 
 }  // namespace
 
-// Whether layer_gemm's large tiles are the faster ones. Both kernels' times in us as fitted to 70 shapes (K and dim 128 to 2048, 256 to
-// 131072 rows): here rounds of 256 workgroups, growing with K; there rounds of 256 tiles of 256 x 256, 1 us per 64 columns of K. Four
-// projections, dim = K, this kernel / the other: K=128 4096 rows 7.6 / 9.6, 16384 rows 21 / 10; K=512 1024 rows 11.9 / 16.7, 2048 rows
-// 19.8 / 16.8; K=1024 256 rows 11.8 / 24, 1024 rows 37 / 26; K=2048 256 rows 36 / 41, 1024 rows 112 / 44.
-static bool takes_large_tiles(const LayerLinearArgs& p, int groups) {
-  if (!layer_gemm_takes(p)) return false;
-  long tiles = 0;
-  for (int j = 0; j < p.jobs; ++j) tiles += (p.N[j] + 255) / 256;
-  tiles *= (p.M + 255) / 256;
+// Which kernel is the fastest, by their times in us as fitted to 56 shapes (dim 128 to 2048, 256 to 16384 rows): here rounds of 256
+// workgroups, growing with K; in layer_gemm tiles of 128 x 128, 0.47 us per 64 columns of K while each compute unit has one, twice that for
+// two; tiles of 256 x 256, 1 us. Four projections, dim = K, here / 128 / 256: K=128 1024 rows 5.0 / 5.2 / 9.1, 8192 rows 12.5 / 6.1 / 9.9; K=512
+// 256 rows 6.1 / 7.9 / 16.2, 1024 rows 11.9 / 8.3 / 16.8, 8192 rows 56 / 21 / 19; K=1024 256 rows 11.3 / 11.6 / 24, 2048 rows 61 / 20 / 28, 4096
+// rows 106 / 36 / 29; K=2048 1024 rows 111 / 34 / 46.
+enum class Kernel { kHere, kMid, kLarge };
+
+static Kernel fastest(const LayerLinearArgs& p, int groups) {
+  if (!layer_gemm_takes(p)) return Kernel::kHere;
+  auto tiles = [&](long side) {
+    long n = 0;
+    for (int j = 0; j < p.jobs; ++j) n += (p.N[j] + side - 1) / side;
+    return n * ((p.M + side - 1) / side);
+  };
+  const int steps = (p.K + 63) / 64;
+  const long small_tiles = tiles(128);
   const double here = 4.0 + (0.7 + 0.0098 * p.K) * (double)groups * ((p.M + 63) / 64) / 256;
-  const double there = 8.0 + (double)((tiles + 255) / 256) * (1.0 + (p.K + 63) / 64);
-  return there < here;
+  const double mid = 4.2 + steps * (small_tiles <= 256 ? 0.47 : 1.0 * (double)((small_tiles + 511) / 512));
+  const double large = 8.0 + (double)((tiles(256) + 255) / 256) * (1.0 + steps);
+  return here <= mid && here <= large ? Kernel::kHere : mid <= large ? Kernel::kMid : Kernel::kLarge;
 }
 
 hipError_t layer_linear(const LayerLinearArgs& p, hipStream_t s) {
   int groups = 0;
   for (int j = 0; j < p.jobs; ++j) groups += (p.N[j] + 63) / 64;
   if (groups == 0 || p.M == 0) return hipSuccess;
-  if (takes_large_tiles(p, groups)) return layer_gemm(p, s);
+  if (const Kernel k = fastest(p, groups); k != Kernel::kHere) return layer_gemm(p, k == Kernel::kMid ? LayerTiles::kMid : LayerTiles::kLarge, s);
   // as layer_token chooses: as many workgroups as there are while they are few
   const long pairs = (long)groups * ((p.M + 15) / 16);
   if (pairs <= 256) launch<1, 4>(p, groups, s);

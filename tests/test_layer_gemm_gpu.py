@@ -21,7 +21,7 @@ def assert_product(got, x, w, bias, label):
     assert over.max().item() <= 0, f"{label}: {over.max().item():.3e} over the bound"
 
 
-# M, K, columns of the projections (bias on all but every third). The rows make the large tiles the faster choice: remainders of 256 rows and
+# M, K, columns of the projections (bias on all but every third). The rows make the tiles the faster choice, of 256 x 256 first: remainders of 256 rows and
 # columns, of 64 columns of K, widths of 128 and less (half tiles), not a multiple of 8 (element stores), several tiles per workgroup and
 # more than one group of row panels, two steps of K.
 SHAPES = [
@@ -31,7 +31,12 @@ SHAPES = [
     (16400, 136, (256, 272, 16, 5)),
     (20000, 72, (1024, 130)),
     (9000, 1000, (640,)),
-    (1024, 2048, (2048, 512, 512, 128)),
+    (8192, 2048, (2048, 512, 512, 128)),
+    # 128 x 128 tiles, fewer and more of them than compute units
+    (1003, 592, (592, 592, 592, 37)),
+    (129, 1000, (1040, 130, 129, 24)),
+    (2048, 72, (1024, 1024, 1024, 64)),
+    (2049, 1032, (1032, 1040, 1041, 5)),
 ]
 
 
