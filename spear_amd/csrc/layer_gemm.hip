@@ -62,7 +62,6 @@ struct Rows {
   i32x4_t of;             // descriptor, ends with the tile's last row
   uint32_t at[4], piece;
   int further, left;      // bytes of a row asked for, and left
-  uint32_t now[4];        // offsets of the step being asked for: `at`, or nowhere past the end of K
 };
 
 __device__ __forceinline__ void aim(Rows& r, const uint16_t* first, int rows, int ld, int K) {
@@ -71,12 +70,13 @@ __device__ __forceinline__ void aim(Rows& r, const uint16_t* first, int rows, in
   r.left = 2 * K;
 }
 
-__device__ __forceinline__ void prepare(Rows& r) {
-#pragma unroll
-  for (int i = 0; i < 4; ++i) r.now[i] = r.at[i];
+// Ahead of the request that meets the end of K: nowhere from there on. The empty asm keeps this, and what else is done a few times per tile,
+// out of the steps between (the compiler would work it out every time and select).
+__device__ __forceinline__ void end_rows(Rows& r) {
   if (r.left < 2 * kStepK) {
+    asm volatile("");
 #pragma unroll
-    for (int i = 0; i < 4; ++i) r.now[i] = (int)(i & 1 ? r.piece ^ 64 : r.piece) < r.left ? r.at[i] : kNowhere;
+    for (int i = 0; i < 4; ++i) r.at[i] = (int)(i & 1 ? r.piece ^ 64 : r.piece) < r.left ? r.at[i] : kNowhere;
   }
 }
 
@@ -87,9 +87,8 @@ __device__ __forceinline__ void advance(Rows& r) {
 
 // The next 64 columns into LDS from address `to` on.
 __device__ __forceinline__ void request(Rows& r, uint32_t to) {
-  prepare(r);
   asm volatile(SPEAR_REQUEST4("%4", "%0", "%1", "%2", "%3", "%5", "%6")
-               :: "v"(r.now[0]), "v"(r.now[1]), "v"(r.now[2]), "v"(r.now[3]), "s"(to), "s"(r.of), "s"(r.further) : "memory", "m0", "scc");
+               :: "v"(r.at[0]), "v"(r.at[1]), "v"(r.at[2]), "v"(r.at[3]), "s"(to), "s"(r.of), "s"(r.further) : "memory", "m0", "scc");
   advance(r);
 }
 
@@ -112,7 +111,6 @@ __device__ __forceinline__ void read_fragments(uint32_t x, uint32_t w, i32x4_t (
 // reads of all four wavefronts 192 and their latency. One after the other they take longer than the 512 cycles in which the other group
 // multiplies.
 __device__ __forceinline__ void read_fragments(uint32_t x, uint32_t w, i32x4_t (&fx)[8], i32x4_t (&fw)[4], Rows& r, uint32_t to) {
-  prepare(r);
   asm volatile(
       "ds_read_b128 %8, %13\n ds_read_b128 %9, %13 offset:2048\n ds_read_b128 %10, %13 offset:4096\n ds_read_b128 %11, %13 offset:6144\n"
       "ds_read_b128 %0, %12\n ds_read_b128 %1, %12 offset:2048\n ds_read_b128 %2, %12 offset:4096\n ds_read_b128 %3, %12 offset:6144\n"
@@ -122,7 +120,7 @@ __device__ __forceinline__ void read_fragments(uint32_t x, uint32_t w, i32x4_t (
       "s_waitcnt lgkmcnt(0)"
       : "=&v"(fx[0]), "=&v"(fx[1]), "=&v"(fx[2]), "=&v"(fx[3]), "=&v"(fx[4]), "=&v"(fx[5]), "=&v"(fx[6]), "=&v"(fx[7]),
         "=&v"(fw[0]), "=&v"(fw[1]), "=&v"(fw[2]), "=&v"(fw[3])
-      : "v"(x), "v"(w), "v"(r.now[0]), "v"(r.now[1]), "v"(r.now[2]), "v"(r.now[3]), "s"(to), "s"(r.of), "s"(r.further)
+      : "v"(x), "v"(w), "v"(r.at[0]), "v"(r.at[1]), "v"(r.at[2]), "v"(r.at[3]), "s"(to), "s"(r.of), "s"(r.further)
       : "memory", "m0", "scc");
   advance(r);
 }
@@ -144,10 +142,10 @@ __global__ __launch_bounds__(512) void layer_gemm_kernel(const LayerLinearArgs p
   const int row = 32 * wave + (lane >> 3);
   Rows rx, rw;
   rx.piece = rw.piece = ((lane & 7) ^ (lane >> 4)) * 16;  // rows 8 further have it 64 bytes across
-#pragma unroll
-  for (int i = 0; i < 4; ++i) rx.at[i] = (row + 8 * i) * ldx * 2 + (i & 1 ? rx.piece ^ 64 : rx.piece);
   auto aim_x = [&](const Tile& t) {
     aim(rx, p.x + (long)t.panel * kTileRows * ldx, min(kTileRows, p.M - t.panel * kTileRows), ldx, K);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) rx.at[i] = (row + 8 * i) * ldx * 2 + (i & 1 ? rx.piece ^ 64 : rx.piece);
   };
   auto aim_w = [&](const Tile& t) {
     const int cols = min(kTileCols, p.N[t.job] - t.col);
@@ -168,7 +166,10 @@ __global__ __launch_bounds__(512) void layer_gemm_kernel(const LayerLinearArgs p
   Tile cur = tile_at(p, tiles_n, id);
   aim_x(cur);
   aim_w(cur);
-  request(rx, x_to); request(rw, w_to); request(rx, x_to + kStage); request(rw, w_to + kStage);
+  request(rx, x_to); request(rw, w_to);
+  end_rows(rx);
+  end_rows(rw);
+  request(rx, x_to + kStage); request(rw, w_to + kStage);
   wait_vm<8>();
   phase_barrier();
   if (wm == 1) phase_barrier();
@@ -198,12 +199,22 @@ __global__ __launch_bounds__(512) void layer_gemm_kernel(const LayerLinearArgs p
     const int span = full ? 64 : 32, across = full ? 32 : 128;  // first column of column tile j: span wn + across (j / 2) + 16 (j % 2)
     const bool more = id + slots < last;
     const Tile next = more ? tile_at(p, tiles_n, id + slots) : cur;  // past the last tile its first steps are asked for again, for nothing
-    auto multiply = [&]() {
+    // The steps of an operand run on into the next tile's. That is seen to while the matrix units have work: reading is the longer part of a
+    // phase.
+    auto follow = [&](Rows& r, auto&& aim_at) {
+      if (r.left < 2 * kStepK) {
+        asm volatile("");
+        if (r.left <= 0) aim_at(next);
+        end_rows(r);
+      }
+    };
+    auto multiply = [&](auto&& meanwhile) {
       __builtin_amdgcn_s_setprio(1);
 #pragma unroll
       for (int j = 0; j < 2; ++j)
 #pragma unroll
         for (int i = 0; i < 8; ++i) acc[i][j] = mfma(fw[j], fx[i], acc[i][j]);
+      meanwhile();
       if (full) {
 #pragma unroll
         for (int j = 2; j < 4; ++j)
@@ -217,22 +228,17 @@ __global__ __launch_bounds__(512) void layer_gemm_kernel(const LayerLinearArgs p
     do {
       // The weights of step t + 1 (the first ones of a tile have been asked for already) go where those of step t - 1 were, x of step
       // t + 2 where that of step t - 1 was: both groups of wavefronts have read them.
-      if (t > 0) {
-        if (t == steps - 1) aim_w(next);
-        read_fragments(x_at + sx * kStage, w_at + sw * kStage, fx, fw, rw, w_to + (sw ^ 1) * kStage);
-      } else {
-        read_fragments(x_at + sx * kStage, w_at + sw * kStage, fx, fw);
-      }
+      if (t > 0) read_fragments(x_at + sx * kStage, w_at + sw * kStage, fx, fw, rw, w_to + (sw ^ 1) * kStage);
+      else read_fragments(x_at + sx * kStage, w_at + sw * kStage, fx, fw);
       phase_barrier();
-      multiply();
-      if (t == steps - 2) aim_x(next);
+      multiply([&]() { follow(rx, aim_x); });
       read_fragments((x_at ^ 64) + sx * kStage, (w_at ^ 64) + sw * kStage, fx, fw, rx, x_to + (sx == 0 ? 2 : sx - 1) * kStage);
       // step t + 1 has landed: all but the request just made, and the stores if they came after step t + 1 was asked for
       if (stored) wait_vm<20>();
       else wait_vm<4>();
       stored = false;
       phase_barrier();
-      multiply();
+      multiply([&]() { follow(rw, aim_w); });
       sx = sx == 2 ? 0 : sx + 1;
       sw ^= 1;
     } while (++t < steps);
@@ -288,20 +294,21 @@ constexpr int kMidSide = 128, kMidStage = kMidSide * kStepK * 2;
 
 // The fragments of 32 columns, four tiles of either operand, with a request as above.
 __device__ __forceinline__ void read_fragments(uint32_t x, uint32_t w, i32x4_t (&fx)[4], i32x4_t (&fw)[4], Rows& r, uint32_t to) {
-  prepare(r);
   asm volatile(
       "ds_read_b128 %4, %9\n ds_read_b128 %5, %9 offset:2048\n ds_read_b128 %6, %9 offset:4096\n ds_read_b128 %7, %9 offset:6144\n"
       "ds_read_b128 %0, %8\n ds_read_b128 %1, %8 offset:2048\n ds_read_b128 %2, %8 offset:4096\n ds_read_b128 %3, %8 offset:6144\n"
       SPEAR_REQUEST4("%14", "%10", "%11", "%12", "%13", "%15", "%16")
       "s_waitcnt lgkmcnt(0)"
       : "=&v"(fx[0]), "=&v"(fx[1]), "=&v"(fx[2]), "=&v"(fx[3]), "=&v"(fw[0]), "=&v"(fw[1]), "=&v"(fw[2]), "=&v"(fw[3])
-      : "v"(x), "v"(w), "v"(r.now[0]), "v"(r.now[1]), "v"(r.now[2]), "v"(r.now[3]), "s"(to), "s"(r.of), "s"(r.further)
+      : "v"(x), "v"(w), "v"(r.at[0]), "v"(r.at[1]), "v"(r.at[2]), "v"(r.at[3]), "s"(to), "s"(r.of), "s"(r.further)
       : "memory", "m0", "scc");
   advance(r);
 }
 
+// Launched with 256 threads. The bound of 512 leaves a wavefront 256 registers: given 512, the compiler keeps the sums in accumulation
+// registers and copies them to and fro between matrix instructions (0.7 us per step instead of 0.45).
 template <int kStages>
-__global__ __launch_bounds__(256, 2) void layer_gemm_mid_kernel(const LayerLinearArgs p, int tiles_n, int tiles) {
+__global__ __launch_bounds__(512) void layer_gemm_mid_kernel(const LayerLinearArgs p, int tiles_n, int tiles) {
   __shared__ __attribute__((aligned(1024))) char lds[2 * kStages * kMidStage];  // the stages of x, then those of the weights
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
   const int n = lane & 15, q = lane >> 4, wm = wave >> 1, wn = wave & 1;
@@ -338,9 +345,13 @@ __global__ __launch_bounds__(256, 2) void layer_gemm_mid_kernel(const LayerLinea
   const uint32_t x_to = lds_address(lds) + wave * 4096, w_to = x_to + kStages * kMidStage;
 #pragma unroll
   for (int t = 0; t < kStages - 1; ++t) {
+    end_rows(rx);
+    end_rows(rw);
     request(rx, x_to + t * kMidStage);
     request(rw, w_to + t * kMidStage);
   }
+  end_rows(rx);
+  end_rows(rw);
   int stage = 0;
   for (int t = 0; t < steps; ++t) {
     wait_vm<8 * (kStages - 2)>();  // step t has landed, the ones after it may be under way
@@ -355,6 +366,8 @@ __global__ __launch_bounds__(256, 2) void layer_gemm_mid_kernel(const LayerLinea
       for (int j = 0; j < 4; ++j)
 #pragma unroll
         for (int i = 0; i < 4; ++i) acc[i][j] = mfma(fw[kk][j], fx[kk][i], acc[i][j]);
+    end_rows(rx);
+    end_rows(rw);
     stage = stage == kStages - 1 ? 0 : stage + 1;
   }
 

@@ -5,6 +5,9 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+// The asm blocks below write m0, which the compiler keeps for itself and sets anew before each of its own uses.
+#pragma clang diagnostic ignored "-Winline-asm"
+
 namespace spear_btp {
 
 namespace {
@@ -47,6 +50,10 @@ __device__ __forceinline__ i32x4_t words_of(const void* p, int bytes) {
   "s_add_u32 m0, " lds ", 0x400\n s_nop 0\n buffer_load_dwordx4 " o1 ", " desc ", " further " offen lds\n" \
   "s_add_u32 m0, " lds ", 0x800\n s_nop 0\n buffer_load_dwordx4 " o2 ", " desc ", " further " offen lds\n" \
   "s_add_u32 m0, " lds ", 0xc00\n s_nop 0\n buffer_load_dwordx4 " o3 ", " desc ", " further " offen lds\n"
+
+#define SPEAR_REQUEST2(lds, o0, o1, desc)                                                \
+  "s_mov_b32 m0, " lds "\n s_nop 0\n buffer_load_dwordx4 " o0 ", " desc ", 0 offen lds\n" \
+  "s_add_u32 m0, " lds ", 0x400\n s_nop 0\n buffer_load_dwordx4 " o1 ", " desc ", 0 offen lds\n"
 
 __device__ __forceinline__ uint32_t lds_address(char* p) { return (uint32_t)(uintptr_t)(lds_void_t*)p; }
 

@@ -60,34 +60,35 @@ __device__ __forceinline__ Unit unit_at(const LayerWgradArgs& p, const Share& sh
 
 // Fragments of 32 tokens: `a` .. `d` are the lane's addresses of four column tiles, 4 tokens further 2 KiB on. The waits are part of the
 // blocks: the registers are written when they end.
-__device__ __forceinline__ void read_tiles(uint32_t a, uint32_t b, uint32_t c, uint32_t d, u32x2_t (&f)[4][2]) {
+// Between the reads and their wait two requests (load_to_lds): `at` are the lane's offsets, `of` the descriptor, `to` the LDS address.
+__device__ __forceinline__ void read_tiles(uint32_t a, uint32_t b, uint32_t c, uint32_t d, u32x2_t (&f)[4][2], const uint32_t (&at)[2], i32x4_t of,
+                                           uint32_t to) {
   asm volatile(
-      "ds_read_b64_tr_b16 %0, %8\n ds_read_b64_tr_b16 %1, %8 offset:2048\n"
-      "ds_read_b64_tr_b16 %2, %9\n ds_read_b64_tr_b16 %3, %9 offset:2048\n"
-      "ds_read_b64_tr_b16 %4, %10\n ds_read_b64_tr_b16 %5, %10 offset:2048\n"
-      "ds_read_b64_tr_b16 %6, %11\n ds_read_b64_tr_b16 %7, %11 offset:2048\n"
+      "ds_read_b64_tr_b16 %0, %8\n ds_read_b64_tr_b16 %1, %8 offset:2048\n ds_read_b64_tr_b16 %2, %9\n ds_read_b64_tr_b16 %3, %9 offset:2048\n"
+      "ds_read_b64_tr_b16 %4, %10\n ds_read_b64_tr_b16 %5, %10 offset:2048\n ds_read_b64_tr_b16 %6, %11\n"
+      "ds_read_b64_tr_b16 %7, %11 offset:2048\n"
+      SPEAR_REQUEST2("%14", "%12", "%13", "%15")
       "s_waitcnt lgkmcnt(0)"
       : "=&v"(f[0][0]), "=&v"(f[0][1]), "=&v"(f[1][0]), "=&v"(f[1][1]), "=&v"(f[2][0]), "=&v"(f[2][1]), "=&v"(f[3][0]), "=&v"(f[3][1])
-      : "v"(a), "v"(b), "v"(c), "v"(d)
-      : "memory");
+      : "v"(a), "v"(b), "v"(c), "v"(d), "v"(at[0]), "v"(at[1]), "s"(to), "s"(of)
+      : "memory", "m0", "scc");
 }
 
 __device__ __forceinline__ void read_tiles(uint32_t a, uint32_t b, uint32_t c, uint32_t d, uint32_t a2, uint32_t b2, uint32_t c2, uint32_t d2,
-                                           u32x2_t (&f)[4][2], u32x2_t (&g)[4][2]) {
+                                           u32x2_t (&f)[4][2], u32x2_t (&g)[4][2], const uint32_t (&at)[2], i32x4_t of, uint32_t to) {
   asm volatile(
-      "ds_read_b64_tr_b16 %0, %16\n ds_read_b64_tr_b16 %1, %16 offset:2048\n"
-      "ds_read_b64_tr_b16 %2, %17\n ds_read_b64_tr_b16 %3, %17 offset:2048\n"
-      "ds_read_b64_tr_b16 %4, %18\n ds_read_b64_tr_b16 %5, %18 offset:2048\n"
-      "ds_read_b64_tr_b16 %6, %19\n ds_read_b64_tr_b16 %7, %19 offset:2048\n"
-      "ds_read_b64_tr_b16 %8, %20\n ds_read_b64_tr_b16 %9, %20 offset:2048\n"
-      "ds_read_b64_tr_b16 %10, %21\n ds_read_b64_tr_b16 %11, %21 offset:2048\n"
-      "ds_read_b64_tr_b16 %12, %22\n ds_read_b64_tr_b16 %13, %22 offset:2048\n"
-      "ds_read_b64_tr_b16 %14, %23\n ds_read_b64_tr_b16 %15, %23 offset:2048\n"
+      "ds_read_b64_tr_b16 %0, %16\n ds_read_b64_tr_b16 %1, %16 offset:2048\n ds_read_b64_tr_b16 %2, %17\n"
+      "ds_read_b64_tr_b16 %3, %17 offset:2048\n ds_read_b64_tr_b16 %4, %18\n ds_read_b64_tr_b16 %5, %18 offset:2048\n"
+      "ds_read_b64_tr_b16 %6, %19\n ds_read_b64_tr_b16 %7, %19 offset:2048\n ds_read_b64_tr_b16 %8, %20\n"
+      "ds_read_b64_tr_b16 %9, %20 offset:2048\n ds_read_b64_tr_b16 %10, %21\n ds_read_b64_tr_b16 %11, %21 offset:2048\n"
+      "ds_read_b64_tr_b16 %12, %22\n ds_read_b64_tr_b16 %13, %22 offset:2048\n ds_read_b64_tr_b16 %14, %23\n"
+      "ds_read_b64_tr_b16 %15, %23 offset:2048\n"
+      SPEAR_REQUEST2("%26", "%24", "%25", "%27")
       "s_waitcnt lgkmcnt(0)"
       : "=&v"(f[0][0]), "=&v"(f[0][1]), "=&v"(f[1][0]), "=&v"(f[1][1]), "=&v"(f[2][0]), "=&v"(f[2][1]), "=&v"(f[3][0]), "=&v"(f[3][1]),
         "=&v"(g[0][0]), "=&v"(g[0][1]), "=&v"(g[1][0]), "=&v"(g[1][1]), "=&v"(g[2][0]), "=&v"(g[2][1]), "=&v"(g[3][0]), "=&v"(g[3][1])
-      : "v"(a), "v"(b), "v"(c), "v"(d), "v"(a2), "v"(b2), "v"(c2), "v"(d2)
-      : "memory");
+      : "v"(a), "v"(b), "v"(c), "v"(d), "v"(a2), "v"(b2), "v"(c2), "v"(d2), "v"(at[0]), "v"(at[1]), "s"(to), "s"(of)
+      : "memory", "m0", "scc");
 }
 
 __device__ __forceinline__ i32x4_t whole(const u32x2_t (&f)[2]) { return i32x4_t{(int)f[0][0], (int)f[0][1], (int)f[1][0], (int)f[1][1]}; }
@@ -114,48 +115,59 @@ __global__ __launch_bounds__(512) void layer_wgrad_kernel(const LayerWgradArgs p
     const int t = token + 2 * i, value = (t & 3) | ((((t >> 3) ^ (t >> 4)) & 1) << 2);
     return ((lane & 31) ^ (value << 1)) * 16;
   };
-  // One operand of the unit whose steps are asked for: where its next step's first token lies, tokens from there to the last one, the
-  // lane's offsets (nowhere past the operand's columns), bytes of a row and of the tile's columns.
+  // One operand of the unit whose steps are asked for: the descriptor of its next step's rows, the lane's offsets (nowhere past the
+  // operand's columns), bytes of a step, and the bytes that the operand's last step has.
   struct Side {
-    const char* from;
-    int rows, ld, columns;
+    i32x4_t of;
     uint32_t at[2];
+    int stride, last_bytes;
   } dy, x;
   auto aim = [&](Side& s, const uint16_t* p0, int ld, int columns, int c0, int step) {
-    const long first = (long)step * kTokens;
-    s.from = reinterpret_cast<const char*>(p0 + first * ld + c0);
-    s.rows = (int)min(p.M - first, 1l << 30);  // only the operand's last step looks at it
-    s.ld = 2 * ld;
-    s.columns = 2 * min(kSide, columns - c0);
+    const int width = 2 * min(kSide, columns - c0), rows = (int)((p.M - 1) % kTokens) + 1;
+    s.of = words_of(p0 + (long)step * kTokens * ld + c0, (kTokens - 1) * 2 * ld + width);
+    s.stride = kTokens * 2 * ld;
+    s.last_bytes = (rows - 1) * 2 * ld + width;
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
       const int piece = piece_of(i);
-      s.at[i] = piece < s.columns ? (uint32_t)((token + 2 * i) * s.ld + piece) : kNowhere;
+      s.at[i] = piece < width ? (uint32_t)((token + 2 * i) * 2 * ld + piece) : kNowhere;
     }
   };
-  auto request = [&](char* to, Side& s) {
-    const auto desc = buffer_of(s.from, (min(s.rows, kTokens) - 1) * s.ld + s.columns);
-#pragma unroll
-    for (int i = 0; i < 2; ++i) load_to_lds(desc, to + wave * 2048 + i * 1024, s.at[i]);
-    s.from += kTokens * s.ld;
-    s.rows -= kTokens;
+  auto advance = [&](Side& s) {
+    const uint32_t low = (uint32_t)s.of[0] + (uint32_t)s.stride;
+    s.of[1] += low < (uint32_t)s.stride ? 1 : 0;
+    s.of[0] = (int)low;
   };
   // The next step to ask for: unit and step in it; past the last unit its steps again (for nothing, so that the counts of the waits hold).
   Unit cur = unit_at(p, share, id);
-  int feed_id = id, feed_left = cur.steps;
+  int feed_id = id, feed_left = 0;
+  bool feed_ends = false;  // the unit's last step is the operands'
+  auto last_step = [&]() {
+    if (feed_ends) {
+      dy.of[2] = dy.last_bytes;
+      x.of[2] = x.last_bytes;
+    }
+  };
   auto aim_at = [&](const Unit& u) {
     const LayerWgradJob& j = p.job[u.job];
     aim(dy, j.dy, j.ld_dy, j.cols_dy, u.n0, u.step);
     aim(x, j.x, j.K, j.K, u.k0, u.step);
     feed_left = u.steps;
+    feed_ends = (long)(u.step + u.steps) * kTokens >= p.M;
+    if (feed_left == 1) last_step();
   };
   aim_at(cur);
-  auto request_step = [&](int stage) {
-    request(lds + stage * kStage, dy);
-    request(lds + (kStages + stage) * kStage, x);
-    if (--feed_left == 0) {
-      if (feed_id + slots < last) feed_id += slots;
-      aim_at(unit_at(p, share, feed_id));
+  const uint32_t to = lds_address(lds) + wave * 2048;
+  auto next_step = [&]() {
+    advance(dy);
+    advance(x);
+    if (--feed_left <= 1) {
+      if (feed_left == 1) {
+        last_step();
+      } else {
+        if (feed_id + slots < last) feed_id += slots;
+        aim_at(unit_at(p, share, feed_id));
+      }
     }
   };
 
@@ -165,7 +177,12 @@ __global__ __launch_bounds__(512) void layer_wgrad_kernel(const LayerWgradArgs p
   f32x4_t acc[8][4];  // [tile of dy's columns][tile of x's columns]; lane 16 q + n: x columns 4 q .. 4 q + 3 of dy column n
   u32x2_t fa[4][2], fb[4][2], fc[4][2];
 
-  for (int i = 0; i < kStages - 1; ++i) request_step(i);
+  for (int i = 0; i < kStages - 1; ++i) {
+    asm volatile(SPEAR_REQUEST2("%2", "%0", "%1", "%3") ::"v"(dy.at[0]), "v"(dy.at[1]), "s"(to + i * kStage), "s"(dy.of) : "memory", "m0", "scc");
+    asm volatile(SPEAR_REQUEST2("%2", "%0", "%1", "%3")
+                 ::"v"(x.at[0]), "v"(x.at[1]), "s"(to + (kStages + i) * kStage), "s"(x.of) : "memory", "m0", "scc");
+    next_step();
+  }
   wait_vm<12>();
   phase_barrier();
   if (wm == 1) phase_barrier();
@@ -183,11 +200,11 @@ __global__ __launch_bounds__(512) void layer_wgrad_kernel(const LayerWgradArgs p
     const int x_tile = full ? 4 * wn : 2 * wn;
     int t = 0;
     do {
-      request_step(stage == 0 ? kStages - 1 : stage - 1);  // four steps ahead, where the step before this one was
       const uint32_t a = y_at + stage * kStage, c = base + (kStages + stage) * kStage;
+      const uint32_t into = to + (stage == 0 ? kStages - 1 : stage - 1) * kStage;  // four steps ahead, where the step before this one was
       auto xa = [&](int j) { return c + (uint32_t)(((x_tile + j) ^ value) * 32); };
-      read_tiles(xa(0), xa(1), xa(2), xa(3), a, a ^ 32, a ^ 64, a ^ 96, fc, fa);
-      read_tiles(a ^ 128, a ^ 160, a ^ 192, a ^ 224, fb);
+      read_tiles(xa(0), xa(1), xa(2), xa(3), a, a ^ 32, a ^ 64, a ^ 96, fc, fa, dy.at, dy.of, into);
+      read_tiles(a ^ 128, a ^ 160, a ^ 192, a ^ 224, fb, x.at, x.of, into + kStages * kStage);
       // the next step has landed: all but the three after it, and the stores if those came after the next step was asked for
       if (stored > 0) wait_vm<44>();
       else wait_vm<12>();
@@ -195,17 +212,18 @@ __global__ __launch_bounds__(512) void layer_wgrad_kernel(const LayerWgradArgs p
       stage = stage == kStages - 1 ? 0 : stage + 1;
       phase_barrier();
       __builtin_amdgcn_s_setprio(1);
+      auto multiply = [&](int j) {
+#pragma unroll
+        for (int i = 0; i < 8; ++i) acc[i][j] = mfma(whole(fc[j]), whole(i < 4 ? fa[i] : fb[i - 4]), acc[i][j]);
+      };
       if (some) {
-#pragma unroll
-        for (int j = 0; j < 2; ++j)
-#pragma unroll
-          for (int i = 0; i < 8; ++i) acc[i][j] = mfma(whole(fc[j]), whole(i < 4 ? fa[i] : fb[i - 4]), acc[i][j]);
-        if (full) {
-#pragma unroll
-          for (int j = 2; j < 4; ++j)
-#pragma unroll
-            for (int i = 0; i < 8; ++i) acc[i][j] = mfma(whole(fc[j]), whole(i < 4 ? fa[i] : fb[i - 4]), acc[i][j]);
-        }
+        multiply(0);
+        multiply(1);
+      }
+      next_step();  // here, where the matrix units have work: reading is the longer part of a phase
+      if (some && full) {
+        multiply(2);
+        multiply(3);
       }
       __builtin_amdgcn_s_setprio(0);
       phase_barrier();
