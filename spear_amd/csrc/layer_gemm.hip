@@ -56,42 +56,6 @@ __device__ __forceinline__ Tile tile_at(const LayerLinearArgs& p, int tiles_n, i
   return t;
 }
 
-// One operand's rows of a tile, asked for 64 columns of K at a time: the lane's offsets of four requests (rows 8 apart; a row's pieces are
-// exchanged, see the top), and what is left of K.
-struct Rows {
-  i32x4_t of;             // descriptor, ends with the tile's last row
-  uint32_t at[4], piece;
-  int further, left;      // bytes of a row asked for, and left
-};
-
-__device__ __forceinline__ void aim(Rows& r, const uint16_t* first, int rows, int ld, int K) {
-  r.of = words_of(first, ((rows - 1) * ld + K) * 2);
-  r.further = 0;
-  r.left = 2 * K;
-}
-
-// Ahead of the request that meets the end of K: nowhere from there on. The empty asm keeps this, and what else is done a few times per tile,
-// out of the steps between (the compiler would work it out every time and select).
-__device__ __forceinline__ void end_rows(Rows& r) {
-  if (r.left < 2 * kStepK) {
-    asm volatile("");
-#pragma unroll
-    for (int i = 0; i < 4; ++i) r.at[i] = (int)(i & 1 ? r.piece ^ 64 : r.piece) < r.left ? r.at[i] : kNowhere;
-  }
-}
-
-__device__ __forceinline__ void advance(Rows& r) {
-  r.further += 2 * kStepK;
-  r.left -= 2 * kStepK;
-}
-
-// The next 64 columns into LDS from address `to` on.
-__device__ __forceinline__ void request(Rows& r, uint32_t to) {
-  asm volatile(SPEAR_REQUEST4("%4", "%0", "%1", "%2", "%3", "%5", "%6")
-               :: "v"(r.at[0]), "v"(r.at[1]), "v"(r.at[2]), "v"(r.at[3]), "s"(to), "s"(r.of), "s"(r.further) : "memory", "m0", "scc");
-  advance(r);
-}
-
 // The fragments of 32 columns: 8 row tiles of x, 4 column tiles of the weights, 2 KiB apart. The wait is part of the block: the
 // registers are written when it ends.
 __device__ __forceinline__ void read_fragments(uint32_t x, uint32_t w, i32x4_t (&fx)[8], i32x4_t (&fw)[4]) {

@@ -51,9 +51,9 @@ __device__ __forceinline__ i32x4_t words_of(const void* p, int bytes) {
   "s_add_u32 m0, " lds ", 0x800\n s_nop 0\n buffer_load_dwordx4 " o2 ", " desc ", " further " offen lds\n" \
   "s_add_u32 m0, " lds ", 0xc00\n s_nop 0\n buffer_load_dwordx4 " o3 ", " desc ", " further " offen lds\n"
 
-#define SPEAR_REQUEST2(lds, o0, o1, desc)                                                \
-  "s_mov_b32 m0, " lds "\n s_nop 0\n buffer_load_dwordx4 " o0 ", " desc ", 0 offen lds\n" \
-  "s_add_u32 m0, " lds ", 0x400\n s_nop 0\n buffer_load_dwordx4 " o1 ", " desc ", 0 offen lds\n"
+#define SPEAR_REQUEST2(lds, o0, o1, desc, further)                                                   \
+  "s_mov_b32 m0, " lds "\n s_nop 0\n buffer_load_dwordx4 " o0 ", " desc ", " further " offen lds\n"     \
+  "s_add_u32 m0, " lds ", 0x400\n s_nop 0\n buffer_load_dwordx4 " o1 ", " desc ", " further " offen lds\n"
 
 __device__ __forceinline__ uint32_t lds_address(char* p) { return (uint32_t)(uintptr_t)(lds_void_t*)p; }
 
@@ -69,6 +69,44 @@ __device__ __forceinline__ void phase_barrier() {
   __builtin_amdgcn_sched_barrier(0);
   __builtin_amdgcn_s_barrier();
   __builtin_amdgcn_sched_barrier(0);
+}
+
+constexpr int kRowsStep = 64;  // columns of K asked for at a time
+
+// One operand's rows of a tile, asked for 64 columns of K at a time: the lane's offsets of four requests (rows 8 apart; a row's pieces are
+// exchanged by ((row >> 1) & 7), so that the reads of a fragment touch every bank once), and what is left of K.
+struct Rows {
+  i32x4_t of;             // descriptor, ends with the tile's last row
+  uint32_t at[4], piece;
+  int further, left;      // bytes of a row asked for, and left
+};
+
+__device__ __forceinline__ void aim(Rows& r, const uint16_t* first, int rows, int ld, int K) {
+  r.of = words_of(first, ((rows - 1) * ld + K) * 2);
+  r.further = 0;
+  r.left = 2 * K;
+}
+
+// Ahead of the request that meets the end of K: nowhere from there on. The empty asm keeps this, and what else is done a few times per tile,
+// out of the steps between (the compiler would work it out every time and select).
+__device__ __forceinline__ void end_rows(Rows& r) {
+  if (r.left < 2 * kRowsStep) {
+    asm volatile("");
+#pragma unroll
+    for (int i = 0; i < 4; ++i) r.at[i] = (int)(i & 1 ? r.piece ^ 64 : r.piece) < r.left ? r.at[i] : kNowhere;
+  }
+}
+
+__device__ __forceinline__ void advance(Rows& r) {
+  r.further += 2 * kRowsStep;
+  r.left -= 2 * kRowsStep;
+}
+
+// The next 64 columns into LDS from address `to` on.
+__device__ __forceinline__ void request(Rows& r, uint32_t to) {
+  asm volatile(SPEAR_REQUEST4("%4", "%0", "%1", "%2", "%3", "%5", "%6")
+               :: "v"(r.at[0]), "v"(r.at[1]), "v"(r.at[2]), "v"(r.at[3]), "s"(to), "s"(r.of), "s"(r.further) : "memory", "m0", "scc");
+  advance(r);
 }
 
 }  // namespace

@@ -18,23 +18,64 @@
 // `kChunk` steps of 32 columns are in flight while the chunk before is multiplied. Neighbouring workgroups take other heads, so an
 // XCD's L2 sees an eighth of the weights where 8 divides the heads.
 //
-// Measured in a HIP graph, us, this kernel / four library products and the step kernel: B=1 8 heads 5.5 / 23.8, B=1 128 heads
-// 10.8 / 30.1, B=256 32 heads 7.7 / 25.7, B=1024 32 heads 14.0 / 25.8 (1.7 GFLOP), B=1024 64 heads 33.7 / 43.0, 128 heads 111 / 64:
-// every workgroup reads its weights and tokens through L2 once, which the library's larger tiles do less often, so the caller
-// takes the library from B H K > 2^26 on. The whole step as a call at B=1024, 32 heads: 122 -> 23 us, with
-// the output projection in layer_linear.
+// Many tokens go through tiles in LDS (below): there the chain of loads from L2 and their number bound the kernel above.
+//
+// Measured in a HIP graph, us, here / four library products and the step kernel: B=1 8 heads 4.4 / 23.8, B=1 128 heads 9.5 / 30.1, B=256
+// 32 heads 6.3 / 25.7, B=1024 32 heads 8.6 / 25.8 (1.7 GFLOP; 12.9 without the tiles), B=1024 64 heads 21 / 43, 128 heads 60 / 64. The
+// caller takes the library from B H K > 2^26 on. The whole step as a call at B=1024, 32 heads: 122 us as products and a step.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
 #include "btp_device.h"
 #include "btp_launch.h"
 #include "layer_mfma.h"
+#include "layer_tile.h"
 
 namespace spear_btp {
 
 namespace {
 
 __device__ __forceinline__ float sigmoid(float z) { return __builtin_amdgcn_rcpf(1.0f + __expf(-z)); }
+
+// The mixing stage's step for features 4 q .. 4 q + 3 of `head` of a token, with `sum` the products of v, b, c and a, on state and biases
+// that the lane has loaded.
+struct TokenState {
+  float4 h, c_prev;
+  float r, ba;
+  int at;
+  uint2 bb, bc;
+};
+
+__device__ __forceinline__ TokenState load_token(const LayerTokenArgs& p, int token, int head, int kv, int q) {
+  const long unit = (long)token * p.H + head;
+  return {*reinterpret_cast<const float4*>(p.h + unit * 16 + 4 * q), *reinterpret_cast<const float4*>(p.c_prev + unit * 16 + 4 * q),
+          p.r[unit], Bf16::lo(p.b_a[head]), p.pos[token], *reinterpret_cast<const uint2*>(p.b_b + kv * 16 + 4 * q),
+          *reinterpret_cast<const uint2*>(p.b_c + kv * 16 + 4 * q)};
+}
+
+__device__ __forceinline__ void step_token(const LayerTokenArgs& p, int token, int head, int q, const f32x4_t (&sum)[4], const TokenState& s) {
+  const long unit = (long)token * p.H + head;
+  const float bias_b[4] = {Bf16::lo(s.bb.x), Bf16::hi(s.bb.x), Bf16::lo(s.bb.y), Bf16::hi(s.bb.y)};
+  const float bias_c[4] = {Bf16::lo(s.bc.x), Bf16::hi(s.bc.x), Bf16::lo(s.bc.y), Bf16::hi(s.bc.y)};
+  const bool boundary = s.at == p.block_len - 1;
+  const float gate = sigmoid(sum[3][0] + s.ba), a = gate > kCoeffFloor ? gate : 0.0f;
+  const float r_new = a * s.r;
+  float hf[4] = {s.h.x, s.h.y, s.h.z, s.h.w}, of[4];
+  const float pf[4] = {s.c_prev.x, s.c_prev.y, s.c_prev.z, s.c_prev.w};
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    hf[i] = fmaf(a, hf[i], sigmoid(sum[1][i] + bias_b[i]) * sum[0][i]);
+    of[i] = fmaf(fmaf(r_new, pf[i], hf[i]), sum[2][i] + bias_c[i], sum[0][i]);
+  }
+  *reinterpret_cast<uint2*>(p.out + unit * 16 + 4 * q) = make_uint2(Bf16::pack2(of[0], of[1]), Bf16::pack2(of[2], of[3]));
+  float4 next = make_float4(hf[0], hf[1], hf[2], hf[3]);
+  if (boundary) {
+    *reinterpret_cast<float4*>(p.c_prev + unit * 16 + 4 * q) = next;
+    next = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+  }
+  *reinterpret_cast<float4*>(p.h + unit * 16 + 4 * q) = next;
+  if (q == 0) p.r[unit] = boundary ? 1.0f : r_new;
+}
 
 template <int kNT, int kChunk>
 __global__ __launch_bounds__(256) void layer_token_kernel(const LayerTokenArgs p) {
@@ -54,46 +95,122 @@ __global__ __launch_bounds__(256) void layer_token_kernel(const LayerTokenArgs p
   // wavefront t finishes token tile t; the state travels with the first operands
   const int token = first + 16 * wave + n;
   const bool mine = wave < kNT && token < p.B;
-  const long unit = (long)token * p.H + head;
-  float4 h = make_float4(0.0f, 0.0f, 0.0f, 0.0f), c_prev = h;
-  float r = 0.0f, ba = 0.0f;
-  int at = 0;
-  uint2 bb = make_uint2(0, 0), bc = bb;
-  if (mine) {
-    h = *reinterpret_cast<const float4*>(p.h + unit * 16 + 4 * q);
-    c_prev = *reinterpret_cast<const float4*>(p.c_prev + unit * 16 + 4 * q);
-    r = p.r[unit];
-    at = p.pos[token];
-    bb = *reinterpret_cast<const uint2*>(p.b_b + kv * 16 + 4 * q);
-    bc = *reinterpret_cast<const uint2*>(p.b_c + kv * 16 + 4 * q);
-    ba = Bf16::lo(p.b_a[head]);
-  }
+  TokenState state{};
+  if (mine) state = load_token(p, token, head, kv, q);
 
   f32x4_t acc[4][kNT], sum[4];
   quarter_product<kNT, kChunk>(w, x, K, wave, q, acc);
   add_quarters<kNT>(partial, acc, wave, lane, sum);
-  if (!mine) return;
+  if (mine) step_token(p, token, head, q, sum, state);
+}
 
-  const float bias_b[4] = {Bf16::lo(bb.x), Bf16::hi(bb.x), Bf16::lo(bb.y), Bf16::hi(bb.y)};
-  const float bias_c[4] = {Bf16::lo(bc.x), Bf16::hi(bc.x), Bf16::lo(bc.y), Bf16::hi(bc.y)};
-  const bool boundary = at == p.block_len - 1;
-  const float gate = sigmoid(sum[3][0] + ba), a = gate > kCoeffFloor ? gate : 0.0f;
-  const float r_new = a * r;
-  float hf[4] = {h.x, h.y, h.z, h.w}, of[4];
-  const float pf[4] = {c_prev.x, c_prev.y, c_prev.z, c_prev.w};
+// ---- many tokens ----------------------------------------------------------------------------------------------------------------------
+// Two heads and 64 tokens to a workgroup, operands through LDS (layer_tile.h): four stages of 64 columns, the tokens' rows and of every
+// matrix the two heads' 16 rows (of W_a the head's row sixteen times). Wavefront w asks for matrix w's rows and a quarter of the tokens';
+// it multiplies head w & 1 with tokens 32 (w >> 1) .. + 31, so that v, b, c and a of a (feature, token) pair meet in one lane as above.
+// Each workgroup reads its weights once for 64 tokens and its tokens once for two heads where the kernel above reads either per 64 by
+// one, without the latency of every load in the chain.
+constexpr int kTokenStages = 4, kTokenRows = 64, kTokenX = kTokenRows * 128, kTokenW = 128 * 128;  // bytes of a stage
+
+// The fragments of 32 columns: two token tiles, one tile of each matrix; between the reads and their wait the requests of a part of a step.
+__device__ __forceinline__ void read_token_fragments(uint32_t x, uint32_t w, i32x4_t (&fx)[2], i32x4_t (&fw)[4], Rows& r, uint32_t to) {
+  asm volatile(
+      "ds_read_b128 %2, %7\n ds_read_b128 %3, %7 offset:4096\n ds_read_b128 %4, %7 offset:8192\n ds_read_b128 %5, %7 offset:12288\n"
+      "ds_read_b128 %0, %6\n ds_read_b128 %1, %6 offset:2048\n"
+      SPEAR_REQUEST4("%12", "%8", "%9", "%10", "%11", "%13", "%14")
+      "s_waitcnt lgkmcnt(0)"
+      : "=&v"(fx[0]), "=&v"(fx[1]), "=&v"(fw[0]), "=&v"(fw[1]), "=&v"(fw[2]), "=&v"(fw[3])
+      : "v"(x), "v"(w), "v"(r.at[0]), "v"(r.at[1]), "v"(r.at[2]), "v"(r.at[3]), "s"(to), "s"(r.of), "s"(r.further)
+      : "memory", "m0", "scc");
+  advance(r);
+}
+
+__device__ __forceinline__ void read_token_fragments_x(uint32_t x, uint32_t w, i32x4_t (&fx)[2], i32x4_t (&fw)[4], Rows& r, uint32_t to) {
+  asm volatile(
+      "ds_read_b128 %2, %7\n ds_read_b128 %3, %7 offset:4096\n ds_read_b128 %4, %7 offset:8192\n ds_read_b128 %5, %7 offset:12288\n"
+      "ds_read_b128 %0, %6\n ds_read_b128 %1, %6 offset:2048\n"
+      SPEAR_REQUEST2("%10", "%8", "%9", "%11", "%12")
+      "s_waitcnt lgkmcnt(0)"
+      : "=&v"(fx[0]), "=&v"(fx[1]), "=&v"(fw[0]), "=&v"(fw[1]), "=&v"(fw[2]), "=&v"(fw[3])
+      : "v"(x), "v"(w), "v"(r.at[0]), "v"(r.at[1]), "s"(to), "s"(r.of), "s"(r.further)
+      : "memory", "m0", "scc");
+  advance(r);
+}
+
+// Launched with 256 threads; the bound of 512 keeps the sums out of the accumulation registers (see layer_gemm.hip).
+__global__ __launch_bounds__(512) void layer_token_tile_kernel(const LayerTokenArgs p, int pairs) {
+  __shared__ __attribute__((aligned(1024))) char lds[kTokenStages * (kTokenX + kTokenW)];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  const int n = lane & 15, q = lane >> 4, K = p.K, ldx = (int)p.ldx, steps = (K + kRowsStep - 1) / kRowsStep;
+  const int pair = (int)blockIdx.x % pairs, first = (int)blockIdx.x / pairs * kTokenRows;
+
+  Rows rx, rw;
+  rx.piece = rw.piece = ((lane & 7) ^ (lane >> 4)) * 16;
+  aim(rx, p.x + (long)first * ldx, min(kTokenRows, p.B - first), ldx, K);
+  const uint16_t* const matrix = wave == 0 ? p.w_v : wave == 1 ? p.w_b : wave == 2 ? p.w_c : p.w_a;
+  aim(rw, matrix, wave == 0 ? p.H * 16 : wave == 3 ? p.H : p.H / p.kv_groups * 16, K, K);
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
-    hf[i] = fmaf(a, hf[i], sigmoid(sum[1][i] + bias_b[i]) * sum[0][i]);
-    of[i] = fmaf(fmaf(r_new, pf[i], hf[i]), sum[2][i] + bias_c[i], sum[0][i]);
+    const int piece = i & 1 ? rx.piece ^ 64 : rx.piece, head = min(2 * pair + (i >> 1), p.H - 1);
+    const int of_head = wave == 3 ? head : (wave == 0 ? head : head / p.kv_groups) * 16 + 8 * (i & 1) + (lane >> 3);
+    rx.at[i] = (16 * wave + 8 * (i & 1) + (lane >> 3)) * ldx * 2 + piece;  // the first two are used
+    rw.at[i] = of_head * K * 2 + piece;
   }
-  *reinterpret_cast<uint2*>(p.out + unit * 16 + 4 * q) = make_uint2(Bf16::pack2(of[0], of[1]), Bf16::pack2(of[2], of[3]));
-  float4 next = make_float4(hf[0], hf[1], hf[2], hf[3]);
-  if (boundary) {
-    *reinterpret_cast<float4*>(p.c_prev + unit * 16 + 4 * q) = next;
-    next = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+  const int mine = 2 * pair + (wave & 1), head = min(mine, p.H - 1), kv = head / p.kv_groups;
+  const uint32_t x_to = lds_address(lds) + wave * 2048, w_to = lds_address(lds) + kTokenStages * kTokenX + wave * 4096;
+  const uint32_t fragment = lds_address(lds) + n * 128 + (q ^ (n >> 1)) * 16;
+  const uint32_t x_at = fragment + (wave >> 1) * 4096, w_at = fragment + kTokenStages * kTokenX + (wave & 1) * 2048;
+  auto request_x = [&](uint32_t to) {
+    asm volatile(SPEAR_REQUEST2("%2", "%0", "%1", "%3", "%4") ::"v"(rx.at[0]), "v"(rx.at[1]), "s"(to), "s"(rx.of), "s"(rx.further)
+                 : "memory", "m0", "scc");
+    advance(rx);
+  };
+  for (int t = 0; t < kTokenStages - 1; ++t) {
+    end_rows(rx);
+    end_rows(rw);
+    request(rw, w_to + t * kTokenW);
+    request_x(x_to + t * kTokenX);
   }
-  *reinterpret_cast<float4*>(p.h + unit * 16 + 4 * q) = next;
-  if (q == 0) p.r[unit] = boundary ? 1.0f : r_new;
+  end_rows(rx);
+  end_rows(rw);
+  TokenState state[2] = {};  // travels with the first operands
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const int token = first + 32 * (wave >> 1) + 16 * i + n;
+    if (mine < p.H && token < p.B) state[i] = load_token(p, token, head, kv, q);
+  }
+  f32x4_t acc[2][4];  // [token tile][v, b, c, a]
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int m = 0; m < 4; ++m) acc[i][m] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+  i32x4_t fx[2][2], fw[2][4];
+  int stage = 0;
+  for (int t = 0; t < steps; ++t) {
+    wait_vm<6 * (kTokenStages - 2)>();  // step t has landed, the ones after it may be under way
+    phase_barrier();                    // in all wavefronts, and all have read step t - 1
+    const int into = stage == 0 ? kTokenStages - 1 : stage - 1;  // where step t - 1 was
+    const uint32_t x = x_at + stage * kTokenX, w = w_at + stage * kTokenW;
+    read_token_fragments(x, w, fx[0], fw[0], rw, w_to + into * kTokenW);
+    read_token_fragments_x(x ^ 64, w ^ 64, fx[1], fw[1], rx, x_to + into * kTokenX);
+#pragma unroll
+    for (int kk = 0; kk < 2; ++kk)
+#pragma unroll
+      for (int m = 0; m < 4; ++m)
+#pragma unroll
+        for (int i = 0; i < 2; ++i) acc[i][m] = mfma(fw[kk][m], fx[kk][i], acc[i][m]);
+    end_rows(rx);
+    end_rows(rw);
+    stage = stage == kTokenStages - 1 ? 0 : stage + 1;
+  }
+  if (mine < p.H) {
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const int token = first + 32 * (wave >> 1) + 16 * i + n;
+      if (token < p.B) step_token(p, token, head, q, acc[i], state[i]);
+    }
+  }
+  wait_vm<0>();  // the requests past the last step write LDS
 }
 
 template <int kNT, int kChunk>
@@ -105,14 +222,19 @@ void launch(const LayerTokenArgs& p, hipStream_t s) {
 }  // namespace
 
 hipError_t layer_token(const LayerTokenArgs& p, hipStream_t s) {
-  // Few workgroups: as many as there are. Else more tokens to a workgroup, which reads the weights less often. One / two / four
-  // token tiles, us: B=32 128 heads (256 pairs) 12.5 / 14.3 / 15.2; B=256 32 heads (512) 8.8 / 7.7 / 8.9; B=1024 32 heads (2048)
-  // 22.6 / 21.3 / 14.0; B=256 128 heads (2048) 65 / 48 / 32.
+  // Few workgroups: as many as there are; then two token tiles each, which read the weights less often (one / two, us: B=32 128 heads,
+  // 256 pairs, 12.5 / 14.3; B=256 32 heads, 512 pairs, 8.8 / 7.7); then the tile kernel. Two token tiles / it: B=256 37 heads (592 pairs) 7.3 /
+  // 8.5, B=200 48 heads (624) 9.8 / 9.2, B=128 64 heads (512) 9.0 / 10.5, B=200 64 heads (832) 11.5 / 10.7, B=512 32 heads (1024) 8.7 / 8.1,
+  // B=1024 32 heads 12.9 / 8.6, B=1024 128 heads 111 / 60.
   const long pairs = (long)p.H * ((p.B + 15) / 16);
-  const int nt = pairs <= 256 ? 1 : pairs <= 512 ? 2 : 4;
-  if (nt == 1) launch<1, 4>(p, s);
-  else if (nt == 2) launch<2, 4>(p, s);
-  else launch<4, 2>(p, s);
+  if (pairs <= 256) {
+    launch<1, 4>(p, s);
+  } else if (pairs <= 600) {
+    launch<2, 4>(p, s);
+  } else {
+    const int head_pairs = (p.H + 1) / 2;
+    hipLaunchKernelGGL(layer_token_tile_kernel, dim3((unsigned)(head_pairs * ((p.B + kTokenRows - 1) / kTokenRows))), dim3(256), 0, s, p, head_pairs);
+  }
   if (const hipError_t err = hipGetLastError(); err != hipSuccess) return err;
   // every wavefront of a row has to have read pos: a launch of its own (4.4 us), or with the next kernel on the stream
   return p.advance ? advance_block_positions(p.pos, p.B, p.block_len, s) : hipSuccess;

@@ -67,7 +67,7 @@ __device__ __forceinline__ void read_tiles(uint32_t a, uint32_t b, uint32_t c, u
       "ds_read_b64_tr_b16 %0, %8\n ds_read_b64_tr_b16 %1, %8 offset:2048\n ds_read_b64_tr_b16 %2, %9\n ds_read_b64_tr_b16 %3, %9 offset:2048\n"
       "ds_read_b64_tr_b16 %4, %10\n ds_read_b64_tr_b16 %5, %10 offset:2048\n ds_read_b64_tr_b16 %6, %11\n"
       "ds_read_b64_tr_b16 %7, %11 offset:2048\n"
-      SPEAR_REQUEST2("%14", "%12", "%13", "%15")
+      SPEAR_REQUEST2("%14", "%12", "%13", "%15", "0")
       "s_waitcnt lgkmcnt(0)"
       : "=&v"(f[0][0]), "=&v"(f[0][1]), "=&v"(f[1][0]), "=&v"(f[1][1]), "=&v"(f[2][0]), "=&v"(f[2][1]), "=&v"(f[3][0]), "=&v"(f[3][1])
       : "v"(a), "v"(b), "v"(c), "v"(d), "v"(at[0]), "v"(at[1]), "s"(to), "s"(of)
@@ -83,7 +83,7 @@ __device__ __forceinline__ void read_tiles(uint32_t a, uint32_t b, uint32_t c, u
       "ds_read_b64_tr_b16 %9, %20 offset:2048\n ds_read_b64_tr_b16 %10, %21\n ds_read_b64_tr_b16 %11, %21 offset:2048\n"
       "ds_read_b64_tr_b16 %12, %22\n ds_read_b64_tr_b16 %13, %22 offset:2048\n ds_read_b64_tr_b16 %14, %23\n"
       "ds_read_b64_tr_b16 %15, %23 offset:2048\n"
-      SPEAR_REQUEST2("%26", "%24", "%25", "%27")
+      SPEAR_REQUEST2("%26", "%24", "%25", "%27", "0")
       "s_waitcnt lgkmcnt(0)"
       : "=&v"(f[0][0]), "=&v"(f[0][1]), "=&v"(f[1][0]), "=&v"(f[1][1]), "=&v"(f[2][0]), "=&v"(f[2][1]), "=&v"(f[3][0]), "=&v"(f[3][1]),
         "=&v"(g[0][0]), "=&v"(g[0][1]), "=&v"(g[1][0]), "=&v"(g[1][1]), "=&v"(g[2][0]), "=&v"(g[2][1]), "=&v"(g[3][0]), "=&v"(g[3][1])
@@ -178,8 +178,8 @@ __global__ __launch_bounds__(512) void layer_wgrad_kernel(const LayerWgradArgs p
   u32x2_t fa[4][2], fb[4][2], fc[4][2];
 
   for (int i = 0; i < kStages - 1; ++i) {
-    asm volatile(SPEAR_REQUEST2("%2", "%0", "%1", "%3") ::"v"(dy.at[0]), "v"(dy.at[1]), "s"(to + i * kStage), "s"(dy.of) : "memory", "m0", "scc");
-    asm volatile(SPEAR_REQUEST2("%2", "%0", "%1", "%3")
+    asm volatile(SPEAR_REQUEST2("%2", "%0", "%1", "%3", "0") ::"v"(dy.at[0]), "v"(dy.at[1]), "s"(to + i * kStage), "s"(dy.of) : "memory", "m0", "scc");
+    asm volatile(SPEAR_REQUEST2("%2", "%0", "%1", "%3", "0")
                  ::"v"(x.at[0]), "v"(x.at[1]), "s"(to + (kStages + i) * kStage), "s"(x.of) : "memory", "m0", "scc");
     next_step();
   }

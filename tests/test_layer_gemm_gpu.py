@@ -160,3 +160,54 @@ def test_weight_gradients_over_splits_against_float64(M, products, splits):
     # 70 fp32 additions, then half a step of the result
     want = tall.double().sum(0)
     assert ((sums.double() - want).abs() <= want.abs() * 2.0**-8 + tall.double().abs().sum(0) * 71 * 2.0**-24).all()
+
+
+# Rows of tokens and pairs of heads that end inside a tile, an odd number of heads, shared kv heads, one and a half steps of 64 columns and
+# a remainder of them; all with more than 600 (head, 16 tokens) pairs, where the tiles are taken.
+@pytest.mark.parametrize("B,H,Hkv,K", [(1030, 37, 37, 592), (2049, 8, 2, 128), (333, 33, 11, 528), (200, 48, 12, 768), (5000, 2, 1, 96), (700, 32, 32, 520)])
+def test_token_tiles_against_float64(B, H, Hkv, K):
+    from spear_amd import _btp
+
+    g = torch.Generator(device=DEV).manual_seed(B + H)
+    normal = lambda *shape: torch.randn(*shape, generator=g, device=DEV)
+    x = normal(B, K).bfloat16()
+    w_a, w_b, w_c, w_v = ((normal(n, K) * K**-0.5).bfloat16() for n in (H, 16 * Hkv, 16 * Hkv, 16 * H))
+    b_a, b_b, b_c = (normal(n).bfloat16() for n in (H, 16 * Hkv, 16 * Hkv))
+    h, r, c_prev = normal(B, H, 16), torch.rand(B, H, generator=g, device=DEV), normal(B, H, 16)
+    pos = torch.randint(0, 16, (B,), generator=g, device=DEV, dtype=torch.int32)
+    state = [t.clone() for t in (h, r, c_prev, pos)]
+    print(f"token tiles B={B} H={H} Hkv={Hkv} K={K}", flush=True)
+    out = _btp.load_extension().layer_token(x, w_a, b_a, w_b, b_b, w_c, b_c, w_v, *state, 16, H, Hkv, False)
+    # products in float64, and what K + 1 fp32 additions may be off by
+    xd = x.double()
+    per_head = lambda t: t.view(B, Hkv, 1, 16).expand(B, Hkv, H // Hkv, 16).reshape(B, H, 16)
+
+    def product(w, b):
+        y, e = xd @ w.double().t(), (xd.abs() @ w.double().abs().t()) * (K + 1) * 2.0**-24
+        return (y, e) if b is None else (y + b.double(), e + (y + b.double()).abs() * 2.0**-24)
+
+    (a, ea), (b, eb), (c, ec), (v, ev) = product(w_a, b_a), product(w_b, b_b), product(w_c, b_c), product(w_v, None)
+    b, eb, c, ec = per_head(b), per_head(eb), per_head(c), per_head(ec)
+    v, ev, a, ea = v.view(B, H, 16), ev.view(B, H, 16), torch.sigmoid(a)[..., None], ea[..., None]
+    gate = torch.sigmoid(b)
+    fast = 2.0**-20  # exp and reciprocal of the hardware, relative, some roundings of the step with it
+    new = a * h.double() + gate * v
+    e_new = (ea / 4 + fast) * h.double().abs() + (eb / 4 + fast) * v.abs() + ev + new.abs() * 2.0**-22
+    r_new = a[..., 0] * r.double()
+    e_r = (ea[..., 0] / 4 + fast) * r.double()
+    sum_ = new + r_new[..., None] * c_prev.double()
+    e_sum = e_new + e_r[..., None] * c_prev.double().abs() + sum_.abs() * 2.0**-22
+    want = sum_ * c + v
+    e_out = e_sum * (c.abs() + ec) + sum_.abs() * ec + ev + (sum_ * c).abs() * 2.0**-22
+    end = (pos == 15)[:, None]
+    got_h, got_r, got_c, got_pos = (t.double() for t in state)
+    zero = torch.zeros_like(new)
+
+    def within(got, want, error, name):
+        assert ((got - want).abs() <= error).all(), f"{name}: {((got - want).abs() - error).max().item():.3e} over the bound"
+
+    within(out.double().view(B, H, 16), want, e_out + (want.abs() + e_out) * 2.0**-8, "out")
+    within(got_h, torch.where(end[..., None], zero, new), e_new, "h")
+    within(got_r, torch.where(end, torch.ones_like(r_new), r_new), e_r, "r")
+    within(got_c, torch.where(end[..., None], new, c_prev.double()), e_new, "c_prev")
+    assert torch.equal(state[3], pos)
