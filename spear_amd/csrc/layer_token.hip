@@ -227,9 +227,11 @@ hipError_t layer_token(const LayerTokenArgs& p, hipStream_t s) {
   // 8.5, B=200 48 heads (624) 9.8 / 9.2, B=128 64 heads (512) 9.0 / 10.5, B=200 64 heads (832) 11.5 / 10.7, B=512 32 heads (1024) 8.7 / 8.1,
   // B=1024 32 heads 12.9 / 8.6, B=1024 128 heads 111 / 60.
   const long pairs = (long)p.H * ((p.B + 15) / 16);
+  // the tile kernel's offsets are 32 bits: the largest matrix and 64 rows of tokens below 1 GiB
+  const bool near = 32l * p.H * p.K < 1l << 30 && 2l * kTokenRows * p.ldx < 1l << 30;
   if (pairs <= 256) {
     launch<1, 4>(p, s);
-  } else if (pairs <= 600) {
+  } else if (pairs <= 600 || !near) {
     launch<2, 4>(p, s);
   } else {
     const int head_pairs = (p.H + 1) / 2;
