@@ -466,9 +466,15 @@ bool small_product(int64_t M, int64_t columns, int64_t K) { return M > 0 && K > 
 // 203 / 238, 65536 rows 772 / 742, K=2048 4096 rows 95 / 114, 8192 rows 193 / 174: all below K = 1024, and few tiles from there on.
 // One: K=512 65536 rows 40 / 43, 16384 rows 13.7 / 15.5, K=1024 1024 rows 11.2 / 8.2, 4096 rows 13.5 / 13.5, 16384 rows 34 / 30, K=2048 1024 rows
 // 20 / 16. On the GPU it is up to 4 us slower up to 9 G multiply-adds, and saves the 15 us that a library product costs the host, which is
-// what bounds calls of that size.
+// what bounds calls of that size. The tiles start at K = 72; up to 64 the few-row kernel is left, which reads its operands too often for
+// many rows (a layer's forward at 1048576 rows, it / the library: K=32 541 / 384, K=64 838 / 470; 8192 rows within 5 %).
 bool own_products(int64_t M, const std::vector<at::Tensor>& weights, int64_t K) {
   if (M <= 0 || K <= 0 || K % 8 != 0) return false;
+  if (K <= 64) {
+    int64_t columns = 0;
+    for (const at::Tensor& w : weights) columns += w.size(0);
+    return M * columns * K <= (weights.size() > 1 ? 1600000000 : 300000000);
+  }
   if (weights.size() == 1) return K <= 512 || M * weights[0].size(0) * K <= 9000000000;
   int64_t tiles = 0;
   for (const at::Tensor& w : weights) tiles += (w.size(0) + 255) / 256;
@@ -617,12 +623,13 @@ struct LayerNode : public torch::autograd::Function<LayerNode> {
     if (front) {
       const int64_t used = 2 * Fkv + F + heads, ld = (used + 63) / 64 * 64;  // [b | c | v | a | padding]
       // Input gradients against the weights transposed, through spear_layer_linear; as the library's products with the weights as they lie
-      // only for a gradient off the 16-byte grid. Measured, us, spear_layer_linear / the library: proj_out's at K=512 131072 rows 75 / 91,
+      // only for a gradient off the 16-byte grid and for many tokens of a narrow layer. Measured, us, spear_layer_linear / the library: proj_out's at K=512 131072 rows 75 / 91,
       // 8192 rows 9 / 12, 1024 rows 6.1 / 7.2, K=1024 131072 rows 251 / 268, 1024 rows 11.2 / 9.7, K=2048 65536 rows 453 / 470, 2048 rows 22 /
       // 26; that of the four input projections at K=512 131072 rows 198 / 208, 1024 rows 14 / 11, K=1024 131072 rows 663 / 697, 4096 rows 30 /
       // 35, 1024 rows 27 / 22, K=2048 65536 rows 1213 / 1299, 1024 rows 51 / 49. The transposing launch takes 3 to 6 us, half of
       // which layer_stack took too. Where it is the slower one on the GPU the host's 15 us per library product count for more.
-      const bool own = K % 8 == 0 && (reinterpret_cast<uintptr_t>(dy.data_ptr()) & 15u) == 0;
+      // Up to K = 64 (see own_products) a step of 131072 tokens takes 324 / 260 us at K=32 and 335 / 285 at K=48, of 8192 tokens 220 / 253.
+      const bool own = K % 8 == 0 && (K > 64 || M <= 32768) && (reinterpret_cast<uintptr_t>(dy.data_ptr()) & 15u) == 0;
       const at::Tensor packed = at::empty({B, L, ld}, v.options());
       const at::Tensor stacked = own ? at::empty({K, ld}, v.options()) : at::empty({ld, K}, v.options());
       at::Tensor dmixed;
