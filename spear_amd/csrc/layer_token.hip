@@ -22,7 +22,7 @@
 //
 // Measured in a HIP graph, us, here / four library products and the step kernel: B=1 8 heads 4.4 / 23.8, B=1 128 heads 9.5 / 30.1, B=256
 // 32 heads 6.3 / 25.7, B=1024 32 heads 8.6 / 25.8 (1.7 GFLOP; 12.9 without the tiles), B=1024 64 heads 21 / 43, 128 heads 60 / 64. The
-// caller takes the library from B H K > 2^26 on. The whole step as a call at B=1024, 32 heads: 122 us as products and a step.
+// caller takes the library from B H K > 3 2^26 on. The whole step as a call at B=1024, 32 heads: 122 us as products and a step.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 

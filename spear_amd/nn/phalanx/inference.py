@@ -318,15 +318,16 @@ def _layer_operands(layer, x: torch.Tensor):
 def _token_operands(layer, x: torch.Tensor):
     """Weights and biases for the compiled step, whose first kernel runs the input projections and the step, or None where the
     call is for the general path: what ``plain_operands`` leaves to the modules, rows that 16-byte accesses do not fit or that overlap, and sizes
-    from which the library's products are faster on the GPU (B=1024 with 64 heads 33.7 against 43.0 us, 700 with 100 heads 61
-    against 52): a limit for steps in a graph. As a call, host included, the step takes 44 us with 64 heads, and 132 with 65 through the
-    modules, as it took for any size before there was a compiled one."""
+    from which the library's products are faster on the GPU: a limit for steps in a graph. Us, here / modules: B=1024 with 65 heads 47 / 78,
+    96 heads 53 / 67 (kv heads shared by four 53 / 57), 700 with 100 heads 56 / 67, 8192 with 32 heads 61 / 64 (shared 61 / 58), past the line
+    1024 with 128 heads 79 / 80 (shared 78 / 67), 4096 with 64 heads 86 / 79. As a call, host included, the modules take 135."""
     if x.dim() != 2 or x.shape[0] == 0 or x.stride(1) != 1 or x.stride(0) % 8 != 0 or x.data_ptr() % 16 != 0:
         return None
     if x.shape[0] > 1 and x.stride(0) < x.shape[1]:  # one token expanded over the batch, windows of a longer row
         return None
     p = layer.param
-    if x.shape[0] * layer.heads * x.shape[1] > 1 << 26:
+    few_products = layer.kv_heads < layer.heads and x.shape[0] > 2048  # the kernel computes shared b and c once per head
+    if x.shape[0] * layer.heads * x.shape[1] > (1 << 26 if few_products else 3 << 26):
         return None
     return _layer_operands(layer, x)
 

@@ -349,6 +349,27 @@ def test_step_with_the_output_projection_of_the_library():
         assert one.pos.tolist() == two.pos.tolist() == [(b + t + 1) % 16 for b in range(B)]
 
 
+@pytest.mark.parametrize("B,H,Hkv", [(1030, 65, 65), (700, 100, 25)])
+def test_steps_of_many_wide_sequences_equal_the_modules(B, H, Hkv):
+    """Between 2^26 and 3 2^26 of batch x heads x dim, where the compiled step runs the projections in tiles."""
+    from spear_amd import Phalanx
+    from spear_amd.nn.phalanx.inference import PhalanxStepState, phalanx_step
+
+    torch.manual_seed(16)
+    layer = Phalanx(dim=16 * H, length=128, method="fused", dtype=torch.bfloat16, kv_heads=Hkv).to(DEV)
+    x = torch.randn(18, B, 16 * H, generator=torch.Generator().manual_seed(17)).bfloat16().to(DEV)
+    one, two = PhalanxStepState.zeros(B, H, DEV), PhalanxStepState.zeros(B, H, DEV)
+    for t in range(18):
+        print(f"step {t} B={B} H={H} Hkv={Hkv}", flush=True)
+        y = phalanx_step(layer, x[t], one)
+        handle = layer.param.proj_a.register_forward_hook(lambda *a: None)  # the projections as modules
+        want = phalanx_step(layer, x[t], two)
+        handle.remove()
+        assert_close(f64(y), f64(want), 2e-2, 2e-2, f"y[{t}]")
+        assert torch.equal(one.pos, two.pos)
+    assert_close(f64(one.h_loc), f64(two.h_loc), 2e-2, 2e-2, "h")
+
+
 @pytest.mark.parametrize("B,L,dim", [(2, 48, 64), (1, 33, 1040)])
 def test_prompts_off_the_16_byte_grid_and_on_another_stream(B, L, dim):
     from spear_amd.nn.phalanx.inference import phalanx_prefill
