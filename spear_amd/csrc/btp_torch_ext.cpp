@@ -556,7 +556,7 @@ bool own_weight_grads(int64_t M, int64_t multiply_adds_per_token) { return M <= 
 // A whole layer call on plain bf16 tensors: the four input projections, the mixing stage and the output projection, with one
 // autograd node. Backward is what spear_amd/nn/phalanx/projections.py does with _ProjectAndMix and _Linear (one product each for the
 // input and weight gradients of the four projections, against the packed gradient buffer), without Python frames and with
-// layer_stack and layer_sums around the products: 10 launches for forward and backward of a small layer where separate modules had 29.
+// layer_transpose and layer_sums around the products: 9 launches for forward and backward of a small layer where separate modules had 29.
 // The mixing kernels are the same.
 struct LayerNode : public torch::autograd::Function<LayerNode> {
   static at::Tensor forward(torch::autograd::AutogradContext* ctx, const at::Tensor& x, const at::Tensor& w_a, const at::Tensor& b_a,
