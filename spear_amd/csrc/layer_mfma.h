@@ -21,6 +21,9 @@ __device__ __forceinline__ f32x4_t mfma(uint4 a, uint4 b, f32x4_t acc) {
 constexpr int kStep = 32;  // columns of one matrix instruction
 constexpr int kParts = 4;  // wavefronts of a workgroup: quarters of the columns
 
+// Matrix instructions along a quarter of K columns (the last quarter may have fewer).
+__host__ __device__ inline int quarter_steps(int K) { return ((K + kStep - 1) / kStep + kParts - 1) / kParts; }
+
 template <int kNT, int kChunk>
 struct Operands {
   uint4 w[kChunk][4];  // v, b, c, a
@@ -37,7 +40,7 @@ __device__ __forceinline__ void quarter_product(const uint16_t* const (&w)[4], c
 #pragma unroll
     for (int i = 0; i < 4; ++i) acc[i][t] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
   }
-  const int steps = (K + kStep - 1) / kStep, share = (steps + kParts - 1) / kParts;
+  const int steps = (K + kStep - 1) / kStep, share = quarter_steps(K);
   const int from = wave * share, to = min(from + share, steps);
   auto load = [&](Operands<kNT, kChunk>& o, int s0) {
 #pragma unroll

@@ -26,6 +26,15 @@ __device__ __forceinline__ f32x4_t mfma(i32x4_t a, i32x4_t b, f32x4_t acc) {
   return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, a), __builtin_bit_cast(bf16x8_t, b), acc, 0, 0, 0);
 }
 
+// acc[i][j] += w[j] x[i] over 32 columns of K.
+template <int kRowTiles, int kColTiles>
+__device__ __forceinline__ void multiply(f32x4_t (&acc)[kRowTiles][kColTiles], const i32x4_t (&w)[kColTiles], const i32x4_t (&x)[kRowTiles]) {
+#pragma unroll
+  for (int j = 0; j < kColTiles; ++j)
+#pragma unroll
+    for (int i = 0; i < kRowTiles; ++i) acc[i][j] = mfma(w[j], x[i], acc[i][j]);
+}
+
 // A buffer of `bytes` bytes (none if negative), which the hardware checks every access against.
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t buffer_of(const void* p, int bytes) {
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, max(bytes, 0), 0x00020000);

@@ -179,35 +179,47 @@ __global__ __launch_bounds__(512) void layer_token_tile_kernel(const LayerTokenA
     const int token = first + 32 * (wave >> 1) + 16 * i + n;
     if (mine < p.H && token < p.B) state[i] = load_token(p, token, head, kv, q);
   }
-  f32x4_t acc[2][4];  // [token tile][v, b, c, a]
+  // [quarter of K][token tile][v, b, c, a]. Added up as the kernel above adds its wavefronts' quarters: a token's state does not depend on how
+  // many others come with it, and is as far from 64 bits as there (h off by 9.2e-8 of its norm at K = 512, 1.1e-7 at 1024; in one chain over K
+  // 1.4e-7 and 1.9e-7).
+  f32x4_t acc[kParts][2][4];
 #pragma unroll
-  for (int i = 0; i < 2; ++i)
+  for (int u = 0; u < kParts; ++u)
 #pragma unroll
-    for (int m = 0; m < 4; ++m) acc[i][m] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int m = 0; m < 4; ++m) acc[u][i][m] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
   i32x4_t fx[2][2], fw[2][4];
-  int stage = 0;
-  for (int t = 0; t < steps; ++t) {
+  int stage = 0, t = 0;
+  auto step = [&](f32x4_t (&first)[2][4], f32x4_t (&second)[2][4]) {
     wait_vm<6 * (kTokenStages - 2)>();  // step t has landed, the ones after it may be under way
     phase_barrier();                    // in all wavefronts, and all have read step t - 1
     const int into = stage == 0 ? kTokenStages - 1 : stage - 1;  // where step t - 1 was
     const uint32_t x = x_at + stage * kTokenX, w = w_at + stage * kTokenW;
     read_token_fragments(x, w, fx[0], fw[0], rw, w_to + into * kTokenW);
     read_token_fragments_x(x ^ 64, w ^ 64, fx[1], fw[1], rx, x_to + into * kTokenX);
-#pragma unroll
-    for (int kk = 0; kk < 2; ++kk)
-#pragma unroll
-      for (int m = 0; m < 4; ++m)
-#pragma unroll
-        for (int i = 0; i < 2; ++i) acc[i][m] = mfma(fw[kk][m], fx[kk][i], acc[i][m]);
+    multiply(first, fw[0], fx[0]);
+    multiply(second, fw[1], fx[1]);
     end_rows(rx);
     end_rows(rw);
     stage = stage == kTokenStages - 1 ? 0 : stage + 1;
+    ++t;
+  };
+#pragma unroll
+  for (int u = 0; u < kParts; ++u) {
+    const int end = quarter_steps(K) * (u + 1), whole = u + 1 < kParts ? min(end / 2, steps) : steps;  // a step is two instructions along K
+    while (t < whole) step(acc[u], acc[u]);
+    if (u + 1 < kParts && end % 2 != 0 && t < steps) step(acc[u], acc[u + 1 < kParts ? u + 1 : u]);
   }
   if (mine < p.H) {
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
       const int token = first + 32 * (wave >> 1) + 16 * i + n;
-      if (token < p.B) step_token(p, token, head, q, acc[i], state[i]);
+#pragma unroll
+      for (int u = 1; u < kParts; ++u)
+#pragma unroll
+        for (int m = 0; m < 4; ++m) acc[0][i][m] += acc[u][i][m];
+      if (token < p.B) step_token(p, token, head, q, acc[0][i], state[i]);
     }
   }
   wait_vm<0>();  // the requests past the last step write LDS

@@ -214,3 +214,32 @@ def test_token_tiles_against_float64(B, H, Hkv, K, ldx):
     within(got_r, torch.where(end, torch.ones_like(r_new), r_new), e_r, "r")
     within(got_c, torch.where(end[..., None], new, c_prev.double()), e_new, "c_prev")
     assert torch.equal(state[3], pos)
+
+
+# As above, and widths of one step of 64 columns (fewer than the stages asked for ahead), of an odd number of instructions per quarter, and
+# of quarters that end inside a step.
+@pytest.mark.parametrize("B,H,Hkv,K", [(1024, 32, 32, 512), (700, 37, 37, 592), (333, 33, 11, 528), (200, 64, 16, 1024), (2049, 8, 2, 128),
+                                       (10007, 1, 1, 16), (5003, 3, 1, 48), (4099, 4, 4, 64), (3001, 5, 5, 80)])
+def test_a_token_is_the_same_whatever_number_comes_with_it(B, H, Hkv, K):
+    """The tiles add up a token's products as the kernel for few tokens does: the state, which is kept in fp32, and the result are equal."""
+    from spear_amd import _btp
+
+    g = torch.Generator(device=DEV).manual_seed(B)
+    normal = lambda *shape: torch.randn(*shape, generator=g, device=DEV)
+    x = normal(B, K).bfloat16()
+    weights = [(normal(n, K) * K**-0.5).bfloat16() for n in (H, 16 * Hkv, 16 * Hkv, 16 * H)]
+    b_a, b_b, b_c = (normal(n).bfloat16() for n in (H, 16 * Hkv, 16 * Hkv))
+    state = [normal(B, H, 16), torch.rand(B, H, generator=g, device=DEV), normal(B, H, 16),
+             torch.randint(0, 16, (B,), generator=g, device=DEV, dtype=torch.int32)]
+
+    def step(rows):
+        of = [t[rows].clone() for t in state]
+        out = _btp.load_extension().layer_token(x[rows], weights[0], b_a, weights[1], b_b, weights[2], b_c, weights[3], *of, 16, H, Hkv, False)
+        return out, *of
+
+    print(f"tokens B={B} H={H} Hkv={Hkv} K={K}", flush=True)
+    all_at_once = step(slice(0, B))
+    for first in (0, 16 * (B // 32), B - B % 16 if B % 16 else B - 16):
+        few = step(slice(first, min(B, first + 16)))
+        for got, want in zip(all_at_once, few):
+            assert torch.equal(got[first:first + 16], want)
