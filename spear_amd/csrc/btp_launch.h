@@ -137,7 +137,8 @@ hipError_t layer_linear(const LayerLinearArgs& p, hipStream_t s);
 // The same at large sizes (layer_gemm.hip), for the operands that layer_gemm_takes: K past 64, no positions.
 bool layer_gemm_takes(const LayerLinearArgs& p);
 enum class LayerTiles { kMid, kLarge };  // 128 x 128, 256 x 256
-hipError_t layer_gemm(const LayerLinearArgs& p, LayerTiles size, hipStream_t s);
+// quarters: kMid adds up K in quarters, as the kernel for few rows does.
+hipError_t layer_gemm(const LayerLinearArgs& p, LayerTiles size, bool quarters, hipStream_t s);
 
 // out[c] <- sum over the rows of in[rows, cols] (dense fp32), rounded to 16 bits (layer_grad.hip)
 struct LayerSumJob {

@@ -32,6 +32,7 @@
 
 #include "btp_device.h"
 #include "btp_launch.h"
+#include "layer_mfma.h"
 #include "layer_tile.h"
 
 namespace spear_btp {
@@ -271,7 +272,7 @@ __device__ __forceinline__ void read_fragments(uint32_t x, uint32_t w, i32x4_t (
 
 // Launched with 256 threads. The bound of 512 leaves a wavefront 256 registers: given 512, the compiler keeps the sums in accumulation
 // registers and copies them to and fro between matrix instructions (0.7 us per step instead of 0.45).
-template <int kStages>
+template <int kStages, bool kQuarters>
 __global__ __launch_bounds__(512) void layer_gemm_mid_kernel(const LayerLinearArgs p, int tiles_n, int tiles) {
   __shared__ __attribute__((aligned(1024))) char lds[2 * kStages * kMidStage];  // the stages of x, then those of the weights
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
@@ -300,11 +301,11 @@ __global__ __launch_bounds__(512) void layer_gemm_mid_kernel(const LayerLinearAr
 
   const uint32_t fragment = lds_address(lds) + n * 128 + (q ^ (n >> 1)) * 16;
   const uint32_t x_at = fragment + wm * 64 * 128, w_at = fragment + kStages * kMidStage + wn * 64 * 128;
-  f32x4_t acc[4][4];
+  f32x4_t acc[4][4], sum[4][4];  // kQuarters: of the quarter of K under way, and of those before it
 #pragma unroll
   for (int i = 0; i < 4; ++i)
 #pragma unroll
-    for (int j = 0; j < 4; ++j) acc[i][j] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+    for (int j = 0; j < 4; ++j) acc[i][j] = sum[i][j] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
   i32x4_t fx[2][4], fw[2][4];
   const uint32_t x_to = lds_address(lds) + wave * 4096, w_to = x_to + kStages * kMidStage;
 #pragma unroll
@@ -316,23 +317,32 @@ __global__ __launch_bounds__(512) void layer_gemm_mid_kernel(const LayerLinearAr
   }
   end_rows(rx);
   end_rows(rw);
-  int stage = 0;
+  const int share = quarter_steps(K);
+  int stage = 0, left = share;  // instructions along K until the next quarter
+  auto starts = [&]() {
+    if (!kQuarters) return false;
+    const bool first = left == 0;
+    left = (first ? share : left) - 1;
+    return first;
+  };
   for (int t = 0; t < steps; ++t) {
     wait_vm<8 * (kStages - 2)>();  // step t has landed, the ones after it may be under way
     phase_barrier();               // in all wavefronts, and all have read step t - 1
     // Step t + kStages - 1 goes where step t - 1 was. Past the last step nothing is asked for (nowhere), so that the waits' counts hold.
     const uint32_t at = stage * kMidStage, to = (stage == 0 ? kStages - 1 : stage - 1) * kMidStage;
     read_fragments(x_at + at, w_at + at, fx[0], fw[0], rx, x_to + to);
+    multiply_quarters(acc, sum, fw[0], fx[0], starts());
     read_fragments((x_at ^ 64) + at, (w_at ^ 64) + at, fx[1], fw[1], rw, w_to + to);
-#pragma unroll
-    for (int kk = 0; kk < 2; ++kk)
-#pragma unroll
-      for (int j = 0; j < 4; ++j)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) acc[i][j] = mfma(fw[kk][j], fx[kk][i], acc[i][j]);
+    multiply_quarters(acc, sum, fw[1], fx[1], starts());
     end_rows(rx);
     end_rows(rw);
     stage = stage == kStages - 1 ? 0 : stage + 1;
+  }
+  if (kQuarters) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) acc[i][j] += sum[i][j];
   }
 
   if (const uint16_t* bias = p.bias[job]; bias != nullptr) {
@@ -383,7 +393,7 @@ bool layer_gemm_takes(const LayerLinearArgs& p) {
   return tiles * ((p.M + kMidSide - 1) / kMidSide) < 1l << 28;
 }
 
-hipError_t layer_gemm(const LayerLinearArgs& p, LayerTiles size, hipStream_t s) {
+hipError_t layer_gemm(const LayerLinearArgs& p, LayerTiles size, bool quarters, hipStream_t s) {
   const int side = size == LayerTiles::kMid ? kMidSide : kTileRows;
   int tiles_n = 0;
   for (int j = 0; j < p.jobs; ++j) tiles_n += (p.N[j] + side - 1) / side;
@@ -391,8 +401,9 @@ hipError_t layer_gemm(const LayerLinearArgs& p, LayerTiles size, hipStream_t s) 
   if (tiles == 0) return hipSuccess;
   if (size == LayerTiles::kMid) {
     const dim3 grid((unsigned)((tiles + 7) / 8 * 8)), block(256);
-    if (tiles <= 256) hipLaunchKernelGGL(layer_gemm_mid_kernel<4>, grid, block, 0, s, p, tiles_n, tiles);
-    else hipLaunchKernelGGL(layer_gemm_mid_kernel<2>, grid, block, 0, s, p, tiles_n, tiles);
+    auto* const kernel = tiles <= 256 ? (quarters ? layer_gemm_mid_kernel<4, true> : layer_gemm_mid_kernel<4, false>)
+                                      : (quarters ? layer_gemm_mid_kernel<2, true> : layer_gemm_mid_kernel<2, false>);
+    hipLaunchKernelGGL(kernel, grid, block, 0, s, p, tiles_n, tiles);
     return hipGetLastError();
   }
   const dim3 grid(256), block(512);  // a workgroup for every compute unit

@@ -96,11 +96,22 @@ static Kernel fastest(const LayerLinearArgs& p, int groups) {
   return here <= mid && here <= large ? Kernel::kHere : mid <= large ? Kernel::kMid : Kernel::kLarge;
 }
 
+// Up to here 128 x 128 tiles add up K in the four quarters that the kernel here has in four wavefronts: a call of such a size gives the same
+// bits whichever of the two it goes to, and loses nothing against the shorter chains (of [2048, 1024] x [1024, 1024] 9.2e-5 of the
+// results are not the nearest 16-bit value in quarters, 1.1e-4 in one chain over K). It takes 0.4 to 1.4 us more (a layer's forward at 1024
+// rows, dim 512, 21.4 / 20.7 us; 4096 rows, 256, 21.5 / 20.1). Larger calls are added up in one chain by tiles of either size, as the library does.
+static bool few(const LayerLinearArgs& p) {
+  long columns = 0;
+  for (int j = 0; j < p.jobs; ++j) columns += p.N[j];
+  return p.jobs > 1 ? p.M * columns * p.K <= 1600000000 : p.K <= 512 && p.M * columns * p.K <= 300000000;
+}
+
 hipError_t layer_linear(const LayerLinearArgs& p, hipStream_t s) {
   int groups = 0;
   for (int j = 0; j < p.jobs; ++j) groups += (p.N[j] + 63) / 64;
   if (groups == 0 || p.M == 0) return hipSuccess;
-  if (const Kernel k = fastest(p, groups); k != Kernel::kHere) return layer_gemm(p, k == Kernel::kMid ? LayerTiles::kMid : LayerTiles::kLarge, s);
+  if (const Kernel k = fastest(p, groups); k != Kernel::kHere)
+    return layer_gemm(p, k == Kernel::kMid ? LayerTiles::kMid : LayerTiles::kLarge, few(p), s);
   // as layer_token chooses: as many workgroups as there are while they are few
   const long pairs = (long)groups * ((p.M + 15) / 16);
   if (pairs <= 256) launch<1, 4>(p, groups, s);

@@ -35,6 +35,23 @@ __device__ __forceinline__ void multiply(f32x4_t (&acc)[kRowTiles][kColTiles], c
     for (int i = 0; i < kRowTiles; ++i) acc[i][j] = mfma(w[j], x[i], acc[i][j]);
 }
 
+// The same where `first` says that a quarter of K starts here: the sums so far go to `sum` and acc starts again, beside the matrix instructions.
+template <int kRowTiles, int kColTiles>
+__device__ __forceinline__ void multiply_quarters(f32x4_t (&acc)[kRowTiles][kColTiles], f32x4_t (&sum)[kRowTiles][kColTiles],
+                                                  const i32x4_t (&w)[kColTiles], const i32x4_t (&x)[kRowTiles], bool first) {
+  if (first) {
+#pragma unroll
+    for (int j = 0; j < kColTiles; ++j)
+#pragma unroll
+      for (int i = 0; i < kRowTiles; ++i) {
+        sum[i][j] += acc[i][j];
+        acc[i][j] = mfma(w[j], x[i], f32x4_t{0.0f, 0.0f, 0.0f, 0.0f});
+      }
+  } else {
+    multiply(acc, w, x);
+  }
+}
+
 // A buffer of `bytes` bytes (none if negative), which the hardware checks every access against.
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t buffer_of(const void* p, int bytes) {
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, max(bytes, 0), 0x00020000);

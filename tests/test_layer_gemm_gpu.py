@@ -243,3 +243,19 @@ def test_a_token_is_the_same_whatever_number_comes_with_it(B, H, Hkv, K):
         few = step(slice(first, min(B, first + 16)))
         for got, want in zip(all_at_once, few):
             assert torch.equal(got[first:first + 16], want)
+
+
+# Sizes that 128 x 128 tiles take up to which K is added up in quarters: quarters that end inside a step of 64 columns, and of one instruction.
+@pytest.mark.parametrize("M,K,columns", [(1024, 512, (512, 512, 512, 32)), (1003, 592, (592, 592, 257, 37)), (600, 1040, (1040, 130, 129, 24)), (1500, 72, (1024, 130))])
+def test_a_row_is_the_same_whatever_number_comes_with_it(M, K, columns):
+    """The tiles add up a row's products as the kernel for few rows does: the results are equal."""
+    from spear_amd import _btp
+
+    g = torch.Generator(device=DEV).manual_seed(M)
+    normal = lambda *shape: torch.randn(*shape, generator=g, device=DEV).bfloat16()
+    x, weights, biases = normal(M, K), [normal(n, K) for n in columns], [normal(n) for n in columns]
+    print(f"rows M={M} K={K} columns={columns}", flush=True)
+    out = _btp.load_extension().linears(x, weights, biases)
+    for first in (0, 16 * (M // 32), M - 16):
+        for y, few in zip(out, _btp.load_extension().linears(x[first:first + 16], weights, biases)):
+            assert torch.equal(y[first:first + 16], few)
