@@ -20,9 +20,10 @@
 //
 // Many tokens go through tiles in LDS (below): there the chain of loads from L2 and their number bound the kernel above.
 //
-// Measured in a HIP graph, us, here / four library products and the step kernel: B=1 8 heads 4.4 / 23.8, B=1 128 heads 9.5 / 30.1, B=256
-// 32 heads 6.3 / 25.7, B=1024 32 heads 8.6 / 25.8 (1.7 GFLOP; 12.9 without the tiles), B=1024 64 heads 21 / 43, 128 heads 60 / 64. The
-// caller takes the library from B H K > 3 2^26 on. The whole step as a call at B=1024, 32 heads: 122 us as products and a step.
+// Measured in a HIP graph, us, here / four library products and the step kernel: B=1 8 heads 4.0 / 23.8, B=1 128 heads 9.3 / 30.1, B=256
+// 32 heads 5.9 / 25.7, B=1024 32 heads 8.2 / 25.8 (1.7 GFLOP; 11.8 without the tiles), B=1024 64 heads 20 / 43, 128 heads 60 / 64. The
+// caller takes the library from B H K > 3 2^26 on, with kv heads shared and more than 2048 tokens from 2^26 on. The whole step as a call at
+// B=1024, 32 heads: 122 us as products and a step.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -233,19 +234,27 @@ void launch(const LayerTokenArgs& p, hipStream_t s) {
 
 }  // namespace
 
-hipError_t layer_token(const LayerTokenArgs& p, hipStream_t s) {
-  // Few workgroups: as many as there are; then two token tiles each, which read the weights less often (one / two, us: B=32 128 heads,
-  // 256 pairs, 12.5 / 14.3; B=256 32 heads, 512 pairs, 8.8 / 7.7); then the tile kernel. Two token tiles / it: B=256 37 heads (592 pairs) 7.3 /
-  // 8.5, B=200 48 heads (624) 9.8 / 9.2, B=128 64 heads (512) 9.0 / 10.5, B=200 64 heads (832) 11.5 / 10.7, B=512 32 heads (1024) 8.7 / 8.1,
-  // B=1024 32 heads 12.9 / 8.6, B=1024 128 heads 111 / 60.
-  const long pairs = (long)p.H * ((p.B + 15) / 16);
+// Whether the tile kernel takes less time than four token tiles per wavefront, past 512 pairs. Both as fitted to 51 shapes (1 to 256 heads,
+// 40 to 20000 tokens): tiles in rounds of 256 workgroups, longer with K; the other in proportion to its workgroups and K. Four token tiles /
+// the tile kernel, us: 1 head B=20000 4.0 / 7.2, 3 heads B=4096 4.3 / 5.0, 8 heads B=2048 5.7 / 5.4, B=20000 28.4 / 24.3, 9 heads B=5000 8.9 / 10.8,
+// 16 heads B=1024 6.1 / 6.6, B=1500 8.0 / 6.8, 32 heads B=512 7.9 / 7.9, B=1024 11.8 / 8.2, 37 heads B=300 6.7 / 8.3, B=500 9.7 / 8.7, 64 heads
+// B=200 10.8 / 10.6, B=1024 32 / 20, 128 heads B=1024 110 / 60.
+static bool tiles_win(const LayerTokenArgs& p) {
   // the tile kernel's offsets are 32 bits: the largest matrix and 64 rows of tokens below 1 GiB
-  const bool near = 32l * p.H * p.K < 1l << 30 && 2l * kTokenRows * p.ldx < 1l << 30;
-  if (pairs <= 256) {
-    launch<1, 4>(p, s);
-  } else if (pairs <= 600 || !near) {
-    launch<2, 4>(p, s);
-  } else {
+  if (32l * p.H * p.K >= 1l << 30 || 2l * kTokenRows * p.ldx >= 1l << 30) return false;
+  const long row_tiles = (p.B + kTokenRows - 1) / kTokenRows, rounds = ((p.H + 1) / 2 * row_tiles + 255) / 256;
+  const double tiles = 1.0 + (double)rounds * (4.2 + 0.36 * ((p.K + kRowsStep - 1) / kRowsStep));
+  return tiles < 3.5 + (1.6 + 0.0059 * p.K) * (double)(p.H * row_tiles) / 256;
+}
+
+hipError_t layer_token(const LayerTokenArgs& p, hipStream_t s) {
+  // Few workgroups: as many as there are. Else more tokens to a workgroup, which reads the weights less often, or the tile kernel where it is the
+  // faster one. One / two token tiles, us: B=32 128 heads (256 pairs) 12.5 / 14.3; B=256 32 heads (512) 8.8 / 7.7.
+  const long pairs = (long)p.H * ((p.B + 15) / 16);
+  if (pairs <= 256) launch<1, 4>(p, s);
+  else if (pairs <= 512) launch<2, 4>(p, s);
+  else if (!tiles_win(p)) launch<4, 2>(p, s);
+  else {
     const int head_pairs = (p.H + 1) / 2;
     hipLaunchKernelGGL(layer_token_tile_kernel, dim3((unsigned)(head_pairs * ((p.B + kTokenRows - 1) / kTokenRows))), dim3(256), 0, s, p, head_pairs);
   }
