@@ -134,7 +134,7 @@ struct LayerLinearArgs {
   int block_len;
 };
 hipError_t layer_linear(const LayerLinearArgs& p, hipStream_t s);
-// The same at large sizes (layer_gemm.hip), for the operands that layer_gemm_takes: K past 64, no positions.
+// The same at large sizes (layer_gemm.hip), for the operands that layer_gemm_takes: K past 64. Only kMid moves positions.
 bool layer_gemm_takes(const LayerLinearArgs& p);
 enum class LayerTiles { kMid, kLarge };  // 128 x 128, 256 x 256
 // quarters: kMid adds up K in quarters, as the kernel for few rows does.

@@ -456,10 +456,6 @@ std::vector<at::Tensor> linears(const at::Tensor& x, const std::vector<at::Tenso
   return out;
 }
 
-// Whether one projection is taken by spear_layer_linear's kernel for few rows although the library's product is no slower on the GPU (the
-// sizes measured at layer_linear.hip).
-bool small_product(int64_t M, int64_t columns, int64_t K) { return M > 0 && K > 0 && K % 8 == 0 && K <= 512 && M * columns * K <= 300000000; }
-
 // Whether projections of M rows are faster through spear_layer_linear than as the library's products. Measured in HIP graphs, us, dim = K,
 // spear_layer_linear / the library. The four input projections: K=128 131072 rows 49 / 67, K=512 1024 rows 8 / 22, 131072 rows 229 / 284,
 // K=768 65536 rows 230 / 239, K=1024 8192 rows 54 / 72, 131072 rows 729 / 717 (with kv heads shared by four 401 / 405), K=1536 16384 rows
@@ -802,11 +798,12 @@ std::vector<at::Tensor> layer_prefill(const at::Tensor& x, const at::Tensor& w_a
 at::Tensor layer_step(const at::Tensor& x, const at::Tensor& w_a, const at::Tensor& b_a, const at::Tensor& w_b, const at::Tensor& b_b,
                       const at::Tensor& w_c, const at::Tensor& b_c, const at::Tensor& w_v, const at::Tensor& w_out, at::Tensor h,
                       at::Tensor r, at::Tensor c_prev, at::Tensor pos, int64_t block_len, int64_t heads, int64_t kv_heads) {
-  // the positions move on with the output projection where that is a kernel of this library
+  // the positions move on with the output projection where that is a kernel of this library: a launch less, which makes up for what the
+  // product takes longer than the library's (see own_products)
   const auto in = [&](bool advance) { return layer_token(x, w_a, b_a, w_b, b_b, w_c, b_c, w_v, h, r, c_prev, pos, block_len, heads, kv_heads, advance); };
-  if (small_product(x.size(0), w_out.size(0), w_out.size(1)))
+  if (own_products(x.size(0), {w_out}, w_out.size(1)))
     return linears(in(false), {w_out}, {at::Tensor()}, pos.data_ptr<int>(), block_len)[0];
-  return project(in(true), {w_out}, {at::Tensor()})[0];
+  return at::linear(in(true), w_out);
 }
 
 }  // namespace

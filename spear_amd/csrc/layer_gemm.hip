@@ -298,6 +298,10 @@ __global__ __launch_bounds__(512) void layer_gemm_mid_kernel(const LayerLinearAr
   }
   aim(rx, p.x + (long)panel * kMidSide * ldx, rows, ldx, K);
   aim(rw, p.w[job] + (long)col * K, cols, K, K);
+  // the first tile of a panel's rows moves their positions on; read here, ahead of the requests, and written with the results
+  const bool moves = p.pos != nullptr && job == 0 && col == 0 && (int)threadIdx.x < rows;
+  int* const pos = p.pos + (long)panel * kMidSide + threadIdx.x;
+  const int was = moves ? *pos : 0;
 
   const uint32_t fragment = lds_address(lds) + n * 128 + (q ^ (n >> 1)) * 16;
   const uint32_t x_at = fragment + wm * 64 * 128, w_at = fragment + kStages * kMidStage + wn * 64 * 128;
@@ -378,13 +382,14 @@ __global__ __launch_bounds__(512) void layer_gemm_mid_kernel(const LayerLinearAr
       }
     }
   }
+  if (moves) *pos = was + 1 >= p.block_len ? 0 : was + 1;
   wait_vm<0>();  // the requests past the last step write LDS
 }
 
 }  // namespace
 
 bool layer_gemm_takes(const LayerLinearArgs& p) {
-  if (p.K <= kStepK || p.K % 8 != 0 || p.ldx % 8 != 0 || p.pos != nullptr || p.K >= 1 << 21 || p.ldx >= 1 << 21) return false;
+  if (p.K <= kStepK || p.K % 8 != 0 || p.ldx % 8 != 0 || p.K >= 1 << 21 || p.ldx >= 1 << 21) return false;
   long tiles = 0;
   for (int j = 0; j < p.jobs; ++j) {
     if (p.N[j] >= 1 << 21) return false;

@@ -93,6 +93,7 @@ static Kernel fastest(const LayerLinearArgs& p, int groups) {
   const double here = 4.0 + (0.7 + 0.0098 * p.K) * (double)groups * ((p.M + 63) / 64) / 256;
   const double mid = 4.2 + steps * (small_tiles <= 256 ? 0.47 : 1.0 * (double)((small_tiles + 511) / 512));
   const double large = 8.0 + (double)((tiles(256) + 255) / 256) * (1.0 + steps);
+  if (p.pos != nullptr) return here <= mid ? Kernel::kHere : Kernel::kMid;  // the large tiles move no positions
   return here <= mid && here <= large ? Kernel::kHere : mid <= large ? Kernel::kMid : Kernel::kLarge;
 }
 

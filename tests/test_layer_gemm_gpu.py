@@ -260,3 +260,25 @@ def test_a_row_is_the_same_whatever_number_comes_with_it(M, K, columns):
     for first in (0, 16 * (M // 32), M - 16):
         for y, few in zip(out, _btp.load_extension().linears(x[first:first + 16], weights, biases)):
             assert torch.equal(y[first:first + 16], few)
+
+
+# The kernel for few rows and 128 x 128 tiles, in each of which one workgroup of a panel of rows moves their positions.
+@pytest.mark.parametrize("M,K,N", [(17, 528, 528), (129, 1024, 1024), (1003, 1040, 1040), (5000, 768, 768), (40000, 136, 136)])
+def test_positions_move_on_with_a_projection(M, K, N):
+    import ctypes
+
+    from spear_amd import _btp
+
+    lib = _btp.load_library()
+    g = torch.Generator(device=DEV).manual_seed(M)
+    x, w = torch.randn(M, K, generator=g, device=DEV).bfloat16(), (torch.randn(N, K, generator=g, device=DEV) * K**-0.5).bfloat16()
+    y = torch.empty(M, N, device=DEV, dtype=torch.bfloat16)
+    pos = torch.randint(0, 16, (M + 1,), generator=g, device=DEV, dtype=torch.int32)
+    was = pos.clone()
+    one = lambda t: (ctypes.c_void_p * 1)(t.data_ptr())
+    print(f"positions with a projection M={M} K={K} N={N}", flush=True)
+    assert lib.spear_layer_linear(1, ctypes.c_void_p(x.data_ptr()), ctypes.c_longlong(K), M, K, one(w), (ctypes.c_void_p * 1)(None), one(y), (ctypes.c_int * 1)(N),
+                                  ctypes.c_void_p(pos.data_ptr()), 16, ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)) == 0
+    torch.cuda.synchronize()
+    assert_product(y, x, w, None, f"M={M} K={K}")
+    assert torch.equal(pos[:M], (was[:M] + 1) % 16) and pos[M] == was[M]

@@ -330,11 +330,9 @@ def test_step_takes_tokens_in_any_layout(layout, B):
     assert one.pos.tolist() == [2] * B
 
 
-def test_step_with_the_output_projection_of_the_library():
-    """Wider than the output projection's kernel takes: the token kernel moves the block positions on itself, also past a block's end."""
+def _steps_equal_the_modules(B, dim):
     from spear_amd.nn.phalanx.inference import PhalanxStepState, phalanx_step
 
-    B, dim = 17, 528
     layer = _layer(dim=dim, seed=12)
     x = torch.randn(20, B, dim, generator=torch.Generator().manual_seed(13)).bfloat16().to(DEV)
     one, two = PhalanxStepState.zeros(B, dim // 16, DEV), PhalanxStepState.zeros(B, dim // 16, DEV)
@@ -347,6 +345,28 @@ def test_step_with_the_output_projection_of_the_library():
         handle.remove()
         assert_close(f64(y), f64(want), 2e-2, 2e-2, f"y[{t}]")
         assert one.pos.tolist() == two.pos.tolist() == [(b + t + 1) % 16 for b in range(B)]
+
+
+def test_step_with_the_output_projection_of_the_library():
+    """More narrow sequences than the output projection's kernel takes: the token kernel moves the block positions on itself, also past a block's end."""
+    _steps_equal_the_modules(73300, 64)
+
+
+@pytest.mark.parametrize("B,dim", [(17, 528), (1030, 784)])
+def test_a_step_is_two_launches(B, dim):
+    """The output projection moves the block positions on, also past a block's end, in its kernel for few rows and in 128 x 128 tiles."""
+    from spear_amd.nn.phalanx.inference import PhalanxStepState, phalanx_step
+
+    _steps_equal_the_modules(B, dim)
+    layer, state = _layer(dim=dim, seed=12), PhalanxStepState.zeros(B, dim // 16, DEV)
+    x = torch.zeros(B, dim, device=DEV, dtype=torch.bfloat16)
+    phalanx_step(layer, x, state)
+    torch.cuda.synchronize()
+    with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CUDA]) as profile:
+        phalanx_step(layer, x, state)
+        torch.cuda.synchronize()
+    kernels = [e.name for e in profile.events() if e.device_type == torch.autograd.DeviceType.CUDA]
+    assert len(kernels) == 2, kernels
 
 
 @pytest.mark.parametrize("B,H,Hkv", [(1030, 65, 65), (700, 100, 25)])
