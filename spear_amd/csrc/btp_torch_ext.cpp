@@ -460,9 +460,9 @@ std::vector<at::Tensor> linears(const at::Tensor& x, const std::vector<at::Tenso
 // spear_layer_linear / the library. The four input projections: K=128 131072 rows 49 / 67, K=512 1024 rows 8 / 22, 131072 rows 229 / 284,
 // K=768 65536 rows 230 / 239, K=1024 8192 rows 54 / 72, 131072 rows 729 / 717 (with kv heads shared by four 401 / 405), K=1536 16384 rows
 // 203 / 238, 65536 rows 772 / 742, K=2048 4096 rows 95 / 114, 8192 rows 193 / 174: all below K = 1024, and few tiles from there on.
-// One: K=512 65536 rows 40 / 43, 16384 rows 13.7 / 15.5, K=1024 1024 rows 11.2 / 8.2, 4096 rows 13.5 / 13.5, 16384 rows 34 / 30, K=2048 1024 rows
-// 20 / 16. On the GPU it is up to 4 us slower up to 9 G multiply-adds, and saves the 15 us that a library product costs the host, which is
-// what bounds calls of that size. The tiles start at K = 72; up to 64 the few-row kernel is left, which reads its operands too often for
+// One: K=512 65536 rows 40 / 43, 16384 rows 13.7 / 15.5, K=1024 16 rows 4.3 / 4.2, 1024 rows 10.6 / 7.7, 4096 rows 13.5 / 13.5, 16384 rows 34 / 30,
+// K=2048 16 rows 6.0 / 5.3, 1024 rows 19 / 15, K=4096 16 rows 10 / 11, 512 rows 33 / 24. On the GPU it is mostly up to 4 us slower up to 9 G
+// multiply-adds, and saves the 15 us that a library product costs the host, which is what bounds calls of that size. The tiles start at K = 72; up to 64 the few-row kernel is left, which reads its operands too often for
 // many rows (a layer's forward at 1048576 rows, it / the library: K=32 541 / 384, K=64 838 / 470; 8192 rows within 5 %).
 bool own_products(int64_t M, const std::vector<at::Tensor>& weights, int64_t K) {
   if (M <= 0 || K <= 0 || K % 8 != 0) return false;

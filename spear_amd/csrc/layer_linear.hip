@@ -4,15 +4,13 @@
 //     out_j[M, N_j] = x[M, K] w_j[N_j, K]^T + bias_j          bf16, fp32 sums, rounded once
 //
 // The four input projections of a thousand tokens are a GFLOP or two. The library serves them one by one, in 5 to 7 us each on
-// the GPU and about 15 us of host time per call, which is what such a layer is bound by. A workgroup makes 64 columns by 16 kNT
+// the GPU and about 15 us of host time per call, which is what such a layer is bound by. A workgroup makes 16 kW columns by 16 kNT
 // rows (layer_mfma.h: a quarter of K per wavefront), whatever array the columns belong to, so the narrow arrays share the chip with the
 // wide ones.
 //
 // Longer inputs are for the tiles of layer_gemm.hip (`fastest`). One projection (dim x dim) here / as the library's
-// product, us in a HIP graph: M=1024 dim=512 5.7 / 5.8 (0.27 G multiply-adds), M=2048 dim=512 7.6 / 6.2, M=16 dim=512 4.8 / 3.8, M=128
-// dim=768 7.2 / 4.7: alone it is the slower one on the GPU and is taken for the host time it saves (a decode step of 16 sequences 19.7 us
-// as a call at K = 512 with it, 38.5 at K = 1024 with the library's product), up to 0.3 G and K = 512. The line at K is
-// the GPU's, for steps in a graph; between 512 and 768 nothing was timed.
+// product, us in a HIP graph: M=1 dim=512 2.9 / 3.7, dim=2048 4.7 / 5.2; M=16 dim=512 3.3 / 3.8, dim=1024 4.3 / 4.3, dim=2048 6.0 / 5.3; M=64 dim=1024 4.4 /
+// 6.5, dim=2048 7.9 / 7.4; M=128 dim=768 5.2 / 4.7, dim=1024 5.4 / 5.2, dim=2048 9.6 / 6.7. As a call the library's product costs the host 15 us more.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -24,22 +22,23 @@ namespace spear_btp {
 
 namespace {
 
-template <int kNT, int kChunk>
+template <int kNT, int kChunk, int kW>
 __global__ __launch_bounds__(256) void layer_linear_kernel(const LayerLinearArgs p, int groups) {
-  __shared__ f32x4_t partial[kParts][4][kNT][64];
+  constexpr int kCols = 16 * kW;
+  __shared__ f32x4_t partial[kParts][kW][kNT][64];
   const int lane = threadIdx.x & 63, n = lane & 15, q = lane >> 4, wave = threadIdx.x >> 6;
   int group = (int)(blockIdx.x % (unsigned)groups), j = 0;
   const int first = (int)(blockIdx.x / (unsigned)groups) * 16 * kNT;
-  while (group >= (p.N[j] + 63) / 64) group -= (p.N[j++] + 63) / 64;
-  const int N = p.N[j], col = 64 * group, K = p.K;
-  const uint16_t *w[4], *x[kNT];
+  while (group >= (p.N[j] + kCols - 1) / kCols) group -= (p.N[j++] + kCols - 1) / kCols;
+  const int N = p.N[j], col = kCols * group, K = p.K;
+  const uint16_t *w[kW], *x[kNT];
 #pragma unroll
-  for (int i = 0; i < 4; ++i) w[i] = p.w[j] + (long)min(col + 16 * i + n, N - 1) * K;  // past the last row or column: read it, store nothing
+  for (int i = 0; i < kW; ++i) w[i] = p.w[j] + (long)min(col + 16 * i + n, N - 1) * K;  // past the last row or column: read it, store nothing
 #pragma unroll
   for (int t = 0; t < kNT; ++t) x[t] = p.x + (long)min(first + 16 * t + n, p.M - 1) * p.ldx;
-  f32x4_t acc[4][kNT], sum[4];
-  quarter_product<kNT, kChunk>(w, x, K, wave, q, acc);
-  add_quarters<kNT>(partial, acc, wave, lane, sum);
+  f32x4_t acc[kW][kNT], sum[kW];
+  quarter_product<kNT, kChunk, kW>(w, x, K, wave, q, acc);
+  add_quarters<kNT, kW>(partial, acc, wave, lane, sum);
   const int row = first + 16 * wave + n;
   if (wave >= kNT || row >= p.M) return;
   if (p.pos != nullptr && blockIdx.x % (unsigned)groups == 0 && q == 0) {  // one lane of the grid per row
@@ -49,7 +48,7 @@ __global__ __launch_bounds__(256) void layer_linear_kernel(const LayerLinearArgs
   const uint16_t* bias = p.bias[j];
   uint16_t* out = p.out[j] + (long)row * N;
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
+  for (int i = 0; i < kW; ++i) {
     const int c = col + 16 * i + 4 * q;
     float v[4];
 #pragma unroll
@@ -66,31 +65,53 @@ __global__ __launch_bounds__(256) void layer_linear_kernel(const LayerLinearArgs
   }
 }
 
-template <int kNT, int kChunk>
-void launch(const LayerLinearArgs& p, int groups, hipStream_t s) {
+template <int kNT, int kChunk, int kW>
+void launch(const LayerLinearArgs& p, long groups, hipStream_t s) {
   const long tiles = (p.M + 16 * kNT - 1) / (16 * kNT);
-  hipLaunchKernelGGL((layer_linear_kernel<kNT, kChunk>), dim3((unsigned)(groups * tiles)), dim3(256), 0, s, p, groups);
+  hipLaunchKernelGGL((layer_linear_kernel<kNT, kChunk, kW>), dim3((unsigned)(groups * tiles)), dim3(256), 0, s, p, (int)groups);
+}
+
+// Tiles of `cols` columns that the arrays of a call have.
+long groups_of(const LayerLinearArgs& p, int cols) {
+  long groups = 0;
+  for (int j = 0; j < p.jobs; ++j) groups += (p.N[j] + cols - 1) / cols;
+  return groups;
+}
+
+// The instance of the kernel here for a call, 16 kNT rows by 16 kW columns to a workgroup, and its time in us as fitted to their times at K = 256 to
+// 4096. The smallest tile of which each compute unit gets one at most: its operands are the longest part of its time. [M, K] x [K, K], the instance that
+// the rule takes / the next larger tile, us: M=16 K=512 3.3 / 3.8, K=1024 4.3 / 5.3, K=2048 6.0 / 7.8, K=4096 10.1 / 13.6 (64 columns 4.9, 7.3, 11.6, 21.0); M=64
+// K=2048 7.9 / 9.6 (16 columns 9.5); M=128 K=2048 9.6 / 11.7.
+struct Instance {
+  int rows, cols;
+  double us;
+};
+
+Instance instance(const LayerLinearArgs& p) {
+  const double K = p.K;
+  const long g16 = groups_of(p, 16), g32 = groups_of(p, 32), g64 = groups_of(p, 64), r16 = (p.M + 15l) / 16, r32 = (p.M + 31l) / 32, r64 = (p.M + 63l) / 64;
+  if (g16 * r16 <= 256) return {16, 16, 2.2 + 0.0019 * K};
+  if (g32 * r16 <= 256) return {16, 32, 2.7 + 0.0026 * K};
+  if (g32 * r32 <= 256) return {32, 32, 2.8 + 0.0035 * K};
+  if (g64 * r16 <= 256) return {16, 64, 3.6 + 0.0041 * K};
+  if (g64 * r16 <= 512) return {32, 64, 3.5 + 0.0051 * K};
+  return {64, 64, 3.7 + (double)((g64 * r64 + 255) / 256) * (0.5 + 0.0072 * K)};
 }
 
 }  // namespace
 
-// Which kernel is the fastest, by their times in us as fitted to 56 shapes (dim 128 to 2048, 256 to 16384 rows): here rounds of 256
-// workgroups, growing with K; in layer_gemm tiles of 128 x 128, 0.47 us per 64 columns of K while each compute unit has one, twice that for
-// two; tiles of 256 x 256, 1 us. Four projections, dim = K, here / 128 / 256: K=128 1024 rows 5.0 / 5.2 / 9.1, 8192 rows 12.5 / 6.1 / 9.9; K=512
-// 256 rows 6.1 / 7.9 / 16.2, 1024 rows 11.9 / 8.3 / 16.8, 8192 rows 56 / 21 / 19; K=1024 256 rows 11.3 / 11.6 / 24, 2048 rows 61 / 20 / 28, 4096
-// rows 106 / 36 / 29; K=2048 1024 rows 111 / 34 / 46.
+// Which kernel is the fastest, by their times in us as fitted to 56 shapes (dim 128 to 2048, 256 to 16384 rows) for the tiles: of 128 x 128, 0.47 us per
+// 64 columns of K while each compute unit has one, twice that for two; of 256 x 256, 1 us. Four projections, dim = K, here / 128 / 256: K=128
+// 1024 rows 5.0 / 5.2 / 9.1, 8192 rows 12.5 / 6.1 / 9.9; K=512 256 rows 5.7 / 7.9 / 16.2, 1024 rows 11.9 / 8.3 / 16.8, 8192 rows 56 / 21 / 19; K=1024 256 rows
+// 10.7 / 11.6 / 24, 2048 rows 61 / 20 / 28, 4096 rows 106 / 36 / 29; K=2048 128 rows 17.7 / 18.6, 1024 rows 111 / 34 / 46; K=4096 1 row 18.6 / 36, 128 rows 60 / 33.
 enum class Kernel { kHere, kMid, kLarge };
 
-static Kernel fastest(const LayerLinearArgs& p, int groups) {
+static Kernel fastest(const LayerLinearArgs& p) {
   if (!layer_gemm_takes(p)) return Kernel::kHere;
-  auto tiles = [&](long side) {
-    long n = 0;
-    for (int j = 0; j < p.jobs; ++j) n += (p.N[j] + side - 1) / side;
-    return n * ((p.M + side - 1) / side);
-  };
+  auto tiles = [&](long side) { return groups_of(p, (int)side) * ((p.M + side - 1) / side); };
   const int steps = (p.K + 63) / 64;
   const long small_tiles = tiles(128);
-  const double here = 4.0 + (0.7 + 0.0098 * p.K) * (double)groups * ((p.M + 63) / 64) / 256;
+  const double here = instance(p).us;
   const double mid = 4.2 + steps * (small_tiles <= 256 ? 0.47 : 1.0 * (double)((small_tiles + 511) / 512));
   const double large = 8.0 + (double)((tiles(256) + 255) / 256) * (1.0 + steps);
   if (p.pos != nullptr) return here <= mid ? Kernel::kHere : Kernel::kMid;  // the large tiles move no positions
@@ -108,16 +129,16 @@ static bool few(const LayerLinearArgs& p) {
 }
 
 hipError_t layer_linear(const LayerLinearArgs& p, hipStream_t s) {
-  int groups = 0;
-  for (int j = 0; j < p.jobs; ++j) groups += (p.N[j] + 63) / 64;
-  if (groups == 0 || p.M == 0) return hipSuccess;
-  if (const Kernel k = fastest(p, groups); k != Kernel::kHere)
-    return layer_gemm(p, k == Kernel::kMid ? LayerTiles::kMid : LayerTiles::kLarge, few(p), s);
-  // as layer_token chooses: as many workgroups as there are while they are few
-  const long pairs = (long)groups * ((p.M + 15) / 16);
-  if (pairs <= 256) launch<1, 4>(p, groups, s);
-  else if (pairs <= 512) launch<2, 4>(p, groups, s);
-  else launch<4, 2>(p, groups, s);
+  if (p.jobs == 0 || p.M == 0) return hipSuccess;
+  if (const Kernel k = fastest(p); k != Kernel::kHere) return layer_gemm(p, k == Kernel::kMid ? LayerTiles::kMid : LayerTiles::kLarge, few(p), s);
+  const Instance at = instance(p);
+  const long groups = groups_of(p, at.cols);
+  if (at.cols == 16) launch<1, 4, 1>(p, groups, s);
+  else if (at.cols == 32 && at.rows == 16) launch<1, 4, 2>(p, groups, s);
+  else if (at.cols == 32) launch<2, 4, 2>(p, groups, s);
+  else if (at.rows == 16) launch<1, 4, 4>(p, groups, s);
+  else if (at.rows == 32) launch<2, 4, 4>(p, groups, s);
+  else launch<4, 2, 4>(p, groups, s);
   return hipGetLastError();
 }
 

@@ -100,8 +100,8 @@ __global__ __launch_bounds__(256) void layer_token_kernel(const LayerTokenArgs p
   if (mine) state = load_token(p, token, head, kv, q);
 
   f32x4_t acc[4][kNT], sum[4];
-  quarter_product<kNT, kChunk>(w, x, K, wave, q, acc);
-  add_quarters<kNT>(partial, acc, wave, lane, sum);
+  quarter_product<kNT, kChunk, 4>(w, x, K, wave, q, acc);
+  add_quarters<kNT, 4>(partial, acc, wave, lane, sum);
   if (mine) step_token(p, token, head, q, sum, state);
 }
 

@@ -282,3 +282,18 @@ def test_positions_move_on_with_a_projection(M, K, N):
     torch.cuda.synchronize()
     assert_product(y, x, w, None, f"M={M} K={K}")
     assert torch.equal(pos[:M], (was[:M] + 1) % 16) and pos[M] == was[M]
+
+
+# The kernel for few rows in each of its tiles (rows by columns of a workgroup): 16 x 16, 16 x 32, 32 x 32, 16 x 64, 32 x 64, 64 x 64; rows and
+# columns that end inside a tile, a result narrower than one, K that ends inside an instruction's 32 columns and with a quarter that has none.
+@pytest.mark.parametrize("M,K,columns", [(1, 8, (1,)), (17, 520, (513, 16, 7, 130)), (256, 40, (256,)), (40, 264, (1500, 37)), (100, 136, (2000,)), (13, 72, (8300,)),
+                                         (300, 64, (1000,)), (1000, 40, (999, 3))])
+def test_few_rows_against_float64(M, K, columns):
+    from spear_amd import _btp
+
+    g = torch.Generator(device=DEV).manual_seed(M + K)
+    normal = lambda *shape: torch.randn(*shape, generator=g, device=DEV).bfloat16()
+    x, weights, biases = normal(M, K + 8)[:, :K], [normal(n, K) for n in columns], [None if i % 3 == 2 else normal(n) for i, n in enumerate(columns)]
+    print(f"few rows M={M} K={K} columns={columns}", flush=True)
+    for i, y in enumerate(_btp.load_extension().linears(x, weights, biases)):
+        assert_product(y, x, weights[i], biases[i], f"M={M} K={K} projection {i}")
