@@ -61,6 +61,11 @@ int spear_layer_linear(int n, const void* x, long long ldx, int M, int K, const 
 int spear_layer_wgrad(int n, const void* const* dy, const int* ld_dy, const int* cols_dy, const int* N, const void* const* x, const int* K,
                       const int* splits, long long M, float* parts, void* stream);
 
+/* The same with results that need no parts: dw[i] NULL, or with splits[i] = 1 and K[i] below 2^21 the product itself, [N[i], K[i]] dense, rounded to bf16
+ * (8-byte aligned). Such a product takes no room in `parts`, which may be NULL if none does; spear_layer_wgrad_sums is for the others. */
+int spear_layer_wgrad_to(int n, const void* const* dy, const int* ld_dy, const int* cols_dy, const int* N, const void* const* x, const int* K,
+                         const int* splits, long long M, float* parts, void* const* dw, void* stream);
+
 /* The number of splits for one of these products that the library's model of it expects to be fastest. */
 int spear_layer_wgrad_splits(long long M, int N, int K);
 

@@ -64,7 +64,7 @@ int check_common(const char* who, int B, int H, int L, int k, int in_dtype, int 
 
 extern "C" {
 
-int spear_btp_abi_version(void) { return 26; }
+int spear_btp_abi_version(void) { return 27; }
 
 const char* spear_btp_last_error(void) { return g_error; }
 
@@ -329,10 +329,15 @@ static long long wgrad_units(int N, int K, int splits) { return (long long)((N +
 
 int spear_layer_wgrad(int n, const void* const* dy, const int* ld_dy, const int* cols_dy, const int* N, const void* const* x, const int* K,
                       const int* splits, long long M, float* parts, void* stream) {
+  return spear_layer_wgrad_to(n, dy, ld_dy, cols_dy, N, x, K, splits, M, parts, nullptr, stream);
+}
+
+int spear_layer_wgrad_to(int n, const void* const* dy, const int* ld_dy, const int* cols_dy, const int* N, const void* const* x, const int* K,
+                         const int* splits, long long M, float* parts, void* const* dw, void* stream) {
   g_error[0] = '\0';
   const char* who = "spear_layer_wgrad";
   if (n < 1 || n > 2 || M < 1 || M >= (1ll << 31)) return fail(SPEAR_BTP_EINVAL, "%s: bad shape (n=%d M=%lld)", who, n, M);
-  if (!dy || !ld_dy || !cols_dy || !N || !x || !K || !splits || !parts) return fail(SPEAR_BTP_ENULL, "%s: NULL array", who);
+  if (!dy || !ld_dy || !cols_dy || !N || !x || !K || !splits) return fail(SPEAR_BTP_ENULL, "%s: NULL array", who);
   spear_btp::LayerWgradArgs a{{}, (long)M, parts};
   long long units = 0;
   for (int i = 0; i < n; ++i) {
@@ -340,12 +345,15 @@ int spear_layer_wgrad(int n, const void* const* dy, const int* ld_dy, const int*
         ld_dy[i] >= (1 << 23) || K[i] >= (1 << 23))
       return fail(SPEAR_BTP_EINVAL, "%s: bad columns (N=%d of %d in rows of %d, K=%d)", who, N[i], cols_dy[i], ld_dy[i], K[i]);
     if (splits[i] < 1 || splits[i] > (M + 31) / 32) return fail(SPEAR_BTP_EINVAL, "%s: bad number of splits (%d)", who, splits[i]);
-    if (!dy[i] || !x[i]) return fail(SPEAR_BTP_ENULL, "%s: NULL tensor pointer", who);
+    uint16_t* const out = dw ? static_cast<uint16_t*>(dw[i]) : nullptr;
+    if (out && (splits[i] != 1 || K[i] >= (1 << 21) || (reinterpret_cast<uintptr_t>(out) & 7u)))
+      return fail(SPEAR_BTP_EINVAL, "%s: a result without parts needs one split, K below 2^21 and 8-byte alignment (splits=%d K=%d)", who, splits[i], K[i]);
+    if (!dy[i] || !x[i] || (!out && !parts)) return fail(SPEAR_BTP_ENULL, "%s: NULL tensor pointer", who);
     if (!aligned16(dy[i]) || !aligned16(x[i]) || !aligned16(parts)) return fail(SPEAR_BTP_EINVAL, "%s: tensor pointers must be 16-byte aligned", who);
     const long long u = wgrad_units(N[i], K[i], splits[i]);
     units += u;
     if (units >= (1ll << 28)) return fail(SPEAR_BTP_EINVAL, "%s: too many tiles for one launch", who);
-    a.job[i] = {static_cast<const uint16_t*>(dy[i]), static_cast<const uint16_t*>(x[i]), ld_dy[i], cols_dy[i], N[i], K[i], splits[i], (int)u};
+    a.job[i] = {static_cast<const uint16_t*>(dy[i]), static_cast<const uint16_t*>(x[i]), ld_dy[i], cols_dy[i], N[i], K[i], splits[i], (int)u, out};
   }
   const hipError_t err = spear_btp::layer_wgrad(a, static_cast<hipStream_t>(stream));
   if (err != hipSuccess) return fail(SPEAR_BTP_ELAUNCH, "%s: launch failed: %s", who, hipGetErrorString(err));

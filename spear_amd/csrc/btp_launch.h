@@ -159,12 +159,14 @@ hipError_t layer_stack(const LayerStackArgs& p, hipStream_t s);
 
 // Products over the tokens in 256 x 256 tiles and splits of the tokens (layer_wgrad.hip), bf16: dy [M, N] with rows ld_dy elements apart, of
 // which cols_dy may be read, and x [M, K] dense; ld_dy, cols_dy and K multiples of 8, 16-byte aligned. parts: fp32, one dense block of 256 x
-// 256 per unit (split-major, then x's tiles, then dy's), of the first job and then the second, in the order that layer_sums reads.
+// 256 per unit (split-major, then x's tiles, then dy's), of the first job and then the second, in the order that layer_sums reads. A job of one
+// split may have `out` instead: the result itself [N, K], rounded (8-byte aligned, K below 2^21).
 constexpr int kWgradSide = 256;
 struct LayerWgradJob {
   const uint16_t *dy, *x;
   int ld_dy, cols_dy, N, K, splits;
   int units;  // splits * ceil(N / 256) * ceil(K / 256); 0: no job
+  uint16_t* out;
 };
 struct LayerWgradArgs {
   LayerWgradJob job[2];

@@ -498,7 +498,8 @@ at::Tensor weight_grad(const at::Tensor& dy, const at::Tensor& x, int64_t s, std
   return out;
 }
 
-// Weight gradients of one backward pass through spear_layer_wgrad: products dy^T x in one launch, their sums and the bias gradients' in another.
+// Weight gradients of one backward pass through spear_layer_wgrad: products dy^T x in one launch, the sums of those cut into splits and the bias
+// gradients' in another.
 struct WeightGrads {
   std::vector<at::Tensor> dy, x, dw;  // dy [M, N or more], x [M, K], dw [N, K]
 
@@ -511,24 +512,34 @@ struct WeightGrads {
   void run(const std::vector<at::Tensor>& sums_of, const std::vector<at::Tensor>& sums) {
     const int n = (int)dy.size();
     const void *g[2], *o[2];
-    void* w[2];
-    int ld[2], N[2], K[2], splits[2];
+    void *whole[2], *w[2];
+    int ld[2], N[2], K[2], splits[2], rows_of[2], cols_of[2], splits_of[2], parted = 0;  // w and *_of: the products with parts
     const int64_t M = x[0].size(0);
     int64_t blocks = 0;
     for (int i = 0; i < n; ++i) {
       g[i] = dy[i].data_ptr();
       o[i] = x[i].data_ptr();
-      w[i] = dw[i].data_ptr();
       ld[i] = (int)dy[i].size(1);
       N[i] = (int)dw[i].size(0);
       K[i] = (int)dw[i].size(1);
       splits[i] = spear_layer_wgrad_splits(M, N[i], K[i]);
+      whole[i] = splits[i] == 1 && K[i] < 1 << 21 ? dw[i].data_ptr() : nullptr;
+      if (whole[i] != nullptr) continue;
       blocks += (int64_t)((N[i] + 255) / 256) * ((K[i] + 255) / 256) * splits[i];
+      rows_of[parted] = N[i];
+      cols_of[parted] = K[i];
+      splits_of[parted] = splits[i];
+      w[parted++] = dw[i].data_ptr();
     }
-    const at::Tensor parts = at::empty({blocks * 65536}, x[0].options().dtype(at::kFloat));
-    float* const to = static_cast<float*>(parts.data_ptr());
-    int rc = spear_layer_wgrad(n, g, ld, ld, N, o, K, splits, M, to, stream_of(x[0]));
+    at::Tensor parts;
+    if (blocks > 0) parts = at::empty({blocks * 65536}, x[0].options().dtype(at::kFloat));
+    float* const to = blocks > 0 ? static_cast<float*>(parts.data_ptr()) : nullptr;
+    int rc = spear_layer_wgrad_to(n, g, ld, ld, N, o, K, splits, M, to, whole, stream_of(x[0]));
     if (rc != 0) raise_native(rc);
+    if (parted == 0) {
+      if (!sums.empty()) layer_sums(sums_of, sums);
+      return;
+    }
     const float* in[3];
     void* out[3];
     long long rows[3], cols[3];
@@ -538,7 +549,7 @@ struct WeightGrads {
       rows[i] = sums_of[i].size(0);
       cols[i] = sums_of[i].size(1);
     }
-    rc = spear_layer_wgrad_sums(n, to, N, K, splits, w, (int)sums.size(), in, out, rows, cols, SPEAR_BTP_BF16, stream_of(x[0]));
+    rc = spear_layer_wgrad_sums(parted, to, rows_of, cols_of, splits_of, w, (int)sums.size(), in, out, rows, cols, SPEAR_BTP_BF16, stream_of(x[0]));
     if (rc != 0) raise_native(rc);
   }
 };

@@ -15,7 +15,8 @@
 //     tokens at one time, so each is fetched about once for all tiles (720 MB from memory for 537 MB of operands and 1.8 GB of requests
 //     at 131072 tokens, [1568, 512]).
 //   - Steps of 32 tokens, one phase each: five stages of 16 KiB for either operand, asked for four steps ahead.
-//   - A unit's sums are stored as they lie in the accumulators, 1 KiB per store; only layer_sums looks at their order.
+//   - A unit's sums are stored as they lie in the accumulators, 1 KiB per store; only layer_sums looks at their order. A product of one
+//     split (few tokens of a wide layer) is rounded and stored as it is: no fp32 array of its size is written and read.
 //
 // Measured at 131072 tokens, us with the sums, here / the library's batched product in slices and its sums: [1568, 512] 278 / 333, [512, 512]
 // 85 / 92, [3136, 1024] 870 / 1089, [3200, 2048] 1646 / 1756, [2048, 2048] 930 / 993, [784, 256] 82 / 92; 65536 tokens [1813, 592] 209 /
@@ -55,7 +56,7 @@ __device__ __forceinline__ Unit unit_at(const LayerWgradArgs& p, const Share& sh
   // the splits differ by a step at most: the first `more` have one more
   const unsigned all = (unsigned)((p.M + kTokens - 1) / kTokens), least = all / (unsigned)job.splits, more = all - least * (unsigned)job.splits;
   return {j, (int)(tile - kt * tiles_n) * kSide, (int)kt * kSide, (int)(split * least + min(split, more)), (int)(least + (split < more ? 1 : 0)),
-          (int)u + (j ? p.job[0].units : 0)};
+          (int)u + (j && p.job[0].out == nullptr ? p.job[0].units : 0)};
 }
 
 // Fragments of 32 tokens: `a` .. `d` are the lane's addresses of four column tiles, 4 tokens further 2 KiB on. The waits are part of the
@@ -229,11 +230,27 @@ __global__ __launch_bounds__(512) void layer_wgrad_kernel(const LayerWgradArgs p
       phase_barrier();
     } while (++t < cur.steps);
 
-    float* const part = p.parts + ((long)cur.part * 8 + wave) * (8 * 4 * 64 * 4) + lane * 4;
+    if (job.out != nullptr) {
+      // The same number of stores, 8 bytes per lane: columns 4 q .. + 3 of x's tile j, row i16 of dy's tile i
+      const int rows = min(kSide, job.N - cur.n0), cols = min(kSide, job.K - cur.k0);
+      const auto desc = buffer_of(job.out + (long)cur.n0 * job.K + cur.k0, ((rows - 1) * job.K + cols) * 2);
 #pragma unroll
-    for (int i = 0; i < 8; ++i)
+      for (int j = 0; j < 4; ++j) {
+        const int c = 16 * (x_tile + j) + 4 * q;
+        const uint32_t at = c < cols && (full || j < 2) ? (uint32_t)((128 * wm + i16) * job.K + c) * 2 : kNowhere;
 #pragma unroll
-      for (int j = 0; j < 4; ++j) __builtin_nontemporal_store(acc[i][j], reinterpret_cast<f32x4_t*>(part + (i * 4 + j) * 256));
+        for (int i = 0; i < 8; ++i) {
+          const u32x2_t d = {Bf16::pack2(acc[i][j][0], acc[i][j][1]), Bf16::pack2(acc[i][j][2], acc[i][j][3])};
+          __builtin_amdgcn_raw_buffer_store_b64(d, desc, at + (uint32_t)(16 * i * job.K * 2), 0, 0);
+        }
+      }
+    } else {
+      float* const part = p.parts + ((long)cur.part * 8 + wave) * (8 * 4 * 64 * 4) + lane * 4;
+#pragma unroll
+      for (int i = 0; i < 8; ++i)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) __builtin_nontemporal_store(acc[i][j], reinterpret_cast<f32x4_t*>(part + (i * 4 + j) * 256));
+    }
     if (id + slots >= last) break;
     id += slots;
     cur = unit_at(p, share, id);

@@ -297,3 +297,56 @@ def test_few_rows_against_float64(M, K, columns):
     print(f"few rows M={M} K={K} columns={columns}", flush=True)
     for i, y in enumerate(_btp.load_extension().linears(x, weights, biases)):
         assert_product(y, x, weights[i], biases[i], f"M={M} K={K} projection {i}")
+
+
+# Products of one split, which are rounded where they are made: alone, beside one with parts in either place; results narrower than a half tile, that
+# end inside one, and several units per workgroup.
+@pytest.mark.parametrize("M,products,splits", [(1, [(8, 8, 8)], [1]), (33, [(300, 304, 136), (40, 64, 72)], [1, 1]), (1000, [(1813, 1856, 592), (592, 592, 592)], [1, 3]),
+                                               (97, [(257, 264, 264), (1040, 1040, 520)], [3, 1]), (64, [(6272, 6272, 2048), (2048, 2048, 2048)], [1, 1])])
+def test_weight_gradients_of_one_split_against_float64(M, products, splits):
+    import ctypes
+
+    from spear_amd import _btp
+
+    lib, n = _btp.load_library(), len(products)
+    g = torch.Generator(device=DEV).manual_seed(M)
+    dys = [torch.randn(M, ld, generator=g, device=DEV).bfloat16() for _, ld, _ in products]
+    xs = [torch.randn(M, K, generator=g, device=DEV).bfloat16() for _, _, K in products]
+    dws = [torch.full((N + 1, K), 7.0, device=DEV).bfloat16() for N, _, K in products]
+    parted = [i for i in range(n) if splits[i] > 1]
+    units = sum(-(-products[i][0] // 256) * -(-products[i][2] // 256) * splits[i] for i in parted)
+    parts = torch.full((units * 65536,), float("nan"), device=DEV)
+    print(f"weight gradients without parts M={M} {products} splits={splits}", flush=True)
+    ints = lambda values: (ctypes.c_int * len(values))(*values)
+    of = lambda ts: (ctypes.c_void_p * len(ts))(*(t.data_ptr() for t in ts))
+    whole = (ctypes.c_void_p * n)(*(dw.data_ptr() if s == 1 else None for dw, s in zip(dws, splits)))
+    lds, Ns, Ks = (ints([p[k] for p in products]) for k in (1, 0, 2))
+    stream = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    assert lib.spear_layer_wgrad_to(n, of(dys), lds, lds, Ns, of(xs), Ks, ints(splits), ctypes.c_longlong(M), ctypes.c_void_p(parts.data_ptr() if parted else None),
+                                    whole, stream) == 0
+    if parted:
+        pick = lambda k: ints([products[i][k] for i in parted])
+        assert lib.spear_layer_wgrad_sums(len(parted), ctypes.c_void_p(parts.data_ptr()), pick(0), pick(2), ints([splits[i] for i in parted]), of([dws[i] for i in parted]),
+                                          0, None, None, None, None, _btp._BF16, stream) == 0
+    torch.cuda.synchronize()
+    for dy, x, dw, (N, _, K) in zip(dys, xs, dws, products):
+        assert_product(dw[:N], dy[:, :N].t(), x.t(), None, f"M={M} [{N}, {K}]")
+        assert (dw[N] == 7).all()
+
+
+def test_backward_of_few_tokens_of_a_wide_layer_needs_little_room():
+    """No fp32 array of the size of the weight gradients: beside what is left afterwards, the transposed weights and arrays of the tokens."""
+    from spear_amd import Phalanx
+
+    torch.manual_seed(0)
+    layer = Phalanx(dim=2048, length=64, method="fused", dtype=torch.bfloat16).to(DEV)
+    x = torch.randn(1, 64, 2048, device=DEV).bfloat16()
+    layer(x).backward(x)
+    layer.zero_grad(set_to_none=True)
+    y = layer(x)
+    torch.cuda.synchronize()
+    torch.cuda.reset_peak_memory_stats()
+    y.backward(x)
+    torch.cuda.synchronize()
+    weights = sum(p.numel() * p.element_size() for p in layer.parameters())
+    assert torch.cuda.max_memory_allocated() - torch.cuda.memory_allocated() < 1.25 * weights
