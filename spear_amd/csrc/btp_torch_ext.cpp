@@ -557,8 +557,17 @@ struct WeightGrads {
 // Whether the weight gradients of a layer's backward are faster through spear_layer_wgrad than as the library's (sliced) products: up to
 // 32768 tokens, and above from 12 G multiply-adds on. Times of single products at layer_wgrad.hip. A whole step, us (and on the GPU alone),
 // with them here / the library's: 1024 tokens, width 512 124 (86) / 169 (86), 4096 tokens 257 (116) / 291 (134), 1024 tokens, width 1024 259
-// (129) / 298 (130), 131072 tokens, width 128 287 / 280.
+// (129) / 298 (130), 131072 tokens, width 128 287 / 280. Up to 1024 tokens they are the slower ones on the GPU (both of a layer at width 512 16 / 9
+// us, 1024 16 / 11, 2048 27 / 19 at 64 tokens, 24 / 23, 33 / 28, 65 / 52 at 1024) and save the host 30 us, which bounds such a step.
 bool own_weight_grads(int64_t M, int64_t multiply_adds_per_token) { return M <= 32768 || M * multiply_adds_per_token >= 12000000000; }
+
+// Few tokens of a very wide layer, whose step the GPU bounds: there the library's products are the faster ones for all gradients; it takes the
+// weights as they lie, and transposing them reads and writes each once more. A step, us, with the library's / here:
+// 68 M weights (width 4096, kv heads its own) 64 tokens 299 / 309, 256 304 / 394, 512 400 / 489, 1024 550 / 595, 2048 880 / 966, 4096 1489 / 1478;
+// 43 M (width 4096, shared by four) 128 tokens 241 / 216, 256 238 / 252, 512 252 / 288, 2048 553 / 598, 4096 974 / 945; 38 M (width 3072) 128 tokens 307 / 213, 512
+// 305 / 314, 1024 397 / 373, 2048 577 / 609; 17 M (width 2048) 512 tokens 227 / 181, 1024 229 / 227; 270 M (width 8192) 64 tokens 720 / 1037, 2048 2860 / 2972. In a
+// graph the library's would be the faster ones in narrower layers too (17 M weights, 512 tokens 152 / 181; 38 M, 256 216 / 250).
+bool few_tokens_of_many_weights(int64_t M, int64_t weights) { return M <= 2048 && (weights >= 60000000 || (weights >= 40000000 && M >= 256)); }
 
 // A whole layer call on plain bf16 tensors: the four input projections, the mixing stage and the output projection, with one
 // autograd node. Backward is what spear_amd/nn/phalanx/projections.py does with _ProjectAndMix and _Linear (one product each for the
@@ -614,7 +623,8 @@ struct LayerNode : public torch::autograd::Function<LayerNode> {
       front = front || ctx->needs_input_grad(i);
       weights = weights || ((i == 1 || i == 3 || i == 5 || i == 7) && ctx->needs_input_grad(i));
     }
-    const bool own_weights = own_weight_grads(M, (ctx->needs_input_grad(8) ? K * F : 0) + (weights ? (2 * Fkv + F + heads) * K : 0));
+    const bool library = few_tokens_of_many_weights(M, (2 * Fkv + 2 * F + heads) * K);
+    const bool own_weights = !library && own_weight_grads(M, (ctx->needs_input_grad(8) ? K * F : 0) + (weights ? (2 * Fkv + F + heads) * K : 0));
     WeightGrads grads;
     if (ctx->needs_input_grad(8)) {
       if (own_weights && (reinterpret_cast<uintptr_t>(dy.data_ptr()) & 15u) == 0) {
@@ -630,13 +640,13 @@ struct LayerNode : public torch::autograd::Function<LayerNode> {
     if (front) {
       const int64_t used = 2 * Fkv + F + heads, ld = (used + 63) / 64 * 64;  // [b | c | v | a | padding]
       // Input gradients against the weights transposed, through spear_layer_linear; as the library's products with the weights as they lie
-      // only for a gradient off the 16-byte grid and for many tokens of a narrow layer. Measured, us, spear_layer_linear / the library: proj_out's at K=512 131072 rows 75 / 91,
+      // only for a gradient off the 16-byte grid, for few tokens of a very wide layer and for many of a narrow one. Measured, us, spear_layer_linear / the library: proj_out's at K=512 131072 rows 75 / 91,
       // 8192 rows 9 / 12, 1024 rows 6.1 / 7.2, K=1024 131072 rows 251 / 268, 1024 rows 11.2 / 9.7, K=2048 65536 rows 453 / 470, 2048 rows 22 /
       // 26; that of the four input projections at K=512 131072 rows 198 / 208, 1024 rows 14 / 11, K=1024 131072 rows 663 / 697, 4096 rows 30 /
       // 35, 1024 rows 27 / 22, K=2048 65536 rows 1213 / 1299, 1024 rows 51 / 49. The transposing launch takes 3 to 6 us, half of
       // which layer_stack took too. Where it is the slower one on the GPU the host's 15 us per library product count for more.
       // Up to K = 64 (see own_products) a step of 131072 tokens takes 324 / 260 us at K=32 and 335 / 285 at K=48, of 8192 tokens 220 / 253.
-      const bool own = K % 8 == 0 && (K > 64 || M <= 32768) && (reinterpret_cast<uintptr_t>(dy.data_ptr()) & 15u) == 0;
+      const bool own = !library && K % 8 == 0 && (K > 64 || M <= 32768) && (reinterpret_cast<uintptr_t>(dy.data_ptr()) & 15u) == 0;
       const at::Tensor packed = at::empty({B, L, ld}, v.options());
       const at::Tensor stacked = own ? at::empty({K, ld}, v.options()) : at::empty({ld, K}, v.options());
       at::Tensor dmixed;

@@ -347,7 +347,8 @@ def test_calls_that_stay_with_the_stand_alone_kernels():
         layer(x[:, :17])
 
 
-@pytest.mark.parametrize("B,L,dim,kv_heads", [(2, 16, 16, 1), (3, 48, 80, None), (8, 128, 96, 2), (64, 128, 256, 4)])
+# The last one: few tokens of many weights, whose gradients are the library's products.
+@pytest.mark.parametrize("B,L,dim,kv_heads", [(2, 16, 16, 1), (3, 48, 80, None), (8, 128, 96, 2), (64, 128, 256, 4), (1, 48, 4096, None)])
 def test_layer_node_against_separate_modules(B, L, dim, kv_heads):
     """Every gradient of the one-node layer against the modules' own autograd (a hook keeps them separate), for every subset of
     frozen tensors that changes what backward computes; padding columns of the packed gradients at odd head counts included."""
