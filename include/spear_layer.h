@@ -53,6 +53,10 @@ int spear_layer_transpose(const void* w_a, const void* w_b, const void* w_c, con
 int spear_layer_linear(int n, const void* x, long long ldx, int M, int K, const void* const* w, const void* const* bias,
                        void* const* out, const int* N, int* pos, int block_len, void* stream);
 
+/* Which of its kernels spear_layer_linear takes for such a call (without positions): 0 the one for few rows, 1 tiles of 128 x 128, 2 of 256 x 256;
+ * -1 for a shape that it refuses. */
+int spear_layer_linear_choice(int n, long long ldx, int M, int K, const int* N);
+
 /* n (1 .. 2) products over M tokens, bf16, as fp32 parts:  dy[i]^T x[i], [N[i], K[i]], cut into splits[i] runs of tokens.
  *     dy[i] [M, N[i]], rows ld_dy[i] elements apart, cols_dy[i] >= N[i] of which may be read       x[i] [M, K[i]] dense
  *     parts  fp32, 65536 * sum of splits[i] ceil(N[i] / 256) ceil(K[i] / 256) elements; written in the order that

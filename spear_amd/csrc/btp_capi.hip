@@ -64,7 +64,7 @@ int check_common(const char* who, int B, int H, int L, int k, int in_dtype, int 
 
 extern "C" {
 
-int spear_btp_abi_version(void) { return 27; }
+int spear_btp_abi_version(void) { return 28; }
 
 const char* spear_btp_last_error(void) { return g_error; }
 
@@ -323,6 +323,16 @@ int spear_layer_linear(int n, const void* x, long long ldx, int M, int K, const 
   const hipError_t err = spear_btp::layer_linear(a, static_cast<hipStream_t>(stream));
   if (err != hipSuccess) return fail(SPEAR_BTP_ELAUNCH, "%s: launch failed: %s", who, hipGetErrorString(err));
   return 0;
+}
+
+int spear_layer_linear_choice(int n, long long ldx, int M, int K, const int* N) {
+  if (n < 1 || n > 4 || M <= 0 || K <= 0 || K % 8 != 0 || ldx < K || ldx % 8 != 0 || !N) return -1;
+  spear_btp::LayerLinearArgs a{nullptr, (long)ldx, M, K, n, {}, {}, {}, {}, nullptr, 0};
+  for (int i = 0; i < n; ++i) {
+    if (N[i] <= 0) return -1;
+    a.N[i] = N[i];
+  }
+  return spear_btp::layer_linear_choice(a);
 }
 
 static long long wgrad_units(int N, int K, int splits) { return (long long)((N + 255) / 256) * ((K + 255) / 256) * splits; }

@@ -134,6 +134,7 @@ struct LayerLinearArgs {
   int block_len;
 };
 hipError_t layer_linear(const LayerLinearArgs& p, hipStream_t s);
+int layer_linear_choice(const LayerLinearArgs& p);  // its kernel: 0 for few rows, 1 tiles of 128 x 128, 2 of 256 x 256
 // The same at large sizes (layer_gemm.hip), for the operands that layer_gemm_takes: K past 64. Only kMid moves positions.
 bool layer_gemm_takes(const LayerLinearArgs& p);
 enum class LayerTiles { kMid, kLarge };  // 128 x 128, 256 x 256

@@ -128,6 +128,8 @@ static bool few(const LayerLinearArgs& p) {
   return p.jobs > 1 ? p.M * columns * p.K <= 1600000000 : p.K <= 512 && p.M * columns * p.K <= 300000000;
 }
 
+int layer_linear_choice(const LayerLinearArgs& p) { return (int)fastest(p); }
+
 hipError_t layer_linear(const LayerLinearArgs& p, hipStream_t s) {
   if (p.jobs == 0 || p.M == 0) return hipSuccess;
   if (const Kernel k = fastest(p); k != Kernel::kHere) return layer_gemm(p, k == Kernel::kMid ? LayerTiles::kMid : LayerTiles::kLarge, few(p), s);

@@ -294,7 +294,7 @@ def test_qkv_form_backward_against_the_oracle(H, Hkv):
 @pytest.mark.parametrize("B,L,dim,kv_heads", [(1, 16, 16, None), (3, 48, 96, 2), (8, 128, 512, None), (64, 144, 80, 1)])
 def test_default_layer_mixes_in_the_fused_kernels(B, L, dim, kv_heads):
     """A plain bf16 call of a default layer lies as close to the fused layer and to the stand-alone composition as their bf16
-    roundings allow, below and above the 8192 tokens from which the weight gradients are cut into slices."""
+    roundings allow, with weight gradients in one split and in several."""
     from spear_amd import Phalanx, btp
 
     torch.manual_seed(11)
@@ -347,8 +347,10 @@ def test_calls_that_stay_with_the_stand_alone_kernels():
         layer(x[:, :17])
 
 
-# The last one: few tokens of many weights, whose gradients are the library's products.
-@pytest.mark.parametrize("B,L,dim,kv_heads", [(2, 16, 16, 1), (3, 48, 80, None), (8, 128, 96, 2), (64, 128, 256, 4), (1, 48, 4096, None)])
+# The last ones: few tokens of many weights, whose gradients are the library's products; past 32768 tokens a narrow layer, whose weight gradients are the
+# library's in slices, and one of dim 64, whose input gradients are too; products in 256 x 256 tiles; the front's projections by the library.
+@pytest.mark.parametrize("B,L,dim,kv_heads", [(2, 16, 16, 1), (3, 48, 80, None), (8, 128, 96, 2), (64, 128, 256, 4), (1, 48, 4096, None), (264, 128, 128, 2),
+                                              (264, 128, 64, None), (256, 128, 512, None), (93, 128, 1024, None)])
 def test_layer_node_against_separate_modules(B, L, dim, kv_heads):
     """Every gradient of the one-node layer against the modules' own autograd (a hook keeps them separate), for every subset of
     frozen tensors that changes what backward computes; padding columns of the packed gradients at odd head counts included."""

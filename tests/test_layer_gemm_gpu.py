@@ -1,5 +1,5 @@
-"""The layer's projections at sizes of the large-tile kernel (spear_layer_linear on many rows): up to four of them on the same rows,
-against float64 products of the same bf16 operands, at the edges of its 256 x 256 x 64 tiles."""
+"""The layer's projections through spear_layer_linear, up to four of them on the same rows, its weight gradients and a decode token's projections in tiles,
+against float64 products of the same bf16 operands at the edges of the kernels' tiles."""
 
 import pytest
 import torch
@@ -21,29 +21,49 @@ def assert_product(got, x, w, bias, label):
     assert over.max().item() <= 0, f"{label}: {over.max().item():.3e} over the bound"
 
 
-# M, K, columns of the projections (bias on all but every third). The rows make the tiles the faster choice, of 256 x 256 first: remainders of 256 rows and
-# columns, of 64 columns of K, widths of 128 and less (half tiles), not a multiple of 8 (element stores), several tiles per workgroup and
-# more than one group of row panels, two steps of K.
+def kernel_of(M, K, columns, extra=0):
+    """Which kernel spear_layer_linear takes: 0 for few rows, 1 tiles of 128 x 128, 2 of 256 x 256."""
+    import ctypes
+
+    from spear_amd import _btp
+
+    return _btp.load_library().spear_layer_linear_choice(len(columns), ctypes.c_longlong(K + extra), M, K, (ctypes.c_int * len(columns))(*columns))
+
+
+# Kernel, M, K, columns of the projections (bias on all but every third). Remainders of rows, of columns, of 64 columns of K; widths of 128 and
+# less (half of the larger tiles) and not a multiple of 8 (element stores).
 SHAPES = [
-    (4099, 520, (592, 592, 257, 37)),
-    (4096, 512, (512, 512, 512, 32)),
-    (2305, 1032, (1040, 129, 128, 127)),
-    (16400, 136, (256, 272, 16, 5)),
-    (20000, 72, (1024, 130)),
-    (9000, 1000, (640,)),
-    (8192, 2048, (2048, 512, 512, 128)),
-    # 128 x 128 tiles, fewer and more of them than compute units
-    (1003, 592, (592, 592, 592, 37)),
-    (129, 1000, (1040, 130, 129, 24)),
-    (2048, 72, (1024, 1024, 1024, 64)),
-    (2049, 1032, (1032, 1040, 1041, 5)),
+    # 256 x 256 tiles, several per workgroup, ending in another projection and in the last rows; results stored at once (K up to 1024) or not; two
+    # and three steps of K, so that the requests of one tile reach into the next
+    (2, 33027, 520, (592, 592, 257, 37)),
+    (2, 33027, 1032, (1040, 129, 128, 127)),
+    (2, 131077, 72, (1024, 130)),
+    (2, 40007, 1000, (640,)),
+    (2, 65541, 136, (1024, 130)),
+    (2, 50000, 328, (256, 272, 16, 5)),
+    (2, 16500, 1288, (520, 24, 136)),
+    (2, 8192, 2048, (2048, 512, 512, 128)),
+    # 128 x 128 tiles, more and fewer of them than compute units, in one chain over K and in quarters
+    (1, 4099, 520, (592, 592, 257, 37)),
+    (1, 4096, 512, (512, 512, 512, 32)),
+    (1, 2305, 1032, (1040, 129, 128, 127)),
+    (1, 16400, 136, (256, 272, 16, 5)),
+    (1, 20000, 72, (1024, 130)),
+    (1, 9000, 1000, (640,)),
+    (1, 1003, 592, (592, 592, 592, 37)),
+    (1, 700, 1000, (1040, 130, 129, 24)),
+    (1, 2048, 72, (1024, 1024, 1024, 64)),
+    (1, 2049, 1032, (1032, 1040, 1041, 5)),
+    (0, 129, 1000, (1040, 130, 129, 24)),
 ]
 
 
-@pytest.mark.parametrize("M,K,columns", SHAPES)
+@pytest.mark.parametrize("kernel,M,K,columns", SHAPES)
 @pytest.mark.parametrize("extra", [0, 24], ids=["dense", "strided"])
-def test_large_projections_against_float64(M, K, columns, extra):
+def test_large_projections_against_float64(kernel, M, K, columns, extra):
     from spear_amd import _btp
+
+    assert kernel_of(M, K, columns, extra) == kernel
 
     g = torch.Generator(device=DEV).manual_seed(M + K + extra)
 
@@ -59,11 +79,13 @@ def test_large_projections_against_float64(M, K, columns, extra):
         assert_product(y, x, w, b, f"M={M} K={K} projection {i} of {len(columns)}")
 
 
-def test_large_projections_keep_rows_apart():
+@pytest.mark.parametrize("kernel,M", [(1, 4096), (2, 33028)])
+def test_large_projections_keep_rows_apart(kernel, M):
     """What lies beside a row (the next row's first columns, read with a step that K does not fill) must not reach its result."""
     from spear_amd import _btp
 
-    M, K, N = 4096, 520, 1040
+    K, N = 520, 1040
+    assert kernel_of(M, K, [N]) == kernel
     x = torch.randn(M, K, device=DEV).bfloat16()
     x[1::2] = float("nan")
     w = torch.randn(N, K, device=DEV).bfloat16()
@@ -72,10 +94,12 @@ def test_large_projections_keep_rows_apart():
     assert torch.isfinite(y[::2]).all() and torch.isnan(y[1::2]).all()
 
 
-def test_large_projections_in_a_graph_follow_their_inputs():
+@pytest.mark.parametrize("kernel,M", [(1, 4096), (2, 32768)])
+def test_large_projections_in_a_graph_follow_their_inputs(kernel, M):
     from spear_amd import _btp
 
-    M, K, N = 4096, 512, 1024
+    K, N = 512, 1024
+    assert kernel_of(M, K, [N, N]) == kernel
     x, w = torch.randn(M, K, device=DEV).bfloat16(), torch.randn(N, K, device=DEV).bfloat16()
     run = lambda: _btp.load_extension().linears(x, [w, w], [None, None])
     run()
@@ -247,10 +271,12 @@ def test_a_token_is_the_same_whatever_number_comes_with_it(B, H, Hkv, K):
 
 
 # Sizes that 128 x 128 tiles take up to which K is added up in quarters: quarters that end inside a step of 64 columns, and of one instruction.
-@pytest.mark.parametrize("M,K,columns", [(1024, 512, (512, 512, 512, 32)), (1003, 592, (592, 592, 257, 37)), (600, 1040, (1040, 130, 129, 24)), (1500, 72, (1024, 130))])
+@pytest.mark.parametrize("M,K,columns", [(1024, 512, (512, 512, 512, 32)), (1003, 592, (592, 592, 257, 37)), (700, 1040, (1040, 130, 129, 24)), (1500, 72, (1024, 130))])
 def test_a_row_is_the_same_whatever_number_comes_with_it(M, K, columns):
     """The tiles add up a row's products as the kernel for few rows does: the results are equal."""
     from spear_amd import _btp
+
+    assert (kernel_of(M, K, columns), kernel_of(16, K, columns)) == (1, 0)
 
     g = torch.Generator(device=DEV).manual_seed(M)
     normal = lambda *shape: torch.randn(*shape, generator=g, device=DEV).bfloat16()

@@ -244,9 +244,9 @@ def test_prefill_of_any_length_is_one_launch_with_the_state_that_stepping_reache
         assert torch.equal(got, ref), name
 
 
-# (B, H, kv heads): one to four token tiles per wavefront, tiles and head groups that are not full, K = 16 H that ends inside
+# (B, H, kv heads): one, two and four token tiles per wavefront and the tile kernel, tiles and head groups that are not full, K = 16 H that ends inside
 # a matrix instruction's 32 columns and inside a chunk of loads
-@pytest.mark.parametrize("B,H,Hkv", [(1, 1, 1), (16, 3, 1), (17, 5, 5), (33, 32, 8), (1024, 17, 17), (700, 33, 11), (1000, 72, 9)])
+@pytest.mark.parametrize("B,H,Hkv", [(1, 1, 1), (16, 3, 1), (17, 5, 5), (33, 32, 8), (200, 24, 8), (1024, 17, 17), (700, 33, 11), (1000, 72, 9)])
 def test_layer_token_kernel_against_the_oracle(B, H, Hkv):
     from spear_amd import _btp
 
