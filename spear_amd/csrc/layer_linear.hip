@@ -102,7 +102,7 @@ Instance instance(const LayerLinearArgs& p) {
 
 // Which kernel is the fastest, by their times in us as fitted to 56 shapes (dim 128 to 2048, 256 to 16384 rows) for the tiles: of 128 x 128, 0.47 us per
 // 64 columns of K while each compute unit has one, twice that for two; of 256 x 256, 1 us. Four projections, dim = K, here / 128 / 256: K=128
-// 1024 rows 5.0 / 5.2 / 9.1, 8192 rows 12.5 / 6.1 / 9.9; K=512 256 rows 5.7 / 7.9 / 16.2, 1024 rows 11.9 / 8.3 / 16.8, 8192 rows 56 / 21 / 19; K=1024 256 rows
+// 1024 rows 5.0 / 5.2 / 9.1, 8192 rows 12.5 / 6.1 / 9.9; K=512 256 rows 5.7 / 7.9 / 16.2, 1024 rows 11.9 / 8.6 / 16.8, 8192 rows 56 / 21 / 19; K=1024 256 rows
 // 10.7 / 11.6 / 24, 2048 rows 61 / 20 / 28, 4096 rows 106 / 36 / 29; K=2048 128 rows 17.7 / 18.6, 1024 rows 111 / 34 / 46; K=4096 1 row 18.6 / 36, 128 rows 60 / 33.
 enum class Kernel { kHere, kMid, kLarge };
 

@@ -57,20 +57,15 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t buffer_of(const void* p, int b
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, max(bytes, 0), 0x00020000);
 }
 
-// 16 bytes per lane from `offset` (the lane's own, checked against the buffer's size) + `further` (the same in all lanes, not checked) to
-// `to` + 16 lane; `to` is the same in all lanes. Counted by wait_vm.
-__device__ __forceinline__ void load_to_lds(__amdgpu_buffer_rsrc_t from, char* to, uint32_t offset, int further = 0) {
-  __builtin_amdgcn_raw_ptr_buffer_load_lds(from, (lds_void_t*)to, 16, offset, further, 0, 0);
-}
-
 // The same descriptor as four words, for asm.
 __device__ __forceinline__ i32x4_t words_of(const void* p, int bytes) {
   const uint64_t a = reinterpret_cast<uint64_t>(p);
   return i32x4_t{(int)(uint32_t)a, (int)(uint32_t)(a >> 32 & 0xffff), max(bytes, 0), 0x00020000};
 }
 
-// Four requests of load_to_lds inside an asm block: 1 KiB apart from LDS address `lds` on (sgpr), the lane's offsets in o0 .. o3, descriptor
-// `desc`, `further` (sgpr). A write of m0 has to be one instruction ahead of its use.
+// Four requests inside an asm block, counted by wait_vm: 16 bytes per lane from the buffer of `desc` at the lane's offset (o0 .. o3, checked against the
+// buffer's size) + `further` (sgpr, not checked) to 16 lane past LDS addresses 1 KiB apart from `lds` on (sgpr). A write of m0 has to be one
+// instruction ahead of its use.
 #define SPEAR_REQUEST4(lds, o0, o1, o2, o3, desc, further)                                            \
   "s_mov_b32 m0, " lds "\n s_nop 0\n buffer_load_dwordx4 " o0 ", " desc ", " further " offen lds\n"    \
   "s_add_u32 m0, " lds ", 0x400\n s_nop 0\n buffer_load_dwordx4 " o1 ", " desc ", " further " offen lds\n" \

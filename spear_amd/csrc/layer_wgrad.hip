@@ -16,11 +16,13 @@
 //     at 131072 tokens, [1568, 512]).
 //   - Steps of 32 tokens, one phase each: five stages of 16 KiB for either operand, asked for four steps ahead.
 //   - A unit's sums are stored as they lie in the accumulators, 1 KiB per store; only layer_sums looks at their order. A product of one
-//     split (few tokens of a wide layer) is rounded and stored as it is: no fp32 array of its size is written and read.
+//     split (few tokens of a wide layer) is rounded and stored as it is: no fp32 array of its size is written and read (both of a layer at
+//     512 tokens, dim 4096: a step of 487 us in place of 524).
 //
-// Measured at 131072 tokens, us with the sums, here / the library's batched product in slices and its sums: [1568, 512] 278 / 333, [512, 512]
-// 85 / 92, [3136, 1024] 870 / 1089, [3200, 2048] 1646 / 1756, [2048, 2048] 930 / 993, [784, 256] 82 / 92; 65536 tokens [1813, 592] 209 /
-// 239; 16384 tokens [1568, 512] 52 / 60, [512, 512] 29 / 24. The matrix units are busy 0.55 (K=512, at 2.7 TB/s from memory beside the
+// Measured at 131072 tokens, us with the sums, here / the library's batched product in slices and its sums: [1568, 512] 238 / 281, [512, 512]
+// 85 / 93, both 308 / 370, [3136, 1024] 797 / 1064, [3200, 2048] 1536 / 1783, [2048, 2048] 876 / 966, [784, 256] 83 / 90; 65536 tokens [1813, 592]
+// 175 / 218; 16384 tokens [1568, 512] 49 / 57, [512, 512] 31 / 24; one split: 512 tokens [1568, 512] 23 / 9, [6272, 2048] 27 / 24, 4096 tokens
+// [6400, 4096] 209 / 217. The matrix units are busy 0.55 (K=512, at 2.7 TB/s from memory beside the
 // parts) to 0.59 of the time and the chip's clock falls to 2.0 GHz: power and the reads of far tokens bound it. With the addresses of a
 // step computed anew per request the same ring took 334 us at [1568, 512].
 #include <hip/hip_runtime.h>
@@ -61,7 +63,7 @@ __device__ __forceinline__ Unit unit_at(const LayerWgradArgs& p, const Share& sh
 
 // Fragments of 32 tokens: `a` .. `d` are the lane's addresses of four column tiles, 4 tokens further 2 KiB on. The waits are part of the
 // blocks: the registers are written when they end.
-// Between the reads and their wait two requests (load_to_lds): `at` are the lane's offsets, `of` the descriptor, `to` the LDS address.
+// Between the reads and their wait two requests (SPEAR_REQUEST2): `at` are the lane's offsets, `of` the descriptor, `to` the LDS address.
 __device__ __forceinline__ void read_tiles(uint32_t a, uint32_t b, uint32_t c, uint32_t d, u32x2_t (&f)[4][2], const uint32_t (&at)[2], i32x4_t of,
                                            uint32_t to) {
   asm volatile(

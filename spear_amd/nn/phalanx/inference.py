@@ -318,8 +318,8 @@ def _layer_operands(layer, x: torch.Tensor):
 def _token_operands(layer, x: torch.Tensor):
     """Weights and biases for the compiled step, whose first kernel runs the input projections and the step, or None where the
     call is for the general path: what ``plain_operands`` leaves to the modules, rows that 16-byte accesses do not fit or that overlap, and sizes
-    from which the library's products are faster on the GPU: a limit for steps in a graph. Us, here / modules: B=1024 with 65 heads 47 / 78,
-    96 heads 53 / 67 (kv heads shared by four 53 / 57), 700 with 100 heads 56 / 67, 8192 with 32 heads 61 / 64 (shared 61 / 58), past the line
+    from which the library's products are faster on the GPU: a limit for steps in a graph. Us, here / modules: B=1024 with 65 heads 46 / 78,
+    96 heads 53 / 66 (kv heads shared by four 53 / 57), 700 with 100 heads 55 / 66, 8192 with 32 heads 61 / 63 (shared 61 / 58), past the line
     1024 with 128 heads 79 / 80 (shared 78 / 67), 4096 with 64 heads 86 / 79. As a call, host included, the modules take 135."""
     if x.dim() != 2 or x.shape[0] == 0 or x.stride(1) != 1 or x.stride(0) % 8 != 0 or x.data_ptr() % 16 != 0:
         return None
