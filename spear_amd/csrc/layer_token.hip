@@ -234,9 +234,9 @@ void launch(const LayerTokenArgs& p, hipStream_t s) {
 
 }  // namespace
 
-// Whether the tile kernel takes less time than four token tiles per wavefront, past 512 pairs. Both as fitted to 51 shapes (1 to 256 heads,
-// 40 to 20000 tokens): tiles in rounds of 256 workgroups, longer with K; the other in proportion to its workgroups and K. Four token tiles /
-// the tile kernel, us: 1 head B=20000 4.0 / 7.2, 3 heads B=4096 4.3 / 5.0, 8 heads B=2048 5.7 / 5.4, B=20000 28.4 / 24.3, 9 heads B=5000 8.9 / 10.8,
+// Whether the tile kernel takes less time than four token tiles per wavefront, past 512 pairs. Both as fitted to 67 shapes (1 to 256 heads,
+// 40 to 20000 tokens): tiles in rounds of 256 workgroups, longer with K; the other in proportion to its workgroups and K, a tenth more past 256 where
+// four divides the heads (20 heads B=2000 14.3 / 11.7, 13 heads B=2500 8.4 / 10.3 in one chain over K). Four token tiles / the tile kernel, us: 1 head B=20000 4.0 / 7.2, 3 heads B=4096 4.3 / 5.0, 8 heads B=2048 5.7 / 5.4, B=20000 28.4 / 24.3, 9 heads B=5000 8.9 / 10.8,
 // 16 heads B=1024 6.1 / 6.6, B=1500 8.0 / 6.8, 32 heads B=512 7.9 / 7.9, B=1024 11.8 / 8.2, 37 heads B=300 6.7 / 8.3, B=500 9.7 / 8.7, 64 heads
 // B=200 10.8 / 10.6, B=1024 32 / 20, 128 heads B=1024 110 / 60.
 static bool tiles_win(const LayerTokenArgs& p) {
@@ -244,7 +244,9 @@ static bool tiles_win(const LayerTokenArgs& p) {
   if (32l * p.H * p.K >= 1l << 30 || 2l * kTokenRows * p.ldx >= 1l << 30) return false;
   const long row_tiles = (p.B + kTokenRows - 1) / kTokenRows, rounds = ((p.H + 1) / 2 * row_tiles + 255) / 256;
   const double tiles = 1.0 + (double)rounds * (4.2 + 0.36 * ((p.K + kRowsStep - 1) / kRowsStep));
-  return tiles < 3.5 + (1.6 + 0.0059 * p.K) * (double)(p.H * row_tiles) / 256;
+  const long others = p.H * row_tiles;
+  const double four = 3.5 + (1.6 + 0.0059 * p.K) * (double)others / 256;
+  return tiles < (p.H % 4 == 0 && others > 256 ? 1.1 * four : four);
 }
 
 hipError_t layer_token(const LayerTokenArgs& p, hipStream_t s) {

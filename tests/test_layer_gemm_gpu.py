@@ -187,10 +187,11 @@ def test_weight_gradients_over_splits_against_float64(M, products, splits):
 
 
 # Rows of tokens and pairs of heads that end inside a tile, an odd number of heads, shared kv heads and a remainder of the steps of 64 columns, where the
-# tiles are taken (the first five), and sizes past 512 (head, 16 tokens) pairs at which the other kernel with four token tiles per wavefront is.
+# tiles are taken (the first seven; the last two of them have one step of 64 columns), and sizes past 512 (head, 16 tokens) pairs at which the other kernel with four token tiles per wavefront is.
 # The last case's rows of tokens lie so far apart that 64 of them reach past the tiles' 32-bit offsets: it stays with the other kernel.
 @pytest.mark.parametrize("B,H,Hkv,K,ldx", [(700, 37, 37, 592, 592), (4090, 8, 2, 128, 128), (700, 33, 11, 528, 552), (700, 32, 32, 520, 520),
-                                           (16333, 3, 3, 1032, 1032), (1030, 37, 37, 592, 592), (333, 33, 11, 528, 528), (2049, 8, 2, 128, 128), (200, 48, 12, 768, 768),
+                                           (16333, 3, 3, 1032, 1032), (16380, 2, 1, 32, 32),
+                                           (8190, 3, 3, 48, 56), (1030, 37, 37, 592, 592), (333, 33, 11, 528, 528), (2049, 8, 2, 128, 128), (200, 48, 12, 768, 768),
                                            (5000, 2, 1, 96, 96), (20000, 1, 1, 16, 16), (80, 128, 128, 128, 1 << 24)])
 def test_token_tiles_against_float64(B, H, Hkv, K, ldx):
     from spear_amd import _btp
@@ -241,9 +242,10 @@ def test_token_tiles_against_float64(B, H, Hkv, K, ldx):
     assert torch.equal(state[3], pos)
 
 
-# Sizes of the tiles (the first six; quarters of K that end inside a step of 64 columns, of one instruction, of one step, and no columns in the last quarter)
+# Sizes of the tiles (the first eight; quarters of K that end inside a step of 64 columns, of one instruction, of one step, and no columns in the last quarter)
 # and of four token tiles per wavefront.
-@pytest.mark.parametrize("B,H,Hkv,K", [(1024, 32, 32, 512), (700, 37, 37, 592), (200, 64, 16, 1024), (4090, 8, 2, 128), (8001, 4, 4, 64), (3200, 10, 10, 160),
+@pytest.mark.parametrize("B,H,Hkv,K", [(1024, 32, 32, 512), (700, 37, 37, 592), (200, 64, 16, 1024), (4090, 8, 2, 128), (8001, 4, 4, 64), (3200, 10, 10, 160), (16380, 2, 1, 32),
+                                       (8190, 3, 3, 48),
                                        (10007, 1, 1, 16), (5003, 3, 1, 48), (3001, 5, 5, 80)])
 def test_a_token_is_the_same_whatever_number_comes_with_it(B, H, Hkv, K):
     """The tiles add up a token's products as the kernel for few tokens does: the state, which is kept in fp32, and the result are equal."""
