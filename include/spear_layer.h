@@ -72,6 +72,8 @@ int spear_layer_wgrad_to(int n, const void* const* dy, const int* ld_dy, const i
 
 /* The number of splits for one of these products that the library's model of it expects to be fastest. */
 int spear_layer_wgrad_splits(long long M, int N, int K);
+/* The same of `atleast` splits and more, for parts that are sums over fewer tokens. */
+int spear_layer_wgrad_splits_from(long long M, int N, int K, int atleast);
 
 /* The parts added up and rounded to `dtype` (16-bit), dw[i] [N[i], K[i]] dense, and m (0 .. 3) column sums of dense fp32 arrays as
  * spear_layer_sums makes them, in one launch. dw[i] 8-byte aligned. */

@@ -64,7 +64,7 @@ int check_common(const char* who, int B, int H, int L, int k, int in_dtype, int 
 
 extern "C" {
 
-int spear_btp_abi_version(void) { return 28; }
+int spear_btp_abi_version(void) { return 29; }
 
 const char* spear_btp_last_error(void) { return g_error; }
 
@@ -370,7 +370,11 @@ int spear_layer_wgrad_to(int n, const void* const* dy, const int* ld_dy, const i
   return 0;
 }
 
-int spear_layer_wgrad_splits(long long M, int N, int K) { return M > 0 && N > 0 && K > 0 ? spear_btp::layer_wgrad_splits((long)M, N, K) : 1; }
+int spear_layer_wgrad_splits_from(long long M, int N, int K, int atleast) {
+  return M > 0 && N > 0 && K > 0 ? spear_btp::layer_wgrad_splits((long)M, N, K, atleast) : 1;
+}
+
+int spear_layer_wgrad_splits(long long M, int N, int K) { return spear_layer_wgrad_splits_from(M, N, K, 1); }
 
 int spear_layer_wgrad_sums(int n, const float* parts, const int* N, const int* K, const int* splits, void* const* dw, int m,
                            const float* const* in, void* const* out, const long long* rows, const long long* cols, int dtype, void* stream) {

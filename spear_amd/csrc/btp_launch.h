@@ -175,7 +175,7 @@ struct LayerWgradArgs {
   float* parts;
 };
 hipError_t layer_wgrad(const LayerWgradArgs& p, hipStream_t s);
-int layer_wgrad_splits(long M, int N, int K);  // the fastest number of splits as modelled
+int layer_wgrad_splits(long M, int N, int K, int atleast);  // the fastest number of splits as modelled, from `atleast` on
 
 // in [rows, cols] (dense, cols a multiple of 8) as out[c * ld + r], zeros for r = rows .. width - 1 (width and ld multiples of 8; 16-byte
 // aligned), and zeros into the columns used .. ld of packed [M, ld] as layer_stack leaves them (none if used == ld).

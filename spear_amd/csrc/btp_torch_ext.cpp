@@ -502,8 +502,10 @@ at::Tensor weight_grad(const at::Tensor& dy, const at::Tensor& x, int64_t s, std
 // gradients' in another.
 struct WeightGrads {
   std::vector<at::Tensor> dy, x, dw;  // dy [M, N or more], x [M, K], dw [N, K]
+  std::vector<int> slices;            // of the tokens, that the library's product would have: at least as many splits
 
-  void add(const at::Tensor& grad, const at::Tensor& operand, int64_t columns) {
+  void add(const at::Tensor& grad, const at::Tensor& operand, int64_t columns, int64_t least) {
+    slices.push_back((int)least);
     dy.push_back(grad);
     x.push_back(operand);
     dw.push_back(at::empty({columns, operand.size(1)}, operand.options()));
@@ -522,7 +524,7 @@ struct WeightGrads {
       ld[i] = (int)dy[i].size(1);
       N[i] = (int)dw[i].size(0);
       K[i] = (int)dw[i].size(1);
-      splits[i] = spear_layer_wgrad_splits(M, N[i], K[i]);
+      splits[i] = spear_layer_wgrad_splits_from(M, N[i], K[i], slices[i]);
       whole[i] = splits[i] == 1 && K[i] < 1 << 21 ? dw[i].data_ptr() : nullptr;
       if (whole[i] != nullptr) continue;
       blocks += (int64_t)((N[i] + 255) / 256) * ((K[i] + 255) / 256) * splits[i];
@@ -628,7 +630,7 @@ struct LayerNode : public torch::autograd::Function<LayerNode> {
     WeightGrads grads;
     if (ctx->needs_input_grad(8)) {
       if (own_weights && (reinterpret_cast<uintptr_t>(dy.data_ptr()) & 15u) == 0) {
-        grads.add(dy, mixed2, K);
+        grads.add(dy, mixed2, K, ctx->saved_data["slices_out"].toInt());
         out[8] = grads.dw[0];
       } else {
         out[8] = weight_grad(dy, mixed2, ctx->saved_data["slices_out"].toInt(), parts, sums);
@@ -684,7 +686,7 @@ struct LayerNode : public torch::autograd::Function<LayerNode> {
       if (weights) {
         at::Tensor dw;
         if (own_weights) {
-          grads.add(d2, x2, used);
+          grads.add(d2, x2, used, ctx->saved_data["slices_in"].toInt());
           dw = grads.dw.back();
         } else {
           dw = weight_grad(d2, x2, ctx->saved_data["slices_in"].toInt(), parts, sums);
@@ -757,7 +759,7 @@ struct LayerNode : public torch::autograd::Function<LayerNode> {
   }
 };
 
-// y = layer(x) for x [B, L, dim]; round_products: gates and products of the mixing stage in 16 bits, as in tensors of their own; slices: into how many slices of tokens the weight gradients' products are cut.
+// y = layer(x) for x [B, L, dim]; round_products: gates and products of the mixing stage in 16 bits, as in tensors of their own; slices: into how many slices of tokens the weight gradients' products are cut at least.
 at::Tensor layer(const at::Tensor& x, const at::Tensor& w_a, const at::Tensor& b_a, const at::Tensor& w_b, const at::Tensor& b_b,
                  const at::Tensor& w_c, const at::Tensor& b_c, const at::Tensor& w_v, const at::Tensor& w_out, int64_t heads,
                  int64_t kv_heads, int64_t slices_in, int64_t slices_out, bool round_products) {

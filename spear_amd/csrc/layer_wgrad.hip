@@ -14,6 +14,9 @@
 //   - The tiles of one split are neighbours in the order of units, and an XCD takes a run of them: its workgroups go through the same
 //     tokens at one time, so each is fetched about once for all tiles (720 MB from memory for 537 MB of operands and 1.8 GB of requests
 //     at 131072 tokens, [1568, 512]).
+//   - A split's sum is one fp32 chain over its tokens. The layer's backward asks for at least as many splits as the library's slices had, for chains
+//     no longer than theirs (the same number of splits gives the library's bits): of [1568, 512] at 131072 tokens 4.6e-4 of the results are not the
+//     nearest 16-bit value with 36 splits, 4.8e-4 with the library's 32 slices, 6.3e-4 with the 18 that are the fastest (250 / 264 / 231 us).
 //   - Steps of 32 tokens, one phase each: five stages of 16 KiB for either operand, asked for four steps ahead.
 //   - A unit's sums are stored as they lie in the accumulators, 1 KiB per store; only layer_sums looks at their order. A product of one
 //     split (few tokens of a wide layer) is rounded and stored as it is: no fp32 array of its size is written and read (both of a layer at
@@ -27,6 +30,8 @@
 // step computed anew per request the same ring took 334 us at [1568, 512].
 #include <hip/hip_runtime.h>
 #include <stdint.h>
+
+#include <algorithm>
 
 #include "btp_device.h"
 #include "btp_launch.h"
@@ -270,14 +275,15 @@ hipError_t layer_wgrad(const LayerWgradArgs& p, hipStream_t s) {
   return hipGetLastError();
 }
 
-int layer_wgrad_splits(long M, int N, int K) {
+int layer_wgrad_splits(long M, int N, int K, int atleast) {
   const long steps = (M + kTokens - 1) / kTokens, tiles = (long)((N + kSide - 1) / kSide) * ((K + kSide - 1) / kSide);
-  int best = 1;
+  const int from = (int)std::max(1l, std::min({(long)atleast, 256l, steps}));
+  int best = from;
   double least = 0.0;
-  for (int n = 1; n <= 256 && (n == 1 || steps >= 16l * n); ++n) {
+  for (int n = from; n <= 256 && (n == from || steps >= 16l * n); ++n) {
     // rounds of the chip, a step 0.75 us and 4 us to start and store; the sums 256 KiB per unit written and read at 4.5 TB/s
     const double us = (double)((tiles * n + 255) / 256) * (0.75 * (double)((steps + n - 1) / n) + 4.0) + 0.117 * (double)(tiles * n);
-    if (n == 1 || us < least) {
+    if (n == from || us < least) {
       least = us;
       best = n;
     }

@@ -378,3 +378,30 @@ def test_backward_of_few_tokens_of_a_wide_layer_needs_little_room():
     torch.cuda.synchronize()
     weights = sum(p.numel() * p.element_size() for p in layer.parameters())
     assert torch.cuda.max_memory_allocated() - torch.cuda.memory_allocated() < 1.25 * weights
+
+
+@pytest.mark.parametrize("M,N,K", [(65536, 1568, 512), (16384, 6272, 2048)])
+def test_weight_gradients_lose_no_precision_against_the_library_in_slices(M, N, K):
+    """The layer's backward takes splits of no more tokens than the library's slices: as many of the results are the nearest 16-bit value to the sum in
+    64 bits, up to five standard deviations of that number."""
+    import ctypes
+
+    from spear_amd import _btp
+    from spear_amd.nn.phalanx.projections import slice_count
+
+    lib, slices = _btp.load_library(), slice_count(M, N, K)
+    splits = lib.spear_layer_wgrad_splits_from(ctypes.c_longlong(M), N, K, slices)
+    assert slices > 1 and splits >= slices
+    g = torch.Generator(device=DEV).manual_seed(M)
+    dy, x = (torch.randn(M, n, generator=g, device=DEV).bfloat16() for n in (N, K))
+    parts, dw, sliced = torch.empty(-(-N // 256) * -(-K // 256) * splits * 65536, device=DEV), torch.empty(N, K, device=DEV).bfloat16(), torch.empty(N, K, device=DEV).bfloat16()
+    one, of = lambda v: (ctypes.c_int * 1)(v), lambda t: (ctypes.c_void_p * 1)(t.data_ptr())
+    stream = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    print(f"weight gradients M={M} [{N}, {K}] splits={splits} slices={slices}", flush=True)
+    assert lib.spear_layer_wgrad(1, of(dy), one(N), one(N), one(N), of(x), one(K), one(splits), ctypes.c_longlong(M), ctypes.c_void_p(parts.data_ptr()), stream) == 0
+    assert lib.spear_layer_wgrad_sums(1, ctypes.c_void_p(parts.data_ptr()), one(N), one(K), one(splits), of(dw), 0, None, None, None, None, _btp._BF16, stream) == 0
+    of_slices = torch.bmm(dy.view(slices, M // slices, N).transpose(1, 2).contiguous(), x.view(slices, M // slices, K), out_dtype=torch.float32)
+    _btp.load_extension().layer_sums([of_slices.view(slices, N * K)], [sliced])
+    want = sum(dy[i:i + 8192].double().t() @ x[i:i + 8192].double() for i in range(0, M, 8192)).bfloat16()
+    off, off_sliced = ((t != want).sum().item() for t in (dw, sliced))
+    assert off <= off_sliced + 5 * off_sliced**0.5
