@@ -821,10 +821,15 @@ std::vector<at::Tensor> layer_prefill(const at::Tensor& x, const at::Tensor& w_a
 at::Tensor layer_step(const at::Tensor& x, const at::Tensor& w_a, const at::Tensor& b_a, const at::Tensor& w_b, const at::Tensor& b_b,
                       const at::Tensor& w_c, const at::Tensor& b_c, const at::Tensor& w_v, const at::Tensor& w_out, at::Tensor h,
                       at::Tensor r, at::Tensor c_prev, at::Tensor pos, int64_t block_len, int64_t heads, int64_t kv_heads) {
-  // the positions move on with the output projection where that is a kernel of this library: a launch less, which makes up for what the
-  // product takes longer than the library's (see own_products)
+  // The positions move on with the output projection where that is a kernel of this library: a launch (4.4 us) less, which makes up for what the
+  // product takes longer than the library's (see own_products). Not for some tokens of a wide layer: [B, dim] x [dim, dim], us, here / the library's
+  // without that launch: dim 3072 B=16 8.2 / 7.4, 64 14.0 / 10.5, 96 19.8 / 13.8; 4096 16 10.2 / 12.1, 32 14.0 / 10.1, 48 17.6 / 11.5, 128 25.8 / 19.6; 6144 16
+  // 19.5 / 14.5, 17 21.2 / 15.3, 48 36 / 19.6; 8192 8 23.1 / 22.0, 16 33.6 / 28.0 (in a step). At dim 2048 it is 18.8 / 12.1 for 512 tokens, but the host's time bounds
+  // such a step as a call (31 us, 43 with the library's product).
   const auto in = [&](bool advance) { return layer_token(x, w_a, b_a, w_b, b_b, w_c, b_c, w_v, h, r, c_prev, pos, block_len, heads, kv_heads, advance); };
-  if (own_products(x.size(0), {w_out}, w_out.size(1)))
+  const int64_t B = x.size(0), K = w_out.size(1);
+  const bool wide = K >= 3072 && B >= 16 && B * w_out.size(0) * K >= 500000000;
+  if (!wide && own_products(B, {w_out}, K))
     return linears(in(false), {w_out}, {at::Tensor()}, pos.data_ptr<int>(), block_len)[0];
   return at::linear(in(true), w_out);
 }

@@ -347,9 +347,11 @@ def _steps_equal_the_modules(B, dim):
         assert one.pos.tolist() == two.pos.tolist() == [(b + t + 1) % 16 for b in range(B)]
 
 
-def test_step_with_the_output_projection_of_the_library():
-    """More narrow sequences than the output projection's kernel takes: the token kernel moves the block positions on itself, also past a block's end."""
-    _steps_equal_the_modules(73300, 64)
+@pytest.mark.parametrize("B,dim", [(73300, 64), (54, 3072)])
+def test_step_with_the_output_projection_of_the_library(B, dim):
+    """More narrow sequences than the output projection's kernel takes, and some of a wide layer, whose output projection the library has in less time: the
+    token kernel moves the block positions on itself, also past a block's end."""
+    _steps_equal_the_modules(B, dim)
 
 
 @pytest.mark.parametrize("B,dim", [(17, 528), (1030, 784)])
