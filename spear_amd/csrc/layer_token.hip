@@ -242,6 +242,9 @@ void launch(const LayerTokenArgs& p, hipStream_t s) {
 static bool tiles_win(const LayerTokenArgs& p) {
   // the tile kernel's offsets are 32 bits: the largest matrix and 64 rows of tokens below 1 GiB
   if (32l * p.H * p.K >= 1l << 30 || 2l * kTokenRows * p.ldx >= 1l << 30) return false;
+  // Up to 64 tokens either kernel reads each weight once, the tiles with half as many workgroups: 256 heads at K = 4096, four token tiles / the tile
+  // kernel, B=33 25.9 / 31.3, B=40 27.2 / 31.2, B=48 28.6 / 28.4, B=64 31.7 / 31.8; with more heads than compute units the former has a second round.
+  if (p.B <= kTokenRows && p.H <= 256) return false;
   const long row_tiles = (p.B + kTokenRows - 1) / kTokenRows, rounds = ((p.H + 1) / 2 * row_tiles + 255) / 256;
   const double tiles = 1.0 + (double)rounds * (4.2 + 0.36 * ((p.K + kRowsStep - 1) / kRowsStep));
   const long others = p.H * row_tiles;

@@ -272,6 +272,22 @@ def test_a_token_is_the_same_whatever_number_comes_with_it(B, H, Hkv, K):
             assert torch.equal(got[first:first + 16], want)
 
 
+@pytest.mark.parametrize("B,H,tiles", [(33, 256, False), (64, 256, False), (65, 256, True), (33, 272, True)])
+def test_up_to_64_tokens_of_256_heads_stay_with_the_kernel_without_tiles(B, H, tiles):
+    from spear_amd import _btp
+
+    K, g = 4096, torch.Generator(device=DEV).manual_seed(B)
+    normal = lambda *shape: torch.randn(*shape, generator=g, device=DEV)
+    x, weights = normal(B, K).bfloat16(), [normal(n, K).bfloat16() for n in (H, 16 * H, 16 * H, 16 * H)]
+    b_a, b_b, b_c = (normal(n).bfloat16() for n in (H, 16 * H, 16 * H))
+    state = [normal(B, H, 16), torch.rand(B, H, generator=g, device=DEV), normal(B, H, 16), torch.zeros(B, device=DEV, dtype=torch.int32)]
+    with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CUDA]) as profile:
+        _btp.load_extension().layer_token(x, weights[0], b_a, weights[1], b_b, weights[2], b_c, weights[3], *state, 16, H, H, False)
+        torch.cuda.synchronize()
+    kernel, = [e.name for e in profile.events() if e.device_type == torch.autograd.DeviceType.CUDA]
+    assert ("layer_token_tile_kernel" in kernel) == tiles, kernel
+
+
 # Sizes that 128 x 128 tiles take up to which K is added up in quarters: quarters that end inside a step of 64 columns, and of one instruction.
 @pytest.mark.parametrize("M,K,columns", [(1024, 512, (512, 512, 512, 32)), (1003, 592, (592, 592, 257, 37)), (700, 1040, (1040, 130, 129, 24)), (1500, 72, (1024, 130))])
 def test_a_row_is_the_same_whatever_number_comes_with_it(M, K, columns):
