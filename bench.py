@@ -896,7 +896,7 @@ def main() -> int:
             """phalanx_mix(a, b, c, v) + backward on [bs, L, features] tensors: eager through the autograd node compiled
             into the binding, the two custom ops on preallocated outputs, and a HIP-graph replay of those two ops."""
             from spear_amd import phalanx_mix
-            import spear_amd.ops.btp.fused  # noqa: F401  (registers the custom ops)
+            from spear_amd.ops.btp.fused import _PhalanxMix  # registers the custom ops, too
 
             F = H * 16
             gq = torch.Generator(device=dev).manual_seed(seed + 23)
@@ -911,7 +911,7 @@ def main() -> int:
 
             def eager_python_node():  # the torch.autograd.Function over the custom ops (what torch.compile traces)
                 leaves = [t.detach().requires_grad_(True) for t in (a, b, c, v)]
-                spear_amd.ops.btp.fused._PhalanxMix.apply(*leaves, H, H).backward(dout)
+                _PhalanxMix.apply(*leaves, H, H).backward(dout)
 
             def ops_only():
                 torch.ops.spear_btp.mix_forward(a, b, c, v, out, H, H)
