@@ -16,16 +16,17 @@
 //     at 131072 tokens, [1568, 512]).
 //   - A split's sum is one fp32 chain over its tokens. The layer's backward asks for at least as many splits as the library's slices had, for chains
 //     no longer than theirs (the same number of splits gives the library's bits): of [1568, 512] at 131072 tokens 4.6e-4 of the results are not the
-//     nearest 16-bit value with 36 splits, 4.8e-4 with the library's 32 slices, 6.3e-4 with the 18 that are the fastest (250 / 264 / 231 us).
+//     nearest 16-bit value with 36 splits, 4.8e-4 with the library's 32 slices, 6.3e-4 with the 18 of the model alone, which
+//     take as long (239 us either; [3200, 2048] in 12 in place of 7 1525 / 1492).
 //   - Steps of 32 tokens, one phase each: five stages of 16 KiB for either operand, asked for four steps ahead.
 //   - A unit's sums are stored as they lie in the accumulators, 1 KiB per store; only layer_sums looks at their order. A product of one
 //     split (few tokens of a wide layer) is rounded and stored as it is: no fp32 array of its size is written and read (both of a layer at
 //     512 tokens, dim 4096: a step of 487 us in place of 524).
 //
-// Measured at 131072 tokens, us with the sums, here / the library's batched product in slices and its sums: [1568, 512] 238 / 281, [512, 512]
-// 85 / 93, both 308 / 370, [3136, 1024] 797 / 1064, [3200, 2048] 1536 / 1783, [2048, 2048] 876 / 966, [784, 256] 83 / 90; 65536 tokens [1813, 592]
-// 175 / 218; 16384 tokens [1568, 512] 49 / 57, [512, 512] 31 / 24; one split: 512 tokens [1568, 512] 23 / 9, [6272, 2048] 27 / 24, 4096 tokens
-// [6400, 4096] 209 / 217. The matrix units are busy 0.55 (K=512, at 2.7 TB/s from memory beside the
+// Measured at 131072 tokens, us with the sums, here / the library's batched product in slices and its sums: [1568, 512] 239 / 283, [512, 512]
+// 81 / 90, [3136, 1024] 780 / 1041, [3200, 2048] 1525 / 1718, [2048, 2048] 854 / 935, [784, 256] 78 / 88; 65536 tokens [1813, 592] 181 / 208;
+// 16384 tokens [1568, 512] 44 / 53, [512, 512] 29 / 26; one split: 512 tokens [1568, 512] 22 / 9, [6272, 2048] 28 / 24, 4096 tokens [6400, 4096]
+// 213 / 240. The matrix units are busy 0.55 (K=512, at 2.7 TB/s from memory beside the
 // parts) to 0.59 of the time and the chip's clock falls to 2.0 GHz: power and the reads of far tokens bound it. With the addresses of a
 // step computed anew per request the same ring took 334 us at [1568, 512].
 #include <hip/hip_runtime.h>

@@ -246,8 +246,8 @@ def layer_call(x: torch.Tensor, dtype: torch.dtype, proj_a, proj_b, proj_c, proj
     binding (``LayerNode`` in ``btp_torch_ext.cpp``; ``round_products``: gates and gated inputs rounded to 16 bits as the tensors
     that :func:`btp` takes), or None where the call is for the modules and the Python nodes of this file: what
     ``plain_operands`` leaves to them, lengths and sizes that the mixing kernels refuse, and a row of gradients of 2 GiB.
-    Forward + backward, us, modules and Python nodes / compiled: B=8 L=128 dim=512 562 / 174, B=1024 1330 / 1151,
-    B=64 L=2048 dim=2048 8152 / 7395."""
+    Forward + backward, us, modules and Python nodes / compiled: B=8 L=128 dim=512 562 / 180, B=1024 1330 / 1162,
+    B=64 L=2048 dim=2048 8152 / 7282."""
     if not x.is_cuda or x.dim() != 3 or x.numel() == 0 or x.shape[1] % 16 != 0:
         return None
     ld, K = packed_columns(heads, kv_heads)[1], x.shape[2]

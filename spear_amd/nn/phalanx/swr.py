@@ -229,7 +229,7 @@ class Phalanx(nn.Module):
         composition of modules below.
 
         For ``"default"``, whose gates and gated inputs keep the 16 bits in which :func:`btp` takes them, this takes the place of
-        the stand-alone recurrence between about twenty elementwise and transposing passes. Forward + backward, us, stand-alone / one node: B=1024 L=128 dim=512 4692 / 1151, B=8 822 / 174; no size was
+        the stand-alone recurrence between about twenty elementwise and transposing passes. Forward + backward, us, stand-alone / one node: B=1024 L=128 dim=512 4692 / 1162, B=8 822 / 180; no size was
         found where the stand-alone kernels win. They keep every call that the fused ones would answer in another way:
         k = 1, other types than bf16 throughout, autocast, anything that traces or transforms the call, hooked or replaced
         projections (``plain_operands``), the matrix-core and checkpoint-store switches, a replaced recurrence, class or method, empty
